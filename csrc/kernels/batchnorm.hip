@@ -562,7 +562,8 @@ dim3 stream_grid(long R, int C) {
 }
 
 // One launch a direction (1568 rows of 512: 10.0 + 8.0 us) instead of three
-// (14.0 + 15.4), as long as a block's threads can keep their rows.
+// (14.0 + 15.4), as long as a block's threads can keep their rows.  At
+// least one row: the kernels read the last one for lanes behind it.
 bool few_rows(long R) { return R <= FEW; }
 
 }  // namespace
@@ -595,6 +596,12 @@ std::vector<torch::Tensor> bn_fwd(torch::Tensor x,
       mask = torch::empty({R, C / 8}, fopt.dtype(torch::kUInt8));
       mp = mask.data_ptr<unsigned char>();
     }
+  }
+  if (R == 0) {                        // as torch: the statistics stay
+    mean.zero_();
+    rstd.zero_();
+    if (mask.defined()) return {y, mean, rstd, mask};
+    return {y, mean, rstd};
   }
   const StatsOut o{mean.data_ptr<float>(), rstd.data_ptr<float>(),
                    running_mean ? running_mean->data_ptr<float>() : nullptr,
@@ -662,6 +669,12 @@ std::vector<torch::Tensor> bn_bwd(torch::Tensor dy, torch::Tensor x,
   if (has_res) {
     dres = torch::empty_like(x);
     drp = (short*)dres.data_ptr();
+  }
+  if (R == 0) {
+    dw.zero_();
+    db.zero_();
+    if (has_res) return {dx, dres, dw, db};
+    return {dx, dw, db};
   }
   const unsigned char* mp = mask.has_value() ? mask->data_ptr<unsigned char>() : nullptr;
   const short *dp = (const short*)dyc.data_ptr(), *xp = (const short*)x.data_ptr();

@@ -78,3 +78,26 @@ def test_matches_float64(N, C, H, W, relu, use_res):
                 bound = bound + shift
             ok = (g - e).abs() <= bound
             assert (ok | near).all(), (name, (g - e).abs().max())
+
+
+@pytest.mark.parametrize("shape", [(0, 16, 7, 7), (3, 16, 0, 7)])
+@pytest.mark.parametrize("relu", [True, False])
+@pytest.mark.parametrize("use_res", [True, False])
+def test_no_rows(shape, relu, use_res):
+    """An empty batch, as the last one of an epoch can be: nothing is read, and
+    the running statistics stay as on the CPU."""
+    from scaffold import ops
+
+    def image():
+        return torch.randn(shape, device="cuda").bfloat16().requires_grad_()
+
+    x, res = image(), image() if use_res else None
+    w, b = (torch.rand(16, device="cuda").requires_grad_() for _ in range(2))
+    rm, rv = torch.randn(16, device="cuda"), torch.rand(16, device="cuda")
+    kept = rm.clone(), rv.clone()
+    y = ops.batch_norm_act(x, res, w, b, rm, rv, 0.1, 1e-5, relu, True)
+    assert y.shape == shape
+    ins = [x, w, b] + ([res] if use_res else [])
+    for t, g in zip(ins, torch.autograd.grad(y, ins, torch.ones_like(y))):
+        assert g.shape == t.shape and not g.any()
+    assert torch.equal(rm, kept[0]) and torch.equal(rv, kept[1])
