@@ -658,7 +658,11 @@ std::vector<torch::Tensor> bn_bwd(torch::Tensor dy, torch::Tensor x,
               (!mask.has_value() ||
                (mask->scalar_type() == torch::kUInt8 && mask->is_contiguous() &&
                 mask->numel() == R * (C / 8))), "bn_bwd: mask");
-  auto dyc = dy.stride(1) == 1 ? dy : dy.contiguous(at::MemoryFormat::ChannelsLast);
+  // as x lies: a slice of the channels and an expanded gradient have
+  // stride(1) == 1 too
+  TORCH_CHECK(dy.sizes() == x.sizes() && dy.scalar_type() == torch::kBFloat16,
+              "bn_bwd: dy");
+  auto dyc = dy.contiguous(at::MemoryFormat::ChannelsLast);
   auto fopt = torch::TensorOptions().dtype(torch::kFloat32).device(x.device());
   auto dw = torch::empty({C}, fopt);
   auto db = torch::empty({C}, fopt);

@@ -101,3 +101,44 @@ def test_no_rows(shape, relu, use_res):
     for t, g in zip(ins, torch.autograd.grad(y, ins, torch.ones_like(y))):
         assert g.shape == t.shape and not g.any()
     assert torch.equal(rm, kept[0]) and torch.equal(rv, kept[1])
+
+
+@pytest.mark.parametrize("shape", [(2, 16, 4, 4), (2, 16, 33, 34)])
+@pytest.mark.parametrize("use_res", [True, False])
+def test_gradients_of_any_layout(shape, use_res):
+    """What autograd hands back through cat (a slice of the channels), sum over
+    the image (an expanded row) and slices of an image, all of stride(1) == 1,
+    counts as the same numbers laid out like x."""
+    from scaffold import ops
+
+    torch.manual_seed(4)
+    N, C, H, W = shape
+
+    def image():
+        t = torch.randn(N, H, W, C, device="cuda").bfloat16()
+        return t.permute(0, 3, 1, 2).requires_grad_()
+
+    x, res = image(), image() if use_res else None
+    w, b = (torch.rand(C, device="cuda").requires_grad_() for _ in range(2))
+    ins = [x, w, b] + ([res] if use_res else [])
+    y = ops.batch_norm_act(x, res, w, b, torch.zeros(C, device="cuda"),
+                           torch.ones(C, device="cuda"), 0.1, 1e-5, True, True)
+    wide = torch.randn(N, H, W + 3, 3 * C, device="cuda").bfloat16()
+    wide = wide.permute(0, 3, 1, 2)
+    for dy in (wide[:, C:2 * C, :, 1:W + 1], wide[:, :C, :, :W],
+               wide[:, :C, :1, :1].expand(shape), wide[:1, :C, :1, :1].expand(shape)):
+        dense = dy.clone(memory_format=torch.channels_last)
+        assert dy.stride(1) == 1 and dy.stride() != dense.stride()
+        got = torch.autograd.grad(y, ins, dy, retain_graph=True)
+        want = torch.autograd.grad(y, ins, dense, retain_graph=True)
+        for g, e in zip(got, want):
+            assert torch.equal(g, e)
+    z = torch.cat([y, y.detach()], 1)
+    assert torch.equal(torch.autograd.grad(z, x, wide[:, :2 * C, :, :W],
+                                           retain_graph=True)[0],
+                       torch.autograd.grad(y, x, wide[:, :C, :, :W],
+                                           retain_graph=True)[0])
+    rows = torch.randn(N, C, device="cuda").bfloat16()
+    assert torch.equal(torch.autograd.grad(y.sum((2, 3)), x, rows, retain_graph=True)[0],
+                       torch.autograd.grad(y, x, rows.view(N, C, 1, 1).repeat(
+                           1, 1, H, W))[0])
