@@ -528,9 +528,17 @@ bn_small_bwd_kernel(const short* __restrict__ dy, const short* __restrict__ x,
 }
 
 void check_nhwc(const torch::Tensor& t, const char* nm) {
-  TORCH_CHECK(t.dim() == 4 && t.stride(1) == 1, nm,
-              " must be 4-D channels_last (stride(1)==1)");
+  TORCH_CHECK(t.is_cuda() && t.dim() == 4 &&
+              t.is_contiguous(at::MemoryFormat::ChannelsLast), nm,
+              " must be 4-D channels_last on the GPU");
   TORCH_CHECK(t.scalar_type() == torch::kBFloat16, nm, " must be bf16");
+}
+
+// a number for each channel
+void check_channels(const torch::Tensor& t, int C, const char* nm) {
+  TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kFloat32 &&
+              t.is_contiguous() && t.numel() == C, nm,
+              " must be one float32 per channel, contiguous on the GPU");
 }
 
 dim3 row_grid(long R, int C, int ns) {
@@ -579,7 +587,15 @@ std::vector<torch::Tensor> bn_fwd(torch::Tensor x,
   CHECK_CUDA(x);
   check_nhwc(x, "x");
   const int C = (int)x.size(1);
-  TORCH_CHECK(C % 8 == 0, "bn_fwd: C % 8 != 0");
+  TORCH_CHECK(C > 0 && C % 8 == 0, "bn_fwd: C % 8 != 0");
+  check_channels(weight, C, "weight");
+  check_channels(bias, C, "bias");
+  TORCH_CHECK(running_mean.has_value() == running_var.has_value(),
+              "bn_fwd: one running statistic without the other");
+  if (running_mean.has_value()) {
+    check_channels(*running_mean, C, "running_mean");
+    check_channels(*running_var, C, "running_var");
+  }
   const long R = x.numel() / C;
   auto fopt = torch::TensorOptions().dtype(torch::kFloat32).device(x.device());
   auto mean = torch::empty({C}, fopt);
@@ -591,6 +607,7 @@ std::vector<torch::Tensor> bn_fwd(torch::Tensor x,
   unsigned char* mp = nullptr;
   if (res.has_value()) {
     check_nhwc(res.value(), "res");
+    TORCH_CHECK(res->sizes() == x.sizes(), "bn_fwd: res must be as large as x");
     rp = (const short*)res->data_ptr();
     if (relu) {
       mask = torch::empty({R, C / 8}, fopt.dtype(torch::kUInt8));
@@ -653,6 +670,11 @@ std::vector<torch::Tensor> bn_bwd(torch::Tensor dy, torch::Tensor x,
   CHECK_CUDA(dy);
   check_nhwc(x, "x");
   const int C = (int)x.size(1);
+  TORCH_CHECK(C > 0 && C % 8 == 0, "bn_bwd: C % 8 != 0");
+  check_channels(weight, C, "weight");
+  check_channels(bias, C, "bias");
+  check_channels(mean, C, "mean");
+  check_channels(rstd, C, "rstd");
   const long R = x.numel() / C;
   TORCH_CHECK(mask.has_value() == (relu && has_res) &&
               (!mask.has_value() ||

@@ -142,3 +142,40 @@ def test_gradients_of_any_layout(shape, use_res):
     assert torch.equal(torch.autograd.grad(y.sum((2, 3)), x, rows, retain_graph=True)[0],
                        torch.autograd.grad(y, x, rows.view(N, C, 1, 1).repeat(
                            1, 1, H, W))[0])
+
+
+def test_refuses_operands_that_do_not_fit():
+    """Sizes that the kernels would read past: refused on the host."""
+    from scaffold import ops
+
+    C = 16
+    x = torch.randn(2, C, 5, 5, device="cuda").bfloat16()
+    vec = {n: torch.ones(C, device="cuda") for n in ("w", "b", "m", "v")}
+
+    def call(x=x, res=None, **kw):
+        p = {**vec, **kw}
+        return ops.batch_norm_act(x, res, p["w"], p["b"], p["m"], p["v"], 0.1,
+                                  1e-5, True, True)
+
+    call()
+    for n in "wbmv":
+        for bad in (torch.ones(C - 8, device="cuda"), torch.ones(C),
+                    torch.ones(2 * C, device="cuda")[::2]):
+            with pytest.raises(RuntimeError):
+                call(**{n: bad})
+    with pytest.raises(RuntimeError):
+        call(m=None)
+    for bad in (x[:1], x[:, :8], x[..., :4], x.float()):
+        with pytest.raises(RuntimeError):
+            call(res=bad)
+    with pytest.raises(RuntimeError):
+        call(x=x[:, :0], **{n: t[:0] for n, t in vec.items()})
+    ext, nhwc = ops.require_ext(), torch.channels_last
+    x = x.contiguous(memory_format=nhwc)
+    y, mean, rstd = ext.bn_fwd(x, None, vec["w"], vec["b"], None, None, 0.1,
+                               1e-5, True)
+    ext.bn_bwd(y, x, False, None, vec["w"], vec["b"], mean, rstd, True)
+    for dy, xx in ((y[:1], x), (y.float(), x), (y, x.contiguous()),
+                   (y[:, :, 1:], x[:, :, 1:])):
+        with pytest.raises(RuntimeError):
+            ext.bn_bwd(dy, xx, False, None, vec["w"], vec["b"], mean, rstd, True)
