@@ -14,7 +14,7 @@ for N, C, H, W in shapes:
     w = torch.rand(C, device="cuda") + 0.5
     b = torch.randn(C, device="cuda")
     for _ in range(5):
-        y, mean, rstd = m.bn_fwd(x, res, w, b, None, None, 0.1, 1e-5, True)
-        m.bn_bwd(dy, x, res, w, b, mean, rstd, True)
+        y, mean, rstd, mask = m.bn_fwd(x, res, w, b, None, None, 0.1, 1e-5, True)
+        m.bn_bwd(dy, x, True, mask, w, b, mean, rstd, True)
 torch.cuda.synchronize()
 print("done")

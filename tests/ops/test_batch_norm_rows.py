@@ -179,3 +179,11 @@ def test_refuses_operands_that_do_not_fit():
                    (y[:, :, 1:], x[:, :, 1:])):
         with pytest.raises(RuntimeError):
             ext.bn_bwd(dy, xx, False, None, vec["w"], vec["b"], mean, rstd, True)
+
+
+def test_benchmark_runs():
+    """benchmarks/bn_only.py calls the kernels as they are."""
+    import runpy
+    from pathlib import Path
+
+    runpy.run_path(str(Path(__file__).parents[2] / "benchmarks" / "bn_only.py"))
