@@ -34,3 +34,15 @@ inline Strides4 strides_of(const torch::Tensor& t) {
               "expected 4-D tensor with contiguous last dim");
   return {t.stride(0), t.stride(1), t.stride(2)};
 }
+
+// t, or a copy of it, with every row of the last dimension on 16 bytes: what
+// 16-byte loads, and copies into LDS above all, are written for.  Only
+// views at odd places or of odd strides are copied.
+inline torch::Tensor rows16(const torch::Tensor& t) {
+  const long per = 16 / (long)t.element_size(), last = t.dim() - 1;
+  bool ok = (size_t)t.data_ptr() % 16 == 0 &&
+            (t.size(last) == 1 || t.stride(last) == 1);
+  for (long d = 0; d < last; ++d)
+    ok = ok && (t.size(d) == 1 || t.stride(d) % per == 0);
+  return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+}

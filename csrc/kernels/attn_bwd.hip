@@ -286,11 +286,11 @@ std::vector<torch::Tensor> attn_bwd(torch::Tensor dout, torch::Tensor q,
   if (q.scalar_type() == torch::kBFloat16 && (D == 64 || D == 128)) {
     // strided MFMA path; grads produced in (B,S,H,D) physical layout so
     // the upstream view backward (QKV un-transpose) is coalesced
-    auto doc = dout.stride(3) == 1 ? dout : dout.contiguous();
-    auto qc = q.stride(3) == 1 ? q : q.contiguous();
-    auto kc = k.stride(3) == 1 ? k : k.contiguous();
-    auto vc = v.stride(3) == 1 ? v : v.contiguous();
-    auto oc = o.stride(3) == 1 ? o : o.contiguous();
+    auto doc = rows16(dout);
+    auto qc = rows16(q);
+    auto kc = rows16(k);
+    auto vc = rows16(v);
+    auto oc = rows16(o);
     torch::Tensor all, dq, dk, dv;
     if (packed) {
       all = torch::empty({B, S, H + 2l * Hkv, D}, q.options());

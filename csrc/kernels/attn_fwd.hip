@@ -191,9 +191,9 @@ std::vector<torch::Tensor> attn_fwd(torch::Tensor q, torch::Tensor k,
   if (q.scalar_type() == torch::kBFloat16 && (D == 64 || D == 128)) {
     // strided MFMA path: consume permuted views directly; O written in
     // (B,S,H,D) physical layout so the caller's transpose+reshape is free
-    auto qc = q.stride(3) == 1 ? q : q.contiguous();
-    auto kc = k.stride(3) == 1 ? k : k.contiguous();
-    auto vc = v.stride(3) == 1 ? v : v.contiguous();
+    auto qc = rows16(q);
+    auto kc = rows16(k);
+    auto vc = rows16(v);
     auto o = torch::empty({B, S, H, D}, q.options()).permute({0, 2, 1, 3});
     const int mode = attn_fwd_mode();
     const bool use8w = (mode == 8) || (mode == 0 && S >= 256);

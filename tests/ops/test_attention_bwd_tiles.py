@@ -40,3 +40,30 @@ def test_matches_float64(S, D, H, G, causal):
             (dk, fold(T(dS) @ Q), fold(T(eS) @ Q.abs())),
             (dv, fold(T(P) @ dO), fold(T(eP) @ dO.abs()))):
         assert ((got.double() - want).abs() <= err + 2.0 ** -8 * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("S", [64, 300])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("which", ["q", "k", "v", "do", "all"])
+def test_operands_at_odd_places(S, D, which):
+    """Rows of odd stride, and rows that start off 16 bytes, give what the same
+    numbers in dense rows give."""
+    torch.manual_seed(S + D)
+    B, H, G = 2, 4, 2
+    n = {"q": H, "k": G, "v": G, "do": H}
+    dense = {a: torch.randn(B, n[a], S, D, device="cuda").bfloat16() for a in n}
+
+    def run(t):
+        leaves = [t[a].detach().requires_grad_() for a in "qkv"]
+        o = ops.attention(*leaves, True)
+        return o, *torch.autograd.grad(o, leaves, t["do"])
+
+    want = run(dense)
+    for pad, first in ((1, 0), (8, 3), (8, 8)):
+        odd = dict(dense)
+        for a in n if which == "all" else [which]:
+            wide = torch.zeros(B, S, n[a], D + pad, device="cuda").bfloat16()
+            odd[a] = wide[..., first:first + D].transpose(1, 2)
+            odd[a].copy_(dense[a])
+        for g, e in zip(run(odd), want):
+            assert torch.equal(g, e)
