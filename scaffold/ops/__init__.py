@@ -386,7 +386,8 @@ def attention_lse(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 
 def _colsum(dy2: torch.Tensor) -> torch.Tensor:
     m = ext()
-    if m is not None and dy2.is_cuda and dy2.dtype == torch.bfloat16:
+    if (m is not None and dy2.is_cuda and dy2.dtype == torch.bfloat16
+            and not torch.is_grad_enabled()):    # the kernel has no gradient
         return m.colsum(dy2)
     return dy2.sum(0)
 
@@ -515,13 +516,7 @@ class _LinearLib(torch.autograd.Function):
         x2 = x.contiguous().view(-1, x.shape[-1])
         dx = (dy2 @ w).view(x.shape)
         dw = _weight_grad(dy2, x2)
-        db = None
-        if ctx.has_bias:
-            m = ext()
-            if m is not None and dy2.dtype == torch.bfloat16:
-                db = m.colsum(dy2)
-            else:
-                db = dy2.sum(0)
+        db = _colsum(dy2) if ctx.has_bias else None
         return dx, dw, db
 
 
