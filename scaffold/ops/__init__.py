@@ -527,15 +527,22 @@ class _LinearGeluLib(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, b):
         pre = F.linear(x, w, b)
-        ctx.save_for_backward(x, w, pre)
+        ctx.save_for_backward(x, w, b, pre)
         return F.gelu(pre, approximate="tanh")
 
     @staticmethod
     def backward(ctx, dy):
-        x, w, pre = ctx.saved_tensors
+        x, w, b, pre = ctx.saved_tensors
         n = pre.shape[-1]
-        dpre, db = require_ext().gelu_bwd(dy.contiguous().view(-1, n),
-                                          pre.view(-1, n))
+        if torch.is_grad_enabled():
+            # a graph is wanted, through the pre-activation too: torch's own
+            pre = F.linear(x, w, b)
+            dpre = torch.ops.aten.gelu_backward(
+                dy, pre, approximate="tanh").reshape(-1, n)
+            db = dpre.sum(0)
+        else:
+            dpre, db = require_ext().gelu_bwd(dy.contiguous().view(-1, n),
+                                              pre.view(-1, n))
         x2 = x.contiguous().view(-1, x.shape[-1])
         return (dpre @ w).view(x.shape), _weight_grad(dpre, x2), db
 

@@ -44,3 +44,10 @@ def test_linear(n):
 def test_linear_residual(n):
     _check(ops.linear_residual, lambda x, w, b, r: F.linear(x, w, b) + r,
            _operands(n))
+
+
+@pytest.mark.parametrize("n", [100, 200])
+def test_linear_gelu(n):
+    _check(ops.linear_gelu,
+           lambda x, w, b: F.gelu(F.linear(x, w, b), approximate="tanh"),
+           _operands(n)[:3])

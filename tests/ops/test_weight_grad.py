@@ -51,9 +51,11 @@ def test_layers_take_it(T, N, K, own, act, monkeypatch):
     assert len(calls) == own
     if not act:
         _close(dw, dy, x.detach())
-    # a graph of the backward stays with operations that have one
+    # a graph of the backward stays with operations that have one (what such a
+    # graph yields: test_second_derivatives.py): dw is linear in dy
     (dw2,) = torch.autograd.grad(y, w, dy.requires_grad_(), create_graph=True)
-    assert len(calls) == own and dw2.requires_grad
+    (back,) = torch.autograd.grad(dw2, dy, torch.ones_like(dw2))
+    assert len(calls) == own and back.any(0).all()
 
 
 def test_refuses_other_operands():
