@@ -501,23 +501,27 @@ _HAND_GEMM_ALL = False  # flipped by benchmarks once the 8-phase core wins
 class _LinearLib(torch.autograd.Function):
     """Library-GEMM (hipBLASLt) forward with an explicit backward:
     rocBLAS matmuls for dX/dW plus the hand colsum kernel for the bias
-    gradient (torch's generic reduce measured ~1 TB/s there)."""
+    gradient (torch's generic reduce measured ~1 TB/s there).  What is frozen
+    costs nothing: its gradient is not made, and what only that needs not kept."""
 
     @staticmethod
     def forward(ctx, x, w, b):
-        ctx.save_for_backward(x, w)
-        ctx.has_bias = b is not None
+        need_x, need_w, need_b = ctx.needs_input_grad
+        ctx.save_for_backward(x if need_w else None, w if need_x else None)
+        ctx.x_shape = x.shape
+        ctx.need_b = need_b
         return F.linear(x, w, b)
 
     @staticmethod
     def backward(ctx, dy):
         x, w = ctx.saved_tensors
         dy2 = dy.contiguous().view(-1, dy.shape[-1])
-        x2 = x.contiguous().view(-1, x.shape[-1])
-        dx = (dy2 @ w).view(x.shape)
-        dw = _weight_grad(dy2, x2)
-        db = _colsum(dy2) if ctx.has_bias else None
-        return dx, dw, db
+        dx = dw = None
+        if w is not None:
+            dx = (dy2 @ w).view(ctx.x_shape)
+        if x is not None:
+            dw = _weight_grad(dy2, x.contiguous().view(-1, x.shape[-1]))
+        return dx, dw, _colsum(dy2) if ctx.need_b else None
 
 
 class _LinearGeluLib(torch.autograd.Function):
