@@ -586,7 +586,9 @@ def linear_residual(x: torch.Tensor, w: torch.Tensor,
     if x.is_cuda and _tile_ok(x, w) and (
             _HAND_GEMM_ALL or (w.shape[0] <= 1024 and w.shape[1] <= 1024)):
         return _LinearResidualFn.apply(x, w, b, res)
-    if (x.is_cuda and b is not None and x.dtype == torch.bfloat16
+    # one type throughout: autocast's float32 weights need torch's own backward
+    if (x.is_cuda and b is not None
+            and x.dtype == w.dtype == b.dtype == torch.bfloat16
             and torch.is_grad_enabled() and not _transformed()):
         return _LinearLib.apply(x, w, b) + res     # bias gradient: colsum
     return F.linear(x, w, b) + res
