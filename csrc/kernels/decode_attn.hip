@@ -20,7 +20,10 @@
 
 namespace {
 
-constexpr float NONE = -1e30f;   // "no key yet", base-2 scores
+// "no key yet", base-2 scores.  What is not above it weighs nothing, which of
+// a key's scores only -inf is: the comparisons below let NaN pass, so that it
+// shows in the row.
+constexpr float NONE = -3.4028234663852886e38f;
 
 struct DecodeArgs {
   const short *qkv;
@@ -178,8 +181,8 @@ decode_attn_kernel(DecodeArgs a) {
       #pragma unroll
       for (int r = 0; r < R; ++r) {
         // a score of NONE is no key, also where the maximum is none yet
-        const float e = sc[u][r] > NONE
-            ? __builtin_amdgcn_exp2f(sc[u][r] - m[r]) : 0.f;
+        const float e = sc[u][r] <= NONE
+            ? 0.f : __builtin_amdgcn_exp2f(sc[u][r] - m[r]);
         sum[r] += e;
         #pragma unroll
         for (int i = 0; i < 8; ++i) o[r][i] = fmaf(e, vf[i], o[r][i]);
@@ -210,7 +213,7 @@ decode_attn_kernel(DecodeArgs a) {
       d = group_sum<LPK>(d);
       if (g != 0) d = NONE;
       const float t = fmaxf(m[r], d), f = __builtin_amdgcn_exp2f(m[r] - t);
-      const float e = d > NONE ? __builtin_amdgcn_exp2f(d - t) : 0.f;
+      const float e = d <= NONE ? 0.f : __builtin_amdgcn_exp2f(d - t);
       m[r] = t;
       sum[r] = sum[r] * f + e;
       #pragma unroll
@@ -311,7 +314,7 @@ void launch(const DecodeArgs& a, hipStream_t st) {
 
 }  // namespace
 
-// What decode_attention_into takes: see decode_attention.
+// What decode_attention takes: see there.
 bool decode_attention_takes(const torch::Tensor& qkv, const torch::Tensor& k,
                             const torch::Tensor& v) {
   const long D = k.dim() == 4 ? k.size(3) : 0;

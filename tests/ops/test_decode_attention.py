@@ -105,3 +105,54 @@ def test_far_scores_do_not_overflow():
     want = _reference(qkv, k, v, pos, None, H)[0]
     got = ops.require_ext().decode_attention(qkv, k, v, pos, None, None, None, H)
     assert (got.double() - want).norm() / want.norm() < 2 ** -8
+
+
+def _inputs(L, H=4, G=2, D=128):
+    torch.manual_seed(L)
+    qkv = torch.randn(1, (H + 2 * G) * D, device="cuda").bfloat16()
+    k, v = (torch.randn(1, G, L, D, device="cuda").bfloat16() for _ in range(2))
+    return qkv, k, v
+
+
+def _attend(qkv, k, v, depth, H=4):
+    from scaffold import ops
+
+    out = ops.require_ext().decode_attention(
+        qkv, k, v, torch.tensor([depth], device="cuda"), None, None, None, H)
+    return out.view(H, -1)
+
+
+@pytest.mark.parametrize("L", [40, 4096])
+@pytest.mark.parametrize("at", [0, 5, 30, "new"])
+def test_a_score_that_is_no_number_shows(L, at):
+    """NaN in one cached key, or in the new one, is NaN in the heads that see
+    it, and in no other."""
+    qkv, k, v = _inputs(L)
+    if at == "new":
+        qkv[0, 5 * 128 + 3] = float("nan")
+    else:
+        k[0, 1, at, 3] = float("nan")
+    out = _attend(qkv, k, v, L - 2)
+    assert out[:2].isfinite().all() and out[2:].isnan().all()
+
+
+@pytest.mark.parametrize("L", [40, 4096])
+@pytest.mark.parametrize("best", [3, 37, "new"])
+def test_scores_far_below_zero(L, best):
+    """Every score near the lowest float's exponent: the highest still wins."""
+    qkv, k, v = _inputs(L)
+    qkv[:, :512] = 1e17
+    k[:] = -1e18
+    qkv[:, 512:768] = -1e18
+    if best == "new":
+        qkv[:, 512:768] = -9e17
+        want = qkv[0, 768:].view(2, 1, 128)
+    else:
+        k[:, :, best] = -9e17
+        want = v[0, :, best].unsqueeze(1)
+    out = _attend(qkv, k, v, L - 2)
+    assert torch.equal(out.view(2, 2, 128), want.expand(2, 2, 128))
+    k[:] = -1e30                         # -inf throughout: no weights at all
+    qkv[:, :512] = 1e30
+    qkv[:, 512:768] = -1e30
+    assert _attend(qkv, k, v, L - 2).isnan().all()
