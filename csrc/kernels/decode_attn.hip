@@ -145,7 +145,14 @@ decode_attn_kernel(DecodeArgs a) {
     #pragma unroll
     for (int i = 0; i < 8; ++i) o[r][i] = 0.f;
   }
-  auto take = [&](const bf16x8 (&kk)[U], const bf16x8 (&vv)[U], int j0) {
+  auto take = [&](const bf16x8 (&kk)[U], bf16x8 (&vv)[U], int j0) {
+    // no weight makes an infinite value nothing, so those of the repeated
+    // places go; only a row's last tile has some
+    if (j0 + TILE > hi) {
+      #pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (j0 + u * KPI + g >= hi) vv[u] = bf16x8{};
+    }
     float sc[U][R];
     #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -200,11 +207,12 @@ decode_attn_kernel(DecodeArgs a) {
   // the new token, by the last wave's first group of lanes
   if (own && w == WAVES - 1) {
     const bf16x8 nk = turned<D>(a, row + (a.H + kv) * D, c, p);
-    const bf16x8 nv = *(const bf16x8*)(row + (a.H + a.G + kv) * D + 8 * c);
+    bf16x8 nv = *(const bf16x8*)(row + (a.H + a.G + kv) * D + 8 * c);
     if (g == 0 && ch == 0) {
       *(bf16x8*)(kc + (long)p * a.ss) = nk;
       *(bf16x8*)(vc + (long)p * a.ss) = nv;
     }
+    if (g != 0) nv = bf16x8{};
     #pragma unroll
     for (int r = 0; r < R; ++r) {
       float d = 0.f;

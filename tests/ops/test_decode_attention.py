@@ -156,3 +156,19 @@ def test_scores_far_below_zero(L, best):
     qkv[:, :512] = 1e30
     qkv[:, 512:768] = -1e30
     assert _attend(qkv, k, v, L - 2).isnan().all()
+
+
+@pytest.mark.parametrize("L", [18, 40, 49, 4096])
+@pytest.mark.parametrize("back", [0, 1, 2, 17])
+def test_infinite_values(L, back):
+    """An infinite value, cached `back` places before the new one or new, is
+    infinite in its column of the heads that see it, and nothing else is."""
+    qkv, k, v = _inputs(L)
+    if back == 0:
+        qkv[0, 7 * 128 + 3] = float("inf")
+    else:
+        v[0, 1, L - 1 - back, 3] = float("inf")
+    out = _attend(qkv, k, v, L - 1)
+    assert (out[2:, 3] == float("inf")).all()
+    out[2:, 3] = 0
+    assert out.isfinite().all()
