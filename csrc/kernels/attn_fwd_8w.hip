@@ -100,7 +100,12 @@ attn_fwd_8w_kernel(const short* __restrict__ q, const short* __restrict__ k,
   f32x16_t oacc[NDT];
   #pragma unroll
   for (int t = 0; t < NDT; ++t) oacc[t] = {};
-  float m_run = -1e30f, l_run = 0.f;  // base-2 domain
+  // Training counts a score below -1e30 as masked.  Serving, whose scores no
+  // loss keeps small, does not: an unseen key has -inf there, and every row
+  // sees a key of the first tile, so that its maximum is a score from then on.
+  constexpr float LOWEST = SPLIT ? -3.4028234663852886e38f : -1e30f;
+  constexpr float UNSEEN = SPLIT ? -__builtin_inff() : -1e30f;
+  float m_run = LOWEST, l_run = 0.f;  // base-2 domain
 
   const unsigned tr_base0 = lds_byte_off(kv_lds + 64 * D) + 128u * (lq >> 4)
                             + ((l & 15) >> 2) * 32 + (l & 3) * 8
@@ -215,7 +220,7 @@ attn_fwd_8w_kernel(const short* __restrict__ q, const short* __restrict__ k,
 
     // ---- scale (exp2-folded) + mask in place (defer-max THR=0)
     const bool need_mask = (causal && c0 + 63 > qrow_g + off) || (c0 + 63 >= Sk);
-    float mtile = -1e30f;
+    float mtile = LOWEST;
     #pragma unroll
     for (int sub = 0; sub < 2; ++sub)
       #pragma unroll
@@ -224,7 +229,7 @@ attn_fwd_8w_kernel(const short* __restrict__ q, const short* __restrict__ k,
         float sv = sacc[sub][r] * scale2;
         if (need_mask) {
           const int kg = c0 + krel;
-          if (kg >= Sk || (causal && kg > qrow_g + off)) sv = -1e30f;
+          if (kg >= Sk || (causal && kg > qrow_g + off)) sv = UNSEEN;
         }
         sacc[sub][r] = sv;
         mtile = fmaxf(mtile, sv);
@@ -336,7 +341,8 @@ attn_fwd_8w_kernel(const short* __restrict__ q, const short* __restrict__ k,
     cur ^= 1;
   }
 
-  const float inv_l = (l_run > 0.f) ? 1.f / l_run : 0.f;
+  // serving: -inf throughout is NaN, as in a softmax
+  const float inv_l = SPLIT || l_run > 0.f ? 1.f / l_run : 0.f;
   if (qrow_g < S) {
     const long obase = (long)b * os.sb + (long)h * os.sh + (long)qrow_g * os.ss;
     // packed store: each r-quad's four d-values are consecutive in

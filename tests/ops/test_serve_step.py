@@ -35,6 +35,30 @@ def test_prompt_attention_matches_float64(D, H, G, S, Sk):
     assert (got - want).norm() / want.norm() < 2.0 ** -9
 
 
+@pytest.mark.parametrize("D,H,G", [(128, 4, 2), (64, 3, 3)])
+@pytest.mark.parametrize("S,Sk", [(1, 70), (5, 5), (64, 65), (257, 300)])
+def test_prompt_scores_far_below_zero(D, H, G, S, Sk):
+    """Every score near the lowest float's exponent, the highest two keys back
+    (or the first): what follows a row is not seen, and -inf is NaN."""
+    from scaffold import ops
+
+    f = ops.require_ext().prompt_attention
+    torch.manual_seed(S)
+    q = torch.full((2, H, S, D), 1e17, device="cuda").bfloat16()
+    k = torch.full((2, G, Sk, D), -1e18, device="cuda").bfloat16()
+    v = torch.randn(2, G, Sk, D, device="cuda").bfloat16()
+    best = max(Sk - S - 2, 0)
+    k[:, :, best] = -9e17
+    want = v[:, :, best].repeat_interleave(H // G, 1).unsqueeze(2)
+    got = f(q, k, v, Sk)
+    assert torch.equal(got, want.expand_as(got))
+    assert f(q * 1e13, k * 1e13, v, Sk).isnan().all()
+    k[0, 0, best] = float("nan")
+    got = f(q, k, v, Sk)
+    assert got[0, :H // G].isnan().all() and got[0, H // G:].isfinite().all()
+    assert got[1].isfinite().all()
+
+
 def _model(name, **kw):
     from scaffold.config import load_config
     from scaffold.models import build_model
