@@ -76,9 +76,12 @@ __global__ void __launch_bounds__(256)
 softmax_xent_bwd_kernel(const T* __restrict__ logits,
                         const long* __restrict__ targets,
                         const float* __restrict__ lse, T* __restrict__ dlogits,
-                        int V, float scale, const float* __restrict__ dloss) {
+                        int V, long R, double factor,
+                        const float* __restrict__ dloss) {
   const long row = blockIdx.x;
-  if (dloss) scale *= *dloss;    // read here: the host need not wait for it
+  // read here: the host need not wait for it.  Divided in double and rounded
+  // once, as the host does
+  const float scale = (float)((dloss ? (double)*dloss : factor) / (double)R);
   const T* lr = logits + row * (long)V;
   T* dr = dlogits + row * (long)V;
   const float l = lse[row];
@@ -134,8 +137,8 @@ std::vector<torch::Tensor> softmax_xent_fwd(torch::Tensor logits, torch::Tensor 
   return {loss, lse};
 }
 
-// dlogits of the mean over the rows; its gradient is `dloss`, or, if given,
-// the float32 number in dloss_dev.
+// dlogits of the mean over the R rows, whose gradient is `dloss`, or, if given,
+// the float32 number in dloss_dev: dloss / R is a row's factor.
 torch::Tensor softmax_xent_bwd(torch::Tensor logits, torch::Tensor targets,
                                torch::Tensor lse, double dloss,
                                c10::optional<torch::Tensor> dloss_dev) {
@@ -149,22 +152,19 @@ torch::Tensor softmax_xent_bwd(torch::Tensor logits, torch::Tensor targets,
                 dloss_dev->scalar_type() == torch::kFloat32,
                 "softmax_xent_bwd: dloss is one float32 on the GPU");
     dp = dloss_dev->data_ptr<float>();
-    dloss = 1.0;
   }
-  // mean reduction: d(mean)/dlogit_row = dloss / R
-  const float scale = (float)(dloss / (double)R);
   auto stream = scaffold_stream();
   dim3 grid((unsigned)R), block(256);
   if (logits.scalar_type() == torch::kBFloat16) {
     hipLaunchKernelGGL(softmax_xent_bwd_kernel<short>, grid, block, 0, stream,
                        (const short*)logits.data_ptr(), targets.data_ptr<long>(),
                        lse.data_ptr<float>(), (short*)dlogits.data_ptr(), V,
-                       scale, dp);
+                       R, dloss, dp);
   } else {
     hipLaunchKernelGGL(softmax_xent_bwd_kernel<float>, grid, block, 0, stream,
                        logits.data_ptr<float>(), targets.data_ptr<long>(),
                        lse.data_ptr<float>(), dlogits.data_ptr<float>(), V,
-                       scale, dp);
+                       R, dloss, dp);
   }
   HIP_CHECK(hipGetLastError());
   return dlogits;
