@@ -574,6 +574,10 @@ class Generator:
                 and m.lm_head.weight.dtype == torch.bfloat16
                 and os.environ.get("SCAFFOLD_DECODE_GEMV") != "1"):
             return None
+        # The call holds every layer's weights at once, so they have to be there
+        # already: a parametrized one (unmerged LoRA) is made on each access, a
+        # whole second model for the time of a step.  It is no plain parameter
+        # and is left to the blocks, which need one layer's at a time.
         layers, eps = [], []
         for blk in m.blocks:
             a = blk.attn
@@ -582,12 +586,13 @@ class Generator:
                 return None
             if self.is_llama:
                 n1, n2 = blk.attn_norm, blk.mlp_norm
-                layers += (n1.weight, a.wqkv.weight, a.wo.weight, n2.weight,
-                           blk.w_gateup.weight, blk.w_down.weight)
+                mods = n1, a.wqkv, a.wo, n2, blk.w_gateup, blk.w_down
+                layers += [mod._parameters.get("weight") for mod in mods]
             else:
                 n1, n2 = blk.ln1, blk.ln2
                 for mod in (n1, a.qkv, a.proj, n2, blk.fc, blk.proj):
-                    layers += (mod.weight, mod.bias)
+                    layers += (mod._parameters.get("weight"),
+                               mod._parameters.get("bias"))
             eps += (n1.eps, n2.eps)
         if self.is_llama:
             f, embed, wpe = m.norm_f, m.embed.weight, None

@@ -179,3 +179,35 @@ def test_prompt_that_does_not_fit_is_refused():
     with torch.no_grad(), pytest.raises(RuntimeError):
         gen._forward_tokens(torch.zeros(1, 9, dtype=torch.int64,
                                         device="cuda"), cache, 0)
+
+
+@pytest.mark.parametrize("name,kw", [("gpt2", {}),
+                                     ("llama", {"n_kv_heads": 2, "d_ff": 520})])
+def test_parametrized_weights_are_left_to_the_blocks(name, kw):
+    """Unmerged adapters, whose merged weights would all be alive in one call:
+    layer by layer, and the step of the merged model."""
+    from scaffold.generate import Generator
+    from scaffold.lora import LoRAAdapter, apply_lora, merge_lora
+
+    m = _model(name, **kw).cuda()
+    apply_lora(m, r=4)
+    for mod in m.modules():
+        if isinstance(mod, LoRAAdapter):
+            torch.nn.init.normal_(mod.B, std=0.02)
+    gen = Generator(m)
+    tok = torch.tensor([[5], [9]], device="cuda")
+    pos = torch.tensor([0, 3], device="cuda")
+    with torch.no_grad():
+        assert gen._native_step(tok, gen.new_cache(2, 16), pos) is None
+        got = gen.decode_step_varpos(tok, gen.new_cache(2, 16), pos)
+        cache = gen.new_cache(2, 16)
+        ids = torch.arange(10, device="cuda").view(2, 5)
+        prompt = gen._forward_tokens(ids, cache, 0)
+    gen = Generator(merge_lora(m).eval())
+    with torch.no_grad():
+        assert gen._native_step(tok, gen.new_cache(2, 16), pos) is not None
+        want = gen.decode_step_varpos(tok, gen.new_cache(2, 16), pos)
+        merged = gen._forward_tokens(ids, gen.new_cache(2, 16), 0)
+    # two bf16 streams of the same weights: see test_step_matches_float32
+    for g, w in ((got, want), (prompt, merged)):
+        assert (g.float() - w.float()).norm() / w.float().norm() < 6 * 2 ** -7
