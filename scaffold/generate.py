@@ -96,6 +96,17 @@ def _tp_reduce(t: torch.Tensor, holder) -> torch.Tensor:
     return t
 
 
+def _plain_lookup(e: torch.nn.Module) -> bool:
+    """Whether calling embedding `e` is a lookup in its weight and nothing
+    else: no hooks, no forward of its own, no rows rescaled on the way."""
+    every = torch.nn.modules.module
+    return (type(e) is torch.nn.Embedding and e.max_norm is None
+            and "forward" not in e.__dict__
+            and not (e._forward_hooks or e._forward_pre_hooks
+                     or every._global_forward_hooks
+                     or every._global_forward_pre_hooks))
+
+
 class Generator:
     """Greedy / temperature decoding for the scaffold's LM families."""
 
@@ -601,7 +612,9 @@ class Generator:
             f, embed, wpe = m.ln_f, m.wte.weight, m.wpe.weight
             last, tables = [f.weight, f.bias], (None, None)
         if any(t is None for t in layers) or (
-                self.is_llama and not tables[0].is_cuda):
+                self.is_llama and not tables[0].is_cuda) or not all(
+                _plain_lookup(e) for e in
+                ((m.embed,) if self.is_llama else (m.wte, m.wpe))):
             return None
         return ops.require_ext().serve_step(
             tokens.contiguous(), embed, wpe, layers, eps + [f.eps], cache.k,

@@ -211,3 +211,56 @@ def test_parametrized_weights_are_left_to_the_blocks(name, kw):
     # two bf16 streams of the same weights: see test_step_matches_float32
     for g, w in ((got, want), (prompt, merged)):
         assert (g.float() - w.float()).norm() / w.float().norm() < 6 * 2 ** -7
+
+
+@pytest.mark.parametrize("name,kw,embeddings", [
+    ("gpt2", {}, ("wte", "wpe")),
+    ("llama", {"n_kv_heads": 2, "d_ff": 520}, ("embed",))])
+def test_embeddings_that_do_more_than_look_up(name, kw, embeddings):
+    """Hooks fire, an own forward is called, and their results count."""
+    from scaffold.generate import Generator
+
+    tok = torch.tensor([[5], [9]], device="cuda")
+    ids = torch.arange(6, device="cuda").view(2, 3)
+    pos = torch.tensor([3, 3], device="cuda")
+
+    @torch.no_grad()
+    def run(m):
+        gen, out = Generator(m), []
+        cache = gen.new_cache(2, 16)
+        out.append(gen._forward_tokens(ids, cache, 0))
+        out.append(gen.decode_step_varpos(tok, cache, pos))
+        return out, gen._native_step(tok, cache, pos)
+
+    for attr in embeddings:
+        m = _model(name, **kw).cuda()
+        mod, table = getattr(m, attr), getattr(m, attr).weight.detach().clone()
+        plain, native = run(m)
+        assert native is not None
+        hits = []
+        ways = []
+        h = mod.register_forward_hook(lambda *a: hits.append(1))
+        ways.append(run(m))
+        assert len(hits) == 2
+        h.remove()
+        h = mod.register_forward_pre_hook(lambda *a: hits.append(1))
+        ways.append(run(m))
+        assert len(hits) == 4
+        h.remove()
+        h = torch.nn.modules.module.register_module_forward_hook(
+            lambda a, *b: hits.append(1) if a is mod else None)
+        ways.append(run(m))
+        assert len(hits) == 6
+        h.remove()
+        mod.forward = lambda t: torch.nn.functional.embedding(t, table)
+        ways.append(run(m))
+        del mod.forward
+        for out, native in ways:
+            assert native is None
+            for g, w in zip(out, plain):
+                assert (g.float() - w.float()).norm() / w.float().norm() < 6 * 2 ** -7
+        h = mod.register_forward_hook(lambda m, a, out: out * 0 + 1)
+        ones = run(m)[0]
+        h.remove()
+        assert not any(torch.equal(g, w) for g, w in zip(ones, ways[0][0]))
+        assert run(m)[1] is not None
