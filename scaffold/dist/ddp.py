@@ -194,22 +194,31 @@ class BucketedDDP(nn.Module):
         """Bring gradients that autograd made elsewhere into the bucket:
         every .grad is its view afterwards."""
         made, places = [], []
+        own = b.flat.untyped_storage().data_ptr()
         for p, v in zip(b.params, b.views):
             g = p.grad
             if g is v:
                 continue
+            p.grad = v
             if g is None:                # took no part in this backward
                 v.zero_()
-            else:
-                made.append(g)
-                places.append(v)
-            p.grad = v
+                continue
+            if g.layout == torch.strided and \
+                    g.untyped_storage().data_ptr() == own:
+                if g.data_ptr() == v.data_ptr() and g.stride() == v.stride():
+                    continue             # the view under another name
+                g = g.clone()            # in the bucket, but not in place
+            made.append(g)
+            places.append(v)
         if made:
             with torch.no_grad():
                 if b.flat.is_cuda:
                     ops.require_ext().gather_into(made, places)
-                else:
-                    for g, v in zip(made, places):
+                    return
+                for g, v in zip(made, places):
+                    if g.layout == torch.strided:
+                        v.copy_(g)
+                    else:
                         v.zero_().add_(g)
 
     def _launch(self, b: GradBucket) -> None:
