@@ -56,7 +56,7 @@ void gather_into(std::vector<torch::Tensor> from, std::vector<torch::Tensor> to)
     TORCH_CHECK(f.sizes() == t.sizes(), "gather_into: shapes differ");
     if (!t.numel()) continue;
     if (f.layout() != torch::kStrided) {
-      t.zero_().add_(f);
+      t.copy_(f.to_dense());
       continue;
     }
     const bool alike = f.is_cuda() && t.is_cuda() && f.device() == t.device() &&

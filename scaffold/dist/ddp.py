@@ -215,11 +215,10 @@ class BucketedDDP(nn.Module):
                 if b.flat.is_cuda:
                     ops.require_ext().gather_into(made, places)
                     return
+                # (torch's add of a sparse tensor to a view misses the view's
+                # place in its storage)
                 for g, v in zip(made, places):
-                    if g.layout == torch.strided:
-                        v.copy_(g)
-                    else:
-                        v.zero_().add_(g)
+                    v.copy_(g if g.layout == torch.strided else g.to_dense())
 
     def _launch(self, b: GradBucket) -> None:
         if b.launched:

@@ -54,3 +54,11 @@ def test_replaced_by_others(dev):
 
     got = _step(dev, turn)
     assert torch.equal(got[0], want[0].t()) and torch.equal(got[2], want[2])
+
+
+@pytest.mark.parametrize("dev", PLACES)
+def test_sparse_ones(dev):
+    """Also into views that do not start where the bucket does."""
+    want = _step(dev, lambda params: None)
+    for g, w in zip(_step(dev, _replace(lambda g: g.to_sparse())), want):
+        assert torch.equal(g, w)
