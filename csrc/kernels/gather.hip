@@ -4,6 +4,8 @@
 
 #include "../common.h"
 
+#include <c10/core/DeviceGuard.h>
+
 namespace {
 
 constexpr int MOST = 64;               // tensors of a launch
@@ -43,6 +45,10 @@ gather_kernel(GatherArgs a) {
 // laid out alike, torch's copy for the others.
 void gather_into(std::vector<torch::Tensor> from, std::vector<torch::Tensor> to) {
   TORCH_CHECK(from.size() == to.size(), "gather_into: lists differ");
+  if (to.empty()) return;
+  // torch's copies go by their tensors' device, whichever is current
+  const auto dev = to[0].device();
+  const c10::DeviceGuard guard(dev);
   auto st = scaffold_stream();
   GatherArgs a;
   a.n = a.first[0] = 0;
@@ -59,7 +65,7 @@ void gather_into(std::vector<torch::Tensor> from, std::vector<torch::Tensor> to)
       t.copy_(f.to_dense());
       continue;
     }
-    const bool alike = f.is_cuda() && t.is_cuda() && f.device() == t.device() &&
+    const bool alike = dev.is_cuda() && f.device() == dev && t.device() == dev &&
         f.scalar_type() == t.scalar_type() &&
         f.element_size() % 2 == 0 && f.strides() == t.strides() &&
         f.is_non_overlapping_and_dense();

@@ -34,6 +34,23 @@ def test_gather_into(dtype):
         ops.require_ext().gather_into([made[3]], [places[4]])
 
 
+@pytest.mark.parametrize("n", [4, 100003])
+def test_gather_into_goes_by_the_tensors_device(n):
+    """Whichever device is current; without a GPU at hand, by torch's copies."""
+    from scaffold import ops
+
+    gather = ops.require_ext().gather_into
+    gather([], [])
+    last = torch.device("cuda", torch.cuda.device_count() - 1)
+    for dev in (last, torch.device("cpu")):
+        made = [torch.randn(n, device=dev), torch.randn(n).half()]
+        places = [torch.zeros(n, device=dev), torch.zeros(n, device=dev)]
+        with torch.cuda.device(0):
+            gather(made, places)
+        for m, p in zip(made, places):
+            assert torch.equal(m.to(dev).float(), p)
+
+
 class _Net(nn.Module):
     def __init__(self):
         super().__init__()
