@@ -388,7 +388,7 @@ torch::Tensor rope_apply(torch::Tensor x, torch::Tensor cos_t, torch::Tensor sin
   if (total == 0) return y;
   if (x.scalar_type() == torch::kBFloat16 && D % 8 == 0 && D <= 2048 &&
       rows(xc) && rows(y) && table(cos_t) && table(sin_t) &&
-      (long)B * S <= 0x7fffffffl) {
+      (long)B * S < (1l << 24)) {      // a launch has fewer than 2^32 threads
     hipLaunchKernelGGL(rope_rows_kernel, dim3((unsigned)((long)B * S)), dim3(256), 0,
                        stream, (const short*)xc.data_ptr(), cos_t.data_ptr<float>(),
                        sin_t.data_ptr<float>(), (short*)y.data_ptr(), H, S, D,

@@ -59,3 +59,20 @@ def test_vectors_turn_as_pairs_do(B, H, S, D, inverse):
     assert not room[:, :, 0].any() and not room[:, :, H + 1:].any()
     f(x, cos, sin, inverse, out=x)             # in place
     assert torch.equal(x, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [(1 << 24) - 1, 1 << 24])
+def test_turns_any_number_of_positions(S):
+    """More positions than a launch has blocks of a position each."""
+    f = ops.require_ext().rope_apply
+    x = torch.randn(1, 1, S, 8, device="cuda", dtype=torch.bfloat16)
+    cos = torch.full((S, 4), 0.6, device="cuda")
+    sin = torch.full((S, 4), 0.8, device="cuda")
+    y = f(x, cos, sin, False)
+    part = f(x[:, :, -999:].contiguous(), cos[:999], sin[:999], False)
+    assert torch.equal(y[:, :, -999:], part)
+    u, w = x[..., ::2].float(), x[..., 1::2].float()
+    # the result's rounding, half of 2^-8 of up to 1.4 times 6
+    assert (y[..., ::2].float() - (0.6 * u - 0.8 * w)).abs().max() < 2 ** -5
+    assert (y[..., 1::2].float() - (0.8 * u + 0.6 * w)).abs().max() < 2 ** -5
