@@ -80,7 +80,9 @@ def _model(name, **kw):
 @pytest.mark.parametrize("name,kw", [
     ("gpt2", {}), ("gpt2", {"d_ff": 520}),
     ("llama", {"n_kv_heads": 2, "d_ff": 520}),
-    ("llama", {"n_kv_heads": 1, "d_ff": 8200})])
+    ("llama", {"n_kv_heads": 1, "d_ff": 8200}),
+    ("llama", {"n_heads": 8, "n_kv_heads": 1, "d_ff": 520}),
+    ("llama", {"n_heads": 10, "n_kv_heads": 2, "d_model": 640, "d_ff": 520})])
 @pytest.mark.parametrize("B", [1, 7, 17, 65])
 def test_step_matches_float32(name, kw, B):
     """A step at unequal depths and one at a common depth, against the
@@ -136,7 +138,8 @@ def test_unknown_token_shows():
 
 @pytest.mark.parametrize("name,kw", [
     ("gpt2", {"n_heads": 4}), ("llama", {"n_kv_heads": 2, "d_ff": 520}),
-    ("llama", {"n_heads": 2, "n_kv_heads": 1, "d_ff": 520})])
+    ("llama", {"n_heads": 2, "n_kv_heads": 1, "d_ff": 520}),
+    ("llama", {"n_heads": 10, "n_kv_heads": 2, "d_model": 640, "d_ff": 520})])
 @pytest.mark.parametrize("B,S,p0", [(1, 2, 0), (3, 5, 0), (2, 9, 64),
                                     (1, 130, 20), (2, 64, 1), (1, 1, 0)])
 @pytest.mark.parametrize("every", [False, True])
@@ -157,6 +160,7 @@ def test_prompt_matches_float32(name, kw, B, S, p0, every):
     cpu.len = gpu.len = p0
     tok = torch.randint(0, 1003, (B, S))
     with torch.no_grad():
+        assert gen._native_step(tok.cuda(), gpu, None, p0) is not None
         want = ref._forward_tokens(tok, cpu, p0, all_logits=every)
         got = gen._forward_tokens(tok.cuda(), gpu, p0, all_logits=every)
     assert got.shape == want.shape and gpu.len == cpu.len == p0 + S
