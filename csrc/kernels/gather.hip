@@ -41,8 +41,8 @@ gather_kernel(GatherArgs a) {
 
 }  // namespace
 
-// to[i] <- from[i]; same shape and type each.  One launch for all that are
-// laid out alike, torch's copy for the others.
+// to[i] <- from[i], places in one buffer; same shape each.  One launch for all
+// that are laid out alike, torch's copy for the others.
 void gather_into(std::vector<torch::Tensor> from, std::vector<torch::Tensor> to) {
   TORCH_CHECK(from.size() == to.size(), "gather_into: lists differ");
   if (to.empty()) return;
@@ -57,14 +57,26 @@ void gather_into(std::vector<torch::Tensor> from, std::vector<torch::Tensor> to)
       hipLaunchKernelGGL(gather_kernel, dim3(a.first[a.n]), dim3(256), 0, st, a);
     a.n = 0;
   };
+  // what lies in the buffer but not at its place is copied out before others
+  // are copied in
+  auto placed = [](const torch::Tensor& f, const torch::Tensor& t) {
+    return f.data_ptr() == t.data_ptr() && f.strides() == t.strides() &&
+           f.scalar_type() == t.scalar_type();
+  };
+  for (size_t i = 0; i < from.size(); ++i) {
+    TORCH_CHECK(from[i].sizes() == to[i].sizes(), "gather_into: shapes differ");
+    if (from[i].layout() == torch::kStrided && from[i].is_alias_of(to[i]) &&
+        !placed(from[i], to[i]))
+      from[i] = from[i].clone();
+  }
   for (size_t i = 0; i < from.size(); ++i) {
     const auto &f = from[i], &t = to[i];
-    TORCH_CHECK(f.sizes() == t.sizes(), "gather_into: shapes differ");
     if (!t.numel()) continue;
     if (f.layout() != torch::kStrided) {
       t.copy_(f.to_dense());
       continue;
     }
+    if (placed(f, t)) continue;
     const bool alike = dev.is_cuda() && f.device() == dev && t.device() == dev &&
         f.scalar_type() == t.scalar_type() &&
         f.element_size() % 2 == 0 && f.strides() == t.strides() &&

@@ -96,6 +96,27 @@ def partition_buckets(
     return buckets
 
 
+def _gather_into(made, places) -> None:
+    """What gather_into does on the GPU: gradients into the views of a bucket.
+    One that lies in the bucket itself is left where it is the view under
+    another name (p.grad = p.grad.detach()), else copied out before others are
+    copied in."""
+    own = places[0].untyped_storage().data_ptr()
+    todo = []
+    for g, v in zip(made, places):
+        if g.layout != torch.strided:
+            # torch's add of a sparse tensor to a view misses the view's place
+            # in its storage
+            g = g.to_dense()
+        elif g.untyped_storage().data_ptr() == own:
+            if g.data_ptr() == v.data_ptr() and g.stride() == v.stride():
+                continue
+            g = g.clone()
+        todo.append((g, v))
+    for g, v in todo:
+        v.copy_(g)
+
+
 class BucketedDDP(nn.Module):
     def __init__(
         self,
@@ -194,31 +215,22 @@ class BucketedDDP(nn.Module):
         """Bring gradients that autograd made elsewhere into the bucket:
         every .grad is its view afterwards."""
         made, places = [], []
-        own = b.flat.untyped_storage().data_ptr()
         for p, v in zip(b.params, b.views):
             g = p.grad
             if g is v:
                 continue
-            p.grad = v
             if g is None:                # took no part in this backward
                 v.zero_()
-                continue
-            if g.layout == torch.strided and \
-                    g.untyped_storage().data_ptr() == own:
-                if g.data_ptr() == v.data_ptr() and g.stride() == v.stride():
-                    continue             # the view under another name
-                g = g.clone()            # in the bucket, but not in place
-            made.append(g)
-            places.append(v)
+            else:
+                made.append(g)
+                places.append(v)
+            p.grad = v
         if made:
             with torch.no_grad():
                 if b.flat.is_cuda:
                     ops.require_ext().gather_into(made, places)
-                    return
-                # (torch's add of a sparse tensor to a view misses the view's
-                # place in its storage)
-                for g, v in zip(made, places):
-                    v.copy_(g if g.layout == torch.strided else g.to_dense())
+                else:
+                    _gather_into(made, places)
 
     def _launch(self, b: GradBucket) -> None:
         if b.launched:

@@ -506,10 +506,9 @@ class _LinearLib(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w, b):
-        need_x, need_w, need_b = ctx.needs_input_grad
+        need_x, need_w, ctx.need_b = ctx.needs_input_grad
         ctx.save_for_backward(x if need_w else None, w if need_x else None)
         ctx.x_shape = x.shape
-        ctx.need_b = need_b
         return F.linear(x, w, b)
 
     @staticmethod
