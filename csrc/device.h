@@ -117,7 +117,12 @@ DEVINL unsigned lds_byte_off(const void* p) {
 // waits for as many as a matrix instruction needs: against batches behind one
 // wait in assembly, training attention of 2 x 32 x 4096 x 128 took 609 us
 // instead of 646 forward and 1305 instead of 1338 for dK and dV, prompt
-// attention over pages 136 instead of 148 (with packed conversions).
+// attention over pages 136 instead of 148 (with packed conversions).  The
+// others, 1 x 4096 tokens or 64 rows at 4000, builtin and assembly in us: tied
+// prompts 215 and 236, windows 99 and 106, latent prompts 91 and 92, latent
+// decoding 37.2 and 38.0, tied decoding 55 and 55, states of retention 31.3 and
+// 31.1, of Mamba-2 50.5 and 53.2, of gated linear attention 16.5 and 17.6, their
+// outputs 54.7 and 55.8, 86.8 and 88.0, 32.3 and 32.1 (4 x 777: 31.7 and 31.2).
 DEVINL bf16x4 tr_read(unsigned at) {
   typedef __attribute__((address_space(3))) bf16x4* P;
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)at);

@@ -228,9 +228,8 @@ attn_bwd_dq_8w_kernel(const short* __restrict__ dout,
       unsigned dsf[2][4];
       pack_frags(ds, dsf);
 
-      // dQ^T += K^T . dS^T per d-tile (K^T A-fragments by PAIR-batched
-      // tr-read — the quad form's 16 forced-live outputs pushed the
-      // pinned-Q/dO register budget over at D=128)
+      // dQ^T += K^T . dS^T per d-tile, K^T A-fragments by transpose
+      // reads a pair at a time (registers are what D=128 is short of)
       __builtin_amdgcn_s_setprio(1);
       #pragma unroll
       for (int t = 0; t < NDT; ++t) {
@@ -431,9 +430,8 @@ attn_bwd_dkv_8w_kernel(const short* __restrict__ dout,
         pack_frags((const float*)&sacc, pf);
         pack_frags((const float*)&dpacc, dsf);
 
-        // dV^T += P^T . dO_cols ; dK^T += dS^T . Q_cols — PAIR-batched
-        // tr-reads (4 per wait): the quad form's 16 forced-live output
-        // regs were half the dkv spill at the D=128 budget edge
+        // dV^T += P^T . dO_cols ; dK^T += dS^T . Q_cols, transpose reads
+        // a pair at a time (registers are what D=128 is short of)
         __builtin_amdgcn_s_setprio(1);
         #pragma unroll
         for (int t = 0; t < NDT; ++t) {

@@ -705,7 +705,7 @@ template <bool F32, int RP> struct RowTile {
     else return p + (j >> 2) * STRIDE + (c >> 4) * 64 + (j & 3) * 16 + (c & 15);
   }
   DEVINL typename N::Frag row(int j, int c) const { return N::load(at(j, c), 0); }
-  // column tiles ct..ct+CB-1 (16 each) of tokens 32*kb..+31, one wait for all
+  // column tiles ct..ct+CB-1 (16 each) of tokens 32*kb..+31
   template <int CB>
   DEVINL void cols(int ct, int kb, int l, typename N::Frag (&f)[CB]) const {
     static_assert(CB == 1 || CB == 2 || CB == 4, "columns at a time");

@@ -275,11 +275,13 @@ class BucketedDDP(nn.Module):
 
     def zero_grad(self) -> None:
         """Start from no gradients.  On the GPU the params let go of their
-        views and the buckets are filled anew (_collect); on the CPU the
-        flat buffers are zeroed.  Rank-local params (_no_ddp, e.g. EP experts) own ordinary .grad
-        tensors — drop them too, or they silently ACCUMULATE across
-        steps (found via a resume-divergence hunt: the accumulated
-        history is exactly what a checkpoint cannot restore)."""
+        views and the buckets are filled anew (_collect): until then .grad
+        is None and a bucket's flat buffer holds what it held.  On the CPU
+        the flat buffers are zeroed.  Rank-local params (_no_ddp, e.g. EP
+        experts) own ordinary .grad tensors — drop them too, or they
+        silently ACCUMULATE across steps (found via a resume-divergence
+        hunt: the accumulated history is exactly what a checkpoint cannot
+        restore)."""
         for b in self.buckets:
             if not b.flat.is_cuda:
                 b.flat.zero_()
