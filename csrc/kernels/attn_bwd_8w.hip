@@ -1,6 +1,6 @@
 // K4 — 8-wave MFMA flash attention backward (bf16, 32x32x16).
 //
-// Round-2 restructure of attn_bwd_mfma.hip's dq/dkv kernels, same move
+// attn_bwd_mfma.hip's dq/dkv kernels restructured, the same move
 // as the forward's 8-wave rebuild (attn_fwd_8w.hip): 512 threads over a
 // 256-row block (wave w owns interleaved rows base + 8*i + w), 64-row
 // staged tiles shared by all 8 waves (half the staging traffic of the

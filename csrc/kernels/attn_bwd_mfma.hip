@@ -34,8 +34,8 @@ namespace {
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef short bf16x8_t __attribute__((ext_vector_type(8)));
 
-// v_cvt_pk_bf16_f32: ONE VALU op per packed pair (guide T12; the r1
-// manual round-to-nearest-even bit sequence was ~7 VALU per pair).
+// v_cvt_pk_bf16_f32: ONE VALU op per packed pair (the manual
+// round-to-nearest-even bit sequence takes ~7 VALU per pair).
 // The asm form constrains the register allocator: the dkv D=128 kernel
 // (at the 256-reg edge) spilled 264 B/lane with it, so dkv keeps the
 // manual sequence (template flag); dq uses cvt_pk (0 spill there).
@@ -243,8 +243,7 @@ attn_bwd_dq_mfma_kernel(const short* __restrict__ dout,
     unsigned dsf[2][4];
     pack_frags(ds, dsf);
 
-    // dQ^T += K^T . dS^T  per d-tile; K^T A-fragments by batched
-    // tr-read (one LDS wait per 4 fragments — common.h)
+    // dQ^T += K^T . dS^T  per d-tile; K^T A-fragments by transpose reads
     __builtin_amdgcn_s_setprio(1);
     #pragma unroll
     for (int t2 = 0; t2 < NDT; t2 += 2) {
@@ -306,10 +305,10 @@ attn_bwd_dkv_mfma_kernel(const short* __restrict__ dout,
   // [buf][Q tile | dO tile], double-buffered at BOTH head dims: tile
   // t+1's glds issue after this tile's LAST ordinary global load (the
   // lse/delta lane loads moved above the issue point — an ordinary
-  // load beside an in-flight glds drains vmcnt(0), guide trap b, which
-  // was also why the r1 D=128 double-buffer attempt measured
-  // net-slower) and drain under the dV/dK MFMAs.  PMC r2: the
-  // synchronous D=128 staging parked waves 73% of the time.
+  // load beside an in-flight glds drains vmcnt(0), which made an earlier
+  // double buffer at D=128 slower than none) and drain under the dV/dK
+  // MFMAs.  With synchronous staging at D=128 waves were parked 73% of
+  // the time (hardware counters).
   __shared__ __attribute__((aligned(16))) short bwd_lds[2 * 2 * 32 * D];
 
   const int wid = threadIdx.x >> 6;
@@ -434,8 +433,7 @@ attn_bwd_dkv_mfma_kernel(const short* __restrict__ dout,
       pack_frags((const float*)&dpacc, dsf);
 
       // dV^T += P^T . dO_cols ; dK^T += dS^T . Q_cols  (C: lane=d, regs=k)
-      // column B-fragments by batched tr-read: one LDS wait per d-tile
-      // pair covers both tensors' 2 k-slices (common.h)
+      // column B-fragments of both tensors by transpose reads
       __builtin_amdgcn_s_setprio(1);
       #pragma unroll
       for (int t = 0; t < NDT; ++t) {
@@ -530,7 +528,7 @@ void attn_bwd_mfma(torch::Tensor dout, torch::Tensor q, torch::Tensor k,
                        (const short*)dout.data_ptr(), (const short*)o.data_ptr(),
                        dlse_ptr, delta.data_ptr<float>(), H, S, rows, dos, osr);
   const int mode = attn_bwd_mode();
-  // auto (re-measured r2): role-split dkv at D=128 (llama train 6.13 ->
+  // auto: role-split dkv at D=128 (llama train 6.13 ->
   // 5.30 ms); 8-wave at D=64 (rs measured 0.71 vs 8w 0.63 ms there)
   if (mode == 5 || (mode == 0 && D == 128 && S >= 128)) {
     // role-split dkv + the auto dq choice
@@ -558,7 +556,7 @@ void attn_bwd_mfma(torch::Tensor dout, torch::Tensor q, torch::Tensor k,
     return;
   }
   // auto: 8-wave at D=64 (measured ~even to +2%); 4-wave at D=128 where
-  // the 8-wave dkv's 36 B/lane spill measured net-slower (NOTES.md r2)
+  // the 8-wave dkv's 36 B/lane spill measured net-slower
   if ((mode == 8) || (mode == 0 && S >= 256 && D <= 64)) {
     attn_bwd_dq_8w(dout, q, k, v, lse, delta, dq, B, H, Hkv, S, D, scale,
                    causal);

@@ -1,9 +1,8 @@
 // K4 — 8-wave MFMA flash attention forward (bf16, CDNA4 32x32x16).
 //
-// The round-2 restructure of attn_fwd_mfma.hip following the guide's
-// 8-warp ladder (cdna_hip_programming.md §B "fused attention prefill")
-// and the round-1 PMC diagnosis (4-wave kernel latency-bound: MfmaUtil
-// 6-10%, dependent-MFMA chains with too few co-resident waves).
+// attn_fwd_mfma.hip restructured: by hardware counters the 4-wave kernel
+// is latency-bound (MfmaUtil 6-10%, dependent-MFMA chains with too few
+// co-resident waves).
 //
 // Structure vs the 4-wave kernel:
 //  * 8 waves / 512 threads over a 256-row q block (wave w owns the
@@ -11,12 +10,11 @@
 //    INDEPENDENT per-wave softmax phases (T5 role-split pays), and the
 //    8 waves share each staged K/V tile — half the per-wave staging
 //    traffic of the 4-wave kernel.
-//  * T14 register staging (guide: glds grafts onto a register-staged
-//    attention pipeline measure <= 0): next tile's global loads issue
-//    BEFORE the compute phase; the ds_write pass lands after the
-//    barrier.  All loads are ordinary (no glds), so hipcc's counted
-//    vmcnt covers both the staging and the D=128 per-tile Q reloads
-//    (no trap-b vmcnt(0) drain — only mixed load KINDS trigger it).
+//  * D=64 stages through registers: the next tile's global loads issue
+//    BEFORE the compute phase, the ds_write pass lands after the barrier.
+//    D=128, which has no registers to spare, stages by copies into LDS
+//    behind QK^T, whose Q reloads are the tile's last ordinary loads (one
+//    beside a copy on its way waits for it).
 //  * exp2-fold: scale*log2e folded into the pre-softmax scale; softmax
 //    runs in the base-2 domain (v_exp_f32 IS exp2 — saves one VALU
 //    multiply per score), lse converted to natural log at the end.
@@ -38,7 +36,7 @@ namespace {
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef short bf16x8_t __attribute__((ext_vector_type(8)));
 
-// v_cvt_pk_bf16_f32 has no builtin on gfx950 (guide T12): one VALU op
+// v_cvt_pk_bf16_f32 has no builtin on gfx950: one VALU op
 // packing two f32 into a dword of 2 bf16 (RTNE).  Inputs are VALU
 // results (exp2), so no producer wait states are needed.
 DEVINL unsigned cvt_pk_bf16(float lo, float hi) {

@@ -1,8 +1,8 @@
 // Fused bf16 NHWC BatchNorm (+ReLU, +residual) for the ResNet headline
-// config.  Round-2 finding (profiles/resnet_kstats_r2.txt): the r1 step
-// spent 38% in MIOpen's fp32 BatchNorm kernels and 19% more in the
-// bf16<->fp32 cast copies its fp32-only interface forces, vs ~30% in
-// the convs themselves.  These kernels read/write the bf16 activation
+// config.  Without them the step spent 38% in MIOpen's fp32 BatchNorm
+// kernels and 19% more in the bf16<->fp32 cast copies its fp32-only
+// interface forces, vs ~30% in the convs themselves
+// (profiles/resnet_kstats_r2.txt).  These kernels read/write the bf16 activation
 // DIRECTLY (fp32 arithmetic inside), and fold the adjacent elementwise
 // ops into the same pass:
 //   fwd:  y = relu?(gamma*xhat + beta [+ res])     xhat=(x-mean)*rstd

@@ -1,7 +1,6 @@
 // Column sum of a [R][C] bf16 matrix -> [C] (bias gradients in the
-// linear backward).  torch's generic reduce ran these at ~1 TB/s; the
-// r1 version used scalar 2-B loads and 16 slices and measured ~23% of
-// HBM roofline (7% of the GPT-2 step, kstats_gpt2_r2).  This version
+// linear backward).  torch's generic reduce ran these at ~1 TB/s, scalar
+// 2-byte loads in 16 slices at a quarter of the copy rate.  This version
 // is bf16x8-vectorized (G13), 4 rows' loads in flight, with a
 // chip-filling slice count and a second stage whose loads are in flight
 // together: 16384 x 768 in 7.8 us (18.5 with one load at a time), 16384 x
@@ -109,7 +108,7 @@ gelu_bwd_kernel(const short* __restrict__ dy, const short* __restrict__ pre,
   fold(C, s, acc, mid + (long)blockIdx.y * C);
 }
 
-// scalar tail path for C % 8 != 0 (rare; the r1 structure)
+// scalar tail path for C % 8 != 0 (rare)
 __global__ void __launch_bounds__(256)
 colsum_slice_scalar_kernel(const short* __restrict__ x,
                            float* __restrict__ mid, long R, int C) {

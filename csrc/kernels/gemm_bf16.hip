@@ -156,9 +156,8 @@ __global__ __launch_bounds__(256) void linear_fwd_kernel(
 // 8x4 fragments of 16x16x32 MFMA; BK=64; LDS = 2 x 64 KiB
 // double-buffered tiles (A 32K + B 32K each).
 //
-// The r1 4-phase version drained vmcnt(0) once per K-tile — the guide
-// measures counted-vs-drain0 at +38%@4k / +73%@8k (T3/T4), so this
-// version NEVER drains in the loop.  Key idea: each wave stages
+// A 4-phase version drained vmcnt(0) once per K-tile; this version
+// NEVER drains in the loop.  Key idea: each wave stages
 // exactly the data IT will read (its A-half rows and B-quarter cols),
 // split so that the pair of glds issued in phase p carries the data
 // quadrant p of the NEXT tile needs.  Then a per-wave counted

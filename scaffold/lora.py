@@ -16,7 +16,7 @@ not MFMA-bound).  The classic x@A@B factored form would avoid the
 materialization but requires module-call sites; this repo's models
 deliberately call ops with raw weights (docs/KERNELS.md), so the
 parametrization form is the right trade until a fused LoRA epilogue
-kernel exists (r3 candidate).
+kernel exists.
 
 Usage:
     apply_lora(model, r=8, alpha=16)        # or model.lora_r config

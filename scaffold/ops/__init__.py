@@ -490,8 +490,8 @@ class _LinearResidualFn(torch.autograd.Function):
         return dx, dw, db, dy
 
 
-# Per-shape dispatch switch: measured on MI355X (gpurun_out/gemm_bench.log,
-# 2026-09-13) the 2-phase 128^2 hand kernel reaches ~900 TF, below
+# Per-shape dispatch switch: measured on MI355X (benchmarks/gemm_bench.py)
+# the 2-phase 128^2 hand kernel reaches ~900 TF, below
 # hipBLASLt at most benched shapes EXCEPT the small-N residual-fused
 # proj (1.07x).  Until the 256^2 8-phase upgrade lands, only the
 # shapes where the hand kernel measured >= parity route to it.
@@ -766,7 +766,7 @@ def fused_adamw_step(
 # Training-mode bf16 NHWC BatchNorm with fused ReLU and optional fused
 # residual add (csrc/kernels/batchnorm.hip, the autograd node included).
 # Replaces MIOpen's fp32-only BN + the bf16<->fp32 cast copies + separate
-# add/relu passes that together were ~57% of the r1 ResNet step
+# add/relu passes that together were ~57% of the ResNet step
 # (profiles/resnet_kstats_r2.txt).
 def _bn_act_eager(x, res, weight, bias, running_mean, running_var,
                   momentum, eps, relu, training):

@@ -8,10 +8,8 @@ int8 + fp32 scales in one safetensors file (~2x smaller than bf16,
 each row's range).
 
 What this is NOT yet: a quantized COMPUTE path.  The llama decode step
-is weight-read-bound (NOTES r2 serving ladder), so an int8 weight x
-bf16 activation GEMV kernel would ~halve decode step time — that
-kernel is a round-3 item (docs/KERNELS.md conventions apply); until it
-exists, quantization buys artifact size, not speed, and this module
+is weight-read-bound, so an int8 weight x bf16 activation GEMV kernel
+would ~halve decode step time; until it exists, quantization buys artifact size, not speed, and this module
 says so rather than pretending otherwise.
 """
 
