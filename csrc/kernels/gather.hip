@@ -5,6 +5,7 @@
 #include "../common.h"
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
 
 namespace {
 
@@ -49,7 +50,8 @@ void gather_into(std::vector<torch::Tensor> from, std::vector<torch::Tensor> to)
   // torch's copies go by their tensors' device, whichever is current
   const auto dev = to[0].device();
   const c10::DeviceGuard guard(dev);
-  auto st = scaffold_stream();
+  const auto stream = c10::hip::getCurrentHIPStream();
+  auto st = stream.stream();
   GatherArgs a;
   a.n = a.first[0] = 0;
   auto flush = [&] {
@@ -77,6 +79,10 @@ void gather_into(std::vector<torch::Tensor> from, std::vector<torch::Tensor> to)
       continue;
     }
     if (placed(f, t)) continue;
+    // made on another stream, it must not go back to that one's pool before it
+    // has been read here (nothing to do if it is this one)
+    if (f.is_cuda())
+      c10::hip::HIPCachingAllocator::recordStream(f.storage().data_ptr(), stream);
     const bool alike = dev.is_cuda() && f.device() == dev && t.device() == dev &&
         f.scalar_type() == t.scalar_type() &&
         f.element_size() % 2 == 0 && f.strides() == t.strides() &&

@@ -51,6 +51,28 @@ def test_gather_into_goes_by_the_tensors_device(n):
             assert torch.equal(m.to(dev).float(), p)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_gradients_of_another_stream_live_until_they_are_read(dtype):
+    """What was made on a side stream is dropped at once, and that stream gets
+    memory of the same size while the copy still waits."""
+    from scaffold import ops
+
+    side = torch.cuda.Stream()
+    n = 1 << 20
+    places = [torch.zeros(n, device="cuda"), torch.zeros(n, device="cuda")]
+    with torch.cuda.stream(side):
+        made = [torch.full((n,), 3.0, device="cuda", dtype=dtype) for _ in places]
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda._sleep(50_000_000)
+    ops.require_ext().gather_into(made, places)
+    del made
+    with torch.cuda.stream(side):
+        others = [torch.full((n,), 5.0, device="cuda", dtype=dtype)
+                  for _ in range(4)]
+    torch.cuda.synchronize()
+    assert all(p.eq(3).all() for p in places) and others[0].eq(5).all()
+
+
 class _Net(nn.Module):
     def __init__(self):
         super().__init__()
