@@ -19,6 +19,8 @@ Design, MI355X-first:
   stream, so it proceeds concurrently with the remaining backward
   kernels over xGMI.  ``finish()`` waits all works (stream-ordered, no
   host sync).
+* A bucket whose gradients are made on several streams waits for
+  ``finish()``: there the caller's stream is behind all of them.
 * **Averaging** is folded into the optimizer's fused AdamW
   ``grad_scale=1/world`` (one less full-gradient pass).
 * Bucket sizes default to 25 MiB, first bucket 4 MiB — chosen so that
@@ -49,6 +51,8 @@ class GradBucket:
     work: object = None
     launched: bool = False
     ready: bool = False
+    stream: Optional[int] = None         # where its first gradient was made
+    mixed: bool = False                  # others on another stream
 
     @property
     def numel(self) -> int:
@@ -189,7 +193,16 @@ class BucketedDDP(nn.Module):
                 return
             b = self._param_bucket[id(p)]
             b.pending -= 1
-            if b.pending == 0 and self.overlap:
+            if b.flat.is_cuda:
+                # a copy out of this hook is in line with gradients of its own
+                # stream alone; behind the backward the caller's stream is
+                # with those of all
+                s = torch._C._cuda_getCurrentRawStream(b.flat.device.index)
+                if b.stream is None:
+                    b.stream = s
+                elif b.stream != s:
+                    b.mixed = True
+            if b.pending == 0 and self.overlap and not b.mixed:
                 b.ready = True
                 self._launch_ready_in_order()
 
@@ -271,6 +284,8 @@ class BucketedDDP(nn.Module):
             b.work = None
             b.launched = False
             b.ready = False
+            b.stream = None
+            b.mixed = False
         self._next_launch = 0
 
     def zero_grad(self) -> None:

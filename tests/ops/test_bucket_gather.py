@@ -177,3 +177,76 @@ def test_captured_step():
         ref.zero_grad()
         ref(t).backward()
         _check(ddp, ref)
+
+
+class _TwoStreams(nn.Module):
+    """Two layers of one bucket, one of them on a side stream that is late."""
+
+    def __init__(self):
+        super().__init__()
+        self.a, self.b = (nn.Linear(256, 256, bias=False) for _ in range(2))
+        self.side = None
+
+    def forward(self, x):
+        if self.side is None:
+            return (self.a(x) * self.b(x)).sum()
+        cur = torch.cuda.current_stream()
+        self.side.wait_stream(cur)
+        with torch.cuda.stream(self.side):
+            u = _Late.apply(self.a(x))
+        v = self.b(x)
+        cur.wait_stream(self.side)
+        return (u * v).sum()
+
+
+class _Late(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, dy):
+        torch.cuda._sleep(20_000_000)
+        return dy * 1
+
+
+@pytest.mark.parametrize("overlap", [True, False])
+def test_gradients_of_several_streams(overlap):
+    from scaffold.dist.ddp import BucketedDDP
+
+    torch.manual_seed(5)
+    net = _TwoStreams().cuda()
+    ref = _TwoStreams().cuda()
+    ref.load_state_dict(net.state_dict())
+    net.side = torch.cuda.Stream()
+    ddp = BucketedDDP(net, overlap=overlap)
+    for _ in range(3):
+        x = torch.randn(64, 256, device="cuda")
+        ddp.zero_grad()
+        ddp(x).backward()
+        ddp.finish()
+        got = [p.grad.clone() for p in net.parameters()]
+        ref.zero_grad()
+        ref(x).backward()
+        for g, p in zip(got, ref.parameters()):
+            torch.testing.assert_close(g, p.grad)
+
+
+def test_one_stream_launches_from_the_backward():
+    """The overlap is still there where a bucket has one stream."""
+    ddp, _ = _nets()
+    t = torch.randint(0, 11, (4, 24), device="cuda")
+    seen = []
+    launch = ddp._launch
+    ddp._launch = lambda b: seen.append(b.index) or launch(b)
+    side = torch.cuda.Stream()
+    for s in (torch.cuda.current_stream(), side):
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            ddp.zero_grad()
+            del seen[:]
+            ddp(t).backward()
+            early = len(seen)
+            ddp.finish()
+        assert early >= len(ddp.buckets) - 1 > 0     # one param is unused
+    torch.cuda.synchronize()
