@@ -268,3 +268,31 @@ def test_embeddings_that_do_more_than_look_up(name, kw, embeddings):
         h.remove()
         assert not any(torch.equal(g, w) for g, w in zip(ones, ways[0][0]))
         assert run(m)[1] is not None
+
+
+@pytest.mark.parametrize("name,kw", [
+    ("gpt2", {}), ("llama", {"n_kv_heads": 2, "d_ff": 512}),
+    ("llama", {"n_heads": 16, "n_kv_heads": 2, "d_model": 512, "d_ff": 512})])
+@pytest.mark.parametrize("rank", [0, 1])
+def test_a_shard_steps_as_on_the_cpu(name, kw, rank):
+    """One rank's share of a tensor-parallel model (partial sums, since no
+    group is there to add them): layer by layer, attention in one launch."""
+    from scaffold.dist.tp import shard_llama_tp
+    from scaffold.generate import Generator
+
+    ref = Generator(shard_llama_tp(_model(name, **kw), rank, 2).float())
+    gen = Generator(shard_llama_tp(_model(name, **kw), rank, 2).cuda())
+    cpu, gpu = ref.new_cache(3, 40), gen.new_cache(3, 40)
+    ids = torch.randint(0, 1003, (3, 9))
+    tok, pos = torch.randint(0, 1003, (3, 1)), torch.tensor([9, 4, 9])
+    with torch.no_grad():
+        assert gen._native_step(tok.cuda(), gpu, pos.cuda()) is None
+        want = [ref._forward_tokens(ids, cpu, 0),
+                ref.decode_step_varpos(tok, cpu, pos)]
+        got = [gen._forward_tokens(ids.cuda(), gpu, 0),
+               gen.decode_step_varpos(tok.cuda(), gpu, pos.cuda())]
+    for g, w in zip(got, want):
+        # a bf16 stream: about ten roundings of 2^-9 a layer, independent
+        assert (g.cpu().float() - w).norm() / w.norm() < 3 * 2 ** -7
+    for a, b in zip(cpu.k + cpu.v, gpu.k + gpu.v):
+        assert (a - b.cpu().float()).norm() / a.norm() < 3 * 2 ** -7
