@@ -167,6 +167,34 @@ bool few(long rows, long depth) {
   return rows <= 16 || (rows <= 64 && rows * depth <= 96 * 1024);
 }
 
+// Few rows of few heads before many keys: the flash kernel has a block for 256
+// rows of a head, which walks the keys alone, 43 us per 1024 of them with heads
+// of 128 and 38 with 64, while the products of a library, in float32 over keys
+// and values spread to all heads, fill the chip.  In us, flash and library:
+// 32 heads of 128, 2 rows, 4096 keys 182 and 146, 8192 355 and 236, 33 rows 359
+// and 361; 64 heads, 8192 350 and 463; 12 heads of 64, 2 rows, 4096 keys 153 and
+// 108, 8192 301 and 121, 96 heads 310 and 257, 33 rows 313 and 520.  Below 5000
+// keys what the step's one call saves is more than the difference.
+bool few_before_many(long heads, long S, long Sk, long D) {
+  return Sk >= 5000 && (D == 64 ? heads * (S + 20) < 2750
+                                : heads * (S + 45) < 3000);
+}
+
+// q (B, H, S, D), k, v (B, G, Sk, D) -> (B, S, H, D): causal, all in float32
+torch::Tensor float32_attention(const torch::Tensor& q, torch::Tensor k,
+                                torch::Tensor v) {
+  const long rep = q.size(1) / k.size(1), S = q.size(2), Sk = k.size(2);
+  if (rep > 1) {
+    k = k.repeat_interleave(rep, 1);
+    v = v.repeat_interleave(rep, 1);
+  }
+  auto s = at::matmul(q.to(at::kFloat), k.to(at::kFloat).transpose(2, 3)) *
+           (1.0 / std::sqrt((double)q.size(3)));
+  const auto unseen = at::ones({S, Sk}, q.options().dtype(at::kBool)).triu(Sk - S + 1);
+  s.masked_fill_(unseen, -std::numeric_limits<double>::infinity());
+  return at::matmul(at::softmax(s, -1), v.to(at::kFloat)).to(q.scalar_type()).transpose(1, 2);
+}
+
 }  // namespace
 
 // tokens (B, S) -> logits (B, V) of the last token of each row, or of all,
@@ -377,10 +405,15 @@ c10::optional<torch::Tensor> serve_step(
       act = torch::Tensor();
     } else {
       append(i, S, true);
-      o = torch::empty({T, inner}, opt);
-      attn_prompt(qkv.view({B, S, heads + 2 * G, D}).narrow(2, 0, heads).transpose(1, 2),
-                  ks[i], vs[i], o.view({B, S, heads, D}).transpose(1, 2),
-                  (int)(pos0 + S), st);
+      const auto q = qkv.view({B, S, heads + 2 * G, D}).narrow(2, 0, heads).transpose(1, 2);
+      if (few_before_many(B * heads, S, pos0 + S, D)) {
+        o = float32_attention(q, ks[i].narrow(2, 0, pos0 + S),
+                              vs[i].narrow(2, 0, pos0 + S)).reshape({T, inner});
+      } else {
+        o = torch::empty({T, inner}, opt);
+        attn_prompt(q, ks[i], vs[i], o.view({B, S, heads, D}).transpose(1, 2),
+                    (int)(pos0 + S), st);
+      }
     }
     if (!product(o, *wo, bias(wo), x, true, SKINNY_NONE))
       pending = lib(o, *wo, bias(wo));

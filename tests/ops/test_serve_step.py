@@ -296,3 +296,33 @@ def test_a_shard_steps_as_on_the_cpu(name, kw, rank):
         assert (g.cpu().float() - w).norm() / w.norm() < 3 * 2 ** -7
     for a, b in zip(cpu.k + cpu.v, gpu.k + gpu.v):
         assert (a - b.cpu().float()).norm() / a.norm() < 3 * 2 ** -7
+
+
+@pytest.mark.parametrize("name,kw", [
+    ("gpt2", {"n_heads": 4}), ("llama", {"n_heads": 4, "n_kv_heads": 2,
+                                         "d_model": 512, "d_ff": 520})])
+@pytest.mark.parametrize("B,S,Sk", [
+    (1, 2, 4999), (1, 2, 5000), (2, 9, 5003),   # by the number of keys
+    (1, 660, 5000), (1, 670, 5000),             # by rows: heads of 64
+    (1, 700, 5000), (1, 710, 5000)])            # heads of 128
+def test_few_rows_before_many_keys(name, kw, B, S, Sk):
+    """Portions on both sides of the rule that takes the float32 products,
+    against float32 on the CPU."""
+    from scaffold.generate import Generator
+
+    kw = {**kw, "max_seq_len": 5100, "n_layers": 2, "vocab_size": 64}
+    ref = Generator(_model(name, **kw).float())
+    gen = Generator(_model(name, **kw).cuda())
+    cpu, gpu = ref.new_cache(B, Sk + 1), gen.new_cache(B, Sk + 1)
+    for a, b in zip(cpu.k + cpu.v, gpu.k + gpu.v):
+        b.copy_(torch.randn_like(b, dtype=torch.float32))
+        a.copy_(b)
+        b[:, :, Sk:] = float("nan")
+    p0 = cpu.len = gpu.len = Sk - S
+    ids = torch.randint(0, 64, (B, S))
+    with torch.no_grad():
+        want = ref._forward_tokens(ids, cpu, p0, all_logits=True)
+        assert gen._native_step(ids.cuda(), gpu, None, p0) is not None
+        got = gen._forward_tokens(ids.cuda(), gpu, p0, all_logits=True)
+    # a bf16 stream: about ten roundings of 2^-9 a layer, independent
+    assert (got.cpu().float() - want).norm() / want.norm() < 3 * 2 ** -7
