@@ -232,7 +232,10 @@ rope_kernel(const T* x, const float* __restrict__ cos_t,
 // aligned: bound by memory.  A block has one position of one sequence, so the
 // only division is by the vectors of a head, and each lane keeps its angles
 // over the heads.  2 x 4096 positions, 40 heads of 128 (168 MB): 29 us with
-// neighbours in the caches, with a lane for a pair 98.
+// neighbours in the caches, with a lane for a pair 98.  A block's threads want
+// 256 elements at least: 100000 positions, 4 heads of 64 56 us (a lane for a
+// pair 58), 3 heads 55 (44), 1 head of 16 53 (6); and few positions are few
+// blocks: 64 with 40 heads of 128 3.7 us (3.4), 8 positions 3.6 (3.0).
 __global__ void __launch_bounds__(256)
 rope_rows_kernel(const short* x, const float* __restrict__ cos_t,
                  const float* __restrict__ sin_t, short* y, int H, int S, int D,
@@ -386,10 +389,11 @@ torch::Tensor rope_apply(torch::Tensor x, torch::Tensor cos_t, torch::Tensor sin
   };
   auto table = [](const torch::Tensor& t) { return (size_t)t.data_ptr() % 16 == 0; };
   if (total == 0) return y;
+  const long places = (long)B * S;     // a launch has fewer than 2^32 threads
   if (x.scalar_type() == torch::kBFloat16 && D % 8 == 0 && D <= 2048 &&
-      rows(xc) && rows(y) && table(cos_t) && table(sin_t) &&
-      (long)B * S < (1l << 24)) {      // a launch has fewer than 2^32 threads
-    hipLaunchKernelGGL(rope_rows_kernel, dim3((unsigned)((long)B * S)), dim3(256), 0,
+      (long)H * D >= 256 && places >= 256 && places < (1l << 24) &&
+      rows(xc) && rows(y) && table(cos_t) && table(sin_t)) {
+    hipLaunchKernelGGL(rope_rows_kernel, dim3((unsigned)places), dim3(256), 0,
                        stream, (const short*)xc.data_ptr(), cos_t.data_ptr<float>(),
                        sin_t.data_ptr<float>(), (short*)y.data_ptr(), H, S, D,
                        inverse ? 1 : 0, xs, ys);

@@ -66,13 +66,40 @@ def test_vectors_turn_as_pairs_do(B, H, S, D, inverse):
 def test_turns_any_number_of_positions(S):
     """More positions than a launch has blocks of a position each."""
     f = ops.require_ext().rope_apply
-    x = torch.randn(1, 1, S, 8, device="cuda", dtype=torch.bfloat16)
-    cos = torch.full((S, 4), 0.6, device="cuda")
-    sin = torch.full((S, 4), 0.8, device="cuda")
+    x = torch.randn(1, S, 4, 64, device="cuda", dtype=torch.bfloat16)
+    cos = torch.full((S, 32), 0.6, device="cuda")
+    sin = torch.full((S, 32), 0.8, device="cuda")
+    x = x.transpose(1, 2)
     y = f(x, cos, sin, False)
-    part = f(x[:, :, -999:].contiguous(), cos[:999], sin[:999], False)
-    assert torch.equal(y[:, :, -999:], part)
-    u, w = x[..., ::2].float(), x[..., 1::2].float()
-    # the result's rounding, half of 2^-8 of up to 1.4 times 6
-    assert (y[..., ::2].float() - (0.6 * u - 0.8 * w)).abs().max() < 2 ** -5
-    assert (y[..., 1::2].float() - (0.8 * u + 0.6 * w)).abs().max() < 2 ** -5
+    for part in (slice(0, 999), slice(S - 999, S)):
+        t = x[:, :, part]
+        assert torch.equal(y[:, :, part], f(t, cos[:999], sin[:999], False))
+        u, w = t[..., ::2].float(), t[..., 1::2].float()
+        got = y[:, :, part].float()
+        # the result's rounding, half of 2^-8 of up to 1.4 times 6
+        assert (got[..., ::2] - (0.6 * u - 0.8 * w)).abs().max() < 2 ** -5
+        assert (got[..., 1::2] - (0.8 * u + 0.6 * w)).abs().max() < 2 ** -5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,S,D", [
+    (1, 31, 300, 8), (1, 32, 255, 8), (1, 32, 256, 8), (2, 11, 130, 24),
+    (1, 40, 300, 128), (1, 1, 256, 256), (3, 2, 100, 2048), (1, 1, 256, 2056)])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_vectors_turn_as_pairs_do_on_both_sides_of_the_rule(B, H, S, D, inverse):
+    """Enough positions and elements for a block a position, and just not."""
+    f = ops.require_ext().rope_apply
+    torch.manual_seed(D)
+    cos, sin = _tables(S, D, "cuda")
+    odd = torch.randn(B, S, H, D + 1, device="cuda").bfloat16()[..., :D]
+    odd = odd.transpose(1, 2)                  # rows of odd stride: by pairs
+    x = odd.transpose(1, 2).contiguous().transpose(1, 2)
+    want = f(odd, cos, sin, inverse)
+    assert torch.equal(f(x, cos, sin, inverse), want)
+    room = torch.zeros(B, S, H + 3, D, device="cuda").bfloat16()
+    place = room[:, :, 1:H + 1].transpose(1, 2)
+    f(x, cos, sin, inverse, out=place)
+    assert torch.equal(place, want)
+    assert not room[:, :, 0].any() and not room[:, :, H + 1:].any()
+    f(x, cos, sin, inverse, out=x)             # in place
+    assert torch.equal(x, want)
