@@ -397,9 +397,13 @@ def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     where dW has few tiles: in us, library and own kernel, 3072 x 768 out of
     16384 rows 179 and 91, of 8192 81 and 57, of 4096 42 and 42; 1024 x 4096
     (64 tiles of 256 x 256) 185 and 143, 88 and 83, 51 and 57; with 100 tiles
-    8192 rows take 134 and 136."""
+    8192 rows take 134 and 136.  Tiles that are mostly empty are not worth it:
+    8192 rows, 32 x 256 19 and 31, 64 x 64 46 and 29, 64 x 16384 63 and 68, 256 x
+    16384 98 and 87."""
     n, k = dy.shape[1], x.shape[1]
-    if (x.is_cuda and dy.dtype == x.dtype == torch.bfloat16
+    small, large = min(n, k), max(n, k)
+    if (x.is_cuda and small >= 64 and (small >= 256 or large <= 8192)
+            and dy.dtype == x.dtype == torch.bfloat16
             and x.shape[0] >= 8192 and n % 8 == 0 and k % 8 == 0
             and 0 < -(-n // 256) * -(-k // 256) <= 64
             and not torch.is_grad_enabled() and not _transformed()

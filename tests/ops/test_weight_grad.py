@@ -65,3 +65,19 @@ def test_refuses_other_operands():
                   (a.t(), a.t()), (a[:0], a[:0]), (a[:, 0], a)):
         with pytest.raises(RuntimeError):
             f(dy, x)
+
+
+@pytest.mark.parametrize("N,K,own", [
+    (56, 4096, False), (4096, 56, False), (64, 8192, True), (64, 8200, False),
+    (248, 16384, False), (256, 16384, True), (8, 8, False)])
+def test_tiles_that_are_mostly_empty_stay_with_the_library(N, K, own, monkeypatch):
+    ext, calls = ops.require_ext(), []
+    made = ext.weight_grad
+    monkeypatch.setattr(ext, "weight_grad",
+                        lambda *a: calls.append(1) or made(*a))
+    torch.manual_seed(N)
+    dy = torch.randn(8192, N, device="cuda").bfloat16()
+    x = torch.randn(8192, K, device="cuda").bfloat16()
+    with torch.no_grad():
+        _close(ops._weight_grad(dy, x), dy, x)
+    assert len(calls) == own
