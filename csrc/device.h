@@ -134,6 +134,20 @@ DEVINL bf16x8 tr_read_frag(unsigned addr_q0, unsigned addr_q1) {
                                  4, 5, 6, 7);
 }
 
+// A softmax weight as three bf16 parts whose sum it is, to float32's last bit: 8
+// significand bits cut off at a time.  No part of a weight above zero is zero
+// (the smallest normal number stands in), which would make an infinite value
+// NaN.
+struct WeightParts { short hi, mid, lo; };
+
+DEVINL WeightParts weight_parts(float x) {
+  auto bits = [](float y) { return __builtin_bit_cast(unsigned, y); };
+  auto cut = [&](float y) { return __builtin_bit_cast(float, bits(y) & 0xffff0000u); };
+  const float least = x > 0.f ? 1.1754943508222875e-38f : 0.f;
+  const float y = fmaxf(x - cut(x), least), z = fmaxf(y - cut(y), least);
+  return {(short)(bits(x) >> 16), (short)(bits(y) >> 16), (short)(bits(z) >> 16)};
+}
+
 struct bf16x8_quad { bf16x8 f[4]; };
 
 DEVINL bf16x8_quad tr_read_quad(unsigned a0, unsigned a1, unsigned b0,

@@ -632,14 +632,14 @@ attn_decode_tied_kernel(AttnArgs a, const int* __restrict__ pos,
 // up to 128: both products on the matrix cores, up to 16 heads of a kv head a
 // block.  A wave takes every fourth 32 keys of its split, as the tied form
 // does with pages: keys go from memory to registers in the layout of the first
-// product's operand, values through the wave's LDS image, the weights as hi + lo
-// bf16 (against 64 bits as near as float32 products, to six digits).
+// product's operand, values through the wave's LDS image, the weights as three
+// bf16 parts, all of float32's bits.
 //
 // The vector products of four heads, 16 lanes to a key, took half the time, and
 // fetches behind each other most of the rest.  With the merge, in us, here and
 // there: 16 heads of 128 on 4, 32 rows 1000 to 4000 keys deep in chunks of 1024
-// 17.6 and 31, 64 rows 22.8 and 44, 1 row to all of 4000 13.1 and 17.5, 16 rows 26.6
-// and 46, 64 rows below 100 keys 8.9 and 19; 8 heads on 4, 1 row 12.7 and 13.8.
+// 18.1 and 31, 64 rows 23.0 and 44, 64 rows below 100 keys 8.9 and 19; 8 heads on
+// 4, 1 row to all of 4000 12.9 and 13.8.  The third part is 1 to 3 % of that.
 template <int DK>
 __global__ void __launch_bounds__(256, DK == 64 ? 3 : 2)
 attn_decode_mfma_kernel(AttnArgs a, const int* __restrict__ pos,
@@ -796,14 +796,14 @@ attn_decode_mfma_kernel(AttnArgs a, const int* __restrict__ pos,
       for (int k = 0; k < KS; ++k) sc[t] = N::mma(kr[t][k], qf[k], sc[t]);
     }
     if (u + 4 < ue) fetch(u + 4, page_of(it + 1));
-    const float d0 = slope2 * (float)(j0 + 4 * lg - p);
+    const float d0 = (float)(j0 + 4 * lg - p);
     float mx = NEG;
     #pragma unroll
     for (int t = 0; t < 2; ++t)
       #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int j = j0 + 16 * t + 4 * lg + r;
-        float x = sc[t][r] * scale2 + fmaf(slope2, (float)(16 * t + r), d0);
+        float x = fmaf(slope2, d0 + (float)(16 * t + r), sc[t][r] * scale2);
         if (edge && (j > p || j < cs)) x = -INFINITY;
         sc[t][r] = x;
         mx = fmaxf(mx, x);
@@ -813,17 +813,20 @@ attn_decode_mfma_kernel(AttnArgs a, const int* __restrict__ pos,
     const float mn = fmaxf(m, mx), al = __builtin_amdgcn_exp2f(m - mn);
     m = mn;
     ls *= al;
-    bf16x8 hi, lo;
+    bf16x8 hi, mid, lo;
+    float part = 0.f;
     #pragma unroll
     for (int t = 0; t < 2; ++t)
       #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float e = __builtin_amdgcn_exp2f(sc[t][r] - mn);
-        const short eh = cvt_bf16(e);
-        ls += e;
-        hi[4 * t + r] = eh;
-        lo[4 * t + r] = cvt_bf16(e - bf2f(eh));
+        part += e;
+        const WeightParts c = weight_parts(e);
+        hi[4 * t + r] = c.hi;
+        mid[4 * t + r] = c.mid;
+        lo[4 * t + r] = c.lo;
       }
+    ls += part;
     #pragma unroll
     for (int i = 0; i < DT; ++i) o[i] *= al;
     // the wave reads what its own lanes wrote; LDS keeps their order
@@ -836,6 +839,7 @@ attn_decode_mfma_kernel(AttnArgs a, const int* __restrict__ pos,
       };
       const bf16x8 v = tr_read_frag(at(0), at(1));
       o[i] = N::mma(v, hi, o[i]);
+      o[i] = N::mma(v, mid, o[i]);
       o[i] = N::mma(v, lo, o[i]);
     }
     asm volatile("" ::: "memory");

@@ -330,7 +330,8 @@ Tensor attend(AttnArgs& a, const Tensor& qkv, const Tensor& pos,
     // merge takes at most 64 splits.  As stored, on the matrix cores, one to a
     // compute unit: 16 heads of 128 on 4, 64 rows below 100 keys 8.9 us, which
     // need no merge, with two 13.9; 1000 to 4000 keys deep in chunks of 1024, 64
-    // rows 22.8, with two 24.4 and four 28.9, 32 rows 17.6, 16.5 and 22.9.
+    // rows 22.8, with two 24.4 and four 28.9, 32 rows 17.6, 16.5 and 22.9 (weights
+    // in two parts).
     const long hg = a.H / a.G;
     const bool mfma = !f32 && lm_attn_decode_mfma(a);
     const long hc = mfma ? 16 : hg <= 2 ? hg : 4;
