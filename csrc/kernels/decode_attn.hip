@@ -255,12 +255,13 @@ DEVINL f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) {
 // operand, values through an LDS image of the wave's own, whose transpose reads
 // make the value product's: no barrier in the loop, and the next tile's rows
 // are on their way while one is used.  The 16 columns of a matrix instruction
-// are 8 heads twice: the weights enter the value product as two bf16 parts, cut
-// and rest, 16 of float32's 24 significand bits, the rests in the second 8
-// columns.  Of 64 rows, 32 heads of 128 on 8, 1024 to 4096 keys deep, 671 MB:
-// 133 us, 5.1 TB/s (159 with both products on the vector unit, which took half
-// of the time there); one head to a kv head is left to it: 64 rows of 12 heads
-// of 64 to 1024 keys 27.1 and 28.2 us, 1 row to 512 5.4 and 6.9.
+// are 8 heads twice: the weights enter the value product as three bf16 parts, all
+// of float32's bits, the second ones in the second 8 columns, the third ones by
+// an instruction of their own (1 to 5 % of the time).  Of 64 rows, 32 heads of 128
+// on 8, 1024 to 4096 keys deep, 671 MB: 133 us, 5.1 TB/s (159 with both products
+// on the vector unit, which took half of the time there); one head to a kv head
+// is left to it: 64 rows of 12 heads of 64 to 1024 keys 27.1 and 28.2 us, 1 row to
+// 512 5.4 and 6.9.
 constexpr int R = 8;                    // query heads of a block
 constexpr int WAVES = 4;                // of a block
 constexpr int TILE = 32;                // keys of a wave at a time
@@ -422,26 +423,30 @@ decode_group_kernel(DecodeArgs a) {
     }
     // weights of the keys 16 t + 4 lg + r; the value product's sum runs over
     // the keys in this order
-    bf16x8 e;
+    bf16x8 e, f;
+    float part = 0.f;
     #pragma unroll
     for (int t = 0; t < 2; ++t)
       #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float x = __builtin_amdgcn_exp2f(sc[t][r] - m);
-        sum += x;
-        const float cut = __builtin_bit_cast(
-            float, __builtin_bit_cast(unsigned, x) & 0xffff0000u);
-        // a rest of zero would make an infinite value NaN
-        const float rest = x > 0.f ? fmaxf(x - cut, 1.1754943508222875e-38f) : 0.f;
-        e[4 * t + r] = f2bf(lr < R ? cut : rest);
+        part += x;
+        const WeightParts c = weight_parts(x);
+        e[4 * t + r] = lr < R ? c.hi : c.mid;
+        // next to nothing in the columns that have no third part
+        f[4 * t + r] = lr < R ? c.lo : x > 0.f ? 0x0080 : 0;
       }
+    sum += part;
     #pragma unroll
-    for (int t = 0; t < DT; ++t)
-      o[t] = mma(tr_read_frag(tr + 32 * t, tr + 32 * t + 16 * ROW * 2), e, o[t]);
+    for (int t = 0; t < DT; ++t) {
+      const bf16x8 v = tr_read_frag(tr + 32 * t, tr + 32 * t + 16 * ROW * 2);
+      o[t] = mma(v, e, o[t]);
+      o[t] = mma(v, f, o[t]);
+    }
   }
   sum += __shfl_xor(sum, 16, 64);
   sum += __shfl_xor(sum, 32, 64);
-  // cuts and rests, then waves
+  // the parts, then waves
   float* mine = (float*)image;              // [R][D + 2]
   #pragma unroll
   for (int t = 0; t < DT; ++t) {

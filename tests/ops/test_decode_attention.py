@@ -192,6 +192,35 @@ def test_heads_that_share_keys(D, H, G, L):
         k[b, :, p:] = float("nan")
         v[b, :, p:] = float("nan")
     got = ops.require_ext().decode_attention(qkv, k, v, pos, None, None, None, H)
-    # float32 sums and weights of 16 significand bits; one rounding of the
-    # result is at most 2^-9 of each value
+    # float32 sums and weights; one rounding of the result is at most 2^-9 of
+    # each value
+    assert (got.double() - want).norm() / want.norm() < 2 ** -9
+
+
+@pytest.mark.parametrize("D,H,G", [(64, 1, 1), (64, 2, 1), (64, 3, 1), (128, 8, 2),
+                                   (32, 8, 1)])
+def test_weights_keep_the_bits_of_float32(D, H, G):
+    """Two keys whose scores differ by a last bit, below a third one's: what is
+    left of their values, 1 and -1, is the difference of two weights."""
+    from scaffold import ops
+
+    torch.manual_seed(0)
+    R = 256
+    q = torch.rand(R, device="cuda") / 4 + 0.25
+    near = (torch.rand(R, device="cuda") + 1).bfloat16()
+    best = (near + 8 + 24 * torch.rand(R, device="cuda")).bfloat16()
+    qkv = torch.zeros(R, H + 2 * G, D, device="cuda").bfloat16()
+    k, v = (torch.zeros(R, G, 3, D, device="cuda").bfloat16() for _ in range(2))
+    qkv[:, :H, 0] = q[:, None].bfloat16()
+    qkv[:, H:H + G, 0] = (near * (1 + 2 ** -7))[:, None]
+    qkv[:, H + G:] = 1
+    k[:, :, 0, 0] = best[:, None]
+    k[:, :, 1, 0] = near[:, None]
+    v[:, :, 1] = -1
+    pos = torch.full((R,), 2, device="cuda")
+    want = _reference(qkv.view(R, -1), k, v, pos, None, H)[0]
+    got = ops.require_ext().decode_attention(qkv.view(R, -1), k, v, pos, None, None,
+                                             None, H)
+    # one rounding of the result is at most 2^-9 of it; 16 bits of the weights
+    # alone would leave twice that of their difference
     assert (got.double() - want).norm() / want.norm() < 2 ** -9
