@@ -88,7 +88,7 @@ attn_fwd_mfma_kernel(const short* __restrict__ q, const short* __restrict__ k,
   __shared__ __attribute__((aligned(16))) short k0[64 * D], k1[64 * D];
   __shared__ __attribute__((aligned(16))) short v0[64 * D], v1[64 * D];
 
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // 0..7
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // 0..3
   const int l = threadIdx.x & 63;
   const int lq = l & 31;
   const int half = l >> 5;
@@ -246,8 +246,7 @@ attn_fwd_mfma_kernel(const short* __restrict__ q, const short* __restrict__ k,
         #pragma unroll
         for (int j = 0; j < 8; ++j) {
           e[j] = __builtin_amdgcn_exp2f(sacc[sub][8 * s + j] - m_run);
-          if constexpr (SPLIT) l_run += e[j];    // of this lane's keys, until the end
-          else psum += e[j];
+          psum += e[j];
         }
         #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -268,7 +267,9 @@ attn_fwd_mfma_kernel(const short* __restrict__ q, const short* __restrict__ k,
           w[3] = ry[1];
         }
       }
-    if constexpr (!SPLIT) {
+    if constexpr (SPLIT) {
+      l_run += psum;                       // of this lane's keys, until the end
+    } else {
       const float other = other_half(psum);
       const float grown = fmaf(l_run, alpha, psum) + other, same = l_run + (psum + other);
       l_run = alpha < 0.f ? same : grown;

@@ -583,6 +583,7 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
         #pragma unroll
         for (int r = 0; r < 16; ++r) o[i][r] *= al;
     }
+    float ps = 0.f;
     #pragma unroll
     for (int sub = 0; sub < 2; ++sub)
       #pragma unroll
@@ -591,7 +592,7 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
         #pragma unroll
         for (int j = 0; j < 8; ++j) {
           e[j] = __builtin_amdgcn_exp2f(s[sub][8 * x + j] - m_run);
-          l_run += e[j];
+          ps += e[j];
         }
         union { unsigned u[4]; bf16x8 v; } p, q;
         #pragma unroll
@@ -603,6 +604,7 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
         hi[sub][x] = p.v;
         lo[sub][x] = q.v;
       }
+    l_run += ps;
   };
   int now = tab[0], next = tab[min(1, n - 1)];     // pages' places
   auto page = [&](auto odd, auto begin, int it) INLINE {
