@@ -184,17 +184,19 @@ bool few(long rows, long depth) {
   return rows <= 16 || (rows <= 64 && rows * depth <= 96 * 1024);
 }
 
-// Few rows of few heads before many keys: the flash kernel has a block for 128
-// rows of a head, which walks the keys alone, 23 us per 1024 of them with heads
-// of 128 and 17 with 64, while the products of a library, in float32 over keys
-// and values spread to all heads, fill the chip.  In us, flash and library:
-// 32 heads of 128, 2 rows, 8192 keys 188 and 232, 33 rows 193 and 330, 64 heads
-// 187 and 452 (7 us a head, and as much again for 75 rows); 12 heads of 64, 2
-// rows, 4096 keys 70 and 96, 8192 136 and 112, 16384 267 and 126, 64 rows 279
-// and 214, 96 heads 273 and 467.
+// Few rows of few heads before many keys: products of a library, in float32 over
+// keys and values spread to all heads.  The line is where the flash kernel, while
+// it had blocks of 256 rows, took as long; behind it weights are held in float32,
+// of which the flash kernel's two parts keep 16 bits, and that stays so, although
+// its blocks of 128 rows walk 1024 keys in 23 us with heads of 128 and 17 with 64
+// and are ahead again for some.  In us, flash and library: 32 heads of 128, 2 rows,
+// 8192 keys 188 and 232, 33 rows 193 and 330, 64 heads 187 and 452; 12 heads of 64,
+// 2 rows, 8192 keys 136 and 112, 16384 267 and 126, 64 rows 279 and 214, 96 heads
+// 273 and 467.  Below 5000 keys what the step's one call saves is more than the
+// difference.
 bool few_before_many(long heads, long S, long Sk, long D) {
-  return Sk >= 6500 && (D == 64 ? heads * (S + 35) < 1650
-                                : heads * (S + 75) < 1950);
+  return Sk >= 5000 && (D == 64 ? heads * (S + 20) < 2750
+                                : heads * (S + 45) < 3000);
 }
 
 // q (B, H, S, D), k, v (B, G, Sk, D) -> (B, S, H, D): causal, all in float32

@@ -326,3 +326,24 @@ def test_few_rows_before_many_keys(name, kw, B, S, Sk):
         got = gen._forward_tokens(ids.cuda(), gpu, p0, all_logits=True)
     # a bf16 stream: about ten roundings of 2^-9 a layer, independent
     assert (got.cpu().float() - want).norm() / want.norm() < 3 * 2 ** -7
+
+
+@pytest.mark.parametrize("name,kw,S,Sk,products", [
+    ("gpt2", {}, 2, 4999, False), ("gpt2", {}, 2, 5000, True),
+    ("gpt2", {}, 667, 5000, True), ("gpt2", {}, 668, 5000, False),
+    ("llama", {"n_kv_heads": 2, "d_model": 512, "d_ff": 520}, 704, 5000, True),
+    ("llama", {"n_kv_heads": 2, "d_model": 512, "d_ff": 520}, 705, 5000, False)])
+def test_which_rows_take_the_float32_products(name, kw, S, Sk, products):
+    """The rule itself, by the library calls that a step makes."""
+    from scaffold.generate import Generator
+
+    gen = Generator(_model(name, **kw, max_seq_len=5100, n_layers=2,
+                           vocab_size=64).cuda())
+    cache = gen.new_cache(1, Sk + 1)
+    for t in cache.k + cache.v:
+        t.zero_()
+    ids = torch.zeros(1, S, dtype=torch.int64, device="cuda")
+    with torch.no_grad(), torch.autograd.profiler.profile() as prof:
+        assert gen._native_step(ids, cache, None, Sk - S, all_logits=True) is not None
+    calls = [e.key for e in prof.key_averages()]
+    assert ("aten::softmax" in calls) == products
