@@ -33,6 +33,7 @@ struct DecodeArgs {
   float *part;                   // [B*H][spans][D + 2]
   short *out;                    // [B][H*D]
   int B, H, G, spans, span, waves;
+  int matrix;                    // decode_group_kernel
   int rows, eager;               // of a cache; decode_group_kernel
   long limit;                    // positions that exist: cache and tables
   float scale2;                  // of scores, times log2(e)
@@ -90,22 +91,23 @@ template <int N> DEVINL float group_sum(float x) {
   return x;
 }
 
-// Heads with keys of their own.  A lane has 8 columns of a key, 16 lanes a key
-// of 128; a cached row goes from memory to the registers that use it, and each
-// group of lanes keeps a running maximum of its own until the end.
-// D: head size; WAVES: of a block
-template <int D, int WAVES>
+// One or two query heads to a kv head.  A lane has 8 columns of a key, 16 lanes a
+// key of 128; a cached row goes from memory to the registers that use it, and
+// each group of lanes keeps a running maximum of its own until the end.
+// D: head size; N: query heads of a block; WAVES: of a block
+template <int D, int N, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
 decode_head_kernel(DecodeArgs a) {
   constexpr int LPK = D / 8;            // lanes per key
   constexpr int KPI = 64 / LPK;         // keys per load of a wave
   constexpr int U = 4;                  // loads in flight
   constexpr int TILE = KPI * U;
-  __shared__ float sm[WAVES][2], so[WAVES][D];
+  __shared__ float sm[WAVES][N][2], so[WAVES][N][D];
 
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int g = l / LPK, c = l % LPK;   // key within a load, column chunk
-  const int s = blockIdx.x, b = blockIdx.y / a.H, h = blockIdx.y % a.H;
+  const int s = blockIdx.x, b = blockIdx.y / a.G, kv = blockIdx.y % a.G;
+  const int h0 = kv * N;
 
   const long pos = a.pos[(long)b * a.pos_step];
   const bool on = (!a.active || a.active[b]) && pos >= 0 && pos < a.limit;
@@ -113,8 +115,8 @@ decode_head_kernel(DecodeArgs a) {
   if (!on) {
     // nothing is written for the row; a place outside the cache shows
     if (s == 0 && w == 0)
-      for (int i = l; i < D; i += 64)
-        a.out[((long)b * a.H + h) * D + i] = !a.active || a.active[b] ? 0x7fc0 : 0;
+      for (int i = l; i < N * D; i += 64)
+        a.out[((long)b * a.H + h0) * D + i] = !a.active || a.active[b] ? 0x7fc0 : 0;
     return;
   }
   const int p = (int)pos;
@@ -122,8 +124,8 @@ decode_head_kernel(DecodeArgs a) {
   const int hi = min(p, lo + a.span);   // cached keys [lo, hi)
   const bool own = p < lo + a.span;     // the new key's place is here
 
-  short* kc = a.k + b * a.sb + h * a.sh + 8 * c;
-  short* vc = a.v + b * a.sb + h * a.sh + 8 * c;
+  short* kc = a.k + b * a.sb + kv * a.sh + 8 * c;
+  short* vc = a.v + b * a.sb + kv * a.sh + 8 * c;
 
   // the next tile's rows are on their way while one is used; places behind
   // the last key repeat it and do not count
@@ -141,12 +143,17 @@ decode_head_kernel(DecodeArgs a) {
   if (j < hi) fetch(k0, v0, j);
 
   const short* row = a.qkv + (long)b * a.ldq;
-  const bf16x8 turn = turned<D>(a, row + h * D, c, p);
-  float q[8], m = NONE, sum = 0.f, o[8];
+  float q[N][8], m[N], sum[N], o[N][8];
   #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    q[i] = bf2f(turn[i]) * a.scale2;
-    o[i] = 0.f;
+  for (int r = 0; r < N; ++r) {
+    const bf16x8 turn = turned<D>(a, row + (h0 + r) * D, c, p);
+    m[r] = NONE;
+    sum[r] = 0.f;
+    #pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      q[r][i] = bf2f(turn[i]) * a.scale2;
+      o[r][i] = 0.f;
+    }
   }
   auto take = [&](const bf16x8 (&kk)[U], bf16x8 (&vv)[U], int j0) {
     // no weight makes an infinite value nothing, so those of the repeated
@@ -156,29 +163,40 @@ decode_head_kernel(DecodeArgs a) {
       for (int u = 0; u < U; ++u)
         if (j0 + u * KPI + g >= hi) vv[u] = bf16x8{};
     }
-    float sc[U], t = m;
+    float sc[U][N];
     #pragma unroll
     for (int u = 0; u < U; ++u) {
-      float d = 0.f;
+      const bool see = j0 + u * KPI + g < hi;
       #pragma unroll
-      for (int i = 0; i < 8; ++i) d = fmaf(q[i], bf2f(kk[u][i]), d);
-      d = group_sum<LPK>(d);
-      sc[u] = j0 + u * KPI + g < hi ? d : NONE;
-      t = fmaxf(t, sc[u]);
+      for (int r = 0; r < N; ++r) {
+        float d = 0.f;
+        #pragma unroll
+        for (int i = 0; i < 8; ++i) d = fmaf(q[r][i], bf2f(kk[u][i]), d);
+        d = group_sum<LPK>(d);
+        sc[u][r] = see ? d : NONE;
+      }
     }
-    const float f = __builtin_amdgcn_exp2f(m - t);
-    m = t;
-    sum *= f;
     #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] *= f;
-    #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      // a score of NONE is no key, also where the maximum is none yet
-      const float e = sc[u] <= NONE ? 0.f : __builtin_amdgcn_exp2f(sc[u] - m);
-      sum += e;
+    for (int r = 0; r < N; ++r) {
+      float t = m[r];
       #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = fmaf(e, bf2f(vv[u][i]), o[i]);
+      for (int u = 0; u < U; ++u) t = fmaxf(t, sc[u][r]);
+      const float f = __builtin_amdgcn_exp2f(m[r] - t);
+      m[r] = t;
+      sum[r] *= f;
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) o[r][i] *= f;
     }
+    #pragma unroll
+    for (int u = 0; u < U; ++u)
+      #pragma unroll
+      for (int r = 0; r < N; ++r) {
+        // a score of NONE is no key, also where the maximum is none yet
+        const float e = sc[u][r] <= NONE ? 0.f : __builtin_amdgcn_exp2f(sc[u][r] - m[r]);
+        sum[r] += e;
+        #pragma unroll
+        for (int i = 0; i < 8; ++i) o[r][i] = fmaf(e, bf2f(vv[u][i]), o[r][i]);
+      }
   };
   for (; j < hi; j += 2 * WAVES * TILE) {
     const int next = j + WAVES * TILE;
@@ -190,57 +208,65 @@ decode_head_kernel(DecodeArgs a) {
   }
   // the new token, by the last wave's first group of lanes
   if (own && w == WAVES - 1) {
-    const bf16x8 nk = turned<D>(a, row + (a.H + h) * D, c, p);
-    bf16x8 nv = *(const bf16x8*)(row + (2 * a.H + h) * D + 8 * c);
+    const bf16x8 nk = turned<D>(a, row + (a.H + kv) * D, c, p);
+    bf16x8 nv = *(const bf16x8*)(row + (a.H + a.G + kv) * D + 8 * c);
     if (g == 0) {
       *(bf16x8*)(kc + (long)p * a.ss) = nk;
       *(bf16x8*)(vc + (long)p * a.ss) = nv;
     } else {
       nv = bf16x8{};
     }
-    float d = 0.f;
     #pragma unroll
-    for (int i = 0; i < 8; ++i) d = fmaf(q[i], bf2f(nk[i]), d);
-    d = group_sum<LPK>(d);
-    if (g != 0) d = NONE;
-    const float t = fmaxf(m, d), f = __builtin_amdgcn_exp2f(m - t);
-    const float e = d <= NONE ? 0.f : __builtin_amdgcn_exp2f(d - t);
-    m = t;
-    sum = sum * f + e;
-    #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = o[i] * f + e * bf2f(nv[i]);
+    for (int r = 0; r < N; ++r) {
+      float d = 0.f;
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) d = fmaf(q[r][i], bf2f(nk[i]), d);
+      d = group_sum<LPK>(d);
+      if (g != 0) d = NONE;
+      const float t = fmaxf(m[r], d), f = __builtin_amdgcn_exp2f(m[r] - t);
+      const float e = d <= NONE ? 0.f : __builtin_amdgcn_exp2f(d - t);
+      m[r] = t;
+      sum[r] = sum[r] * f + e;
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) o[r][i] = o[r][i] * f + e * bf2f(nv[i]);
+    }
   }
   // groups of lanes, then waves
   #pragma unroll
-  for (int x = LPK; x < 64; x *= 2) {
-    const float mo = __shfl_xor(m, x, 64), t = fmaxf(m, mo);
-    const float f = __builtin_amdgcn_exp2f(m - t);
-    const float fo = __builtin_amdgcn_exp2f(mo - t);
-    sum = sum * f + __shfl_xor(sum, x, 64) * fo;
+  for (int r = 0; r < N; ++r) {
     #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = o[i] * f + __shfl_xor(o[i], x, 64) * fo;
-    m = t;
-  }
-  if (g == 0) {
-    #pragma unroll
-    for (int i = 0; i < 8; ++i) so[w][8 * c + i] = o[i];
-    if (c == 0) {
-      sm[w][0] = m;
-      sm[w][1] = sum;
+    for (int x = LPK; x < 64; x *= 2) {
+      const float mo = __shfl_xor(m[r], x, 64), t = fmaxf(m[r], mo);
+      const float f = __builtin_amdgcn_exp2f(m[r] - t);
+      const float fo = __builtin_amdgcn_exp2f(mo - t);
+      sum[r] = sum[r] * f + __shfl_xor(sum[r], x, 64) * fo;
+      #pragma unroll
+      for (int i = 0; i < 8; ++i)
+        o[r][i] = o[r][i] * f + __shfl_xor(o[r][i], x, 64) * fo;
+      m[r] = t;
+    }
+    if (g == 0) {
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) so[w][r][8 * c + i] = o[r][i];
+      if (c == 0) {
+        sm[w][r][0] = m[r];
+        sm[w][r][1] = sum[r];
+      }
     }
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < D; d += 64 * WAVES) {
+  for (int i = threadIdx.x; i < N * D; i += 64 * WAVES) {
+    const int r = i / D, d = i % D;
     float t = NONE, den = 0.f, num = 0.f;
     #pragma unroll
-    for (int x = 0; x < WAVES; ++x) t = fmaxf(t, sm[x][0]);
+    for (int x = 0; x < WAVES; ++x) t = fmaxf(t, sm[x][r][0]);
     #pragma unroll
     for (int x = 0; x < WAVES; ++x) {
-      const float f = __builtin_amdgcn_exp2f(sm[x][0] - t);
-      den += f * sm[x][1];
-      num += f * so[x][d];
+      const float f = __builtin_amdgcn_exp2f(sm[x][r][0] - t);
+      den += f * sm[x][r][1];
+      num += f * so[x][r][d];
     }
-    put<D>(a, b, h, s, d, t, den, num);
+    put<D>(a, b, h0 + r, s, d, t, den, num);
   }
 }
 
@@ -260,8 +286,8 @@ DEVINL f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) {
 // an instruction of their own (1 to 5 % of the time).  Of 64 rows, 32 heads of 128
 // on 8, 1024 to 4096 keys deep, 671 MB: 133 us, 5.1 TB/s (159 with both products
 // on the vector unit, which took half of the time there); one head to a kv head
-// is left to it: 64 rows of 12 heads of 64 to 1024 keys 27.1 and 28.2 us, 1 row to
-// 512 5.4 and 6.9.
+// is left to it, 64 rows of 12 heads of 64 to 1024 keys 27.1 and 28.2 us, 1 row to
+// 512 5.4 and 6.9, and two where decode_attention() says.
 constexpr int R = 8;                    // query heads of a block
 constexpr int WAVES = 4;                // of a block
 constexpr int TILE = 32;                // keys of a wave at a time
@@ -501,16 +527,26 @@ decode_merge_kernel(DecodeArgs a) {
   a.out[bh * D + d] = f2bf(num / den);
 }
 
+template <int D, int N>
+void launch_heads(const DecodeArgs& a, hipStream_t st) {
+  const dim3 grid(a.spans, a.B * a.G);
+  if (a.waves == 8)
+    hipLaunchKernelGGL((decode_head_kernel<D, N, 8>), grid, dim3(512), 0, st, a);
+  else
+    hipLaunchKernelGGL((decode_head_kernel<D, N, 4>), grid, dim3(256), 0, st, a);
+}
+
 template <int D>
 void launch(const DecodeArgs& a, hipStream_t st) {
-  const int chunks = (a.H / a.G + R - 1) / R;
-  const dim3 grid(a.spans, a.B * a.G * chunks);
-  if (a.H != a.G)
-    hipLaunchKernelGGL((decode_group_kernel<D>), grid, dim3(64 * WAVES), 0, st, a);
-  else if (a.waves == 8)
-    hipLaunchKernelGGL((decode_head_kernel<D, 8>), grid, dim3(512), 0, st, a);
-  else
-    hipLaunchKernelGGL((decode_head_kernel<D, 4>), grid, dim3(256), 0, st, a);
+  if (a.matrix) {
+    const int chunks = (a.H / a.G + R - 1) / R;
+    hipLaunchKernelGGL((decode_group_kernel<D>), dim3(a.spans, a.B * a.G * chunks),
+                       dim3(64 * WAVES), 0, st, a);
+  } else if (a.H == a.G) {
+    launch_heads<D, 1>(a, st);
+  } else {
+    launch_heads<D, 2>(a, st);
+  }
   if (a.spans > 1)
     hipLaunchKernelGGL((decode_merge_kernel<D>), dim3(a.B * a.H),
                        dim3(D < 64 ? 64 : D), 0, st, a);
@@ -591,26 +627,43 @@ torch::Tensor decode_attention(torch::Tensor qkv, torch::Tensor k,
   auto out = torch::empty({a.B, (long)a.H * D}, qkv.options());
   a.out = (short*)out.data_ptr();
   if (a.B == 0) return out;
-  // Spans of whole 64s.  Heads with keys of their own: with 256 of them or
-  // more, 512 blocks of 4 waves fill the chip (64 rows of 12 heads of 64 to
-  // 1024 deep: 27 us); with fewer, 256 blocks of 8 waves.  A cache that 8 waves
-  // walk in 4 steps is one span, which saves the merge (8 rows of 12 heads of
-  // 64 to 1024: 8.8 us, 10.0 us in two spans).
-  // Heads that share keys: a compute unit's misses bound it to 50 KB a
-  // microsecond, so up to 256 blocks share the keys, if that saves more than
-  // the merge's 5 us; in us, one span and several: 1 row of 8 kv heads to
-  // 4096 43 and 16, 4 rows to 1000 17.3 and 13.0, 8 rows to 2048 30 and 21, 16
-  // rows to 1000 19.9 and 19.3, 32 rows to 300 13.7 and 18.0.
-  const int chunks = (a.H / a.G + R - 1) / R;
+  const int rep = a.H / a.G, chunks = (rep + R - 1) / R;
   const int pairs = a.B * a.G * chunks, full = (L + 63) / 64;
+  // Two heads to a kv head use a quarter of the matrix instruction's columns, and
+  // the vector kernel's 8 waves walk a span faster than the other's 4; in us,
+  // vector and matrix kernel: heads of 128, 64 pairs of a row and a kv head, caches
+  // of 128 5.7 and 6.7, 1024 10.5 and 11.5, 512 pairs of 128 7.3 and 9.3; heads of
+  // 64, 64 pairs of 128 5.6 and 5.1, of 1024 9.5 and 10.6; heads of 32, 64 pairs of
+  // 128 5.4 and 4.4, of 1024 7.4 and 9.1, 512 of 4096 32.1 and 32.8.  The matrix
+  // kernel's where it starts sooner, or its products are what counts: heads of
+  // 128, 256 pairs of 1024 21.6 and 19.5, 512 of 4096 130 and 125; of 64, 256 of 1024
+  // 15.1 and 11.7.
+  if (rep == 2)
+    a.matrix = D == 128 ? L > 256 && pairs >= 192 && (long)pairs * L >= 128 * 1024
+                        : L <= 256 || (D == 64 && pairs >= 256);
+  else
+    a.matrix = rep > 2;
+  // Spans of whole 64s.  Vector kernel: with 256 pairs or more, 512 blocks of 4
+  // waves fill the chip (64 rows of 12 heads of 64 to 1024 deep: 27 us); with
+  // fewer, 256 blocks of 8 waves.  A cache that 8 waves walk in 4 steps is one
+  // span, which saves the merge (8 rows of 12 heads of 64 to 1024: 8.8 us, 10.0 us
+  // in two spans); of two heads, what 4 waves do as well (32 rows of 8 pairs of
+  // 128, 128 deep: 6.0 and 8.8).
+  // Matrix kernel: a compute unit's misses bound it to 50 KB a microsecond (what
+  // 32 keys cost aside, which rows of 32 do not come below), so up to 256 blocks
+  // share the keys, if that saves more than the merge's 5 us; in us, one span and
+  // several: 1 row of 8 kv heads to 4096 43 and 16, 4 rows to 1000 17.3 and 13.0, 8
+  // rows to 2048 30 and 21, 16 rows to 1000 19.9 and 19.3, 32 rows to 300 13.7 and
+  // 18.0; 4 heads of 32, 16 rows to 4096 24.8 and 18.7.
   int want;
-  if (a.H == a.G) {
-    a.waves = pairs >= 256 ? 4 : 8;
-    want = a.waves == 8 && L <= 65536 / D ? 1
-        : std::max(1, std::min(full, (a.waves == 4 ? 512 : 256) / pairs));
-  } else {
+  if (a.matrix) {
     want = std::max(1, std::min((full + 1) / 2, 256 / pairs));
-    if (4l * L * D * (want - 1) <= 256l * 1024 * want) want = 1;
+    if (4l * L * std::max(D, 64) * (want - 1) <= 256l * 1024 * want) want = 1;
+  } else {
+    a.waves = pairs >= 256 ? 4 : 8;
+    want = std::max(1, std::min(rep == 1 ? full : (full + 1) / 2,
+                                (a.waves == 4 ? 512 : 256) / pairs));
+    if ((a.waves == 8 && L <= 65536 / D) || (rep == 2 && L <= 32768 / D)) want = 1;
   }
   a.span = (full + want - 1) / want * 64;
   a.spans = (L + a.span - 1) / a.span;

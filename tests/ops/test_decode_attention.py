@@ -224,3 +224,32 @@ def test_weights_keep_the_bits_of_float32(D, H, G):
     # one rounding of the result is at most 2^-9 of it; 16 bits of the weights
     # alone would leave twice that of their difference
     assert (got.double() - want).norm() / want.norm() < 2 ** -9
+
+
+@pytest.mark.parametrize("D,B,G,L", [
+    (32, 3, 2, 256), (32, 3, 2, 257), (32, 64, 4, 1024), (32, 64, 4, 1100),
+    (64, 3, 2, 256), (64, 3, 2, 257), (64, 51, 5, 300), (64, 64, 4, 300),
+    (128, 3, 2, 256), (128, 64, 4, 256), (128, 64, 4, 511), (128, 64, 4, 512),
+    (128, 2, 2, 2100)])
+def test_two_heads_to_a_kv_head(D, B, G, L):
+    """Sizes on both sides of where the matrix kernel takes over, and of where
+    one span does."""
+    from scaffold import ops
+
+    torch.manual_seed(L)
+    H = 2 * G
+    qkv = torch.randn(B, (H + 2 * G) * D, device="cuda").bfloat16()
+    k, v = (torch.randn(B, G, L, D, device="cuda").bfloat16() for _ in range(2))
+    pos = torch.randint(0, L, (B,), device="cuda")
+    pos[0], pos[-1] = L - 1, 0
+    want, wk, wv = _reference(qkv, k, v, pos, None, H)
+    for b, p in enumerate(pos.tolist()):
+        k[b, :, p:] = float("nan")
+        v[b, :, p:] = float("nan")
+    got = ops.require_ext().decode_attention(qkv, k, v, pos, None, None, None, H)
+    # float32 sums and weights; one rounding of the result is at most 2^-9 of
+    # each value
+    assert (got.double() - want).norm() / want.norm() < 2 ** -9
+    for b, p in enumerate(pos.tolist()):
+        assert torch.equal(k[b, :, p].double(), wk[b, :, p])
+        assert torch.equal(v[b, :, p].double(), wv[b, :, p])
