@@ -413,9 +413,12 @@ DEVINL int swapped(int row) {
 // first loads, each behind another: 16 heads of 128 on 4, 8192 tokens in chunks
 // of 1024 (8.5 pages a block) 92 us, against 119 with pages through registers
 // and values behind their own page's softmax; two prompts of 1000 behind 1500
-// 48 against 60.
+// 48 against 60.  Blocks of one head as well: 9 heads of 64 on 3 with values of 128,
+// 8192 tokens in chunks of 1024, 95 against 121, 3 heads of 64 on 1 39 against 50, 5
+// heads of 128 97 against 129; bounds that ask for more waves than LDS has room for
+// are not kept, and 277 registers leave one wave to a SIMD (131, 43, 96).
 template <int DK, int DV, int HPB, bool BIAS>
-__global__ void __launch_bounds__(HPB * 128, 4 / HPB)
+__global__ void __launch_bounds__(HPB * 128, 2)
 attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
   constexpr int NT = HPB * 128;
   constexpr int NSL = DK / 16, NDT = DV / 32;
