@@ -396,7 +396,7 @@ c10::optional<torch::Tensor> serve_step(
     a.w = (const short*)w.data_ptr();
     a.bias = b ? (const short*)b->data_ptr() : nullptr;
     a.ldx = a.K;
-    const long parts = T <= 64 ? skinny_parts(a) : 0;
+    const long parts = T <= 64 && skinny_split_pays(a) ? skinny_parts(a) : 0;
     if (parts) {
       pending = torch::empty({parts, T, W}, opt.dtype(torch::kFloat32));
       skinny_split(a, pending.data_ptr<float>(), parts, st);

@@ -29,4 +29,5 @@ void skinny_gemm(const SkinnyArgs& a, SkinnyAct act, hipStream_t st);
 // blocks whose sums, (parts, M, N) float32 with the bias in the first, the
 // reader adds.  0: not what it is for.
 long skinny_parts(const SkinnyArgs& a);
+bool skinny_split_pays(const SkinnyArgs& a);   // against whole depths, the library
 void skinny_split(const SkinnyArgs& a, float* sums, long parts, hipStream_t st);

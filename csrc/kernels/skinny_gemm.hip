@@ -393,6 +393,20 @@ long skinny_parts(const SkinnyArgs& a) {
   return (chunks + per - 1) / per;
 }
 
+// Where w has many rows, the blocks that take whole depths, or the library's tiles,
+// fill the chip.  A step of two layers, whole (or the library) and split, in us:
+// width 5120, feed-forward 13824, 17 rows 371 and 342, 64 rows 378 and 366; 6144 and
+// 6144, 16 rows 315 and 292, 17 rows 279 and 286, 64 rows 318 and 327; 7168 and 8192,
+// 16 rows 390 and 366; 8192 and 8192, 9 rows 381 and 404, 64 rows 404 and 432; 12288
+// and 8192, 64 rows 683 and 786.  Depths of three times the rows of w and more are
+// worth it a little longer: 6144 and 20480, 17 rows 641 and 528, 8192 and 28672, 48
+// rows 937 and 834, but 7168 and 24576, 17 rows 582 and 616, 10240 and 32768, 33
+// rows 1095 and 1211.
+bool skinny_split_pays(const SkinnyArgs& a) {
+  const bool deep = a.K >= 3l * a.N && a.N <= (a.M <= 32 ? 6144 : 8192);
+  return a.N <= (a.M <= 16 ? 7168 : 5120) || deep;
+}
+
 void skinny_split(const SkinnyArgs& a, float* sums, long parts, hipStream_t st) {
   if (a.M <= 16) launch_split<1, split_chunk(16)>(a, sums, parts, st);
   else if (a.M <= 32) launch_split<2, split_chunk(32)>(a, sums, parts, st);

@@ -113,6 +113,74 @@ def test_step_matches_float32(name, kw, B):
         assert gpu.len == cpu.len == 21
 
 
+# residual products of 16 MB of weights, whose depth is split over blocks and whose
+# parts the next norm adds up
+WIDE = [("llama", {"n_heads": 8, "n_kv_heads": 2, "d_model": 1024, "d_ff": 8200}),
+        ("gpt2", {"n_heads": 8, "d_model": 1024, "d_ff": 8200})]
+
+
+@pytest.mark.parametrize("name,kw", WIDE)
+@pytest.mark.parametrize("B", [9, 17, 64])
+def test_split_products_of_a_step(name, kw, B):
+    from scaffold.generate import Generator
+
+    kw = {**kw, "n_layers": 2, "vocab_size": 64}
+    ref = Generator(_model(name, **kw).float())
+    gen = Generator(_model(name, **kw).cuda())
+    cpu, gpu = ref.new_cache(B, 40), gen.new_cache(B, 40)
+    for a, b in zip(cpu.k + cpu.v, gpu.k + gpu.v):
+        b.copy_(torch.randn_like(b, dtype=torch.float32))
+        a.copy_(b)
+    tok, pos = torch.randint(0, 64, (B, 1)), torch.randint(0, 40, (B,))
+    with torch.no_grad():
+        want = ref.decode_step_varpos(tok, cpu, pos)
+        got = gen._native_step(tok.cuda(), gpu, pos.cuda()).cpu().float()
+    # a bf16 stream: about ten roundings of 2^-9 a layer, independent
+    assert (got - want).norm() / want.norm() < 3 * 2 ** -7
+
+
+@pytest.mark.parametrize("name,kw", WIDE)
+@pytest.mark.parametrize("B,S", [(1, 9), (3, 20), (2, 32), (12, 3)])
+@pytest.mark.parametrize("every", [False, True])
+def test_split_products_of_a_prompt(name, kw, B, S, every):
+    """Without all logits the last layer's rows are fewer than the others',
+    and as few as take whole depths."""
+    from scaffold.generate import Generator
+
+    kw = {**kw, "n_layers": 2, "vocab_size": 64}
+    ref = Generator(_model(name, **kw).float())
+    gen = Generator(_model(name, **kw).cuda())
+    cpu, gpu = ref.new_cache(B, 40), gen.new_cache(B, 40)
+    ids = torch.randint(0, 64, (B, S))
+    with torch.no_grad():
+        want = ref._forward_tokens(ids, cpu, 0, all_logits=every)
+        got = gen._native_step(ids.cuda(), gpu, None, 0, all_logits=every)
+    # a bf16 stream: about ten roundings of 2^-9 a layer, independent
+    assert (got.cpu().float() - want).norm() / want.norm() < 3 * 2 ** -7
+
+
+@pytest.mark.parametrize("rows,width,ff,splits", [
+    (8, 1024, 8200, 0), (9, 1024, 8200, 2), (64, 1024, 8200, 2), (65, 1024, 8200, 0),
+    (16, 7168, 2048, 4), (17, 7168, 2048, 0), (16, 8192, 2048, 0)])
+def test_which_products_are_split(rows, width, ff, splits):
+    """The rule itself, by the kernels that a step of two layers launches."""
+    from torch.profiler import ProfilerActivity, profile
+
+    from scaffold.generate import Generator
+
+    gen = Generator(_model("llama", n_heads=width // 128, n_kv_heads=2, n_layers=2,
+                           vocab_size=64, d_model=width, d_ff=ff).cuda())
+    cache = gen.new_cache(rows, 8)
+    tok = torch.zeros(rows, 1, dtype=torch.int64, device="cuda")
+    pos = torch.zeros(rows, dtype=torch.int64, device="cuda")
+    with torch.no_grad(), profile(activities=[ProfilerActivity.CUDA]) as prof:
+        assert gen._native_step(tok, cache, pos) is not None
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events()]
+    assert any("row_norm_kernel" in n for n in names)
+    assert sum("skinny_split_kernel" in n for n in names) == splits
+
+
 def test_step_is_left_to_the_blocks():
     """Routed feed-forwards and float32 models keep the general step."""
     from scaffold.generate import Generator
