@@ -511,7 +511,8 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
 
   const float scale2 = a.scale * LOG2E;
   const float slope2 = BIAS && a.slopes ? a.slopes[h] * LOG2E : 0.f;
-  float m_run = a.has_sink ? fmaxf(sink_score<false>(a, h) * LOG2E, LOWEST) : LOWEST;
+  float m_run = a.has_sink ? sink_score<false>(a, h) * LOG2E : LOWEST;
+  if (m_run < LOWEST) m_run = LOWEST;          // -inf; NaN stays, and shows
   float l_run = a.has_sink && !half ? 1.f : 0.f;    // of this half's keys
   f32x16 o[NDT], s[2];
   #pragma unroll

@@ -30,3 +30,17 @@ def test_matches_oracle(H, G, d, e, parts, size, sink):
                         sink=s, parts=parts)
     # results are averages of values: one rounding of them and of the weights
     close(got, L.sink_attention(q, k, v, d ** -0.5, size, s), torch.bfloat16)
+
+
+@pytest.mark.parametrize("parts", [(65,), (64, 1)], ids=str)
+def test_a_sink_that_is_no_number_shows(parts):
+    """In its head, and in no other."""
+    T, H, G, d = sum(parts), 4, 2, 64
+    q, k, v = rnd(T, H, d, seed=1), rnd(T, G, d, seed=2), rnd(T, G, d, seed=3)
+    sink = rnd(H, seed=4)
+    sink[1] = math.nan
+    got = run_attention("cuda", torch.bfloat16, q, k, v, scale=d ** -0.5, size=0,
+                        sink=sink, parts=parts)
+    assert got[:, 1].isnan().all()
+    got[:, 1] = 0
+    assert got.isfinite().all()
