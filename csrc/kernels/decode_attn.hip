@@ -627,6 +627,7 @@ torch::Tensor decode_attention(torch::Tensor qkv, torch::Tensor k,
   auto out = torch::empty({a.B, (long)a.H * D}, qkv.options());
   a.out = (short*)out.data_ptr();
   if (a.B == 0) return out;
+  TORCH_CHECK(L > 0, "decode_attention: a cache without places");
   const int rep = a.H / a.G, chunks = (rep + R - 1) / R;
   const int pairs = a.B * a.G * chunks, full = (L + 63) / 64;
   // Two heads to a kv head use a quarter of the matrix instruction's columns, and

@@ -253,3 +253,14 @@ def test_two_heads_to_a_kv_head(D, B, G, L):
     for b, p in enumerate(pos.tolist()):
         assert torch.equal(k[b, :, p].double(), wk[b, :, p])
         assert torch.equal(v[b, :, p].double(), wv[b, :, p])
+
+
+@pytest.mark.parametrize("H", [2, 4, 8])
+def test_a_cache_without_places_is_refused(H):
+    from scaffold import ops
+
+    qkv = torch.zeros(1, (H + 4) * 64, device="cuda").bfloat16()
+    k, v = (torch.zeros(1, 2, 0, 64, device="cuda").bfloat16() for _ in range(2))
+    with pytest.raises(RuntimeError, match="places"):
+        ops.require_ext().decode_attention(
+            qkv, k, v, torch.zeros(1, dtype=torch.int64, device="cuda"), None, None, None, H)
