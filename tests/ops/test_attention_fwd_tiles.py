@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("D,B,H,G", [(64, 1, 3, 3), (128, 2, 8, 4),
                                      (64, 4, 8, 2), (128, 1, 5, 1)])
-@pytest.mark.parametrize("S", [255, 256, 257, 320, 383, 512, 641])
+@pytest.mark.parametrize("S", [1, 31, 33, 64, 65, 127, 129, 192, 255, 256, 257, 320,
+                               383, 512, 641])
 @pytest.mark.parametrize("causal", [True, False])
 def test_matches_float64(D, B, H, G, S, causal):
     from scaffold import ops
