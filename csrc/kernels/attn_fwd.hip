@@ -1,6 +1,5 @@
-// K4 — flash-style causal attention forward (correctness-first tile
-// version; the MFMA 8-wave structure of cdna_hip_programming.md §B
-// replaces the inner loops in a later milestone — same launch contract).
+// K4 — flash-style causal attention forward: float32, and heads that the matrix
+// kernels (attn_fwd_mfma.hip, attn_fwd_short.hip) do not take.
 //
 // Layout: q (B,H,S,D), k/v (B,Hkv,S,D) row-major bf16/fp32; GQA via
 // Hkv | H.  One 256-thread workgroup per (b, h, q-tile of QT rows);
@@ -155,7 +154,8 @@ void launch_fwd(const torch::Tensor& q, const torch::Tensor& k,
 
 }  // namespace
 
-// bf16, D in {64, 128}: attn_fwd_mfma.hip, and attn_fwd_short.hip below 256 rows
+// bf16, D in {64, 128}: attn_fwd_mfma.hip, and below 256 rows attn_fwd_short.hip,
+// where the reason for the line and both sides' times stand
 void attn_fwd_mfma(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                    torch::Tensor o, torch::Tensor lse, double scale, bool causal);
 void attn_fwd_short(torch::Tensor q, torch::Tensor k, torch::Tensor v,

@@ -1,5 +1,11 @@
 // K4 — MFMA flash attention forward (bf16, CDNA4 32x32x16 matrix cores) of
-// fewer than 256 rows, in natural logarithms.
+// fewer than 256 rows: a block has 128 consecutive rows, softmax in natural
+// logarithms.  It stays for the bits of training steps on such rows, which another
+// order of sums and base 2 would change, and for blocks of one head that are many
+// and short; heads of 128 spill 11 registers.  Here and in attn_fwd_mfma.hip, in us:
+// 64 x 32 (8 kv) x 32 x 128 32 and 49, x 128 rows 77 and 79, x 255 191 and 148; 64 x 12
+// x 32 x 64 10.9 and 13.4, x 128 21.0 and 20.4, x 255 45 and 35; 3 x 12 x 128 x 64 8.9
+// and 6.8.
 //
 // Structure (cdna_hip_programming.md §B "fused attention prefill" ladder,
 // adapted to 32x32x16 fragments):

@@ -284,7 +284,7 @@ DEVINL f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) {
 // are 8 heads twice: the weights enter the value product as three bf16 parts, all
 // of float32's bits, the second ones in the second 8 columns, the third ones by
 // an instruction of their own (1 to 5 % of the time).  Of 64 rows, 32 heads of 128
-// on 8, 1024 to 4096 keys deep, 671 MB: 133 us, 5.1 TB/s (159 with both products
+// on 8, 1024 to 4096 keys deep, 671 MB: 128 us, 5.2 TB/s (148 with both products
 // on the vector unit, which took half of the time there); one head to a kv head
 // is left to it, 64 rows of 12 heads of 64 to 1024 keys 27.1 and 28.2 us, 1 row to
 // 512 5.4 and 6.9, and two where decode_attention() says.

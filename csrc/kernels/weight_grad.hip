@@ -8,14 +8,14 @@
 // with their rows along the sum, so they are staged as they are, by copies
 // into LDS up to four stages ahead, and transposed by the reads, which are a
 // stage ahead of the products: a wave that reads at a stage's barrier, as all
-// then do, waits for most of what its products take (102 us below).
+// then do, waits for most of what its products take.
 //
-// 16384 rows, library and this, in us: 3072 x 768 179 and 95 (with the sums), 2304
-// x 768 142 and 70, 768 x 768 91 and 40; 8192 rows, 4096 x 4096 253 (1087 TF/s),
-// 287 with reads at the barrier; with three stages ahead 96, 70, 40 and 259.
-// The second kernel takes 11 of the first three's, writing the parts, 66 MB,
-// as much again; in between the matrix cores are busy 55 % of the time, the
-// waits for copies, 10 TB/s out of the caches, are most of the rest.
+// 16384 rows, library, this and this with reads at the barrier, in us: 3072 x 768
+// 152, 90 (with the sums) and 96, 2304 x 768 121, 68 and 75, 768 x 768 92, 41 and 42;
+// 8192 rows, 4096 x 4096 235, 240 (1145 TF/s) and 259.  Copies three stages ahead
+// are 1 to 2 % slower.  The second kernel takes 11 of the first shape's, writing the
+// parts, 66 MB, as much again; in between the matrix cores are busy 55 % of the
+// time, the waits for copies, 10 TB/s out of the caches, are most of the rest.
 
 #include "../common.h"
 
@@ -35,8 +35,8 @@ DEVINL void each(const F& f) {
 }
 
 // A stage lies as units of 4 rows x 32 columns, 256 bytes: four lanes of a copy
-// take 64 bytes of a row (with units of 16 columns, 32 bytes, 96 us instead of
-// 91).  A transpose read takes 16 columns of a unit; odd quads of rows have
+// take 64 bytes of a row (with units of 16 columns, 32 bytes, 5 % slower, when
+// stages were three ahead).  A transpose read takes 16 columns of a unit; odd quads of rows have
 // its halves swapped, so that the two quads of half a wave's read lie in
 // different banks.
 constexpr int BT = 32;                  // rows of a stage

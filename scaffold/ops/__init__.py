@@ -395,11 +395,11 @@ def _colsum(dy2: torch.Tensor) -> torch.Tensor:
 def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """dy^T x of contiguous rows.  The library splits the rows too little
     where dW has few tiles: in us, library and own kernel, 3072 x 768 out of
-    16384 rows 179 and 91, of 8192 81 and 57, of 4096 42 and 42; 1024 x 4096
-    (64 tiles of 256 x 256) 185 and 143, 88 and 83, 51 and 57; with 100 tiles
-    8192 rows take 134 and 136.  Tiles that are mostly empty are not worth it:
-    8192 rows, 32 x 256 19 and 31, 64 x 64 46 and 29, 64 x 16384 63 and 68, 256 x
-    16384 98 and 87."""
+    16384 rows 152 and 90, of 8192 77 and 55, of 4096 42 and 41; 1024 x 4096
+    (64 tiles of 256 x 256) 166 and 130, 85 and 77, 45 and 51; with 100 tiles
+    8192 rows take 120 and 115.  Tiles that are mostly empty are not worth it:
+    8192 rows, 32 x 256 19 and 30, 64 x 64 45 and 30, 64 x 16384 63 and 75, 256 x
+    16384 108 and 86."""
     n, k = dy.shape[1], x.shape[1]
     small, large = min(n, k), max(n, k)
     if (x.is_cuda and small >= 64 and (small >= 256 or large <= 8192)
