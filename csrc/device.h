@@ -7,9 +7,12 @@
 #include <hip/hip_bf16.h>
 
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #define WAVE 64
 #define DEVINL __device__ __forceinline__
+#define INLINE __attribute__((always_inline))    // of lambdas
 
 using bf16 = __hip_bfloat16;
 
@@ -33,6 +36,36 @@ DEVINL short f2bf(float f) {
   unsigned int rounded = x + 0x7FFF + ((x >> 16) & 1);
   if ((x & 0x7F800000u) == 0x7F800000u) rounded = x;  // inf/nan passthrough
   return (short)(rounded >> 16);
+}
+
+// Two float32 to a dword of two bf16, to nearest even: v_cvt_pk_bf16_f32.  Not
+// in assembly, before which the compiler leaves out the wait that a result of
+// v_exp_f32 needs.
+DEVINL unsigned cvt_pk_bf16(float lo, float hi) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((f2{lo, hi}), b2));
+}
+
+// f(0) ... f(N - 1), each number a constant
+template <typename F, int... I>
+DEVINL void each_of(const F& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+template <int N, typename F>
+DEVINL void each(const F& f) {
+  each_of(f, std::make_integer_sequence<int, N>{});
+}
+
+// a value that is the same in all lanes, where the compiler does not see it (and
+// would loop over the lanes to make a buffer descriptor of it)
+DEVINL unsigned same(unsigned x) { return (unsigned)__builtin_amdgcn_readfirstlane((int)x); }
+
+// Bits 2 and 3 change places: score products of 32 x 32 whose rows are keys in this
+// order leave a lane, in registers 8 i ..., the weights of consecutive keys.
+DEVINL int swapped(int row) {
+  return (row & ~12) | (row & 4) << 1 | (row & 8) >> 1;
 }
 
 // wave-level reductions (wave64)

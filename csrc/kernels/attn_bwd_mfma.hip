@@ -43,17 +43,8 @@ namespace {
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef short bf16x8_t __attribute__((ext_vector_type(8)));
 
-#define INLINE __attribute__((always_inline))
-
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr int ROWS = 128;              // of a block of 4 waves
-
-// Two float32 to a dword of two bf16, to nearest even: v_cvt_pk_bf16_f32.
-DEVINL unsigned cvt_pk_bf16(float lo, float hi) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(unsigned, __builtin_convertvector((f2{lo, hi}), b2));
-}
 
 // What a lane holds of a product's 32 x 32 (a column, 16 rows), as operands of
 // 8 consecutive rows a lane: the halves exchange every other four.
@@ -76,17 +67,6 @@ DEVINL void pack_frags(const f32x16_t& p, bf16x8_t out[2]) {
 
 DEVINL f32x16_t mma(bf16x8_t a, bf16x8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-
-// f(0) ... f(N - 1), each number a constant
-template <typename F, int... I>
-DEVINL void each_of(const F& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-
-template <int N, typename F>
-DEVINL void each(const F& f) {
-  each_of(f, std::make_integer_sequence<int, N>{});
 }
 
 // Image of 64 rows of D: element (row, col) is at row * D + 8 * ((col / 8) ^
@@ -139,10 +119,6 @@ DEVINL unsigned copy_at(long ss) {
   const int row = threadIdx.x / (D / 8), chunk = threadIdx.x % (D / 8);
   return 2u * ((unsigned)row * (unsigned)ss + 8u * (chunk ^ chunk_key<D>(row)));
 }
-
-// a value that is the same in all lanes, where the compiler does not see it and
-// would loop over the lanes
-DEVINL unsigned same(unsigned x) { return (unsigned)__builtin_amdgcn_readfirstlane((int)x); }
 
 template <int D>
 DEVINL void copy_rows(short* img, const short* from, long ss, unsigned lane_at,

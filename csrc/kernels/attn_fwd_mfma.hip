@@ -40,17 +40,6 @@ constexpr int ROWS = 32 * W;       // query rows of a block
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef short bf16x8_t __attribute__((ext_vector_type(8)));
 
-// Two float32 to a dword of two bf16, to nearest even: v_cvt_pk_bf16_f32.  Not
-// in assembly, before which the compiler leaves out the wait that a result of
-// v_exp_f32 needs.
-DEVINL unsigned cvt_pk_bf16(float lo, float hi) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(unsigned, __builtin_convertvector((f2{lo, hi}), b2));
-}
-
-#define INLINE __attribute__((always_inline))
-
 DEVINL bf16x4 tr_at(const short* at) {
   typedef __attribute__((address_space(3))) bf16x4* P;
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)at);
@@ -61,11 +50,6 @@ DEVINL float other_half(float x) {
   const unsigned u = __builtin_bit_cast(unsigned, x);
   const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   return __builtin_bit_cast(float, threadIdx.x & 32 ? r[0] : r[1]);
-}
-
-// bits 2 and 3 change places
-DEVINL int swapped(int row) {
-  return (row & ~12) | (row & 4) << 1 | (row & 8) >> 1;
 }
 
 // S query rows see Sk keys, the last S of them their own places (training:

@@ -23,17 +23,6 @@ namespace {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-// f(0) ... f(N - 1), each number a constant
-template <typename F, int... I>
-DEVINL void each_of(const F& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-
-template <int N, typename F>
-DEVINL void each(const F& f) {
-  each_of(f, std::make_integer_sequence<int, N>{});
-}
-
 // A stage lies as units of 4 rows x 32 columns, 256 bytes: four lanes of a copy
 // take 64 bytes of a row (with units of 16 columns, 32 bytes, 5 % slower, when
 // stages were three ahead).  A transpose read takes 16 columns of a unit; odd quads of rows have
@@ -55,10 +44,6 @@ DEVINL f32x4_t mma(bf16x8 a, bf16x8 b, f32x4_t c) {
       __builtin_bit_cast(__attribute__((ext_vector_type(8))) __bf16, a),
       __builtin_bit_cast(__attribute__((ext_vector_type(8))) __bf16, b), c, 0, 0, 0);
 }
-
-#define INLINE __attribute__((always_inline))
-
-DEVINL unsigned same(unsigned x) { return (unsigned)__builtin_amdgcn_readfirstlane((int)x); }
 
 __global__ void __launch_bounds__(512)
 wgrad_kernel(WgradArgs a) {

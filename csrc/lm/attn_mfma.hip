@@ -39,12 +39,6 @@ DEVINL f32x16 mma32(bf16x8 a, bf16x8 b, f32x16 c) {
       0, 0);
 }
 
-DEVINL unsigned cvt_pk_bf16(float a, float b) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, b16x2));
-}
-
 // B fragments (16 keys each) of 16 consecutive-by-lane P^T values, which p
 // holds afterwards less what went into them
 DEVINL void p_frags(float (&p)[16], bf16x8 (&out)[2]) {
@@ -394,13 +388,6 @@ attn_prefill_form_kernel(AttnArgs a, const int4* __restrict__ tiles,
   }
 }
 
-#define INLINE __attribute__((always_inline))
-
-// bits 2 and 3 change places
-DEVINL int swapped(int row) {
-  return (row & ~12) | (row & 4) << 1 | (row & 8) >> 1;
-}
-
 // As stored, with or without a bias by distance.  A page is S = K(t) Q, O += V(t
 // - 1) P(t - 1), softmax of S, one barrier; K(t + 1) and V(t) come into LDS
 // meanwhile, by buffer loads, which read as zero what lies behind the tile's
@@ -484,9 +471,8 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
         (unsigned long)((const short*)cache + ((long)page * a.G + g) * LM_PAGE * dim);
     const int rows = min(LM_PAGE, p_last - (first + pg) * LM_PAGE + 1);
     const auto src = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)((unsigned long)(unsigned)__builtin_amdgcn_readfirstlane((int)(from >> 32)) << 32 |
-                (unsigned)__builtin_amdgcn_readfirstlane((int)from)), 0,
-        __builtin_amdgcn_readfirstlane(2 * rows * dim), 0x00020000);
+        (void*)((unsigned long)same((unsigned)(from >> 32)) << 32 | same((unsigned)from)), 0,
+        (int)same((unsigned)(2 * rows * dim)), 0x00020000);
     #pragma unroll
     for (int i = 0; i < decltype(count)::value; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
