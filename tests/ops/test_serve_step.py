@@ -173,7 +173,8 @@ def test_which_products_are_split(rows, width, ff, splits):
     cache = gen.new_cache(rows, 8)
     tok = torch.zeros(rows, 1, dtype=torch.int64, device="cuda")
     pos = torch.zeros(rows, dtype=torch.int64, device="cuda")
-    with torch.no_grad(), profile(activities=[ProfilerActivity.CUDA]) as prof:
+    with torch.no_grad(), profile(activities=[ProfilerActivity.CUDA],
+                                  acc_events=True) as prof:
         assert gen._native_step(tok, cache, pos) is not None
         torch.cuda.synchronize()
     names = [e.name for e in prof.events()]
