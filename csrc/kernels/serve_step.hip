@@ -312,10 +312,10 @@ c10::optional<torch::Tensor> serve_step(
                                    // (parts, T, W) float32
   const torch::Tensor* nw = nullptr;   // a norm that the next product takes
   double neps = 0;
-  auto norm = [&](const torch::Tensor* w, double e, bool first) {
+  auto norm = [&](const torch::Tensor* w, double e, bool first, SkinnyAct act) {
     // few rows are normed by the product that reads them (which is one of
     // skinny_gemm's then)
-    const bool later = w != final_norm.data() && skinny_norms(T, W) &&
+    const bool later = w != final_norm.data() && skinny_norm_pays(T, W, act) &&
                        (first || !pending.defined());
     if (later) {
       nw = w;
@@ -426,10 +426,11 @@ c10::optional<torch::Tensor> serve_step(
     }
     hipLaunchKernelGGL(append_kernel, dim3((unsigned)(B * rows)), dim3(256), 0, st, a);
   };
+  const SkinnyAct up_act = gpt2 ? SKINNY_GELU : SKINNY_SWIGLU;
   torch::Tensor act;
   for (size_t i = 0; i < n; ++i) {
     const torch::Tensor* w = &layers[per * i];
-    norm(w, eps[2 * i], i == 0);
+    norm(w, eps[2 * i], i == 0, SKINNY_NONE);
     const torch::Tensor *wq = w + (gpt2 ? 2 : 1), *wo = w + (gpt2 ? 4 : 2);
     const torch::Tensor *w2 = w + (gpt2 ? 6 : 3), *up = w + (gpt2 ? 8 : 4);
     const torch::Tensor* down = w + (gpt2 ? 10 : 5);
@@ -461,15 +462,15 @@ c10::optional<torch::Tensor> serve_step(
       }
     }
     residual(o, *wo, bias(wo));
-    norm(w2, eps[2 * i + 1], false);
+    norm(w2, eps[2 * i + 1], false, up_act);
     if (act.defined() && act.size(1) != down->size(1)) act = torch::Tensor();
-    if (!product(h, *up, bias(up), act, false, gpt2 ? SKINNY_GELU : SKINNY_SWIGLU)) {
+    if (!product(h, *up, bias(up), act, false, up_act)) {
       act = lib(h, *up, bias(up));
       act = gpt2 ? at::gelu(act, "tanh") : swiglu_packed_fwd(act);
     }
     residual(act, *down, bias(down));
   }
-  norm(final_norm.data(), eps[2 * n], false);
+  norm(final_norm.data(), eps[2 * n], false, SKINNY_NONE);
   torch::Tensor logits;
   if (!product(h, head, nullptr, logits, false, SKINNY_NONE))
     logits = lib(h, head, nullptr);

@@ -6,12 +6,15 @@
 
 struct SkinnyArgs {
   const short *x, *w;            // (M, K) rows of ldx, (N or 2N, K)
+  long ldx;
+  int M, N, K;
+  int fours;                     // skinny_gemm: y, bias and res lie for 8-byte access
+  const short *nw, *nb;          // x is normed first: layer norm with nb, else RMS
+                                 // norm; null: as it is
   const short *bias, *res;       // (N) or null; (M, N) rows of ldr or null
   short *y;                      // (M, N) rows of ldy
-  const short *nw, *nb;          // x is normed first: layer norm with nb, else
-  float eps;                     // RMS norm; null: as it is
-  long ldx, ldr, ldy;
-  int M, N, K;
+  long ldr, ldy;
+  float eps;                     // of the norm
 };
 
 enum SkinnyAct {
@@ -23,7 +26,8 @@ enum SkinnyAct {
 // M up to 64, K a multiple of 8, x and w rows 16-byte aligned
 bool skinny_takes(const SkinnyArgs& a);
 bool skinny_norms(long M, long K);     // whether it may have a norm
-void skinny_gemm(const SkinnyArgs& a, SkinnyAct act, hipStream_t st);
+bool skinny_norm_pays(long M, long K, SkinnyAct act);   // against a launch of its own
+void skinny_gemm(SkinnyArgs a, SkinnyAct act, hipStream_t st);
 
 // The same without act, res or norm, the depth split over `parts` groups of
 // blocks whose sums, (parts, M, N) float32 with the bias in the first, the

@@ -1,13 +1,14 @@
 // y = x w^T for few rows x (a decode step: up to 64), bf16, float32 sums.
 //
-// What bounds it is reading w once.  A weight goes from memory to the one
-// wave that multiplies it and nowhere else: a block has 16 rows of w (RT
-// times that), its 8 waves split the depth in spans of 32 * U columns, and
-// the rows of x, which every block reads, come out of the caches as the other
-// operand of the 16x16x32 MFMA.  Each wave has the next span's loads in
-// flight while it multiplies one.  The waves' sums meet in LDS at the end,
-// where bias, residual, GELU or the gate's product join before the only
-// rounding.
+// What bounds it is reading w once, and with little of it the chain of a launch:
+// an empty one takes 1.6 us, one that reads 24 KB a block and adds them up over 8
+// waves 2.8.  A weight goes from memory to the one wave that multiplies it and
+// nowhere else: a block has some rows of w, its 8 waves split the depth, and the
+// rows of x, which every block reads, come out of the caches as the other operand
+// of the 16x16x32 MFMA.  Each wave has the next span's loads in flight while it
+// multiplies one, and what the end needs of bias and residual.  The waves' sums
+// meet in LDS, where bias, residual, GELU or the gate's product join before the
+// only rounding.
 
 #include "../common.h"
 #include "skinny.h"
@@ -23,95 +24,115 @@ DEVINL f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) {
 DEVINL float gelu_tanh(float z) {
   const float u = 0.7978845608028654f * (z + 0.044715f * z * z * z);
   // tanh(u) = 1 - 2 / (exp(2u) + 1), also at both ends
-  return 0.5f * z * (2.f - 2.f / (__expf(2.f * u) + 1.f));
+  return 0.5f * z * (2.f - 2.f * __builtin_amdgcn_rcpf(__expf(2.f * u) + 1.f));
 }
 
-// Rows of x, normed (layer norm with a bias, else RMS norm) and rounded, into
-// LDS; a wave takes a row at a time, up to 4096 columns.
-template <int NW>
-DEVINL void norm_rows(const SkinnyArgs& a, short* xs) {
-  constexpr int NV = 8;
-  const int wid = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const float inv = 1.f / (float)a.K;
-  for (int m = wid; m < a.M; m += NW) {
-    bf16x8 v[NV];
-    float s = 0.f, mean = 0.f;
+// sum over the lanes that are the same but for bit 4, or 5
+DEVINL float pair_sum(float x, std::integral_constant<int, 16>) {
+  const unsigned u = __builtin_bit_cast(unsigned, x);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+DEVINL float pair_sum(float x, std::integral_constant<int, 32>) {
+  const unsigned u = __builtin_bit_cast(unsigned, x);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+// and the lane N places on in its row of 16
+template <int N> DEVINL float turn_sum(float x) {
+  const int i = __builtin_bit_cast(int, x);
+  return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                 0, i, 0x120 + N, 0xf, 0xf, true));
+}
+
+// waits for LDS alone: __syncthreads() would wait for weights on their way too
+DEVINL void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// What a lane needs of bias and residual for 4 outputs, asked for when the
+// kernel starts: behind the products each would be a wait of its own.  Where
+// there is none, or it does not lie for it, any 8 bytes are, for a load in a
+// branch is waited for where the ways meet.
+struct Extra { bf16x4 bias, res; };
+
+DEVINL Extra extra(const SkinnyArgs& a, int row, int n) {
+  const bool b = a.bias && a.fours, r = a.res && a.fours;
+  const int c = min(n, a.N - 4);
+  return {*(const bf16x4*)((b ? a.bias : a.w) + (b ? c : 0)),
+          *(const bf16x4*)((r ? a.res : a.w) + (r ? min(row, a.M - 1) * a.ldr + c : 0))};
+}
+
+// 4 outputs in a row of one row of x
+template <int ACT>
+DEVINL void put(const SkinnyArgs& a, const Extra& e, f32x4 s, int row, int n) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  short* y = a.y + row * a.ldy + n;
+  if (a.fours) {
+    const bf16x4 b = e.bias & (a.bias ? (short)-1 : (short)0);
+    const bf16x4 r = e.res & (a.res ? (short)-1 : (short)0);
     #pragma unroll
-    for (int n = 0; n < NV; ++n) {
-      const int c = (n * 64 + l) * 8;
-      if (n * 512 < a.K)
-        v[n] = *(const bf16x8*)(a.x + m * a.ldx + min(c, a.K - 8));
+    for (int j = 0; j < 4; ++j) {
+      s[j] += bf2f(b[j]);
+      if (ACT == SKINNY_GELU) s[j] = gelu_tanh(s[j]);
+      s[j] += bf2f(r[j]);
     }
-    #pragma unroll
-    for (int n = 0; n < NV; ++n) {
-      const bool in = (n * 64 + l) * 8 < a.K;
-      if (n * 512 < a.K)
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float x = in ? bf2f(v[n][j]) : 0.f;
-          s += a.nb ? x : x * x;
-        }
-    }
-    s = wave_reduce_sum(s) * inv;
-    if (a.nb) {
-      mean = s;
-      s = 0.f;
-      #pragma unroll
-      for (int n = 0; n < NV; ++n) {
-        const bool in = (n * 64 + l) * 8 < a.K;
-        if (n * 512 < a.K)
-          #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float d = in ? bf2f(v[n][j]) - mean : 0.f;
-            s += d * d;
-          }
-      }
-      s = wave_reduce_sum(s) * inv;
-    }
-    const float rstd = rsqrtf(s + a.eps);
-    #pragma unroll
-    for (int n = 0; n < NV; ++n) {
-      const int c = (n * 64 + l) * 8;
-      if (c >= a.K) continue;
-      const bf16x8 w = *(const bf16x8*)(a.nw + c);
-      bf16x8 b = {}, o;
-      if (a.nb) b = *(const bf16x8*)(a.nb + c);
-      #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        o[j] = f2bf((bf2f(v[n][j]) - mean) * rstd * bf2f(w[j]) + bf2f(b[j]));
-      *(bf16x8*)(xs + m * (a.K + 8) + c) = o;
-    }
+    *(u32x2*)y = u32x2{cvt_pk_bf16(s[0], s[1]), cvt_pk_bf16(s[2], s[3])};
+    return;
   }
+  #pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (n + j < a.N) {
+      if (a.bias) s[j] += bf2f(a.bias[n + j]);
+      if (ACT == SKINNY_GELU) s[j] = gelu_tanh(s[j]);
+      if (a.res) s[j] += bf2f(a.res[row * a.ldr + n + j]);
+      y[j] = (short)cvt_pk_bf16(s[j], s[j]);
+    }
 }
 
-// MT tiles of 16 rows of x, RT tiles of 16 rows of w (SWIGLU: half of them
-// gate rows, half the up rows that go with them), NW waves.  NORM: the rows of
-// x are normed first, by every block for itself, into LDS; the first weights
-// are on their way meanwhile.
-template <int MT, int RT, int NW, int ACT, bool NORM>
+// MT tiles of 16 rows of x, RT tiles of rows of w (SWIGLU: half of them gate rows,
+// half the up rows that go with them), NW waves.
+//
+// SEG: the 16 rows and columns of the matrix instruction are 16 / SEG rows of w
+// and of x, each SEG times, at SEG places of the depth; of the products, those
+// of equal places count.  So few rows of w make SEG times the blocks, which
+// read a SEG-th each.
+//
+// S: the rows of x are normed first (layer norm with a bias, else RMS norm), by
+// every block for itself: a wave has its share of the depth of all rows, S steps,
+// in registers as the products take them, and only the sums go through LDS.
+// Such a kernel is as long as its instructions in a row, 8 cycles each, and its
+// waits.  768 to 2304, 1 row, 8 rows: rows normed by a wave each, rounded into LDS
+// and read from there (11 KB of code), and bias asked for at the end 5.1 and 5.4 us;
+// so 3.6 and 4.2; without the norm 3.1 and 3.4.
+template <int MT, int RT, int NW, int ACT, int S, int SEG>
 __global__ void __launch_bounds__(64 * NW)
 skinny_kernel(SkinnyArgs a) {
   constexpr bool PAIR = ACT == SKINNY_SWIGLU;
-  constexpr int U = MT + RT <= 3 ? 4 : 2;
-  constexpr int SPAN = 32 * U;
+  constexpr int U = MT + RT <= 3 ? 4 / SEG : SEG < 4 ? 2 : 1;
+  constexpr int STEP = 32 * SEG;              // columns of a matrix instruction
+  constexpr int SPAN = STEP * U;
   constexpr int OT = PAIR ? RT / 2 : RT;      // output tiles
+  constexpr int R = 16 / SEG;                 // rows of one
+  constexpr int TILES = (MT * OT + NW - 1) / NW;   // of a wave, at the end
+  static_assert((SEG == 1 && !S) || (MT == 1 && NW == 8), "few rows");
   __shared__ __attribute__((aligned(16))) f32x4 part[NW][MT * RT][64];
 
-  const int wid = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
   const int lr = l & 15, lg = l >> 4;
-  const int n0 = blockIdx.x * 16 * OT;
+  const int n0 = blockIdx.x * R * OT;
+  const int at = 8 * lg + 32 * (lr / R);      // of a step's columns, this lane's 8
   const short *wp[RT], *xp[MT];
   #pragma unroll
   for (int r = 0; r < RT; ++r) {
-    const int n = min(n0 + 16 * (r % OT) + lr, a.N - 1) + (r / OT) * a.N;
-    wp[r] = a.w + (long)n * a.K + 8 * lg;
+    const int n = min(n0 + R * (r % OT) + lr % R, a.N - 1) + (r / OT) * a.N;
+    wp[r] = a.w + (long)n * a.K + at;
   }
-  extern __shared__ __attribute__((aligned(16))) short xs[];   // NORM: [M][K + 8]
   #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int row = min(16 * m + lr, a.M - 1);
-    xp[m] = (NORM ? xs + row * (a.K + 8) : a.x + (long)row * a.ldx) + 8 * lg;
-  }
+  for (int m = 0; m < MT; ++m)
+    xp[m] = a.x + (long)min(16 * m + lr % R, a.M - 1) * a.ldx + at;
+  auto w_at = [&](int r, int c) { return *(const bf16x8*)(wp[r] + c); };
+  auto x_at = [&](int m, int c) { return *(const bf16x8*)(xp[m] + c); };
 
   f32x4 acc[MT][RT];
   #pragma unroll
@@ -119,64 +140,163 @@ skinny_kernel(SkinnyArgs a) {
     #pragma unroll
     for (int r = 0; r < RT; ++r) acc[m][r] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  struct Span { bf16x8 w[RT][U], x[NORM ? 1 : MT][U]; };
-  auto fetch = [&](Span& s, int k0) {
+  // where a lane's outputs are: of SEG^2 groups of lanes each has all of them
+  const int orow = SEG == 1 ? lr : SEG == 2 ? l & 7 : l & 3;
+  const int ocol = SEG == 1 ? 4 * lg : SEG == 2 ? (l >> 1) & 4 : 0;
+  Extra ex[TILES];
+  auto ask = [&] {
     #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      #pragma unroll
-      for (int r = 0; r < RT; ++r)
-        s.w[r][u] = *(const bf16x8*)(wp[r] + k0 + 32 * u);
-      if constexpr (!NORM)
-        #pragma unroll
-        for (int m = 0; m < MT; ++m) s.x[m][u] = *(const bf16x8*)(xp[m] + k0 + 32 * u);
+    for (int i = 0; i < TILES; ++i) {
+      const int t = min(wid + i * NW, MT * OT - 1);
+      ex[i] = extra(a, 16 * (t / OT) + orow, n0 + R * (t % OT) + ocol);
     }
   };
-  auto use = [&](const Span& s, int k0) {
+
+  if constexpr (S) {
+    __shared__ __attribute__((aligned(16))) float sums[2][R][NW];
+    // Step i NW + wid of the depth; columns behind the end are read at its last
+    // 8 and count as zero on both sides.  No load stands in a branch: the
+    // compiler waits for all of them where two ways meet.
+    const int last = (a.K - 1) / STEP * STEP;           // columns of the last step
+    const int edge = min(at, a.K - 8 - last);
+    auto col = [&](int i) { return (i * NW + wid) * STEP; };
+    auto in = [&](int i) { return at < a.K - col(i); };
+    auto from = [&](int i) {
+      return min(col(i), last) + (col(i) < last ? 0 : edge - at);
+    };
+    bf16x8 x[S], w[RT][S], nw[S], nb[S];
+    const short* nbp = a.nb ? a.nb : a.nw;
+    auto fetch = [&](int i) {
+      #pragma unroll
+      for (int r = 0; r < RT; ++r) w[r][i] = w_at(r, from(i));
+    };
     #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int i = 0; i < S; ++i) x[i] = x_at(0, from(i));
+    #pragma unroll
+    for (int i = 0; i < S; ++i) fetch(i);
+    #pragma unroll
+    for (int i = 0; i < S; ++i) {
+      nw[i] = *(const bf16x8*)(a.nw + at + from(i));
+      nb[i] = *(const bf16x8*)(nbp + at + from(i));
+    }
+    ask();
+    const float inv = 1.f / (float)a.K;
+    // s: of the wave, by rows of x in 16 columns; to the whole depth's of this lane's row
+    auto total = [&](float s, int n) {
+      if constexpr (SEG == 2) s = turn_sum<8>(s);
+      if constexpr (SEG == 4) s = turn_sum<8>(turn_sum<4>(s));
+      if (l < R) sums[n][l][wid] = s;
+      lds_barrier();
+      const f32x4 lo = *(const f32x4*)&sums[n][lr % R][0];
+      const f32x4 hi = *(const f32x4*)&sums[n][lr % R][4];
+      return ((lo[0] + lo[1]) + (lo[2] + lo[3])) + ((hi[0] + hi[1]) + (hi[2] + hi[3]));
+    };
+    #pragma unroll
+    for (int i = 0; i < S; ++i)
+      if (col(i) >= last && !in(i)) x[i] = bf16x8{};
+    auto normed = [&](auto layer) INLINE {
+      constexpr bool LAYER = decltype(layer)::value;
+      float mean = 0.f, d[S][8], s = 0.f;
+      if constexpr (LAYER) {
+        // the matrix instruction adds the rows up
+        bf16x8 one;
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) one[j] = 0x3f80;
+        f32x4 t = {};
+        #pragma unroll
+        for (int i = 0; i < S; ++i) t = mma(one, x[i], t);
+        mean = total(t[0], 0) * inv;
+      }
+      #pragma unroll
+      for (int i = 0; i < S; ++i) {
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) d[i][j] = bf2f(x[i][j]) - mean;
+        if (!LAYER || col(i) < last || in(i))
+          #pragma unroll
+          for (int j = 0; j < 8; ++j) s += d[i][j] * d[i][j];
+      }
+      s = pair_sum(pair_sum(s, std::integral_constant<int, 16>{}),
+                   std::integral_constant<int, 32>{});
+      const float rstd = rsqrtf(total(s, 1) * inv + a.eps);
+      #pragma unroll
+      for (int i = 0; i < S; ++i) {
+        typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+        u32x4 o;
+        #pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          float y[2];
+          #pragma unroll
+          for (int k = 0; k < 2; ++k)
+            y[k] = d[i][j + k] * rstd * bf2f(nw[i][j + k]) +
+                   (LAYER ? bf2f(nb[i][j + k]) : 0.f);
+          o[j / 2] = cvt_pk_bf16(y[0], y[1]);
+        }
+        bf16x8 h = __builtin_bit_cast(bf16x8, o);
+        if (col(i) >= last) {
+          h = in(i) ? h : bf16x8{};
+          #pragma unroll
+          for (int r = 0; r < RT; ++r) w[r][i] = in(i) ? w[r][i] : bf16x8{};
+        }
+        #pragma unroll
+        for (int r = 0; r < RT; ++r) acc[0][r] = mma(w[r][i], h, acc[0][r]);
+      }
+    };
+    if (a.nb) normed(std::true_type{});
+    else normed(std::false_type{});
+  } else {
+    struct Span { bf16x8 w[RT][U], x[MT][U]; };
+    auto fetch = [&](Span& s, int k0) {
+      #pragma unroll
+      for (int u = 0; u < U; ++u) {
+        #pragma unroll
+        for (int r = 0; r < RT; ++r)
+          s.w[r][u] = w_at(r, k0 + STEP * u);
+        #pragma unroll
+        for (int m = 0; m < MT; ++m) s.x[m][u] = x_at(m, k0 + STEP * u);
+      }
+    };
+    auto use = [&](const Span& s) {
+      #pragma unroll
+      for (int u = 0; u < U; ++u)
+        #pragma unroll
+        for (int m = 0; m < MT; ++m)
+          #pragma unroll
+          for (int r = 0; r < RT; ++r) acc[m][r] = mma(s.w[r][u], s.x[m][u], acc[m][r]);
+    };
+    const int full = a.K / SPAN;               // whole spans
+    Span s0, s1;
+    int i = wid;
+    if (i < full) fetch(s0, i * SPAN);
+    ask();
+    for (; i < full; i += 2 * NW) {
+      if (i + NW < full) fetch(s1, (i + NW) * SPAN);
+      use(s0);
+      if (i + NW >= full) break;
+      if (i + 2 * NW < full) fetch(s0, (i + 2 * NW) * SPAN);
+      use(s1);
+    }
+    // what is left of the depth, a step at a time, by the waves that have had
+    // one span less; columns behind the end are read at its last 8 and count
+    // as zero on both sides
+    const int left = (a.K - full * SPAN + STEP - 1) / STEP;
+    const int mine = (wid - full % NW + NW) % NW;
+    if (mine < left) {
+      const int k0 = full * SPAN + STEP * mine;
+      const bool in = k0 + at < a.K;
+      const int c = in ? k0 : a.K - 8 - at;
+      bf16x8 wv[RT], xv[MT];
+      #pragma unroll
+      for (int r = 0; r < RT; ++r) wv[r] = w_at(r, c);
+      #pragma unroll
+      for (int m = 0; m < MT; ++m) xv[m] = x_at(m, c);
+      #pragma unroll
+      for (int r = 0; r < RT; ++r) wv[r] = in ? wv[r] : bf16x8{};
       #pragma unroll
       for (int m = 0; m < MT; ++m) {
-        const bf16x8 x = NORM ? *(const bf16x8*)(xp[m] + k0 + 32 * u) : s.x[m][u];
+        xv[m] = in ? xv[m] : bf16x8{};
         #pragma unroll
-        for (int r = 0; r < RT; ++r) acc[m][r] = mma(s.w[r][u], x, acc[m][r]);
+        for (int r = 0; r < RT; ++r) acc[m][r] = mma(wv[r], xv[m], acc[m][r]);
       }
-  };
-  const int full = a.K / SPAN;               // whole spans
-  Span s0, s1;
-  int i = wid;
-  if (i < full) fetch(s0, i * SPAN);
-  if constexpr (NORM) {
-    norm_rows<NW>(a, xs);
-    __syncthreads();
-  }
-  for (; i < full; i += 2 * NW) {
-    if (i + NW < full) fetch(s1, (i + NW) * SPAN);
-    use(s0, i * SPAN);
-    if (i + NW >= full) break;
-    if (i + 2 * NW < full) fetch(s0, (i + 2 * NW) * SPAN);
-    use(s1, (i + NW) * SPAN);
-  }
-  // what is left of the depth, 32 columns at a time, by the waves that have
-  // had one span less; columns behind the end are read at its last 8 and
-  // count as zero on both sides
-  const int left = (a.K - full * SPAN + 31) / 32;
-  const int mine = (wid - full % NW + NW) % NW;
-  if (mine < left) {
-    const int k0 = full * SPAN + 32 * mine;
-    const bool in = k0 + 8 * lg < a.K;
-    const int c = in ? k0 : a.K - 8 - 8 * lg;
-    bf16x8 wv[RT], xv[MT];
-    #pragma unroll
-    for (int r = 0; r < RT; ++r) wv[r] = *(const bf16x8*)(wp[r] + c);
-    #pragma unroll
-    for (int m = 0; m < MT; ++m) xv[m] = *(const bf16x8*)(xp[m] + c);
-    #pragma unroll
-    for (int r = 0; r < RT; ++r) wv[r] = in ? wv[r] : bf16x8{};
-    #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      xv[m] = in ? xv[m] : bf16x8{};
-      #pragma unroll
-      for (int r = 0; r < RT; ++r) acc[m][r] = mma(wv[r], xv[m], acc[m][r]);
     }
   }
   #pragma unroll
@@ -185,66 +305,112 @@ skinny_kernel(SkinnyArgs a) {
     for (int r = 0; r < RT; ++r) part[wid][m * RT + r][l] = acc[m][r];
   __syncthreads();
 
-  // a lane has 4 outputs in a row of one row of x
-  for (int t = wid; t < MT * OT; t += NW) {
+  #pragma unroll
+  for (int i = 0; i < TILES; ++i) {
+    const int t = wid + i * NW;
+    if (t >= MT * OT) break;
     const int m = t / OT, o = t % OT;
-    f32x4 s = part[0][m * RT + o][l];
-    #pragma unroll
-    for (int v = 1; v < NW; ++v) s += part[v][m * RT + o][l];
+    // tile r's sums over waves, and over the places of the depth
+    auto whole = [&](int r) {
+      f32x4 s;
+      if constexpr (SEG == 1) {
+        s = part[0][r][l];
+        #pragma unroll
+        for (int v = 1; v < NW; ++v) s += part[v][r][l];
+      } else if constexpr (SEG == 2) {
+        // place c lies at lanes 16 (2 c + quad) + 8 c + row
+        const int from = 16 * (ocol / 4) + orow;
+        s = (part[2 * lg][r][from] + part[2 * lg][r][from + 40]) +
+            (part[2 * lg + 1][r][from] + part[2 * lg + 1][r][from + 40]);
+      } else {
+        // at lanes 16 c + 4 c + row
+        const int v = (l >> 2) & 7, from = (l >> 5) * 40 + orow;
+        s = part[v][r][from] + part[v][r][from + 20];
+        #pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] = turn_sum<8>(turn_sum<4>(s[j]));
+      }
+      if constexpr (SEG > 1)
+        #pragma unroll
+        for (int j = 0; j < 4; ++j)
+          s[j] = pair_sum(pair_sum(s[j], std::integral_constant<int, 16>{}),
+                          std::integral_constant<int, 32>{});
+      return s;
+    };
+    f32x4 s = whole(m * RT + o);
     if constexpr (PAIR) {
-      f32x4 up = part[0][m * RT + OT + o][l];
-      #pragma unroll
-      for (int v = 1; v < NW; ++v) up += part[v][m * RT + OT + o][l];
+      const f32x4 up = whole(m * RT + OT + o);
       #pragma unroll
       for (int j = 0; j < 4; ++j) s[j] = s[j] / (1.f + __expf(-s[j])) * up[j];
     }
-    const int row = 16 * m + lr, n = n0 + 16 * o + 4 * lg;
-    if (row >= a.M) continue;
-    short* y = a.y + row * a.ldy + n;
-    const short* res = a.res ? a.res + row * a.ldr + n : nullptr;
-    bf16x4 out;
-    #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bool in = n + j < a.N;
-      if (a.bias && in) s[j] += bf2f(a.bias[n + j]);
-      if (ACT == SKINNY_GELU) s[j] = gelu_tanh(s[j]);
-      if (res && in) s[j] += bf2f(res[j]);
-      out[j] = f2bf(s[j]);
-    }
-    if (n + 4 <= a.N && a.ldy % 4 == 0 && (size_t)a.y % 8 == 0) {
-      *(bf16x4*)y = out;
-    } else {
-      #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (n + j < a.N) y[j] = out[j];
-    }
+    const int row = 16 * m + orow, n = n0 + R * o + ocol;
+    if (row < a.M && n < a.N && (SEG == 1 || l < 64 / (SEG * SEG)))
+      put<ACT>(a, ex[i], s, row, n);
   }
 }
 
-template <int MT, int RT, int NW, int ACT>
+template <int MT, int RT, int NW, int ACT, int S = 0, int SEG = 1>
 void launch(const SkinnyArgs& a, hipStream_t st) {
-  constexpr int OT = ACT == SKINNY_SWIGLU ? RT / 2 : RT;
-  const dim3 grid((a.N + 16 * OT - 1) / (16 * OT)), block(64 * NW);
-  if constexpr (MT == 1) {
-    if (a.nw) {
-      hipLaunchKernelGGL((skinny_kernel<MT, RT, NW, ACT, true>), grid, block,
-                         (size_t)a.M * (a.K + 8) * 2, st, a);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((skinny_kernel<MT, RT, NW, ACT, false>), grid, block, 0,
-                     st, a);
+  constexpr int OT = ACT == SKINNY_SWIGLU ? RT / 2 : RT, ROWS = 16 / SEG * OT;
+  hipLaunchKernelGGL((skinny_kernel<MT, RT, NW, ACT, S, SEG>),
+                     dim3((a.N + ROWS - 1) / ROWS), dim3(64 * NW), 0, st, a);
 }
 
-// A block takes more rows of w where there are enough of them to fill the
-// chip all the same: x is then read by fewer blocks.  Of 28672 rows of 4096,
-// 16 rows of x: 49 us with 64 rows in a block of 4 waves, 58 with 16 or 32;
-// 8 rows of x: 47 and 49 us.  Of 6144: 17 us with 16 rows a block, 16 with
-// 32, 21 with 64; of 4096: 10 and 14 us.
+template <int RT, int ACT, int SEG>
+void launch_norm(const SkinnyArgs& a, hipStream_t st) {
+  const int steps = (a.K + 256 * SEG - 1) / (256 * SEG);
+  if (steps == 1) launch<1, RT, 8, ACT, 1, SEG>(a, st);
+  else if (steps == 2) launch<1, RT, 8, ACT, 2, SEG>(a, st);
+  else if (steps == 3) launch<1, RT, 8, ACT, 3, SEG>(a, st);
+  else launch<1, RT, 8, ACT, 4, SEG>(a, st);
+}
+
+// Up to 4 rows of x read w at four places of the depth at once, up to 8 at two: a
+// load is whole lines of 128 bytes then (16 rows of w to a load have halves of
+// 64), and x is read as often less.  A block has few rows of w as long as that
+// fills the chip, and where as many blocks as 16 rows make would leave a last wave
+// of them nearly empty.  In us, with 16 rows and more to a block, two waves of
+// loads ahead (before), and now: 768 rows of w of 3072, 1 row of x 6.0 and 3.2, 8
+// rows 7.1 and 5.1; 4096 of 4096, 1 row 9.3 and 8.0, 8 rows 10.0 and 9.1; 5120 of 4096,
+// 2 rows 13.8 and 10.4, 5 rows 14.4 and 13.0; 128256 of 4096, 1 row 198 and 164, 8
+// rows 205 and 182; pairs, 2 x 14336 of 4096, 1 row 52.0 and 41.2, 8 rows 49.9 and
+// 44.6, 2 x 28672 of 8192 198 and 154, 197 and 161 (6.1 and 5.9 TB/s).  Many rows
+// of w of little depth are as many short blocks: 50257 of 768, 1 row, 4 rows of w
+// to a block 20.7, 8 15.0, 64 16.5 (17.7 before), 8 rows of x 16 to a block 21.0 and
+// 64 19.1.
+//
+// More rows of x: a block takes more rows of w where there are enough of them
+// to fill the chip all the same: x is then read by fewer blocks.  Of 28672 rows of
+// 4096, 16 rows of x: 47 us with 64 rows in a block of 4 waves, 58 with 16 or 32.
+//
+// With a norm, which every block makes for itself, 16 rows of w share it: 768 to
+// 2304, 1 row 3.6 us, 4.0 with 8 rows of w; deep rows, of which the loads are the
+// longer part, 8: 4096 to 6144 13.0 and 14.3.
 template <int MT, int ACT>
 void pick(const SkinnyArgs& a, hipStream_t st) {
   constexpr bool PAIR = ACT == SKINNY_SWIGLU;
   const int tiles = (a.N + 15) / 16 * (PAIR ? 2 : 1);
+  if constexpr (MT == 1) {
+    const bool shallow = a.K < 2048 && tiles >= 1280;
+    if (a.nw) {
+      if (a.M <= 4 && (PAIR || a.K <= 2048)) launch_norm<4, ACT, 4>(a, st);
+      else if (a.M <= 4) launch_norm<2, ACT, 4>(a, st);
+      else if (a.M <= 8) launch_norm<2, ACT, 2>(a, st);
+      else launch_norm<PAIR ? 2 : 1, ACT, 1>(a, st);
+      return;
+    }
+    if constexpr (PAIR) {
+      if (a.M <= 8) return launch<1, 2, 8, ACT, 0, 2>(a, st);
+    } else {
+      if (a.M <= 2 && shallow) return launch<1, 2, 8, ACT, 0, 4>(a, st);
+      // rows of w up to which a block has four
+      const int fours = a.M > 4 ? 0 : a.M > 2 ? 1024 : a.K < 2048 ? 2048
+                        : a.M == 2 ? 6144 : a.N;
+      if (a.N <= fours) return launch<1, 1, 8, ACT, 0, 4>(a, st);
+      if (a.M <= 4 && a.N <= 2048) return launch<1, 2, 8, ACT, 0, 4>(a, st);
+      if (a.M <= 8 && a.N <= 2048) return launch<1, 1, 8, ACT, 0, 2>(a, st);
+      if (a.M <= 8 && !shallow) return launch<1, 2, 8, ACT, 0, 2>(a, st);
+    }
+  }
   if (tiles >= 1280) launch<MT, 4, 4, ACT>(a, st);
   else if (PAIR || (MT > 1 && tiles >= 384)) launch<MT, 2, 8, ACT>(a, st);
   else if constexpr (!PAIR) launch<MT, 1, 8, ACT>(a, st);
@@ -419,19 +585,26 @@ bool skinny_takes(const SkinnyArgs& a) {
          (!a.nw || skinny_norms(a.M, a.K));
 }
 
-// A norm of few elements costs a block less than a launch of its own would:
-// the first weights are on their way meanwhile, and a wave has one row or two.
-// With the norm's launch, and without, in us: 768 to 2304, 1 row 5.8 and 4.8,
-// 8 rows 6.5 and 5.1, 16 rows 6.7 and 6.9; 768 to 3072, 1 row 6.0 and 5.0;
-// 4096 to 6144 and to 2 x 14336, 1 row 18.5 + 55.1 and 20.0 + 49.4, 2 rows
-// 19.2 + 56.0 and 20.4 + 50.4.  Where the rows of w are many enough for
-// several blocks a compute unit, each of them norms again: 768 to 50257 takes
-// 20.8 and 22.2, so the last norm of a model stays a launch.
+// A norm of few elements costs a block less than a launch of its own (2.8 us)
+// would: in us, with the norm, and the product alone: 768 to 2304, 1 row 3.6 and 3.1, 10
+// rows 4.2 and 3.4; 1024 to 4096, 8 rows 4.6 and 4.1; 4096 to 6144, 2 rows 13.1 and 11.5.
+// A wave holds up to four steps of the depth.
 bool skinny_norms(long M, long K) {
-  return M >= 1 && M <= 16 && K <= 4096 && M * K <= 8 * 1024;
+  return M >= 1 && M <= 16 && (K <= 1024 || (K <= 4096 && M * K <= 8 * 1024));
 }
 
-void skinny_gemm(const SkinnyArgs& a, SkinnyAct act, hipStream_t st) {
+// Where the rows of w are many and deep, each of the several blocks of a compute
+// unit norms again: 2048 to 2 x 5632, 1 row 11.6 and 9.8 without the norm, 4096 to 2 x
+// 14336 48.4 and 41.0.  768 to 50257 takes 20.8 and 22.2, so the last norm of a model
+// stays a launch.
+bool skinny_norm_pays(long M, long K, SkinnyAct act) {
+  return skinny_norms(M, K) && (act != SKINNY_SWIGLU || K <= 2048);
+}
+
+void skinny_gemm(SkinnyArgs a, SkinnyAct act, hipStream_t st) {
+  auto fours = [&](const short* p, long ld) { return (size_t)p % 8 == 0 && ld % 4 == 0; };
+  a.fours = a.N % 4 == 0 && fours(a.y, a.ldy) && fours(a.bias, 0) &&
+            (!a.res || fours(a.res, a.ldr));
   if (act == SKINNY_GELU) pick<SKINNY_GELU>(a, st);
   else if (act == SKINNY_SWIGLU) pick<SKINNY_SWIGLU>(a, st);
   else pick<SKINNY_NONE>(a, st);

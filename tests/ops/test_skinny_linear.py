@@ -39,8 +39,40 @@ def test_matches_float64(N, K, M, act):
     assert ((got - y).abs() <= 2.0 ** -8 * y.abs() + 2.0 ** -14).all()
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (2, 1028, 776), (3, 1024, 136), (4, 1025, 2056), (4, 2048, 264),
+    (2, 2052, 1000), (2, 6144, 2064), (2, 6148, 2064), (1, 7001, 2048),
+    (5, 2048, 72), (7, 2049, 200), (8, 4100, 2080)])
+@pytest.mark.parametrize("act", [0, 1, 2])
+@pytest.mark.parametrize("off", [0, 2])
+def test_places_of_the_depth(M, N, K, act, off):
+    """Up to 8 rows: the edges of what takes four or two places of the depth at
+    once, depths that do not fill them, bias and residual in and out of line."""
+    from scaffold import ops
+
+    torch.manual_seed(N + K + M)
+    dev = "cuda"
+    x = torch.randn(M, K + 8, device=dev).bfloat16()[:, :K]
+    w = (torch.randn(N * (2 if act == 2 else 1), K, device=dev)
+         / math.sqrt(K)).bfloat16()
+    b = None if act == 2 else torch.randn(N + off, device=dev).bfloat16()[off:]
+    r = torch.randn(M, N + off, device=dev).bfloat16()[:, off:]
+    got = ops.require_ext().skinny_linear(x, w, b, r, act).double()
+    y = x.double() @ w.double().T
+    if act == 2:
+        y = F.silu(y[:, :N]) * y[:, N:]
+    else:
+        y = y + b.double()
+    if act == 1:
+        y = F.gelu(y, approximate="tanh")
+    y = y + r.double()
+    # as above
+    assert ((got - y).abs() <= 2.0 ** -8 * y.abs() + 2.0 ** -14).all()
+
+
 @pytest.mark.parametrize("M,K", [(1, 8), (1, 4096), (2, 4096), (3, 768),
-                                 (10, 768), (16, 504), (16, 512), (9, 520)])
+                                 (10, 768), (16, 504), (16, 512), (9, 520),
+                                 (4, 2048), (5, 1024), (8, 1016), (16, 1024)])
 @pytest.mark.parametrize("N,act", [(48, 0), (2304, 1), (6150, 2), (20483, 0)])
 @pytest.mark.parametrize("kind", ["layer", "rms"])
 def test_norm_of_the_rows(M, K, N, act, kind):
