@@ -44,12 +44,17 @@ struct RowNormArgs {
   float eps;
 };
 
-// A block per row, the row in registers between the sum and the result.
+// A block per row, the row in registers between the sum and the result.  Of few
+// rows it is the chain of waits that counts: all loads are asked for at once, those
+// of the norm's weights before its sums, and none stands in a branch, behind which
+// the compiler would wait for it.  2536 rows of 768 and a residual 7.0 us with the
+// weights behind the sums, 5.9 so.
 template <int C>
 __global__ void __launch_bounds__(256)
 row_norm_kernel(RowNormArgs a) {
-  __shared__ float red[4];
+  __shared__ float red[2][4];
   const long row = blockIdx.x;
+  const int wid = threadIdx.x >> 6;
   short* x = a.x + row * a.W;
   float v[C][8];
   const short *t = nullptr, *p = nullptr;
@@ -61,7 +66,23 @@ row_norm_kernel(RowNormArgs a) {
     t = a.wte + (bad ? 0 : id * a.W);
     p = a.wpe ? a.wpe + (bad ? 0 : at * a.W) : nullptr;
   }
+  const short* from = t ? t : x;
   const short* y = a.y ? a.y + row * a.W : p;
+  const short* also = y ? y : from;
+  const short* bias = a.b ? a.b : a.w;
+  bf16x8 e[C], f[C], w[C], b[C];
+  #pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int i = min((c * 256 + (int)threadIdx.x) * 8, a.W - 8);
+    e[c] = *(const bf16x8*)(from + i);
+    f[c] = *(const bf16x8*)(also + i);
+  }
+  #pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int i = min((c * 256 + (int)threadIdx.x) * 8, a.W - 8);
+    w[c] = *(const bf16x8*)(a.w + i);
+    b[c] = *(const bf16x8*)(bias + i);
+  }
   float s = 0.f;
   #pragma unroll
   for (int c = 0; c < C; ++c) {
@@ -69,12 +90,9 @@ row_norm_kernel(RowNormArgs a) {
     #pragma unroll
     for (int j = 0; j < 8; ++j) v[c][j] = 0.f;
     if (i >= a.W) continue;
-    bf16x8 e = *(const bf16x8*)((t ? t : x) + i);
-    if (y) {
-      const bf16x8 f = *(const bf16x8*)(y + i);
+    if (y)
       #pragma unroll
-      for (int j = 0; j < 8; ++j) e[j] = f2bf(bf2f(e[j]) + bf2f(f[j]));
-    }
+      for (int j = 0; j < 8; ++j) e[c][j] = f2bf(bf2f(e[c][j]) + bf2f(f[c][j]));
     if (a.sums) {
       const float* p = a.sums + row * a.W + i;
       f32x4 lo = {}, hi = {};
@@ -85,23 +103,31 @@ row_norm_kernel(RowNormArgs a) {
       }
       #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        e[j] = f2bf(bf2f(e[j]) + lo[j]);
-        e[4 + j] = f2bf(bf2f(e[4 + j]) + hi[j]);
+        e[c][j] = f2bf(bf2f(e[c][j]) + lo[j]);
+        e[c][4 + j] = f2bf(bf2f(e[c][4 + j]) + hi[j]);
       }
     }
     if (bad) {                           // no such row: let it show
       #pragma unroll
-      for (int j = 0; j < 8; ++j) e[j] = 0x7fc0;
+      for (int j = 0; j < 8; ++j) e[c][j] = 0x7fc0;
     }
-    if (t || y || a.sums) *(bf16x8*)(x + i) = e;
+    if (t || y || a.sums) *(bf16x8*)(x + i) = e[c];
     #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      v[c][j] = bf2f(e[j]);
+      v[c][j] = bf2f(e[c][j]);
       s += a.b ? v[c][j] : v[c][j] * v[c][j];
     }
   }
   if (!a.h) return;
-  s = block_reduce_sum(s, red);
+  // over the block's four waves; waits for LDS alone
+  auto total = [&](float s, int n) {
+    s = wave_reduce_sum(s);
+    if ((threadIdx.x & 63) == 0) red[n][wid] = s;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const f32x4 r = *(const f32x4*)red[n];
+    return (r[0] + r[1]) + (r[2] + r[3]);
+  };
+  s = total(s, 0);
   float mean = 0.f;
   if (a.b) {
     mean = s / a.W;
@@ -112,20 +138,25 @@ row_norm_kernel(RowNormArgs a) {
         #pragma unroll
         for (int j = 0; j < 8; ++j) s += (v[c][j] - mean) * (v[c][j] - mean);
       }
-    s = block_reduce_sum(s, red);
+    s = total(s, 1);
   }
   const float rstd = rsqrtf(s / a.W + a.eps);
   #pragma unroll
   for (int c = 0; c < C; ++c) {
     const int i = (c * 256 + threadIdx.x) * 8;
     if (i >= a.W) continue;
-    const bf16x8 w = *(const bf16x8*)(a.w + i);
-    bf16x8 b = {}, o;
-    if (a.b) b = *(const bf16x8*)(a.b + i);
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 o;
     #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      o[j] = f2bf((v[c][j] - mean) * rstd * bf2f(w[j]) + bf2f(b[j]));
-    *(bf16x8*)(a.h + row * a.W + i) = o;
+    for (int j = 0; j < 8; j += 2) {
+      float h[2];
+      #pragma unroll
+      for (int k = 0; k < 2; ++k)
+        h[k] = (v[c][j + k] - mean) * rstd * bf2f(w[c][j + k]) +
+               (a.b ? bf2f(b[c][j + k]) : 0.f);
+      o[j / 2] = cvt_pk_bf16(h[0], h[1]);
+    }
+    *(u32x4*)(a.h + row * a.W + i) = o;
   }
 }
 

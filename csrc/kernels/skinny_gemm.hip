@@ -196,7 +196,7 @@ skinny_kernel(SkinnyArgs a) {
       if (col(i) >= last && !in(i)) x[i] = bf16x8{};
     auto normed = [&](auto layer) INLINE {
       constexpr bool LAYER = decltype(layer)::value;
-      float mean = 0.f, d[S][8], s = 0.f;
+      float mean = 0.f, s = 0.f;
       if constexpr (LAYER) {
         // the matrix instruction adds the rows up
         bf16x8 one;
@@ -208,13 +208,13 @@ skinny_kernel(SkinnyArgs a) {
         mean = total(t[0], 0) * inv;
       }
       #pragma unroll
-      for (int i = 0; i < S; ++i) {
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) d[i][j] = bf2f(x[i][j]) - mean;
+      for (int i = 0; i < S; ++i)
         if (!LAYER || col(i) < last || in(i))
           #pragma unroll
-          for (int j = 0; j < 8; ++j) s += d[i][j] * d[i][j];
-      }
+          for (int j = 0; j < 8; ++j) {
+            const float d = bf2f(x[i][j]) - mean;
+            s += d * d;
+          }
       s = pair_sum(pair_sum(s, std::integral_constant<int, 16>{}),
                    std::integral_constant<int, 32>{});
       const float rstd = rsqrtf(total(s, 1) * inv + a.eps);
@@ -227,7 +227,7 @@ skinny_kernel(SkinnyArgs a) {
           float y[2];
           #pragma unroll
           for (int k = 0; k < 2; ++k)
-            y[k] = d[i][j + k] * rstd * bf2f(nw[i][j + k]) +
+            y[k] = (bf2f(x[i][j + k]) - mean) * rstd * bf2f(nw[i][j + k]) +
                    (LAYER ? bf2f(nb[i][j + k]) : 0.f);
           o[j / 2] = cvt_pk_bf16(y[0], y[1]);
         }
@@ -587,10 +587,12 @@ bool skinny_takes(const SkinnyArgs& a) {
 
 // A norm of few elements costs a block less than a launch of its own (2.8 us)
 // would: in us, with the norm, and the product alone: 768 to 2304, 1 row 3.6 and 3.1, 10
-// rows 4.2 and 3.4; 1024 to 4096, 8 rows 4.6 and 4.1; 4096 to 6144, 2 rows 13.1 and 11.5.
-// A wave holds up to four steps of the depth.
+// rows 4.2 and 3.4; 1024 to 4096, 8 rows 4.6 and 4.1; 4096 to 6144, 2 rows 13.1 and
+// 11.5, 4 rows 13.6 and 12.9.  A wave holds up to four steps of the depth; with eight,
+// 8 rows of 4096 to 6144 are 18.0 and 14.1, and behind much of the weights a launch is
+// 4.9: as good.
 bool skinny_norms(long M, long K) {
-  return M >= 1 && M <= 16 && (K <= 1024 || (K <= 4096 && M * K <= 8 * 1024));
+  return M >= 1 && K <= (M <= 4 ? 4096 : M <= 8 ? 2048 : M <= 16 ? 1024 : 0);
 }
 
 // Where the rows of w are many and deep, each of the several blocks of a compute

@@ -72,7 +72,7 @@ def test_places_of_the_depth(M, N, K, act, off):
 
 @pytest.mark.parametrize("M,K", [(1, 8), (1, 4096), (2, 4096), (3, 768),
                                  (10, 768), (16, 504), (16, 512), (9, 520),
-                                 (4, 2048), (5, 1024), (8, 1016), (16, 1024)])
+                                 (4, 4096), (5, 1024), (8, 2040), (16, 1024)])
 @pytest.mark.parametrize("N,act", [(48, 0), (2304, 1), (6150, 2), (20483, 0)])
 @pytest.mark.parametrize("kind", ["layer", "rms"])
 def test_norm_of_the_rows(M, K, N, act, kind):
