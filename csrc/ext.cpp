@@ -95,6 +95,8 @@ torch::Tensor prompt_attention(torch::Tensor q, torch::Tensor k,
                                torch::Tensor v, long Sk);
 torch::Tensor skinny_linear_parts(torch::Tensor x, torch::Tensor w,
                                   c10::optional<torch::Tensor> bias);
+c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Tensor& w,
+                                         const c10::optional<torch::Tensor>& bias, long act);
 torch::Tensor skinny_linear(torch::Tensor x, torch::Tensor w,
                             c10::optional<torch::Tensor> bias,
                             c10::optional<torch::Tensor> res, long act,
@@ -176,6 +178,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_linear_parts", &skinny_linear_parts,
         "sums over parts of the depth of a product of few rows", py::arg("x"),
         py::arg("w"), py::arg("bias") = py::none());
+  m.def("tile_linear", &tile_linear,
+        "act(x w^T + b) of some hundred rows, or None; act: 0 none, 1 tanh-GELU, 2 erf-GELU",
+        py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("act") = 0);
   m.def("skinny_linear", &skinny_linear,
         "product of up to 64 rows with bias, residual, GELU or SwiGLU",
         py::arg("x"), py::arg("w"), py::arg("bias") = py::none(),

@@ -9,6 +9,7 @@
 
 #include "../common.h"
 #include "skinny.h"
+#include "tile_gemm.h"
 
 bool decode_attention_takes(const torch::Tensor& qkv, const torch::Tensor& k,
                             const torch::Tensor& v);
@@ -416,6 +417,28 @@ c10::optional<torch::Tensor> serve_step(
     skinny_gemm(a, act, st);
     return true;
   };
+  // many rows: act(in w^T + b) by tiles, or undefined
+  auto tiled = [&](const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor* b,
+                   TileAct act) {
+    TileArgs a = {};
+    a.M = (int)T;
+    a.N = (int)w.size(0);
+    a.K = (int)w.size(1);
+    a.x = (const short*)in.data_ptr();
+    a.w = (const short*)w.data_ptr();
+    a.bias = b ? (const short*)b->data_ptr() : nullptr;
+    a.ldx = a.K;
+    a.ldy = a.N;
+    if (!tile_takes(a, act)) return torch::Tensor();
+    auto y = torch::empty({T, a.N}, opt);
+    a.y = (short*)y.data_ptr();
+    tile_gemm(a, act, st);
+    return y;
+  };
+  auto lib = [&](const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor* b) {
+    auto y = tiled(in, w, b, TILE_NONE);
+    return y.defined() ? y : b ? at::linear(in, w, *b) : at::linear(in, w);
+  };
   // what is to be added to x before the next norm: in w^T + b
   auto residual = [&](const torch::Tensor& in, const torch::Tensor& w,
                       const torch::Tensor* b) {
@@ -432,12 +455,8 @@ c10::optional<torch::Tensor> serve_step(
       pending = torch::empty({parts, T, W}, opt.dtype(torch::kFloat32));
       skinny_split(a, pending.data_ptr<float>(), parts, st);
     } else if (!product(in, w, b, x, true, SKINNY_NONE)) {
-      pending = b ? at::linear(in, w, *b) : at::linear(in, w);
+      pending = lib(in, w, b);
     }
-  };
-  auto lib = [](const torch::Tensor& in, const torch::Tensor& w,
-                const torch::Tensor* b) {
-    return b ? at::linear(in, w, *b) : at::linear(in, w);
   };
   auto append = [&](size_t i, long rows, bool turn_q) {
     AppendArgs a = {};
@@ -496,8 +515,11 @@ c10::optional<torch::Tensor> serve_step(
     norm(w2, eps[2 * i + 1], false, up_act);
     if (act.defined() && act.size(1) != down->size(1)) act = torch::Tensor();
     if (!product(h, *up, bias(up), act, false, up_act)) {
-      act = lib(h, *up, bias(up));
-      act = gpt2 ? at::gelu(act, "tanh") : swiglu_packed_fwd(act);
+      if (gpt2) act = tiled(h, *up, bias(up), TILE_GELU_TANH);
+      if (!gpt2 || !act.defined()) {
+        act = lib(h, *up, bias(up));
+        act = gpt2 ? at::gelu(act, "tanh") : swiglu_packed_fwd(act);
+      }
     }
     residual(act, *down, bias(down));
   }

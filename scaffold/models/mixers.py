@@ -514,7 +514,7 @@ class DenseFF(nn.Module):
         return [("up", self.up.weight), ("down", self.down.weight)]
 
     def step(self, h, plan: StepPlan):
-        return ops.linear(ops.gelu_erf(ops.linear(h, self.up.weight)),
+        return ops.linear(ops.linear_gelu_erf(h, self.up.weight),
                           self.down.weight)
 
 

@@ -33,6 +33,7 @@ __all__ = [
     "attention",
     "linear",
     "linear_gelu",
+    "linear_gelu_erf",
     "linear_residual",
     "swiglu",
     "swiglu_packed",
@@ -502,8 +503,17 @@ class _LinearResidualFn(torch.autograd.Function):
 _HAND_GEMM_ALL = False  # flipped by benchmarks once the 8-phase core wins
 
 
+def _product(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None
+             ) -> torch.Tensor:
+    """F.linear without a graph, of some hundred rows by tiles of our own, which
+    take more of the chip there (both sides' times: csrc/kernels/tile_gemm.hip)."""
+    m = ext()
+    y = m.tile_linear(x, w, b) if m is not None and x.is_cuda else None
+    return F.linear(x, w, b) if y is None else y
+
+
 class _LinearLib(torch.autograd.Function):
-    """Library-GEMM (hipBLASLt) forward with an explicit backward:
+    """Forward by _product() with an explicit backward:
     rocBLAS matmuls for dX/dW plus the hand colsum kernel for the bias
     gradient (torch's generic reduce measured ~1 TB/s there).  What is frozen
     costs nothing: its gradient is not made, and what only that needs not kept."""
@@ -513,7 +523,7 @@ class _LinearLib(torch.autograd.Function):
         need_x, need_w, ctx.need_b = ctx.needs_input_grad
         ctx.save_for_backward(x if need_w else None, w if need_x else None)
         ctx.x_shape = x.shape
-        return F.linear(x, w, b)
+        return _product(x, w, b)
 
     @staticmethod
     def backward(ctx, dy):
@@ -533,7 +543,7 @@ class _LinearGeluLib(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w, b):
-        pre = F.linear(x, w, b)
+        pre = _product(x, w, b)
         ctx.save_for_backward(x, w, b, pre)
         return F.gelu(pre, approximate="tanh")
 
@@ -566,8 +576,22 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None
     if x.is_cuda and _HAND_GEMM_ALL and _tile_ok(x, w):
         return _LinearFn.apply(x, w, b)
     if x.is_cuda and x.dtype == torch.bfloat16:
+        if not torch.is_grad_enabled() and not _transformed():
+            return _product(x, w, b)
         return _LinearLib.apply(x, w, b)
     return F.linear(x, w, b)
+
+
+def linear_gelu_erf(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """gelu(x w^T), the erf form, without a graph; in one kernel where _product()
+    is ours."""
+    m = ext()
+    if (m is not None and x.is_cuda and x.dtype == torch.bfloat16
+            and not torch.is_grad_enabled() and not _transformed()):
+        y = m.tile_linear(x, w, None, 2)
+        if y is not None:
+            return y
+    return gelu_erf(linear(x, w))
 
 
 def linear_gelu(x: torch.Tensor, w: torch.Tensor,

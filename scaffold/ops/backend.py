@@ -47,6 +47,7 @@ _SOURCES = [
     "kernels/decode_gemv.hip",
     "kernels/decode_attn.hip",
     "kernels/skinny_gemm.hip",
+    "kernels/tile_gemm.hip",
     "kernels/serve_step.hip",
     "kernels/probe.hip",
 ]
