@@ -10,12 +10,12 @@
 // stage ahead of the products: a wave that reads at a stage's barrier, as all
 // then do, waits for most of what its products take.
 //
-// 16384 rows, library, this and this with reads at the barrier, in us: 3072 x 768
-// 152, 90 (with the sums) and 96, 2304 x 768 121, 68 and 75, 768 x 768 92, 41 and 42;
-// 8192 rows, 4096 x 4096 235, 240 (1145 TF/s) and 259.  Copies three stages ahead
-// are 1 to 2 % slower.  The second kernel takes 11 of the first shape's, writing the
-// parts, 66 MB, as much again; in between the matrix cores are busy 55 % of the
-// time, the waits for copies, 10 TB/s out of the caches, are most of the rest.
+// 16384 rows, library, this, this with its copies asked for at once and up to the last
+// stage (behind which the compiler waits for all of them once a round), and with reads at
+// the barrier too, in us: 3072 x 768 152, 85 (with the sums), 92 and 96, 2304 x 768 121, 66,
+// 72 and 75, 768 x 768 92, 39, 40 and 42; 8192 rows, 4096 x 4096 235, 241 (1140 TF/s), 256 and
+// 259.  Copies three stages ahead are 1 to 2 % slower.  The second kernel takes 11 of the
+// first shape's, writing the parts, 66 MB, as much again.
 
 #include "../common.h"
 
@@ -76,26 +76,31 @@ wgrad_kernel(WgradArgs a) {
     pa[i] = 2u * ((unsigned)row * a.N + min(n0 + col, a.N - 8));
     pb[i] = 2u * ((unsigned)row * a.K + min(k0 + col, a.K - 8));
   }
-  // rows behind the part's last read as zero
-  auto copy = [&](short* to, const short* from, int width, const unsigned* at, int s) INLINE {
-    const int row = t0 + s * BT;
+  // rows behind the part's last read as zero, and stages behind it, so that what is on
+  // its way is the same in every step: where it may be less, the compiler waits for all of
+  // it once a round
+  auto copy = [&](short* to, const short* from, int width, const unsigned* at, int s, int i) INLINE {
+    const int row = min(t0 + s * BT, t1);
     const unsigned long base = (unsigned long)(from + (long)row * width);
     const auto rows = __builtin_amdgcn_make_buffer_rsrc(
         (void*)((unsigned long)same((unsigned)(base >> 32)) << 32 | same((unsigned)base)), 0,
         (int)same(2u * min(BT, t1 - row) * width), 0x00020000);
-    #pragma unroll
-    for (int i = 0; i < 2; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rows, (__attribute__((address_space(3))) void*)(to + (wid * 2 + i) * 512), 16,
-          at[i], 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rows, (__attribute__((address_space(3))) void*)(to + (wid * 2 + i) * 512), 16,
+        at[i], 0, 0, 0);
   };
   auto image = [&](auto n) INLINE {
     constexpr int I = decltype(n)::value % NB;
     return I == 0 ? s0 : I == 1 ? s1 : I == 2 ? s2 : I == 3 ? s3 : s4;
   };
+  // copy J of four of a stage
+  auto part_of = [&](auto n, int s, auto j) INLINE {
+    constexpr int J = decltype(j)::value;
+    if constexpr (J < 2) copy(image(n), a.dy, a.N, pa, s, J);
+    else copy(image(n) + OPER, a.x, a.K, pb, s, J - 2);
+  };
   auto stage = [&](auto n, int s) INLINE {
-    copy(image(n), a.dy, a.N, pa, s);
-    copy(image(n) + OPER, a.x, a.K, pb, s);
+    each<4>([&](auto j) INLINE { part_of(n, s, j); });
   };
 
   // this lane's quads are g and 4 + g: any order of a stage's rows will do.
@@ -117,13 +122,11 @@ wgrad_kernel(WgradArgs a) {
           (P)(img + wm * 512 + (M & 1 ? o : e) + M / 2 * 128 + R % 2 * 4096));
     }
   };
-  // The copies of stage s have arrived, in all waves, those of up to two later
-  // ones may not; in a form that the compiler's own count takes notice of.
-  auto turn = [&](int s) INLINE {
+  // The copies of the stage after the next have arrived, in all waves, those of two
+  // later ones may not; in a form that the compiler's own count takes notice of.
+  auto turn = [&] INLINE {
     asm volatile("" ::: "memory");
-    if (s + 2 < ns) __builtin_amdgcn_s_waitcnt(0x0f78);        // vmcnt(8)
-    else if (s + 1 < ns) __builtin_amdgcn_s_waitcnt(0x0f74);   // vmcnt(4)
-    else __builtin_amdgcn_s_waitcnt(0x0f70);                   // vmcnt(0)
+    __builtin_amdgcn_s_waitcnt(0x0f78);        // vmcnt(8)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
@@ -134,7 +137,6 @@ wgrad_kernel(WgradArgs a) {
   // are on their way and s + 4 is asked for, where s - 1 lay.
   auto step = [&](auto n, int s) INLINE {
     constexpr int I = decltype(n)::value, X = I & 1;
-    if (s + 4 < ns) stage(std::integral_constant<int, I + 4>{}, s + 4);
     const short* next = image(std::integral_constant<int, I + 1>{});
     each<8>([&](auto m) INLINE {
       constexpr int M = decltype(m)::value;
@@ -144,21 +146,42 @@ wgrad_kernel(WgradArgs a) {
       });
       const bf16x8 am = frag(fa[X][M]);
       each<4>([&](auto k) INLINE { acc[M][k] = mma(frag(fb[X][k]), am, acc[M][k]); });
+      if constexpr (M % 2 == 0)
+        part_of(std::integral_constant<int, I + 4>{}, s + 4, std::integral_constant<int, M / 2>{});
       __builtin_amdgcn_sched_barrier(0);
     });
-    turn(s + 2);
+    turn();
   };
   using std::integral_constant;
   stage(integral_constant<int, 0>{}, 0);
-  if (ns > 1) stage(integral_constant<int, 1>{}, 1);
-  if (ns > 2) stage(integral_constant<int, 2>{}, 2);
-  if (ns > 3) stage(integral_constant<int, 3>{}, 3);
-  turn(1);
+  stage(integral_constant<int, 1>{}, 1);
+  stage(integral_constant<int, 2>{}, 2);
+  stage(integral_constant<int, 3>{}, 3);
+  turn();
   each<24>([&](auto r) INLINE { read(integral_constant<int, 0>{}, s0, r); });
-  for (int s = 0; s < ns; s += 2 * NB)
-    each<2 * NB>([&](auto n) INLINE {
-      if (s + n < ns) step(n, s + n);
-    });
+  static_assert(NB == 5, "ten steps a round");
+  for (int s = 0;;) {
+    step(integral_constant<int, 0>{}, s);
+    if (++s == ns) break;
+    step(integral_constant<int, 1>{}, s);
+    if (++s == ns) break;
+    step(integral_constant<int, 2>{}, s);
+    if (++s == ns) break;
+    step(integral_constant<int, 3>{}, s);
+    if (++s == ns) break;
+    step(integral_constant<int, 4>{}, s);
+    if (++s == ns) break;
+    step(integral_constant<int, 5>{}, s);
+    if (++s == ns) break;
+    step(integral_constant<int, 6>{}, s);
+    if (++s == ns) break;
+    step(integral_constant<int, 7>{}, s);
+    if (++s == ns) break;
+    step(integral_constant<int, 8>{}, s);
+    if (++s == ns) break;
+    step(integral_constant<int, 9>{}, s);
+    if (++s == ns) break;
+  }
 
   // a lane has four columns of a row
   float* to = a.part + (long)part * a.N * a.K;

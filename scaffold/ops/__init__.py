@@ -396,10 +396,10 @@ def _colsum(dy2: torch.Tensor) -> torch.Tensor:
 def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """dy^T x of contiguous rows.  The library splits the rows too little
     where dW has few tiles: in us, library and own kernel, 3072 x 768 out of
-    16384 rows 152 and 90, of 8192 77 and 55, of 4096 42 and 41; 1024 x 4096
-    (64 tiles of 256 x 256) 166 and 130, 85 and 77, 45 and 51; with 100 tiles
-    8192 rows take 120 and 115.  Tiles that are mostly empty are not worth it:
-    8192 rows, 32 x 256 19 and 30, 64 x 64 45 and 30, 64 x 16384 63 and 75, 256 x
+    16384 rows 152 and 85, of 8192 77 and 52, of 4096 42 and 39; 1024 x 4096
+    (64 tiles of 256 x 256) 166 and 126, 85 and 73, 45 and 50; with 100 tiles
+    8192 rows take 120 and 116.  Tiles that are mostly empty are not worth it:
+    8192 rows, 32 x 256 19 and 33, 64 x 64 45 and 30, 64 x 16384 63 and 69, 256 x
     16384 108 and 86."""
     n, k = dy.shape[1], x.shape[1]
     small, large = min(n, k), max(n, k)
