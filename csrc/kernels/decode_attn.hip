@@ -660,6 +660,13 @@ torch::Tensor decode_attention(torch::Tensor qkv, torch::Tensor k,
   if (a.matrix) {
     want = std::max(1, std::min((full + 1) / 2, 256 / pairs));
     if (4l * L * std::max(D, 64) * (want - 1) <= 256l * 1024 * want) want = 1;
+    // A few more blocks than compute units leave some with two and most with one; three
+    // spans a row share them out.  One span and three, us: 32 heads of 128 on 8, caches
+    // of 4096 near their end, 33 rows 98 and 75, 40 104 and 87, 44 109 and 95, 48 111
+    // and 107; while only 512 places are taken, 15.2 and 17.5, 15.9 and 19.6, 16.2 and
+    // 21.3.  Caches of 2048 gain less than their first steps would lose (40 rows: 58
+    // and 51), and so do heads of 64 (40 rows of 4096: 53 and 52).
+    if (pairs > 256 && pairs <= 352 && (long)L * D >= 512l * 1024) want = 3;
   } else {
     a.waves = pairs >= 256 ? 4 : 8;
     want = std::max(1, std::min(rep == 1 ? full : (full + 1) / 2,

@@ -264,3 +264,28 @@ def test_a_cache_without_places_is_refused(H):
     with pytest.raises(RuntimeError, match="places"):
         ops.require_ext().decode_attention(
             qkv, k, v, torch.zeros(1, dtype=torch.int64, device="cuda"), None, None, None, H)
+
+
+@pytest.mark.parametrize("D,B,G,L", [
+    (128, 33, 8, 4096), (128, 43, 6, 4100), (128, 44, 8, 4161), (128, 89, 4, 4096),
+    (64, 257, 1, 8192)])
+def test_a_few_more_blocks_than_compute_units(D, B, G, L):
+    """Rows that fill the chip once and a little walk their keys in three spans;
+    depths at the spans' edges, and rows whose later spans are empty."""
+    from scaffold import ops
+
+    torch.manual_seed(B + L)
+    H, dev = 4 * G, "cuda"
+    span = ((L + 63) // 64 + 2) // 3 * 64
+    edges = [L - 1, 0, 1, span - 1, span, span + 1, 2 * span - 1, 2 * span, 63, 64]
+    qkv = torch.randn(B, (H + 2 * G) * D, device=dev).bfloat16()
+    k, v = (torch.randn(B, G, L, D, device=dev).bfloat16() for _ in range(2))
+    pos = torch.randint(0, L, (B,), device=dev)
+    pos[:len(edges)] = torch.tensor(edges, device=dev)
+    got = ops.require_ext().decode_attention(qkv, k, v, pos, None, None, None, H)
+    for r in range(0, B, 11):                 # float64 of a few rows at a time
+        rows = slice(r, min(B, r + 11))
+        want = _reference(qkv[rows], k[rows], v[rows], pos[rows], None, H)[0]
+        # one rounding of the result: 2^-9
+        err = (got[rows].double() - want).norm(dim=1) / want.norm(dim=1)
+        assert err.max() < 2 * 2 ** -9, err
