@@ -187,3 +187,29 @@ def test_benchmark_runs():
     from pathlib import Path
 
     runpy.run_path(str(Path(__file__).parents[2] / "benchmarks" / "bn_only.py"))
+
+
+@pytest.mark.parametrize("R", [4 * 65535, 4 * 65535 + 1, 300001])
+def test_more_rows_than_a_grid_of_four(R):
+    """Rows of 2048 channels, four to a block, up to and beyond a grid's limit;
+    channels are independent, so that eight of them tell."""
+    from scaffold import ops
+
+    torch.manual_seed(R)
+    C = 2048
+    x, dy, res = (torch.randn(1, R, 1, C, device="cuda", dtype=torch.bfloat16)
+                  .permute(0, 3, 1, 2) for _ in range(3))
+    w, b = torch.rand(C, device="cuda") + 0.5, torch.randn(C, device="cuda") * 0.1
+    rm, rv = torch.zeros(C, device="cuda"), torch.ones(C, device="cuda")
+    some = [0, 7, 8, 1023, 1024, 2039, 2040, 2047]
+    want, pre = _exact(*(t[:, some] for t in (x, res)),
+                       *(t[some] for t in (w, b, rm, rv)), True, dy[:, some])
+    ins = [t.requires_grad_() for t in (x, w, b, res)]
+    y = ops.batch_norm_act(x, res, w, b, rm, rv, 0.1, 1e-5, True, True)
+    dx, _, _, dres = torch.autograd.grad(y, ins, dy)
+    for name, g, e in (("y", y, want[0]), ("dx", dx, want[1]), ("dres", dres, want[4])):
+        # one bf16 rounding (2^-9), float32 statistics behind it; a sign within
+        # float32's error of zero may fall on either side
+        g = g.detach()[:, some].double()
+        bound = 2.0 ** -8 * e.abs() + 1e-4 * e.abs().max()
+        assert (((g - e).abs() <= bound) | (pre.abs() < 1e-5)).all(), name
