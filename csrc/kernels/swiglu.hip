@@ -4,7 +4,7 @@
 //        du = dh * silu(g)
 // vs eager (separate silu + mul + their backwards) this halves the HBM
 // passes over the (M, d_ff) activations.  Pure-bandwidth kernel:
-// bf16x8 vector loads (G13), grid-stride, fp32 math.
+// bf16x8 vector loads (G13), fp32 math.
 
 #include "../common.h"
 
@@ -56,40 +56,49 @@ swiglu_bwd_kernel(const short* __restrict__ dh, const short* __restrict__ g,
 
 // packed variant: gate|up live in ONE [M][2F] buffer (the fused
 // gate+up GEMM's output); h = silu(gu[:, :F]) * gu[:, F:].
+//
+// A block has 256 eights of the (rows, F8) next to each other and ends: 8192 x 14336,
+// bwd 231 -> 209 us (5.6 TB/s), fwd 126 -> 115 (6.1), against 2048 blocks that walk
+// with the grid's stride and divide 64 bits at each step; two eights a thread 207
+// and 121, four 212 and 119.
+struct Place { long gu, h; bool in; };
+
+DEVINL Place place(long first, long total, int F8) {
+  const long row = first / F8;                  // the block's: uniform
+  const unsigned at = (unsigned)(first - row * F8) + threadIdx.x;
+  const unsigned r = at / (unsigned)F8, c8 = at - r * F8;
+  return {((row + r) * 2 * F8 + c8) * 8, ((row + r) * F8 + c8) * 8,
+          first + threadIdx.x < total};
+}
+
 __global__ void __launch_bounds__(256)
 swiglu_packed_fwd_kernel(const short* __restrict__ gu, short* __restrict__ h,
-                         long rows, int F8) {
-  const long stride = grid_stride();
-  const long total = rows * F8;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-    const long row = i / F8;
-    const int c8 = (int)(i % F8);
-    const short* gp = gu + row * (2L * 8 * F8) + c8 * 8;
-    bf16x8 gv = *(const bf16x8*)gp;
-    bf16x8 uv = *(const bf16x8*)(gp + 8L * F8);
+                         long total, int F8) {
+  for (long first = blockIdx.x * 256l; first < total; first += gridDim.x * 256l) {
+    const Place p = place(first, total, F8);
+    if (!p.in) return;
+    const bf16x8 gv = *(const bf16x8*)(gu + p.gu);
+    const bf16x8 uv = *(const bf16x8*)(gu + p.gu + 8L * F8);
     bf16x8 out;
     #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float x = bf2f(gv[j]);
       out[j] = f2bf(x * sigm(x) * bf2f(uv[j]));
     }
-    *(bf16x8*)(h + row * (8L * F8) + c8 * 8) = out;
+    *(bf16x8*)(h + p.h) = out;
   }
 }
 
 __global__ void __launch_bounds__(256)
 swiglu_packed_bwd_kernel(const short* __restrict__ dh,
                          const short* __restrict__ gu,
-                         short* __restrict__ dgu, long rows, int F8) {
-  const long stride = grid_stride();
-  const long total = rows * F8;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-    const long row = i / F8;
-    const int c8 = (int)(i % F8);
-    const short* gp = gu + row * (2L * 8 * F8) + c8 * 8;
-    bf16x8 gv = *(const bf16x8*)gp;
-    bf16x8 uv = *(const bf16x8*)(gp + 8L * F8);
-    bf16x8 dhv = *(const bf16x8*)(dh + row * (8L * F8) + c8 * 8);
+                         short* __restrict__ dgu, long total, int F8) {
+  for (long first = blockIdx.x * 256l; first < total; first += gridDim.x * 256l) {
+    const Place p = place(first, total, F8);
+    if (!p.in) return;
+    const bf16x8 gv = *(const bf16x8*)(gu + p.gu);
+    const bf16x8 uv = *(const bf16x8*)(gu + p.gu + 8L * F8);
+    const bf16x8 dhv = *(const bf16x8*)(dh + p.h);
     bf16x8 dgv, duv;
     #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -101,10 +110,14 @@ swiglu_packed_bwd_kernel(const short* __restrict__ dh,
       dgv[j] = f2bf(d * bf2f(uv[j]) * dsi);
       duv[j] = f2bf(d * si);
     }
-    short* op = dgu + row * (2L * 8 * F8) + c8 * 8;
-    *(bf16x8*)op = dgv;
-    *(bf16x8*)(op + 8L * F8) = duv;
+    *(bf16x8*)(dgu + p.gu) = dgv;
+    *(bf16x8*)(dgu + p.gu + 8L * F8) = duv;
   }
+}
+
+// all of them, up to a launch's limit of 2^32 threads
+unsigned packed_blocks(long total) {
+  return (unsigned)std::min<long>((total + 255) / 256, 1 << 23);
 }
 
 }  // namespace
@@ -119,9 +132,9 @@ torch::Tensor swiglu_packed_fwd(torch::Tensor gu) {
   shape.back() = F;
   auto h = torch::empty(shape, gu.options());
   auto stream = scaffold_stream();
-  hipLaunchKernelGGL(swiglu_packed_fwd_kernel, dim3(capped_blocks(rows * (F / 8))),
+  hipLaunchKernelGGL(swiglu_packed_fwd_kernel, dim3(packed_blocks(rows * (F / 8))),
                      dim3(256), 0, stream, (const short*)gu.data_ptr(),
-                     (short*)h.data_ptr(), rows, (int)(F / 8));
+                     (short*)h.data_ptr(), rows * (F / 8), (int)(F / 8));
   HIP_CHECK(hipGetLastError());
   return h;
 }
@@ -132,10 +145,10 @@ torch::Tensor swiglu_packed_bwd(torch::Tensor dh, torch::Tensor gu) {
   const long rows = gu.numel() / (2 * F);
   auto dgu = torch::empty_like(gu);
   auto stream = scaffold_stream();
-  hipLaunchKernelGGL(swiglu_packed_bwd_kernel, dim3(capped_blocks(rows * (F / 8))),
+  hipLaunchKernelGGL(swiglu_packed_bwd_kernel, dim3(packed_blocks(rows * (F / 8))),
                      dim3(256), 0, stream, (const short*)dh.data_ptr(),
                      (const short*)gu.data_ptr(), (short*)dgu.data_ptr(),
-                     rows, (int)(F / 8));
+                     rows * (F / 8), (int)(F / 8));
   HIP_CHECK(hipGetLastError());
   return dgu;
 }
