@@ -58,7 +58,7 @@ swiglu_bwd_kernel(const short* __restrict__ dh, const short* __restrict__ g,
 // gate+up GEMM's output); h = silu(gu[:, :F]) * gu[:, F:].
 //
 // A block has 256 eights of the (rows, F8) next to each other and ends: 8192 x 14336,
-// bwd 231 -> 209 us (5.6 TB/s), fwd 126 -> 115 (6.1), against 2048 blocks that walk
+// bwd 231 -> 210 us (5.6 TB/s), fwd 126 -> 119 (5.9), against 2048 blocks that walk
 // with the grid's stride and divide 64 bits at each step; two eights a thread 207
 // and 121, four 212 and 119.
 struct Place { long gu, h; bool in; };
