@@ -216,7 +216,9 @@ void pick(const TileArgs& a, int tile, hipStream_t st) {
 // The tile, or -1 where a library is faster.  In us, library and this: little of all but the
 // depth, 1024 from 4096, 256 rows 10.7 and 14.4, 400 13.8 and 14.6, 700 17.8 and 15.1; 768 to
 // 768, 65 rows 4.8 and 5.4, 100 6.0 and 5.5.  Tiles of 128 x 128: 4096 from 4096, 700 rows 30.4
-// and 31.6, 2048 from 8192, 1500 rows 56.9 and 66.0, 2048 from 2048 19.2 and 16.5.  Of 128 x 256
+// and 31.6, 2048 from 8192, 1500 rows (192 tiles) 56 and 66, 1600 (208) 67.2 and 65.2, 1700
+// 64 and 53, 2032 73 and 69, 4096 from 14336, 700 rows (192) 97 and 106, 850 (224) 131 and 121,
+// 8192 from 4096, 500 rows (256) 43 and 40, 2048 from 2048 19.2 and 16.5.  Of 128 x 256
 // with nothing behind them: 3072 from 1024, 1500 rows (144 tiles) 15.9 and 17.8, 2304 from 768,
 // 2536 (180) 15.7 and 15.1; with a GELU, of which a launch is saved, 4096 from 1024, 1500 rows
 // (192) 26.4 and 20.9, 3072 from 768, 4096 rows (384) 38.4 and 31.2, but 6400 from 1600, 1500
@@ -227,7 +229,8 @@ int tile_of(const TileArgs& a, TileAct act) {
   if (a.M < 96 || few * 32 < a.K) return -1;
   if (few <= 256) return 0;
   if (tiles(128, 64) <= 256) return 1;
-  if (tiles(128, 128) <= 256) return a.K <= 2048 ? 2 : -1;
+  const long square = tiles(128, 128);
+  if (square <= 256) return a.K <= 2048 || square >= 208 ? 2 : -1;
   const long wide = tiles(128, 256);
   if (act != TILE_NONE) return wide <= 256 || (wide <= 512 && a.K <= 1024) ? 3 : -1;
   return wide >= 180 && wide <= 256 && a.K <= 1024 ? 3 : -1;

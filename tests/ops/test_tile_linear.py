@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
     (96, 2048, 64), (97, 1000, 128), (127, 1544, 192), (129, 5000, 320),
     (1024, 1024, 576), (1025, 1024, 64), (1000, 2056, 704), (2047, 1032, 128),
     (2048, 2040, 64), (1153, 3072, 192), (1920, 2048, 448), (2049, 2816, 64),
-    (2300, 2560, 128), (4096, 3000, 320)])
+    (2300, 2560, 128), (4096, 3000, 320), (1665, 2040, 2112), (641, 4600, 4160)])
 @pytest.mark.parametrize("act", [0, 1, 2])
 @pytest.mark.parametrize("bias", [False, True])
 def test_matches_float64(M, N, K, act, bias):
