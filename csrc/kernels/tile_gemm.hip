@@ -255,7 +255,9 @@ void tile_gemm(const TileArgs& a, TileAct act, hipStream_t st) {
 // act(x w^T + b) of rows (..., K), act as TileAct; None: not what it is for
 c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Tensor& w,
                                          const c10::optional<torch::Tensor>& bias, long act) {
-  // what a plain kernel would not see: gradients, transforms, tensors of Python classes
+  // what a plain kernel would not see: gradients, transforms, tensors of Python classes,
+  // modes that watch each call
+  if (c10::impl::dispatch_mode_enabled()) return c10::nullopt;
   auto plain = [&](const torch::Tensor& t) {
     const auto keys = t.key_set();
     return t.is_cuda() && t.scalar_type() == torch::kBFloat16 && t.device() == x.device() &&

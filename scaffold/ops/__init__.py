@@ -507,8 +507,9 @@ def _product(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None
              ) -> torch.Tensor:
     """F.linear without a graph, of some hundred rows by tiles of our own, which
     take more of the chip there (both sides' times: csrc/kernels/tile_gemm.hip)."""
-    m = ext()
-    y = m.tile_linear(x, w, b) if m is not None and x.is_cuda else None
+    y = None
+    if x.is_cuda and not torch.compiler.is_compiling() and ext() is not None:
+        y = ext().tile_linear(x, w, b)
     return F.linear(x, w, b) if y is None else y
 
 
@@ -576,7 +577,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None
     if x.is_cuda and _HAND_GEMM_ALL and _tile_ok(x, w):
         return _LinearFn.apply(x, w, b)
     if x.is_cuda and x.dtype == torch.bfloat16:
-        if not torch.is_grad_enabled() and not _transformed():
+        if (not torch.is_grad_enabled() and not torch.compiler.is_compiling()
+                and not _transformed()):
             return _product(x, w, b)
         return _LinearLib.apply(x, w, b)
     return F.linear(x, w, b)
@@ -585,10 +587,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None
 def linear_gelu_erf(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """gelu(x w^T), the erf form, without a graph; in one kernel where _product()
     is ours."""
-    m = ext()
-    if (m is not None and x.is_cuda and x.dtype == torch.bfloat16
-            and not torch.is_grad_enabled() and not _transformed()):
-        y = m.tile_linear(x, w, None, 2)
+    if (x.is_cuda and x.dtype == torch.bfloat16 and not torch.is_grad_enabled()
+            and not torch.compiler.is_compiling() and not _transformed()
+            and ext() is not None):
+        y = ext().tile_linear(x, w, None, 2)
         if y is not None:
             return y
     return gelu_erf(linear(x, w))

@@ -78,3 +78,20 @@ def test_leaves_what_it_is_not_for():
     for g, r in ((gx, rx), (gw, rw)):
         # y rounded, and the gradient of it, and the result: 2^-9 each
         assert (g.double() - r.double()).norm() <= 3 * 2.0 ** -9 * r.double().norm()
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_seen_by_modes_and_by_the_compiler(grad):
+    """A product stays a product for what counts or traces calls."""
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from scaffold import ops
+
+    x, w = (torch.randn(n, 768, device="cuda").bfloat16() for n in (256, 2304))
+    with torch.set_grad_enabled(grad):
+        with FlopCounterMode(display=False) as flops:
+            y = ops.linear(x, w)
+        assert flops.get_total_flops() == 2 * 256 * 768 * 2304
+        whole = torch.compile(lambda t: ops.linear(t, w), backend="eager", fullgraph=True)
+        # one rounding either way
+        torch.testing.assert_close(whole(x), y, rtol=2 ** -7, atol=2 ** -10)
