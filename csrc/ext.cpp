@@ -68,6 +68,8 @@ void save_shard_pinned(std::string path, std::vector<std::string> names,
                        std::vector<std::string> meta_keys,
                        std::vector<std::string> meta_vals);
 torch::Tensor weight_grad(torch::Tensor dy, torch::Tensor x);
+c10::optional<torch::Tensor> wide_weight_grad(const torch::Tensor& dy, const torch::Tensor& x);
+c10::optional<torch::Tensor> input_grad(const torch::Tensor& dy, const torch::Tensor& w);
 std::vector<torch::Tensor> linear_fwd(torch::Tensor x, torch::Tensor w,
                                       c10::optional<torch::Tensor> bias,
                                       long epilogue,
@@ -116,6 +118,15 @@ std::vector<torch::Tensor> bn_bwd(torch::Tensor dy, torch::Tensor x,
                                   torch::Tensor mean, torch::Tensor rstd,
                                   bool relu);
 
+// f of two tensors, or None: classes and modes that override functions see torch's product
+template <typename F>
+c10::optional<torch::Tensor> exact(F f, const py::object& a, const py::object& b) {
+  if (at::impl::torch_function_mode_enabled() || !THPVariable_CheckExact(a.ptr()) ||
+      !THPVariable_CheckExact(b.ptr()))
+    return c10::nullopt;
+  return f(a.cast<torch::Tensor>(), b.cast<torch::Tensor>());
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_adamw", &fused_adamw, "fused multi-tensor AdamW (K1)");
   m.def("adamw_build_meta", &adamw_build_meta,
@@ -161,6 +172,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "stream tensors to a safetensors shard via pinned D2H (C6)");
   m.def("weight_grad", &weight_grad, "dY^T X of few tiles, split over rows",
         py::arg("dy"), py::arg("x"));
+  m.def("wide_weight_grad", [](py::object dy, py::object x) { return exact(wide_weight_grad, dy, x); },
+        "weight_grad where that is faster than a library, or None", py::arg("dy"),
+        py::arg("x"));
+  m.def("input_grad", [](py::object dy, py::object w) { return exact(input_grad, dy, w); },
+        "dY W where that is faster than a library, or None", py::arg("dy"), py::arg("w"));
   m.def("linear_fwd", &linear_fwd,
         "MFMA linear fwd, fused bias+GELU/residual epilogue (K5)");
   m.def("bn_fwd", &bn_fwd,

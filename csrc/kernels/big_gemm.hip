@@ -1,0 +1,107 @@
+// Large products on the matrix cores: where they are faster than a library's, and how
+// they are split.  The kernel, and what bounds it: big_gemm.h.
+
+#include <c10/core/DeviceGuard.h>
+
+#include "../common.h"
+#include "../plain.h"
+#include "big_gemm.h"
+
+namespace {
+
+constexpr long UNITS = 256;          // compute units, each with one block
+
+long up(long a, long b) { return (a + b - 1) / b; }
+
+// Results that the caches would not keep go past them: in us, through and past, 4096 x 28672
+// x 4096 731 and 685, 8192 x 8192 x 8192 757 and 741, 16384 x 3072 x 768 64 and 68.
+template <bool ACOL, bool BCOL, int NT, int ACT>
+void launch(BigArgs a, hipStream_t st) {
+  a.tiles = (unsigned)(up(a.M, 256) * up(a.N, 32 * NT));
+  a.stream = 2l * a.M * a.N > 112l << 20;
+  hipLaunchKernelGGL((big::gemm_kernel<ACOL, BCOL, NT, ACT>),
+                     dim3(std::min<unsigned>(a.tiles, UNITS)), dim3(256), 0, st, a);
+}
+
+// Tiles of 256 x 256, or of 256 x 192 where these leave less of the chip idle: a round of
+// them takes 0.82 of the time.  In us, 256 and 192 wide: x w^T, 16384 x 2304 x 768 62 and 51,
+// 16384 x 768 x 3072 71 and 65, 8192 x 3072 x 2048 97 and 81, 8192 x 2048 x 2048 54 and 78.
+double rounds(const BigArgs& a, int nt) {
+  return (double)up(up(a.M, 256) * up(a.N, 32 * nt), UNITS) * (nt == 6 ? 0.82 : 1.);
+}
+
+int columns(const BigArgs& a) { return rounds(a, 6) < rounds(a, 8) ? 6 : 8; }
+
+// the chip's part that full tiles take over that many rounds
+double at_work(const BigArgs& a, double rounds) {
+  return (double)a.M * (double)a.N / (65536. * UNITS * rounds);
+}
+
+}  // namespace
+
+// dW[N][K] = sum over t of dY[t][N] X[t][K] where that is faster than a library's, else None:
+// where tiles keep two thirds of the chip at work.  In us, library and this: 28672 x 4096 out
+// of 8192 rows 1646 and 1272, of 500 176 and 106; 4096 x 4096 out of 8192 240 and 188; 6144 x
+// 4096 out of 1000 66 and 52; but 608 x 12888 out of 11800 (0.60) 225 and 236.
+//
+// Sums run in the library's order, and the gradients are the same bits, but where it splits
+// the tiles of a last round.  Deep sums of few rounds whose last is half empty stay with it:
+// 4096 x 14336 out of 8192 rows would take 721 instead of 982, but 5000 of its 59 million
+// gradients are rounded otherwise, after which a step of AdamW leaves the next gradients
+// 2 % apart, the most that bf16 lets them.  (128256 x 4096, the head, of 31 rounds, 7361 and
+// 5691: 5000 of 525 million, and 0.7 %.)
+c10::optional<torch::Tensor> wide_weight_grad(const torch::Tensor& dy, const torch::Tensor& x) {
+  if (watched() || !dy.is_cuda() || !plain(dy, dy.device()) || !plain(x, dy.device()) ||
+      dy.dim() != 2 || x.dim() != 2 || dy.size(0) != x.size(0) || !dy.is_contiguous() ||
+      !x.is_contiguous() || ((size_t)dy.data_ptr() | (size_t)x.data_ptr()) % 16)
+    return c10::nullopt;
+  const long T = x.size(0), N = dy.size(1), K = x.size(1);
+  if (T < 256 || T >= 1l << 30 || N < 256 || K < 256 || N % 8 || K % 8 || N > 1l << 22 ||
+      K > 1l << 22)
+    return c10::nullopt;
+  BigArgs a = {};
+  a.a = (const short*)dy.data_ptr();
+  a.b = (const short*)x.data_ptr();
+  a.M = (int)N; a.N = (int)K; a.K = (int)T;
+  a.lda = N; a.ldb = a.ldy = K;
+  const long tiles = up(N, 256) * up(K, 256), last = tiles % UNITS;
+  if (at_work(a, rounds(a, 8)) < 0.66 ||
+      (T >= 8192 && tiles < 4 * UNITS && last > 0 && last <= UNITS / 2))
+    return c10::nullopt;
+  // the operands' device, whichever is current: torch's product goes by it too
+  const c10::DeviceGuard guard(dy.device());
+  auto dw = torch::empty({N, K}, x.options());
+  a.y = (short*)dw.data_ptr();
+  launch<true, true, 8, BIG_NONE>(a, scaffold_stream());
+  HIP_CHECK(hipGetLastError());
+  return dw;
+}
+
+// dX[M][K] = sum over n of dY[M][n] W[n][K] where that is faster than a library's, else None:
+// where tiles keep 0.72 of the chip at work, of 150 sizes every one.  In us, library and this:
+// 16384 rows, 768 from 3072 86 and 68, 3072 from 768 85 and 68, 8192 rows, 4096 from 28672 1400
+// and 1302, 14336 from 4096 716 and 642; but 2000 rows, 4096 from 28672 (0.60) 394 and 472.
+c10::optional<torch::Tensor> input_grad(const torch::Tensor& dy, const torch::Tensor& w) {
+  if (watched() || !dy.is_cuda() || !plain(dy, dy.device()) || !plain(w, dy.device()) ||
+      dy.dim() != 2 || w.dim() != 2 || dy.size(1) != w.size(0) || !dy.is_contiguous() ||
+      !w.is_contiguous() || ((size_t)dy.data_ptr() | (size_t)w.data_ptr()) % 16)
+    return c10::nullopt;
+  const long M = dy.size(0), N = w.size(0), K = w.size(1);
+  if (M < 256 || M >= 1l << 30 || N < 128 || N % 128 || N > 1l << 22 || K < 256 || K % 8 ||
+      K > 1l << 22)
+    return c10::nullopt;
+  BigArgs a = {};
+  a.a = (const short*)dy.data_ptr();
+  a.b = (const short*)w.data_ptr();
+  a.M = (int)M; a.N = (int)K; a.K = (int)N;
+  a.lda = N; a.ldb = a.ldy = K;
+  const int nt = columns(a);
+  if (at_work(a, rounds(a, nt)) < 0.72) return c10::nullopt;
+  const c10::DeviceGuard guard(dy.device());
+  auto dx = torch::empty({M, K}, dy.options());
+  a.y = (short*)dx.data_ptr();
+  if (nt == 6) launch<false, true, 6, BIG_NONE>(a, scaffold_stream());
+  else launch<false, true, 8, BIG_NONE>(a, scaffold_stream());
+  HIP_CHECK(hipGetLastError());
+  return dx;
+}

@@ -17,11 +17,10 @@
 // 12.4, 2536 20.1 and 19.4; 2048 to 8192, GELU behind it, 256 rows 28.4 and 17.5, 1024 rows 46.0
 // and 36.6; 2048 to 2048, 1600 rows 20.4 and 18.4; 4096 to 6144, 256 rows 37.4 and 24.7.
 
-#include <ATen/TracerMode.h>
-#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 
 #include "../common.h"
+#include "../plain.h"
 #include "tile_gemm.h"
 
 namespace {
@@ -270,23 +269,9 @@ void tile_gemm(const TileArgs& a, TileAct act, hipStream_t st) {
 // act(x w^T + b) of rows (..., K), act as TileAct; None: not what it is for
 c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Tensor& w,
                                          const c10::optional<torch::Tensor>& bias, long act) {
-  // what a plain kernel would not see: gradients, transforms, tensors of Python classes,
-  // modes that watch each call, autocast to another type, and a trace, which would hold the
-  // memory of the result without what was written to it
-  if (c10::impl::dispatch_mode_enabled() || at::tracer::impl::is_dispatch_enabled() ||
-      (at::autocast::is_autocast_enabled(at::kCUDA) &&
-       at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16))
-    return c10::nullopt;
-  auto plain = [&](const torch::Tensor& t) {
-    // nothing but memory on the device: no wrapper, no batch, no tensor of zeros without
-    // any
-    const auto keys = t.key_set() - c10::autograd_dispatch_keyset -
-                      c10::autocast_dispatch_keyset -
-                      c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView);
-    return keys == c10::DispatchKeySet(c10::DispatchKey::CUDA) &&
-           t.scalar_type() == torch::kBFloat16 && t.device() == x.device() &&
-           !t._fw_grad(0).defined() && !(at::GradMode::is_enabled() && t.requires_grad());
-  };
+  // what a plain kernel would not see: gradients, transforms, tensors of Python classes
+  if (watched()) return c10::nullopt;
+  auto plain = [&](const torch::Tensor& t) { return ::plain(t, x.device()); };
   if (!x.defined() || x.dim() < 2 || w.dim() != 2 || act < 0 || act > 2 || !plain(x) || !plain(w) ||
       (bias.has_value() && !plain(*bias)) || x.size(-1) != w.size(1) || !w.is_contiguous() ||
       x.stride(-1) != 1 || (x.dim() > 2 && !x.is_contiguous()) ||

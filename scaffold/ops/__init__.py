@@ -400,17 +400,34 @@ def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     (64 tiles of 256 x 256) 166 and 126, 85 and 73, 45 and 50; with 100 tiles
     8192 rows take 120 and 116.  Tiles that are mostly empty are not worth it:
     8192 rows, 32 x 256 19 and 30, 64 x 64 45 and 30, 64 x 16384 63 and 75, 256 x
-    16384 108 and 86."""
+    16384 108 and 86.  Where tiles fill the chip, another: csrc/kernels/big_gemm.hip."""
     n, k = dy.shape[1], x.shape[1]
-    small, large = min(n, k), max(n, k)
-    if (x.is_cuda and small >= 64 and (small >= 256 or large <= 8192)
-            and dy.dtype == x.dtype == torch.bfloat16
-            and x.shape[0] >= 8192 and n % 8 == 0 and k % 8 == 0
-            and 0 < -(-n // 256) * -(-k // 256) <= 64
-            and not torch.is_grad_enabled() and not _transformed()
-            and dy.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0):
-        return require_ext().weight_grad(dy, x)
+    many = n * k >= 11_000_000                 # tiles for two thirds of the chip
+    if (x.is_cuda and (many or x.shape[0] >= 8192)
+            and not torch.is_grad_enabled() and not _transformed()):
+        small, large = min(n, k), max(n, k)
+        if (small >= 64 and (small >= 256 or large <= 8192)
+                and dy.dtype == x.dtype == torch.bfloat16
+                and x.shape[0] >= 8192 and n % 8 == 0 and k % 8 == 0
+                and 0 < -(-n // 256) * -(-k // 256) <= 64
+                and dy.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0):
+            return require_ext().weight_grad(dy, x)
+        dw = require_ext().wide_weight_grad(dy, x) if many else None
+        if dw is not None:
+            return dw
     return dy.t() @ x
+
+
+def _input_grad(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """dy w of contiguous rows, by a kernel of our own where that is faster
+    than the library's (both sides' times: csrc/kernels/big_gemm.hip)."""
+    if (dy.shape[0] * w.shape[1] >= 9_900_000  # tiles for most of the chip
+            and dy.is_cuda and not torch.is_grad_enabled()
+            and not _transformed()):
+        dx = require_ext().input_grad(dy, w)
+        if dx is not None:
+            return dx
+    return dy @ w
 
 
 # ------------------------------------------------- K5 hand MFMA linear
@@ -623,10 +640,10 @@ def linear_residual(x: torch.Tensor, w: torch.Tensor,
             _HAND_GEMM_ALL or (w.shape[0] <= 1024 and w.shape[1] <= 1024)):
         return _LinearResidualFn.apply(x, w, b, res)
     # one type throughout: autocast's float32 weights need torch's own backward
-    if (x.is_cuda and b is not None
-            and x.dtype == w.dtype == b.dtype == torch.bfloat16
+    if (x.is_cuda and x.dtype == w.dtype == torch.bfloat16
+            and (b is None or b.dtype == torch.bfloat16)
             and torch.is_grad_enabled() and not _transformed()):
-        return _LinearLib.apply(x, w, b) + res     # bias gradient: colsum
+        return _LinearLib.apply(x, w, b) + res     # gradients by own kernels
     return F.linear(x, w, b) + res
 
 

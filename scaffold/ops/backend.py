@@ -40,6 +40,7 @@ _SOURCES = [
     "kernels/attn_bwd_mfma.hip",
     "kernels/gemm_bf16.hip",
     "kernels/weight_grad.hip",
+    "kernels/big_gemm.hip",
     "kernels/swiglu.hip",
     "kernels/colsum.hip",
     "kernels/gather.hip",

@@ -1,0 +1,58 @@
+"""Large products by tiles: at the edges of tiles, over several tiles a block,
+past the caches."""
+
+import pytest
+import torch
+
+from scaffold import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(got, a, b):
+    """got = a b, of which every partial sum is below the sum of sizes: the
+    result's rounding, and that of depth / 32 + 32 float32 sums."""
+    a, b = a.double(), b.double()
+    want, size = a @ b, a.abs() @ b.abs()
+    lim = 2.0 ** -8 * want.abs() + (a.shape[1] / 32 + 32) * 2.0 ** -24 * size
+    assert got.shape == want.shape and ((got.double() - want).abs() <= lim).all()
+
+
+def _rows(n, m, mean=0.0):
+    """n rows of m, and NaN behind the last"""
+    t = torch.full((n + 64, m), torch.nan, device="cuda").bfloat16()
+    t[:n] = torch.randn(n, m, device="cuda") + mean
+    return t[:n]
+
+
+@pytest.mark.parametrize("T,N,K", [
+    (257, 5128, 8200),        # three tiles a block, the last ones partly empty
+    (4097, 3080, 3600),       # one tile a block, the last ones of eight rows
+    (300, 8192, 7432),        # a result that goes past the caches
+    (385, 10000, 1280)])
+def test_weight_gradients(T, N, K):
+    torch.manual_seed(T)
+    dy, x = _rows(T, N), _rows(T, K, 0.5)
+    got = ops.require_ext().wide_weight_grad(dy, x)
+    _close(got, dy.t(), x)
+    assert torch.equal(got, ops.require_ext().wide_weight_grad(dy, x))
+
+
+def test_weight_gradients_of_other_operands_are_left():
+    f = ops.require_ext().wide_weight_grad
+    dy, x = _rows(2048, 3328), _rows(2048, 3584)
+    assert f(dy, x) is not None
+    for a, b in ((dy.half(), x.half()), (dy, x[:-1]), (dy[:, :-4], x),
+                 (dy.t().contiguous().t(), x), (dy.cpu(), x), (dy[:128], x[:128]),
+                 (dy.clone().requires_grad_(), x)):
+        assert f(a, b) is None
+
+
+def test_infinite_rows_stay_where_they_are():
+    torch.manual_seed(3)
+    dy, x = _rows(2048, 3328), _rows(2048, 3584)
+    dy[:, 300] = torch.inf
+    got = ops.require_ext().wide_weight_grad(dy, x)
+    assert not got[300].isfinite().any()
+    rest = torch.cat([got[:300], got[301:]])
+    _close(rest, torch.cat([dy[:, :300], dy[:, 301:]], 1).t(), x)
