@@ -183,9 +183,10 @@ gemm_kernel(BigArgs a) {
   // beside the first products; then (FREE) all waves have what they need of its place, and
   // the copies of the stage after the next go there; when (HERE) the next stage has come,
   // in all waves, its first half is read.
-  constexpr int READ1 = R > 16 ? 1 : 2, FREE = READ1 * (R - 1) + 2 + (R > 24 ? 4 : 0);
-  constexpr int COPY = NT == 8 ? 5 : 4, READ2 = READ1;
-  constexpr int HERE = NT == 8 ? (R > 16 ? 84 : 88) : 56;
+  constexpr int READ1 = R <= 16 || R == 24 ? 2 : 1, READ2 = READ1;
+  constexpr int FREE = READ1 * (R - 1) + (R > 24 ? 6 : R == 24 ? 4 : 2);
+  constexpr int COPY = NT == 8 ? 5 : 4;
+  constexpr int HERE = NT < 8 ? 56 : R > 24 ? 84 : R == 24 ? 64 : 88;
   static_assert(FREE + 1 + COPY * (C - 1) < 2 * Q1 && HERE + 1 + READ2 * (R - 1) < 2 * Q1 &&
                 HERE + 1 >= Q1, "schedule");
   // stores of a tile, of which the first stage behind it takes no notice

@@ -457,7 +457,7 @@ class _LinearFn(torch.autograd.Function):
         x, w = ctx.saved_tensors
         dy2 = dy.contiguous().view(-1, dy.shape[-1])
         x2 = x.view(-1, x.shape[-1])
-        dx = (dy2 @ w).view(x.shape)
+        dx = _input_grad(dy2, w).view(x.shape)
         dw = _weight_grad(dy2, x2)
         db = _colsum(dy2) if ctx.has_bias else None
         return dx, dw, db
@@ -482,7 +482,7 @@ class _LinearGeluFn(torch.autograd.Function):
         dpre = torch.ops.aten.gelu_backward(dy, pre, approximate="tanh")
         dpre2 = dpre.contiguous().view(-1, dpre.shape[-1])
         x2 = x.view(-1, x.shape[-1])
-        dx = (dpre2 @ w).view(x.shape)
+        dx = _input_grad(dpre2, w).view(x.shape)
         dw = _weight_grad(dpre2, x2)
         db = _colsum(dpre2) if ctx.has_bias else None
         return dx, dw, db
@@ -506,7 +506,7 @@ class _LinearResidualFn(torch.autograd.Function):
         x, w = ctx.saved_tensors
         dy2 = dy.contiguous().view(-1, dy.shape[-1])
         x2 = x.view(-1, x.shape[-1])
-        dx = (dy2 @ w).view(x.shape)
+        dx = _input_grad(dy2, w).view(x.shape)
         dw = _weight_grad(dy2, x2)
         db = _colsum(dy2) if ctx.has_bias else None
         return dx, dw, db, dy
@@ -556,7 +556,7 @@ class _LinearLib(torch.autograd.Function):
         dy2 = dy.contiguous().view(-1, dy.shape[-1])
         dx = dw = None
         if w is not None:
-            dx = (dy2 @ w).view(ctx.x_shape)
+            dx = _input_grad(dy2, w).view(ctx.x_shape)
         if x is not None:
             dw = _weight_grad(dy2, x.contiguous().view(-1, x.shape[-1]))
         return dx, dw, _colsum(dy2) if ctx.need_b else None
@@ -587,7 +587,7 @@ class _LinearGeluLib(torch.autograd.Function):
             dpre, db = require_ext().gelu_bwd(dy.contiguous().view(-1, n),
                                               pre.view(-1, n))
         x2 = x.contiguous().view(-1, x.shape[-1])
-        return (dpre @ w).view(x.shape), _weight_grad(dpre, x2), db
+        return _input_grad(dpre, w).view(x.shape), _weight_grad(dpre, x2), db
 
 
 def _transformed() -> bool:

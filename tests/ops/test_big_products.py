@@ -56,3 +56,48 @@ def test_infinite_rows_stay_where_they_are():
     assert not got[300].isfinite().any()
     rest = torch.cat([got[:300], got[301:]])
     _close(rest, torch.cat([dy[:, :300], dy[:, 301:]], 1).t(), x)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (505, 128, 32760),        # one stage of each half, edges both ways
+    (5003, 256, 2568),        # tiles of 256 columns, the last of eight
+    (16001, 384, 760),        # of 192, one of them of one row
+    (16000, 2304, 760),
+    (8192, 640, 7432)])       # past the caches
+def test_input_gradients(M, N, K):
+    torch.manual_seed(M)
+    dy = _rows(M, N)
+    w = _rows(N, K, 0.5)
+    got = ops.require_ext().input_grad(dy, w)
+    _close(got, dy, w)
+    assert torch.equal(got, ops.require_ext().input_grad(dy, w))
+
+
+def test_input_gradients_of_other_operands_are_left():
+    f = ops.require_ext().input_grad
+    dy, w = _rows(4096, 512), _rows(512, 4096)
+    assert f(dy, w) is not None
+    for a, b in ((dy.half(), w.half()), (dy[:, :-8], w), (dy, w.t()),
+                 (dy[:, :448].contiguous(), w[:448].contiguous()), (dy.cpu(), w),
+                 (dy[:128], w), (dy, w.clone().requires_grad_())):
+        assert f(a, b) is None
+
+
+@pytest.mark.parametrize("act", [False, True])
+def test_layers_take_it(act, monkeypatch):
+    ext, calls = ops.require_ext(), []
+    made = ext.input_grad
+    monkeypatch.setattr(ext, "input_grad",
+                        lambda *a: calls.append(1) or made(*a))
+    torch.manual_seed(1)
+    x = torch.randn(4096, 4096, device="cuda").bfloat16().requires_grad_()
+    w = (torch.randn(512, 4096, device="cuda") / 64).bfloat16().requires_grad_()
+    b = torch.zeros(512, device="cuda").bfloat16().requires_grad_()
+    y = (ops.linear_gelu if act else ops.linear)(x, w, b)
+    dy = torch.randn_like(y)
+    (dx,) = torch.autograd.grad(y, x, dy, retain_graph=True)
+    assert len(calls) == 1
+    if not act:
+        _close(dx, dy, w.detach())
+    torch.autograd.grad(y, x, dy.requires_grad_(), create_graph=True)
+    assert len(calls) == 1
