@@ -122,7 +122,26 @@ DEVINL f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) {
       __builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
 }
 
-DEVINL float gelu_erf(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
+// z Phi(z), with Phi(-t) = 2^P(t), t = |z|: P of degree 10, P(0) = -1, fitted on [0, 7] to the
+// logarithm in 64 bits, weighted with Phi(-t), by least squares whose weights follow the
+// largest error (Lawson's method); behind 7 it only falls, and 2^P(16) is 0.  Largest errors
+// against 64 bits 5.6e-8 up to 1 and 2.4e-7 up to 12, where 0.5 z (1 + erff(z / sqrt 2)) has
+// 8.5e-8 and 4.5e-7, and 5e-5 of the value down to -5, there 5 %.
+DEVINL float gelu_erf(float z) {
+  const float t = fminf(fabsf(z), 16.f);
+  float p = -2.1855125709180358e-8f;
+  p = fmaf(p, t, 7.03961745784909e-7f);
+  p = fmaf(p, t, -9.565534128341824e-6f);
+  p = fmaf(p, t, 6.97065843269229e-5f);
+  p = fmaf(p, t, -2.606377238407731e-4f);
+  p = fmaf(p, t, -3.2546609872952104e-5f);
+  p = fmaf(p, t, 6.980439648032188e-3f);
+  p = fmaf(p, t, -5.246090516448021e-2f);
+  p = fmaf(p, t, -4.592151641845703e-1f);
+  p = fmaf(p, t, -1.1511048078536987f);
+  p = fmaf(p, t, -1.f);
+  return fmaf(z > 0.f ? -t : z, __builtin_amdgcn_exp2f(p), fmaxf(z, 0.f));
+}
 
 // tanh(u) = 1 - 2 / (exp(2u) + 1), also at both ends.  The reciprocal with a Newton step,
 // for which its operand stays finite: errors against 64 bits are those of a division to

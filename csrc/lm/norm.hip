@@ -267,22 +267,49 @@ void dispatch_norm(const NormArgs& a, bool f32, hipStream_t st) {
   else v4 ? launch_norm<false, 4>(a, st) : launch_norm<false, 1>(a, st);
 }
 
-template <bool F32>
+// Memory bounds it: 8192 x 8192 of bf16, read and written, 57 us with 8 bytes a load, blocks
+// with the whole grid's stride and erff(), whose instructions took as long; 42 (6.4 TB/s)
+// with U loads of 16 bytes in flight, a block's next to each other.  One load where that
+// leaves few blocks: 1000 x 1000 4.4 us with four, 3.8 with one.
+template <bool F32, int V, int U>
 __global__ void __launch_bounds__(256)
-gelu_erf_kernel(const void* in, void* out, long n4, long n) {
-  const long step = grid_stride();
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n4; i += step) {
-    Pack<4> p = ldv<F32, 4>(in, i * 4);
-    #pragma unroll
-    for (int j = 0; j < 4; ++j) p.v[j] = gelu_erf(p.v[j]);
-    stv<F32, 4>(out, i * 4, p);
+gelu_erf_kernel(const void* in, void* out, long n) {
+  typedef typename Num<F32>::E E;
+  struct alignas(V * sizeof(E)) Vec { E e[V]; };
+  const long first = ((long)blockIdx.x * U * 256 + threadIdx.x) * V;
+  Vec p[U];
+  #pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (first + u * 256 * V + V <= n) p[u] = *(const Vec*)((const E*)in + first + u * 256 * V);
+  #pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const long at = first + u * 256 * V;
+    if (at + V <= n) {
+      #pragma unroll
+      for (int j = 0; j < V; ++j) p[u].e[j] = Num<F32>::down(gelu_erf(Num<F32>::up(p[u].e[j])));
+      *(Vec*)((E*)out + at) = p[u];
+    } else {
+      for (long i = at; i < n; ++i)              // the last few
+        ((E*)out)[i] = Num<F32>::down(gelu_erf(Num<F32>::up(((const E*)in)[i])));
+    }
   }
-  const long tail = n4 * 4 + (long)blockIdx.x * 256 + threadIdx.x;
-  if (tail < n) {
-    Pack<1> p = ldv<F32, 1>(in, tail);
-    p.v[0] = gelu_erf(p.v[0]);
-    stv<F32, 1>(out, tail, p);
-  }
+}
+
+template <bool F32>
+void launch_gelu_erf(const void* in, void* out, long n, hipStream_t st) {
+  constexpr int V = F32 ? 4 : 8;
+  auto go = [&](auto v, auto u) {
+    constexpr int VEC = decltype(v)::value, U = decltype(u)::value;
+    const long each = 256 * VEC * U;
+    hipLaunchKernelGGL((gelu_erf_kernel<F32, VEC, U>), dim3((unsigned)((n + each - 1) / each)),
+                       dim3(256), 0, st, in, out, n);
+  };
+  constexpr std::integral_constant<int, V> wide;
+  constexpr std::integral_constant<int, 4> four;
+  constexpr std::integral_constant<int, 1> one;
+  if (((size_t)in | (size_t)out) % 16) go(one, four);
+  else if (n >= 1024 * 1024 * V) go(wide, four);
+  else go(wide, one);
 }
 
 // act(g) * u of rows [g | u], each n wide
@@ -418,12 +445,8 @@ void lm_replace_norm(float* x, const void* y, bool y_f32, const void* step,
 void lm_gelu_erf(const void* in, void* out, long n, bool f32,
                  hipStream_t stream) {
   if (n <= 0) return;
-  const long n4 = n / 4;
-  const dim3 grid(capped_blocks(std::max<long>(n4, 256), 256, 4096));
-  if (f32)
-    hipLaunchKernelGGL((gelu_erf_kernel<true>), grid, dim3(256), 0, stream, in, out, n4, n);
-  else
-    hipLaunchKernelGGL((gelu_erf_kernel<false>), grid, dim3(256), 0, stream, in, out, n4, n);
+  if (f32) launch_gelu_erf<true>(in, out, n, stream);
+  else launch_gelu_erf<false>(in, out, n, stream);
 }
 
 void lm_gated_act(const void* in, void* out, long rows, int n, int act,
