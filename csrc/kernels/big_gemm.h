@@ -29,7 +29,7 @@
 
 struct BigArgs {
   const short *a, *b;            // operands, of rows of lda and ldb
-  const short* bias;             // (N) or null
+  const short* bias;             // (N) or null; x w^T only
   short* y;                      // (M, N) of rows of ldy
   long lda, ldb, ldy;
   int M, N, K;
@@ -37,7 +37,7 @@ struct BigArgs {
   bool stream;                   // the result goes past the caches
 };
 
-enum BigAct { BIG_NONE, BIG_GELU_TANH, BIG_GELU_ERF };
+enum BigAct { BIG_NONE, BIG_GELU_ERF };
 
 namespace big {
 
@@ -277,7 +277,7 @@ gemm_kernel(BigArgs a) {
       return n0 + col < a.N ? 2 * (unsigned)(row * (int)a.ldy + col) : 0xfffffff0u;
     };
     auto act = [](float v) INLINE {
-      return ACT == BIG_GELU_TANH ? gelu_tanh(v) : ACT == BIG_GELU_ERF ? gelu_erf(v) : v;
+      return ACT == BIG_GELU_ERF ? gelu_erf(v) : v;
     };
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
     typedef unsigned u32x3 __attribute__((ext_vector_type(3)));

@@ -6,6 +6,7 @@
 #include "../common.h"
 #include "../plain.h"
 #include "big_gemm.h"
+#include "tile_gemm.h"
 
 namespace {
 
@@ -37,7 +38,47 @@ double at_work(const BigArgs& a, double rounds) {
   return (double)a.M * (double)a.N / (65536. * UNITS * rounds);
 }
 
+BigArgs of(const TileArgs& t) {
+  BigArgs a = {};
+  a.a = t.x; a.b = t.w; a.bias = t.bias; a.y = t.y;
+  a.lda = t.ldx; a.ldb = t.K; a.ldy = t.ldy;
+  a.M = t.M; a.N = t.N; a.K = t.K;
+  return a;
+}
+
+// columns of x w^T, whose lanes store as many as a block has products across
+int width(const BigArgs& a) { return a.N % 24 ? 8 : columns(a); }
+
 }  // namespace
+
+// Where it is faster than a library, of 120 sizes of 512 to 16384 rows next to every one.  In
+// us, library and this.  Shallow products, whose stores a library waits for: 16384 rows, 768 to
+// 2304 69 and 53, to 3072 78 and 67; 9208 x 1656 x 512 35 and 20; 1152 x 28168 x 896 (0.64) 79
+// and 74; but 8360 x 14088 x 128 83 and 92.  Deeper ones with tiles left over, for which 192
+// columns or persistent blocks are better: 8192 x 3072 x 2048 91 and 82, 13360 x 2304 x 3072 246
+// and 143, 5080 x 18216 x 3328 436 and 432; but full rounds, 8192 x 2048 x 2048, 51 and 54,
+// and 10024 x 5752 x 6016 488 and 488.  With the erf GELU behind it a pass over memory is
+// saved: 8192 x 8192 x 2048 244 and 221, 2032 x 8192 x 2048 69 and 61, 11728 x 8352 x 5888 (0.97)
+// 0.92 of it, but 6152 x 7760 x 6784 (0.71) 1.02, 2064 x 4528 x 3072 (0.56) 1.05.
+bool big_takes(const TileArgs& t, TileAct act) {
+  const BigArgs a = of(t);
+  if (act == TILE_GELU_TANH || t.M < 256 || t.N < 128 || t.N % 8 || t.K < 128 || t.K % 128 ||
+      t.K > 1 << 22 || t.ldx % 8 || t.ldx < t.K || t.ldx > 1 << 22 || t.ldy % 8 ||
+      t.ldy > 1 << 22 || ((size_t)t.x | (size_t)t.w | (size_t)t.y) % 16 || (size_t)t.bias % 2)
+    return false;
+  const double busy = at_work(a, rounds(a, width(a)));
+  if (act == TILE_GELU_ERF) return t.K <= 4096 ? busy >= 0.62 : t.K <= 8192 && busy >= 0.75;
+  return t.K <= 1280 ? t.K >= 256 && busy >= 0.6 : t.K <= 4096 && busy >= 0.72 && busy <= 0.97;
+}
+
+void big_gemm(const TileArgs& t, TileAct act, hipStream_t st) {
+  const BigArgs a = of(t);
+  const int nt = width(a);
+  if (act == TILE_GELU_ERF && nt == 6) launch<false, false, 6, BIG_GELU_ERF>(a, st);
+  else if (act == TILE_GELU_ERF) launch<false, false, 8, BIG_GELU_ERF>(a, st);
+  else if (nt == 6) launch<false, false, 6, BIG_NONE>(a, st);
+  else launch<false, false, 8, BIG_NONE>(a, st);
+}
 
 // dW[N][K] = sum over t of dY[t][N] X[t][K] where that is faster than a library's, else None:
 // where tiles keep two thirds of the chip at work.  In us, library and this: 28672 x 4096 out

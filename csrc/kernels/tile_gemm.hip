@@ -266,7 +266,8 @@ void tile_gemm(const TileArgs& a, TileAct act, hipStream_t st) {
   else pick<TILE_NONE>(a, tile, st);
 }
 
-// act(x w^T + b) of rows (..., K), act as TileAct; None: not what it is for
+// act(x w^T + b) of rows (..., K), act as TileAct, by these or by large tiles; None: not
+// what they are for
 c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Tensor& w,
                                          const c10::optional<torch::Tensor>& bias, long act) {
   // what a plain kernel would not see: gradients, transforms, tensors of Python classes
@@ -288,14 +289,16 @@ c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Te
   a.bias = bias.has_value() ? (const short*)bias->data_ptr() : nullptr;
   a.ldx = x.dim() == 2 ? x.stride(0) : a.K;
   a.ldy = a.N;
-  if (!tile_takes(a, (TileAct)act)) return c10::nullopt;
+  const bool big = big_takes(a, (TileAct)act);
+  if (!big && !tile_takes(a, (TileAct)act)) return c10::nullopt;
   // the operands' device, whichever is current: torch's product goes by it too
   const c10::DeviceGuard guard(x.device());
   auto shape = x.sizes().vec();
   shape.back() = a.N;
   auto y = torch::empty(shape, x.options());
   a.y = (short*)y.data_ptr();
-  tile_gemm(a, (TileAct)act, scaffold_stream());
+  if (big) big_gemm(a, (TileAct)act, scaffold_stream());
+  else tile_gemm(a, (TileAct)act, scaffold_stream());
   HIP_CHECK(hipGetLastError());
   return y;
 }

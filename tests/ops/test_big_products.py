@@ -3,6 +3,7 @@ past the caches."""
 
 import pytest
 import torch
+import torch.nn.functional as F
 
 from scaffold import ops
 
@@ -101,3 +102,33 @@ def test_layers_take_it(act, monkeypatch):
         _close(dx, dy, w.detach())
     torch.autograd.grad(y, x, dy.requires_grad_(), create_graph=True)
     assert len(calls) == 1
+
+
+@pytest.mark.parametrize("M,N,K,act,bias", [
+    (16129, 2056, 256, 0, True),      # tiles of 256 columns, several a block
+    (16001, 768, 768, 0, True),       # of 192, the last of one row
+    (2500, 8184, 1408, 0, False),     # of 192, the last of 120 columns
+    (9000, 6664, 256, 0, False),      # past the caches
+    (4100, 5128, 1152, 2, False),
+    (16001, 768, 768, 2, True),
+    (2040, 8192, 2048, 2, False)])
+def test_products(M, N, K, act, bias):
+    torch.manual_seed(M)
+    x, w = _rows(M, K), _rows(N, K, 0.5) / K ** 0.5
+    b = torch.randn(N, device="cuda").bfloat16() if bias else None
+    got = ops.require_ext().tile_linear(x, w.contiguous(), b, act)
+    a, v = x.double(), w.double().t()
+    size = a.abs() @ v.abs() + (b.double().abs() if bias else 0)
+    want = a @ v + (b.double() if bias else 0)
+    lim = (K / 32 + 34) * 2.0 ** -24 * size
+    if act:                           # whose slope is below 1.13
+        want, lim = F.gelu(want), 1.13 * lim + 1e-7 * want.abs().clamp(min=0.5)
+    assert ((got.double() - want).abs() <= lim + 2.0 ** -8 * want.abs()).all()
+
+
+def test_rows_that_lie_far_apart():
+    torch.manual_seed(5)
+    both = _rows(8000, 1024)
+    w = _rows(2048, 512)
+    got = ops.require_ext().tile_linear(both[:, 512:], w)
+    _close(got, both[:, 512:], w.t())
