@@ -69,6 +69,9 @@ void save_shard_pinned(std::string path, std::vector<std::string> names,
                        std::vector<std::string> meta_vals);
 torch::Tensor weight_grad(torch::Tensor dy, torch::Tensor x);
 c10::optional<torch::Tensor> wide_weight_grad(const torch::Tensor& dy, const torch::Tensor& x);
+c10::optional<torch::Tensor> head_logits(const torch::Tensor& x, const torch::Tensor& w);
+std::vector<torch::Tensor> head_grads(const torch::Tensor& d, const torch::Tensor& x,
+                                      const torch::Tensor& w, bool want_x, bool want_w);
 c10::optional<torch::Tensor> input_grad(const torch::Tensor& dy, const torch::Tensor& w);
 std::vector<torch::Tensor> linear_fwd(torch::Tensor x, torch::Tensor w,
                                       c10::optional<torch::Tensor> bias,
@@ -177,6 +180,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("x"));
   m.def("input_grad", [](py::object dy, py::object w) { return exact(input_grad, dy, w); },
         "dY W where that is faster than a library, or None", py::arg("dy"), py::arg("w"));
+  m.def("head_logits", [](py::object x, py::object w) { return exact(head_logits, x, w); },
+        "x W^T in rows of whole lines, or None", py::arg("x"), py::arg("w"));
+  m.def("head_grads", &head_grads, "dL W and dL^T x of such logits", py::arg("d"),
+        py::arg("x"), py::arg("w"), py::arg("want_x"), py::arg("want_w"));
   m.def("linear_fwd", &linear_fwd,
         "MFMA linear fwd, fused bias+GELU/residual epilogue (K5)");
   m.def("bn_fwd", &bn_fwd,

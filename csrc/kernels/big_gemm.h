@@ -33,6 +33,7 @@ struct BigArgs {
   short* y;                      // (M, N) of rows of ldy
   long lda, ldb, ldy;
   int M, N, K;
+  int am, bn;                    // of a and of b that there are to read, M and N or more or less
   unsigned tiles;
   bool stream;                   // the result goes past the caches
 };
@@ -114,8 +115,8 @@ gemm_kernel(BigArgs a) {
     return Place{(unsigned long)(from + at), (unsigned)(2 * size)};
   };
   auto seek = [&]() INLINE {
-    ca = where(std::integral_constant<bool, ACOL>{}, a.a, a.lda, mc, a.M);
-    cb = where(std::integral_constant<bool, BCOL>{}, a.b, a.ldb, nc, a.N);
+    ca = where(std::integral_constant<bool, ACOL>{}, a.a, a.lda, mc, a.am);
+    cb = where(std::integral_constant<bool, BCOL>{}, a.b, a.ldb, nc, a.bn);
   };
   place(tc, mc, nc);
   seek();

@@ -19,6 +19,8 @@ long up(long a, long b) { return (a + b - 1) / b; }
 template <bool ACOL, bool BCOL, int NT, int ACT>
 void launch(BigArgs a, hipStream_t st) {
   a.tiles = (unsigned)(up(a.M, 256) * up(a.N, 32 * NT));
+  if (!a.am) a.am = a.M;
+  if (!a.bn) a.bn = a.N;
   a.stream = 2l * a.M * a.N > 112l << 20;
   hipLaunchKernelGGL((big::gemm_kernel<ACOL, BCOL, NT, ACT>),
                      dim3(std::min<unsigned>(a.tiles, UNITS)), dim3(256), 0, st, a);
@@ -145,4 +147,83 @@ c10::optional<torch::Tensor> input_grad(const torch::Tensor& dy, const torch::Te
   else launch<false, true, 8, BIG_NONE>(a, scaffold_stream());
   HIP_CHECK(hipGetLastError());
   return dx;
+}
+
+// The head of a language model whose vocabulary is no multiple of eight: rows of logits and of
+// their gradients, 16 bytes apart at odd places, are what a library reads and writes slowly.
+// Here they lie in rows of whole lines.  In us, library with rows of 50257 and this: 16384
+// rows of 768, logits 1154 and 1001, dx 1203 and 989, dW 1352 and 1031.
+//
+// x (R, K) w (V, K)^T, as (R, V) with rows of V rounded up to 128; None where it is not for that.
+c10::optional<torch::Tensor> head_logits(const torch::Tensor& x, const torch::Tensor& w) {
+  if (watched() || !x.is_cuda() || !plain(x.detach(), x.device()) ||
+      !plain(w.detach(), x.device()) || x.dim() != 2 || w.dim() != 2 ||
+      x.size(1) != w.size(1) || !x.is_contiguous() || !w.is_contiguous())
+    return c10::nullopt;
+  const long V = w.size(0), K = w.size(1), R = x.size(0), ld = up(V, 128) * 128;
+  if (V % 8 == 0 || V >= 1l << 22 || R >= 1l << 30) return c10::nullopt;
+  TileArgs t = {};
+  t.x = (const short*)x.data_ptr();
+  t.w = (const short*)w.data_ptr();
+  t.M = (int)R; t.N = (int)(up(V, 8) * 8); t.K = (int)K;
+  t.ldx = K; t.ldy = ld;
+  if (!big_takes(t, TILE_NONE)) return c10::nullopt;
+  const c10::DeviceGuard guard(x.device());
+  auto y = torch::empty({R, ld}, x.options());
+  t.y = (short*)y.data_ptr();
+  BigArgs a = of(t);
+  a.bn = (int)V;
+  if (width(a) == 6) launch<false, false, 6, BIG_NONE>(a, scaffold_stream());
+  else launch<false, false, 8, BIG_NONE>(a, scaffold_stream());
+  HIP_CHECK(hipGetLastError());
+  return y.narrow(1, 0, V);
+}
+
+// {d w, d^T x} of such logits' gradient d, zero behind its last column; undefined where not
+// wanted
+std::vector<torch::Tensor> head_grads(const torch::Tensor& d, const torch::Tensor& x,
+                                      const torch::Tensor& w, bool want_x, bool want_w) {
+  const long R = d.size(0), V = w.size(0), K = w.size(1), ld = d.stride(0);
+  TORCH_CHECK(d.is_cuda() && d.scalar_type() == torch::kBFloat16 && d.dim() == 2 &&
+              d.size(1) == V && d.stride(1) == 1 && ld == up(V, 128) * 128 &&
+              d.storage_offset() == 0 && (long)d.storage().nbytes() >= 2 * R * ld &&
+              x.is_contiguous() && w.is_contiguous() && x.size(0) == R && x.size(1) == K &&
+              x.scalar_type() == torch::kBFloat16 && w.scalar_type() == torch::kBFloat16 &&
+              K % 8 == 0 && ((size_t)x.data_ptr() | (size_t)w.data_ptr()) % 16 == 0,
+              "head_grads: operands");
+  const c10::DeviceGuard guard(d.device());
+  auto st = scaffold_stream();
+  torch::Tensor dx, dw;
+  BigArgs a = {};
+  a.a = (const short*)d.data_ptr();
+  a.lda = ld;
+  if (want_x) {
+    a.b = (const short*)w.data_ptr();
+    a.M = (int)R; a.N = (int)K; a.K = (int)V;
+    a.ldb = a.ldy = K;
+    const int nt = columns(a);
+    if (at_work(a, rounds(a, nt)) >= 0.72) {
+      dx = torch::empty({R, K}, x.options());
+      a.y = (short*)dx.data_ptr();
+      if (nt == 6) launch<false, true, 6, BIG_NONE>(a, st);
+      else launch<false, true, 8, BIG_NONE>(a, st);
+    } else {
+      dx = at::mm(d, w);
+    }
+  }
+  if (want_w) {
+    a.b = (const short*)x.data_ptr();
+    a.M = (int)V; a.N = (int)K; a.K = (int)R;
+    a.am = (int)ld; a.bn = 0;
+    a.ldb = a.ldy = K;
+    if (at_work(a, rounds(a, 8)) >= 0.66) {
+      dw = torch::empty({V, K}, w.options());
+      a.y = (short*)dw.data_ptr();
+      launch<true, true, 8, BIG_NONE>(a, st);
+    } else {
+      dw = at::mm(d.t(), x);
+    }
+  }
+  HIP_CHECK(hipGetLastError());
+  return {dx, dw};
 }

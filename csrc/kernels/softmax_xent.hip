@@ -33,10 +33,10 @@ __global__ void __launch_bounds__(256)
 softmax_xent_fwd_kernel(const T* __restrict__ logits,
                         const long* __restrict__ targets,
                         float* __restrict__ loss, float* __restrict__ lse_out,
-                        int V) {
+                        int V, long ld) {
   __shared__ float red[8];
   const long row = blockIdx.x;
-  const T* lr = logits + row * (long)V;
+  const T* lr = logits + row * ld;
   const int V8 = V & ~7;
 
   float m = -INFINITY, s = 0.f;
@@ -76,14 +76,14 @@ __global__ void __launch_bounds__(256)
 softmax_xent_bwd_kernel(const T* __restrict__ logits,
                         const long* __restrict__ targets,
                         const float* __restrict__ lse, T* __restrict__ dlogits,
-                        int V, long R, double factor,
+                        int V, long ld, long R, double factor,
                         const float* __restrict__ dloss) {
   const long row = blockIdx.x;
   // read here: the host need not wait for it.  Divided in double and rounded
   // once, as the host does
   const float scale = (float)((dloss ? (double)*dloss : factor) / (double)R);
-  const T* lr = logits + row * (long)V;
-  T* dr = dlogits + row * (long)V;
+  const T* lr = logits + row * ld;
+  T* dr = dlogits + row * ld;
   const float l = lse[row];
   const long tgt = targets[row];
   const int V8 = V & ~7;
@@ -110,14 +110,25 @@ softmax_xent_bwd_kernel(const T* __restrict__ logits,
     if constexpr (std::is_same<T, short>::value) dr[i] = f2bf(d);
     else dr[i] = d;
   }
+  for (long i = V + threadIdx.x; i < ld; i += blockDim.x) dr[i] = 0;
 }
+
+// rows that lie one behind the other, or farther apart
+void check_rows(const torch::Tensor& t) {
+  CHECK_CUDA(t);
+  TORCH_CHECK(t.is_contiguous() ||
+              (t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1)),
+              "logits must be contiguous, or rows of contiguous numbers");
+}
+
+long row_length(const torch::Tensor& t) { return t.is_contiguous() ? t.size(1) : t.stride(0); }
 
 }  // namespace
 
 std::vector<torch::Tensor> softmax_xent_fwd(torch::Tensor logits, torch::Tensor targets) {
-  CHECK_CUDA(logits); CHECK_CONTIG(logits);
+  check_rows(logits);
   TORCH_CHECK(targets.scalar_type() == torch::kInt64);
-  const long R = logits.size(0);
+  const long R = logits.size(0), ld = row_length(logits);
   const int V = (int)logits.size(1);
   auto fopt = torch::TensorOptions().dtype(torch::kFloat32).device(logits.device());
   auto loss = torch::empty({R}, fopt);
@@ -127,25 +138,26 @@ std::vector<torch::Tensor> softmax_xent_fwd(torch::Tensor logits, torch::Tensor 
   if (logits.scalar_type() == torch::kBFloat16) {
     hipLaunchKernelGGL(softmax_xent_fwd_kernel<short>, grid, block, 0, stream,
                        (const short*)logits.data_ptr(), targets.data_ptr<long>(),
-                       loss.data_ptr<float>(), lse.data_ptr<float>(), V);
+                       loss.data_ptr<float>(), lse.data_ptr<float>(), V, ld);
   } else {
     hipLaunchKernelGGL(softmax_xent_fwd_kernel<float>, grid, block, 0, stream,
                        logits.data_ptr<float>(), targets.data_ptr<long>(),
-                       loss.data_ptr<float>(), lse.data_ptr<float>(), V);
+                       loss.data_ptr<float>(), lse.data_ptr<float>(), V, ld);
   }
   HIP_CHECK(hipGetLastError());
   return {loss, lse};
 }
 
 // dlogits of the mean over the R rows, whose gradient is `dloss`, or, if given,
-// the float32 number in dloss_dev: dloss / R is a row's factor.
+// the float32 number in dloss_dev: dloss / R is a row's factor.  They lie as the logits
+// do, with zeros between rows that are apart.
 torch::Tensor softmax_xent_bwd(torch::Tensor logits, torch::Tensor targets,
                                torch::Tensor lse, double dloss,
                                c10::optional<torch::Tensor> dloss_dev) {
-  CHECK_CUDA(logits); CHECK_CONTIG(logits);
-  const long R = logits.size(0);
+  check_rows(logits);
+  const long R = logits.size(0), ld = row_length(logits);
   const int V = (int)logits.size(1);
-  auto dlogits = torch::empty_like(logits);
+  auto dlogits = torch::empty({R, ld}, logits.options()).narrow(1, 0, V);
   const float* dp = nullptr;
   if (dloss_dev.has_value()) {
     TORCH_CHECK(dloss_dev->is_cuda() && dloss_dev->numel() == 1 &&
@@ -159,12 +171,12 @@ torch::Tensor softmax_xent_bwd(torch::Tensor logits, torch::Tensor targets,
     hipLaunchKernelGGL(softmax_xent_bwd_kernel<short>, grid, block, 0, stream,
                        (const short*)logits.data_ptr(), targets.data_ptr<long>(),
                        lse.data_ptr<float>(), (short*)dlogits.data_ptr(), V,
-                       R, dloss, dp);
+                       ld, R, dloss, dp);
   } else {
     hipLaunchKernelGGL(softmax_xent_bwd_kernel<float>, grid, block, 0, stream,
                        logits.data_ptr<float>(), targets.data_ptr<long>(),
                        lse.data_ptr<float>(), dlogits.data_ptr<float>(), V,
-                       R, dloss, dp);
+                       ld, R, dloss, dp);
   }
   HIP_CHECK(hipGetLastError());
   return dlogits;

@@ -695,6 +695,32 @@ class _LmHeadCE(torch.autograd.Function):
         return dh, dw, None
 
 
+class _HeadCE(torch.autograd.Function):
+    """Final projection and cross-entropy, with logits (of head_logits) and
+    their gradients in rows of whole lines."""
+
+    @staticmethod
+    def forward(ctx, x, w, logits, targets):
+        loss, lse = require_ext().softmax_xent_fwd(logits, targets)
+        ctx.save_for_backward(x, w, logits, targets, lse)
+        return loss.mean()
+
+    @staticmethod
+    def backward(ctx, dloss):
+        x, w, logits, targets, lse = ctx.saved_tensors
+        m = require_ext()
+        need_x, need_w = ctx.needs_input_grad[:2]
+        h = x.view(-1, x.shape[-1])
+        d = m.softmax_xent_bwd(
+            logits, targets, lse,
+            dloss_dev=dloss.to(logits.device, torch.float32))
+        if torch.is_grad_enabled():                # a graph is wanted
+            dx, dw = d @ w if need_x else None, d.t() @ h if need_w else None
+        else:
+            dx, dw = m.head_grads(d, h, w, need_x, need_w)
+        return dx.view(x.shape) if need_x else None, dw, None, None
+
+
 import os as _os_env
 
 # Measured A/B (2x25-step runs each, GPT-2 bs16): unfused 444.4
@@ -712,6 +738,12 @@ def lm_head_ce(x: torch.Tensor, w: torch.Tensor, targets: torch.Tensor
     t = targets.contiguous().view(-1)
     if x.is_cuda and _FUSED_CE:
         return _LmHeadCE.apply(x, w, t)
+    if x.is_cuda and not _transformed() and not torch.compiler.is_compiling():
+        x = x.contiguous()
+        logits = require_ext().head_logits(x.detach().view(-1, x.shape[-1]),
+                                           w.detach())
+        if logits is not None:
+            return _HeadCE.apply(x, w, logits, t)
     if x.is_cuda:
         # unfused: full logits through blaslt + K3 CE kernels
         return softmax_cross_entropy(linear(x, w), t)

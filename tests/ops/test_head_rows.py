@@ -1,0 +1,77 @@
+"""The head of a vocabulary that is no multiple of eight: logits and gradients
+in rows of whole lines."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from scaffold import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _made(R, V, K):
+    torch.manual_seed(R)
+    x = torch.randn(R, K, device="cuda").bfloat16().requires_grad_()
+    w = (torch.randn(V, K, device="cuda") / K ** 0.5).bfloat16().requires_grad_()
+    return x, w, torch.randint(0, V, (R,), device="cuda")
+
+
+def _calls(monkeypatch):
+    ext, calls = ops.require_ext(), []
+    made = ext.head_grads
+    monkeypatch.setattr(ext, "head_grads", lambda *a: calls.append(1) or made(*a))
+    return calls
+
+
+@pytest.mark.parametrize("R,V,K", [
+    (2047, 10001, 256),      # both gradients by the library
+    (16384, 3001, 768),      # dx by the kernel
+    (2048, 15001, 768),      # dW by the kernel
+    (2049, 15007, 768)])
+def test_loss_and_gradients(R, V, K, monkeypatch):
+    calls = _calls(monkeypatch)
+    x, w, t = _made(R, V, K)
+    loss = ops.lm_head_ce(x.view(1, R, K), w, t)
+    got = torch.autograd.grad(loss, (x, w), torch.tensor(3.0, device="cuda"))
+    assert calls
+    u, v = (s.detach().double().requires_grad_() for s in (x, w))
+    want_loss = F.cross_entropy(u @ v.t(), t)
+    want = torch.autograd.grad(3 * want_loss, (u, v))
+    assert abs(loss.item() - want_loss.item()) < 1e-3
+    for g, h in zip(got, want):
+        assert g.shape == h.shape and g.is_contiguous()
+        # logits rounded to 8 bits move each weight by 2^-9 |logit|, gradients once more
+        assert (g.double() - h).norm() < 0.01 * h.norm()
+    # what lies between the rows does not count, frozen operands cost nothing
+    (only,) = torch.autograd.grad(ops.lm_head_ce(x, w.detach(), t), x)
+    assert (3 * only.double() - want[0]).norm() < 0.01 * want[0].norm()
+    with torch.no_grad():
+        assert abs(ops.lm_head_ce(x, w, t).item() - loss.item()) < 1e-6
+
+
+def test_the_same_bits_as_one_row_behind_the_other(monkeypatch):
+    calls = _calls(monkeypatch)
+    x, w, t = _made(16384, 3001, 768)
+    a = torch.autograd.grad(ops.lm_head_ce(x, w, t), (x, w))
+    assert calls
+    b = torch.autograd.grad(ops.softmax_cross_entropy(F.linear(x, w), t), (x, w))
+    for g, h in zip(a, b):
+        assert (g.double() - h.double()).norm() < 1e-3 * h.double().norm()
+
+
+def test_small_or_other_operands_go_the_general_way(monkeypatch):
+    calls = _calls(monkeypatch)
+    for R, V, K, dtype in ((100, 3001, 768, torch.bfloat16), (16384, 3000, 768, torch.bfloat16),
+                           (16384, 301, 768, torch.float32)):
+        x, w, t = _made(R, V, K)
+        x, w = (s.detach().to(dtype).requires_grad_() for s in (x, w))
+        torch.autograd.grad(ops.lm_head_ce(x, w, t), (x, w))
+    assert not calls
+
+
+def test_a_graph_of_the_gradients(monkeypatch):
+    calls = _calls(monkeypatch)
+    x, w, t = _made(2047, 10001, 256)
+    (dx,) = torch.autograd.grad(ops.lm_head_ce(x, w, t), x, create_graph=True)
+    assert not calls and torch.autograd.grad(dx.float().sum(), w)[0].any()
