@@ -58,6 +58,20 @@ DEVINL void each(const F& f) {
   each_of(f, std::make_integer_sequence<int, N>{});
 }
 
+// Past the caches, or through them: for what is read or written once and is more than the
+// memory-side cache holds, 256 MB, so that this keeps what will be asked for again, and does
+// not have to write back before it takes something in.
+template <bool PAST, typename V>
+DEVINL void put_to(V* to, V v) {
+  if constexpr (PAST) __builtin_nontemporal_store(v, to);
+  else *to = v;
+}
+template <bool PAST, typename V>
+DEVINL V get_from(const V* from) {
+  if constexpr (PAST) return __builtin_nontemporal_load(from);
+  else return *from;
+}
+
 // a value that is the same in all lanes, where the compiler does not see it (and
 // would loop over the lanes to make a buffer descriptor of it)
 DEVINL unsigned same(unsigned x) { return (unsigned)__builtin_amdgcn_readfirstlane((int)x); }

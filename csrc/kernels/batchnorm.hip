@@ -13,7 +13,7 @@
 //         bit per element, so that the residual is neither saved nor read)
 //
 // What bounds these is memory: 256 x 256 x 56 x 56 with a residual is 10.1
-// passes over 411 MB.  A thread has UN rows' loads in flight at a time, and
+// passes over 411 MB, 657 us.  A thread has UN rows' loads in flight at a time, and
 // every second pass walks the rows backwards, so that it starts with what
 // the pass before has left in the memory-side cache.  Few rows are bound by
 // launches instead: there one launch per direction does everything
@@ -229,7 +229,8 @@ DEVINL bf16x8_t bn_out(const Channel8& p, bf16x8_t x, bf16x8_t res,
   return out;
 }
 
-template <bool RELU, bool RES>
+// PAST: see past_caches()
+template <bool RELU, bool RES, bool PAST>
 __global__ void __launch_bounds__(256)
 bn_apply_kernel(const short* __restrict__ x, const short* __restrict__ res,
                 const float* __restrict__ mean, const float* __restrict__ rstd,
@@ -245,11 +246,11 @@ bn_apply_kernel(const short* __restrict__ x, const short* __restrict__ res,
   walk<UN, true>(r0 + m.g, m.G, min(R, r0 + span), R,
       [&](int u, long r) {
         xs[u] = *(const bf16x8_t*)(x + r * C + m.vc * 8);
-        if (RES) rs[u] = *(const bf16x8_t*)(res + r * C + m.vc * 8);
+        if (RES) rs[u] = get_from<PAST>((const bf16x8_t*)(res + r * C + m.vc * 8));
       },
       [&](int u, long r) {
         unsigned bits;
-        *(bf16x8_t*)(y + r * C + m.vc * 8) = bn_out<RELU, RES>(p, xs[u], rs[u], bits);
+        put_to<PAST>((bf16x8_t*)(y + r * C + m.vc * 8), bn_out<RELU, RES>(p, xs[u], rs[u], bits));
         if (RELU && RES) mask[r * (C / 8) + m.vc] = (unsigned char)bits;
       });
 }
@@ -333,7 +334,7 @@ DEVINL bf16x8_t bn_dx(const Channel8& p, const float (&mdb)[8],
   return dx;
 }
 
-template <bool RELU, bool MASK>
+template <bool RELU, bool MASK, bool PAST>
 __global__ void __launch_bounds__(256)
 bn_bwd_dx_kernel(const short* __restrict__ dy, const short* __restrict__ x,
                  const unsigned char* __restrict__ mask,
@@ -364,9 +365,9 @@ bn_bwd_dx_kernel(const short* __restrict__ dy, const short* __restrict__ x,
       },
       [&](int u, long r) {
         bf16x8_t dr;
-        *(bf16x8_t*)(dx + r * C + m.vc * 8) =
-            bn_dx<RELU, MASK>(p, mdb, mdw, ds[u], xs[u], ms[u], dr);
-        if (dres) *(bf16x8_t*)(dres + r * C + m.vc * 8) = dr;
+        put_to<PAST>((bf16x8_t*)(dx + r * C + m.vc * 8),
+                     bn_dx<RELU, MASK>(p, mdb, mdw, ds[u], xs[u], ms[u], dr));
+        if (dres) put_to<PAST>((bf16x8_t*)(dres + r * C + m.vc * 8), dr);
       });
 }
 
@@ -585,6 +586,14 @@ Stream stream_grid(long R, int C) {
   return {dim3(cvb, (unsigned)((R + span - 1) / span)), span};
 }
 
+// Large results go past the caches, and so does the residual, which is read once: what the
+// first pass has left in the memory-side cache of x and dy stays for the second, and the next
+// first pass does not wait for lines to be written back.  Both directions in us, through the
+// caches and past them, alone and with the results read once more behind it: 411 MB with a
+// residual 728 and 657, 1126 and 1085, 206 MB 371 and 328, 584 and 559, 103 MB 186 and 167, 311
+// and 289; but 51 MB without one 75 and 75, 111 and 113, 26 MB 49 and 48, 67 and 69.
+bool past_caches(long R, int C) { return R * C >= 32l << 20; }
+
 // One launch a direction instead of three, as long as a block's threads can
 // keep their rows.  GPU time of forward + backward in us, one launch and three:
 // 1568 rows of 512 channels 18.1 and 21.6, of 2048 29 and 36; 2048 rows of 512
@@ -669,8 +678,10 @@ std::vector<torch::Tensor> bn_fwd(torch::Tensor x,
     hipLaunchKernelGGL(bn_stats_final_kernel, dim3((C + 15) / 16), dim3(256),
                        0, st, mid.data_ptr<float>(), o, ns, R, C);
     by_kind([&](auto rl, auto rs) {
-      hipLaunchKernelGGL((bn_apply_kernel<decltype(rl)::value, decltype(rs)::value>),
-                         stream.grid, dim3(256), 0, st, xp, rp, o.mean,
+      constexpr bool RL = decltype(rl)::value, RS = decltype(rs)::value;
+      auto* kernel = past_caches(R, C) ? &bn_apply_kernel<RL, RS, true>
+                                       : &bn_apply_kernel<RL, RS, false>;
+      hipLaunchKernelGGL(kernel, stream.grid, dim3(256), 0, st, xp, rp, o.mean,
                          o.rstd, wp, bp, yp, mp, R, C, stream.span);
     });
   }
@@ -753,8 +764,10 @@ std::vector<torch::Tensor> bn_bwd(torch::Tensor dy, torch::Tensor x,
     hipLaunchKernelGGL(bn_bwd_final_kernel, dim3((C + 15) / 16), dim3(256), 0,
                        st, mid.data_ptr<float>(), dwp, dbp, ns, C);
     by_kind([&](auto rl, auto mk) {
-      hipLaunchKernelGGL((bn_bwd_dx_kernel<decltype(rl)::value, decltype(mk)::value>),
-                         stream.grid, dim3(256), 0, st, dp, xp, mp, mn,
+      constexpr bool RL = decltype(rl)::value, MK = decltype(mk)::value;
+      auto* kernel = past_caches(R, C) ? &bn_bwd_dx_kernel<RL, MK, true>
+                                       : &bn_bwd_dx_kernel<RL, MK, false>;
+      hipLaunchKernelGGL(kernel, stream.grid, dim3(256), 0, st, dp, xp, mp, mn,
                          rs, wp, bp, dwp, dbp, dxp, drp, R, C, stream.span);
     });
   }
