@@ -6,9 +6,9 @@
 // elements of a virtual concatenation of all tensors; it looks its chunk up once, and
 // a thread has the loads of four places on their way together.  Only chunks with
 // several tensors in them, or a tensor's odd end, look up each place.  A block a chunk:
-// 4096 blocks that walk them are 7 % slower.  GPT-2-small (124 M) 664 us, 5.2 TB/s, 1.92 G
-// elements of Llama's sizes 10.28 ms, 5.2 TB/s; a place a thread, looked up in 32 KB of LDS
-// each, 2048 blocks, 767 us and 11.45 ms.
+// 4096 blocks that walk them are 7 % slower.  GPT-2-small (124 M) in its step 583 us, 6.0 TB/s, 1.92 G
+// elements of Llama's sizes 9.89 ms, 5.4 TB/s; a place a thread, looked up in 32 KB of LDS
+// each, 2048 blocks, through the caches, 767 us and 11.45 ms.
 
 #include "../common.h"
 
@@ -33,18 +33,19 @@ struct Four {
   f32x4 p, m, v, g;
 };
 
-template <bool BF16>
+// PAST: see PAST_CACHES
+template <bool BF16, bool PAST>
 DEVINL Four fetch(const Place& t, long e0, float scale) {
   Four f;
-  f.p = *(const f32x4*)(t.master + e0);
-  f.m = *(const f32x4*)(t.m + e0);
-  f.v = *(const f32x4*)(t.v + e0);
+  f.p = get_from<PAST>((const f32x4*)(t.master + e0));
+  f.m = get_from<PAST>((const f32x4*)(t.m + e0));
+  f.v = get_from<PAST>((const f32x4*)(t.v + e0));
   if constexpr (BF16) {
-    const bf16x4 g = *(const bf16x4*)((const short*)t.grad + e0);
+    const bf16x4 g = get_from<PAST>((const bf16x4*)((const short*)t.grad + e0));
     #pragma unroll
     for (int j = 0; j < 4; ++j) f.g[j] = bf2f(g[j]);
   } else {
-    f.g = *(const f32x4*)((const float*)t.grad + e0);
+    f.g = get_from<PAST>((const f32x4*)((const float*)t.grad + e0));
   }
   #pragma unroll
   for (int j = 0; j < 4; ++j) f.g[j] *= scale;
@@ -59,6 +60,7 @@ DEVINL void update(const AdamwArgs& a, float& p, float& m, float& v, float g) {
   p = p * (1.f - a.lr * a.wd) - a.lr * mhat / (sqrtf(vhat) + a.eps);
 }
 
+template <bool PAST>
 DEVINL void put(const AdamwArgs& a, const Place& t, long e0, Four& f, bool has_out) {
   bf16x4 o;
   #pragma unroll
@@ -70,9 +72,9 @@ DEVINL void put(const AdamwArgs& a, const Place& t, long e0, Four& f, bool has_o
     f.v[j] = v;
     o[j] = f2bf(p);
   }
-  *(f32x4*)(t.master + e0) = f.p;
-  *(f32x4*)(t.m + e0) = f.m;
-  *(f32x4*)(t.v + e0) = f.v;
+  put_to<PAST>((f32x4*)(t.master + e0), f.p);
+  put_to<PAST>((f32x4*)(t.m + e0), f.m);
+  put_to<PAST>((f32x4*)(t.v + e0), f.v);
   if (has_out) *(bf16x4*)(t.out + e0) = o;
 }
 
@@ -90,8 +92,8 @@ DEVINL void one(const AdamwArgs& a, const long* meta, int n, int t, long vi, boo
   const Place at = place_of(meta, n, t);
   const long e0 = (vi - meta[t]) * 4, numel = meta[n + 1 + 5l * n + t];
   if (e0 + 4 <= numel) {
-    Four f = fetch<BF16>(at, e0, a.grad_scale);
-    put(a, at, e0, f, has_out);
+    Four f = fetch<BF16, false>(at, e0, a.grad_scale);
+    put<false>(a, at, e0, f, has_out);
     return;
   }
   for (long e = e0; e < numel; ++e) {
@@ -139,7 +141,14 @@ adamw_few_kernel(const long* __restrict__ meta, int n, long total_vec4,
   }
 }
 
-template <bool BF16>
+// More places than this: moments and masters are more than the memory-side cache holds, and go
+// past it both ways, so that nothing is written back before something is read.  The new weights
+// go through it.  Through the cache and past, in us: 10 million elements 45 and 53, 25 million
+// 137 and 120, 60 million 320 and 265, 124 million 700 and 565 (6.2 TB/s), 400 million 2354 and
+// 2186; with the stores alone past it 717 for 124 million, with the loads alone 678.
+constexpr long PAST_CACHES = 4 << 20;    // places
+
+template <bool BF16, bool PAST>
 __global__ void __launch_bounds__(256)
 adamw_mt_kernel(const long* __restrict__ meta, int n, long total_vec4,
                 AdamwArgs a, int has_out, const int* __restrict__ step_dev) {
@@ -163,9 +172,9 @@ adamw_mt_kernel(const long* __restrict__ meta, int n, long total_vec4,
       const long e0 = (first + threadIdx.x) * 4;
       Four f[4];
       #pragma unroll
-      for (int u = 0; u < 4; ++u) f[u] = fetch<BF16>(at, e0 + u * 1024, a.grad_scale);
+      for (int u = 0; u < 4; ++u) f[u] = fetch<BF16, PAST>(at, e0 + u * 1024, a.grad_scale);
       #pragma unroll
-      for (int u = 0; u < 4; ++u) put(a, at, e0 + u * 1024, f[u], has_out);
+      for (int u = 0; u < 4; ++u) put<PAST>(a, at, e0 + u * 1024, f[u], has_out);
       continue;
     }
     const long end = min(total_vec4, (c + 1) * CHUNK);
@@ -250,7 +259,9 @@ void fused_adamw_run(torch::Tensor meta_dev, long n, long total_vec4,
                        total_vec4, a, has_out ? 1 : 0, sd);
   };
   if (few) grad_bf16 ? run(adamw_few_kernel<true>) : run(adamw_few_kernel<false>);
-  else grad_bf16 ? run(adamw_mt_kernel<true>) : run(adamw_mt_kernel<false>);
+  else if (total_vec4 < PAST_CACHES)
+    grad_bf16 ? run(adamw_mt_kernel<true, false>) : run(adamw_mt_kernel<false, false>);
+  else grad_bf16 ? run(adamw_mt_kernel<true, true>) : run(adamw_mt_kernel<false, true>);
   HIP_CHECK(hipGetLastError());
 }
 
