@@ -404,18 +404,26 @@ attn_prefill_form_kernel(AttnArgs a, const int4* __restrict__ tiles,
 // 8192 tokens in chunks of 1024, 95 against 121, 3 heads of 64 on 1 39 against 50, 5
 // heads of 128 97 against 129; bounds that ask for more waves than LDS has room for
 // are not kept, and 277 registers leave one wave to a SIMD (131, 43, 96).
-template <int DK, int DV, int HPB, bool BIAS>
-__global__ void __launch_bounds__(HPB * 128, 2)
+//
+// KS = 2, where blocks are no more than compute units: a page's keys are split over two
+// waves of a SIMD, which add their results up at the end, for one wave alone has 8 cycles
+// an instruction and waits between products and softmax.  Two prompts of 1000 behind 1500,
+// 256 blocks, 47.6 -> 41.3 us.  (There, copies two pages ahead into three images take 51.)
+template <int DK, int DV, int HPB, bool BIAS, int KS>
+__global__ void __launch_bounds__(HPB * 128 * KS, KS == 1 ? 2 : 1)
 attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
-  constexpr int NT = HPB * 128;
+  constexpr int NT = HPB * 128 * KS, WAVES = NT / 64, SUBS = 2 / KS;
   constexpr int NSL = DK / 16, NDT = DV / 32;
   constexpr int KC = 64 * DK / 8 / NT, VC = 64 * DV / 8 / NT;
   constexpr float LOWEST = -3.4028234663852886e38f;
   __shared__ __attribute__((aligned(16))) short k0[64 * DK], k1[64 * DK];
   __shared__ __attribute__((aligned(16))) short v0[64 * DV], v1[64 * DV];
+  __shared__ float other[KS > 1 ? HPB * 2 : 1][KS > 1 ? 16 * NDT + 2 : 1][64];
 
   const int tid = threadIdx.x, l = tid & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int place = __builtin_amdgcn_readfirstlane(tid >> 6);      // among the waves
+  const int wid = KS > 1 ? place >> 1 : place;                     // of a head's rows
+  const int part = KS > 1 ? place & 1 : 0, k32 = 32 * part;        // of a page's keys
   const int lq = l & 31, half = l >> 5;
   int bx, by;
   xcd_tile_map(n_tiles, &bx, &by);
@@ -476,7 +484,7 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
     #pragma unroll
     for (int i = 0; i < decltype(count)::value; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          src, (__attribute__((address_space(3))) void*)(to + (i * 2 * HPB + wid) * 512),
+          src, (__attribute__((address_space(3))) void*)(to + (i * WAVES + place) * 512),
           16, at[i], 0, 0, 0);
   };
   auto copy_k = [&](short* to, int page, int pg) INLINE {
@@ -497,34 +505,35 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
 
   const float scale2 = a.scale * LOG2E;
   const float slope2 = BIAS && a.slopes ? a.slopes[h] * LOG2E : 0.f;
-  float m_run = a.has_sink ? sink_score<false>(a, h) * LOG2E : LOWEST;
+  const bool sink = a.has_sink && !part;
+  float m_run = sink ? sink_score<false>(a, h) * LOG2E : LOWEST;
   if (m_run < LOWEST) m_run = LOWEST;          // -inf; NaN stays, and shows
-  float l_run = a.has_sink && !half ? 1.f : 0.f;    // of this half's keys
-  f32x16 o[NDT], s[2];
+  float l_run = sink && !half ? 1.f : 0.f;          // of this half's keys
+  f32x16 o[NDT], s[SUBS];
   #pragma unroll
   for (int i = 0; i < NDT; ++i) o[i] = {};
-  bf16x8 hi[2][2], lo[2][2];                        // weights, [sub][16 keys]
+  bf16x8 hi[SUBS][2], lo[SUBS][2];                  // weights, [sub][16 keys]
 
   auto scores = [&](const short* kimg) INLINE {
-    s[0] = {};
-    s[1] = {};
+    #pragma unroll
+    for (int sub = 0; sub < SUBS; ++sub) s[sub] = {};
     #pragma unroll
     for (int i = 0; i < NSL; ++i)
       #pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-        s[sub] = mma32(*(const bf16x8*)(kimg + (32 * sub + swapped(lq)) * DK +
+      for (int sub = 0; sub < SUBS; ++sub)
+        s[sub] = mma32(*(const bf16x8*)(kimg + (k32 + 32 * sub + swapped(lq)) * DK +
                                         ((2 * i + half) ^ (lq & 7)) * 8),
                        qf[i], s[sub]);
   };
   const int tr = 64 * (lq >> 4) + ((l & 15) >> 2) * 16 + (l & 3) * 4 +
-                 (half ? 128 * (DV / 16) : 0);
+                 (half ? 128 * (DV / 16) : 0) + k32 * DV;
   auto values = [&](const short* vimg) INLINE {
     typedef __attribute__((address_space(3))) bf16x4* P;
     auto quad = [&](int at) INLINE {
       return __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)(vimg + tr + at));
     };
     #pragma unroll
-    for (int sub = 0; sub < 2; ++sub)
+    for (int sub = 0; sub < SUBS; ++sub)
       #pragma unroll
       for (int i = 0; i < NDT; ++i)
         #pragma unroll
@@ -537,9 +546,9 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
         }
   };
   auto softmax = [&](int j0) INLINE {
-    const float d0 = slope2 * (float)(j0 + 8 * half - ip);
+    const float d0 = slope2 * (float)(j0 + k32 + 8 * half - ip);
     #pragma unroll
-    for (int sub = 0; sub < 2; ++sub)
+    for (int sub = 0; sub < SUBS; ++sub)
       #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int jr = 32 * sub + 16 * (r >> 3) + (r & 7);
@@ -548,9 +557,9 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
       }
     if (j0 + LM_PAGE - 1 > w0 || j0 < wcs1) {
       asm volatile("");        // a branch, not 32 selects in every page
-      const int from = cs - j0 - 8 * half, to = ip - j0 - 8 * half;
+      const int from = cs - j0 - k32 - 8 * half, to = ip - j0 - k32 - 8 * half;
       #pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
+      for (int sub = 0; sub < SUBS; ++sub)
         #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int jr = 32 * sub + 16 * (r >> 3) + (r & 7);
@@ -559,7 +568,7 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
     }
     float top = s[0][0];
     #pragma unroll
-    for (int sub = 0; sub < 2; ++sub)
+    for (int sub = 0; sub < SUBS; ++sub)
       #pragma unroll
       for (int r = 0; r < 16; ++r) top = fmaxf(top, s[sub][r]);
     if (__any(top > m_run)) {
@@ -575,7 +584,7 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
     }
     float ps = 0.f;
     #pragma unroll
-    for (int sub = 0; sub < 2; ++sub)
+    for (int sub = 0; sub < SUBS; ++sub)
       #pragma unroll
       for (int x = 0; x < 2; ++x) {
         float e[8];
@@ -610,7 +619,7 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
       // operands come from LDS four ahead of the product that takes them
       __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
       #pragma unroll
-      for (int i = 0; i < 2 * NSL - 4; ++i) {
+      for (int i = 0; i < SUBS * NSL - 4; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
@@ -621,7 +630,7 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
           __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         }
         #pragma unroll
-        for (int i = 0; i < 4 * NDT - 4; ++i) {
+        for (int i = 0; i < 2 * SUBS * NDT - 4; ++i) {
           __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
           __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         }
@@ -640,25 +649,51 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
     page(yes, no, it);
     if (it + 1 < n) page(no, no, it + 1);
   }
-  if (!w_any) return;
+  if (KS == 1 && !w_any) return;
   if (n & 1) values(v0);
   else values(v1);
 
   l_run = over_halves(l_run, [](float x, float y) { return x + y; });
+  if constexpr (KS > 1) {
+    float(&to)[16 * NDT + 2][64] = other[wid];
+    if (part) {
+      #pragma unroll
+      for (int i = 0; i < NDT; ++i)
+        #pragma unroll
+        for (int r = 0; r < 16; ++r) to[16 * i + r][l] = o[i][r];
+      to[16 * NDT][l] = m_run;
+      to[16 * NDT + 1][l] = l_run;
+    }
+    __syncthreads();
+    if (part || !w_any) return;
+    const float m1 = to[16 * NDT][l], mn = fmaxf(m_run, m1);
+    const float al = __builtin_amdgcn_exp2f(m_run - mn), be = __builtin_amdgcn_exp2f(m1 - mn);
+    l_run = l_run * al + to[16 * NDT + 1][l] * be;
+    #pragma unroll
+    for (int i = 0; i < NDT; ++i)
+      #pragma unroll
+      for (int r = 0; r < 16; ++r) o[i][r] = o[i][r] * al + to[16 * i + r][l] * be;
+  }
   if (row < t.y) {
     const float inv = l_run > 0.f ? a.out_scale / l_run : 0.f;
     store_row<NDT>(a, o, inv, t.x + row, h, half);
   }
 }
 
+constexpr unsigned UNITS = 256;          // compute units
+
 // FORM 0: as stored; 1: with a bias by distance; 2: tied, with one; 3: window
 template <int DK, int DV, int HPB, int FORM>
 void go(const AttnArgs& a, const int4* tiles, int n, hipStream_t st) {
   const dim3 grid((unsigned)((long)n * a.G * (a.H / a.G / HPB)));
-  if constexpr (FORM < 2)
-    hipLaunchKernelGGL((attn_prefill_kernel<DK, DV, HPB, FORM == 1>), grid,
-                       dim3(HPB * 128), 0, st, a, tiles, n);
-  else
+  if constexpr (FORM < 2) {
+    if (grid.x <= UNITS)
+      hipLaunchKernelGGL((attn_prefill_kernel<DK, DV, HPB, FORM == 1, 2>), grid,
+                         dim3(HPB * 256), 0, st, a, tiles, n);
+    else
+      hipLaunchKernelGGL((attn_prefill_kernel<DK, DV, HPB, FORM == 1, 1>), grid,
+                         dim3(HPB * 128), 0, st, a, tiles, n);
+  } else
     hipLaunchKernelGGL((attn_prefill_form_kernel<DK, DV, HPB, FORM == 2>), grid,
                        dim3(HPB * 128), 0, st, a, tiles, n);
 }

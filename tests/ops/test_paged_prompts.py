@@ -32,6 +32,24 @@ def test_matches_oracle(H, G, d, e, parts, size, sink):
     close(got, L.sink_attention(q, k, v, d ** -0.5, size, s), torch.bfloat16)
 
 
+@pytest.mark.parametrize("H,G,d", [(32, 32, 64), (64, 32, 128)])
+@pytest.mark.parametrize("parts", [(512,), (513,), (400, 120)], ids=str)
+def test_as_many_blocks_as_units_and_more(H, G, d, parts):
+    """8 and 9 tiles of 32 blocks, for which a page's keys are split or not."""
+    T, size = sum(parts), 200
+    q, k, v = rnd(T, H, d, seed=1), rnd(T, G, d, seed=2), rnd(T, G, d, seed=3)
+    s = rnd(H, seed=4, scale=2)
+    got = run_attention("cuda", torch.bfloat16, q, k, v, scale=d ** -0.5, size=size,
+                        sink=s, parts=parts)
+    i, j = torch.arange(T).unsqueeze(1), torch.arange(T)
+    seen = (j <= i) & (j >= i - i % size)
+    kk, vv = (t.repeat_interleave(H // G, 1).transpose(0, 1).double() for t in (k, v))
+    x = q.transpose(0, 1).double() @ kk.transpose(1, 2) * d ** -0.5
+    x = torch.cat([x.masked_fill(~seen, -math.inf), s.double().view(H, 1, 1).expand(H, T, 1)], 2)
+    want = (torch.softmax(x, 2)[..., :-1] @ vv).transpose(0, 1)
+    close(got, want.to(got.dtype).reshape(got.shape), torch.bfloat16)
+
+
 @pytest.mark.parametrize("parts", [(65,), (64, 1)], ids=str)
 def test_a_sink_that_is_no_number_shows(parts):
     """In its head, and in no other."""
