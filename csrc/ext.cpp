@@ -26,7 +26,8 @@ std::vector<torch::Tensor> layernorm_fwd(torch::Tensor x, torch::Tensor w,
                                          torch::Tensor b, double eps);
 std::vector<torch::Tensor> layernorm_bwd(torch::Tensor dy, torch::Tensor x,
                                          torch::Tensor w, torch::Tensor mean,
-                                         torch::Tensor rstd);
+                                         torch::Tensor rstd,
+                                         c10::optional<torch::Tensor> res);
 std::vector<torch::Tensor> softmax_xent_fwd(torch::Tensor logits,
                                             torch::Tensor targets);
 torch::Tensor softmax_xent_bwd(torch::Tensor logits, torch::Tensor targets,
@@ -35,7 +36,8 @@ torch::Tensor softmax_xent_bwd(torch::Tensor logits, torch::Tensor targets,
 std::vector<torch::Tensor> rmsnorm_fwd(torch::Tensor x, torch::Tensor w,
                                        double eps);
 std::vector<torch::Tensor> rmsnorm_bwd(torch::Tensor dy, torch::Tensor x,
-                                       torch::Tensor w, torch::Tensor rstd);
+                                       torch::Tensor w, torch::Tensor rstd,
+                                       c10::optional<torch::Tensor> res);
 torch::Tensor rope_apply(torch::Tensor x, torch::Tensor cos_t,
                          torch::Tensor sin_t, bool inverse,
                          c10::optional<torch::Tensor> out);
@@ -137,13 +139,16 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_adamw_run", &fused_adamw_run,
         "AdamW step on a prebuilt meta (graph-capturable; optional device step)");
   m.def("layernorm_fwd", &layernorm_fwd, "LayerNorm forward (K2)");
-  m.def("layernorm_bwd", &layernorm_bwd, "LayerNorm backward (K2)");
+  m.def("layernorm_bwd", &layernorm_bwd, "LayerNorm backward (K2)", py::arg("dy"),
+        py::arg("x"), py::arg("w"), py::arg("mean"), py::arg("rstd"),
+        py::arg("res") = py::none());
   m.def("softmax_xent_fwd", &softmax_xent_fwd, "softmax cross-entropy fwd (K3)");
   m.def("softmax_xent_bwd", &softmax_xent_bwd, "softmax cross-entropy bwd (K3)",
         py::arg("logits"), py::arg("targets"), py::arg("lse"),
         py::arg("dloss") = 1.0, py::arg("dloss_dev") = py::none());
   m.def("rmsnorm_fwd", &rmsnorm_fwd, "RMSNorm forward (K7)");
-  m.def("rmsnorm_bwd", &rmsnorm_bwd, "RMSNorm backward (K7)");
+  m.def("rmsnorm_bwd", &rmsnorm_bwd, "RMSNorm backward (K7)", py::arg("dy"),
+        py::arg("x"), py::arg("w"), py::arg("rstd"), py::arg("res") = py::none());
   m.def("rope_apply", &rope_apply, "RoPE apply/inverse (K7)", py::arg("x"),
         py::arg("cos"), py::arg("sin"), py::arg("inverse"),
         py::arg("out") = py::none());

@@ -265,15 +265,23 @@ std::vector<torch::Tensor> layernorm_fwd(torch::Tensor x, torch::Tensor w,
 }
 
 bool norm_bwd_takes(const torch::Tensor& dy, const torch::Tensor& x,
-                    const torch::Tensor& w);
+                    const torch::Tensor& w, const c10::optional<torch::Tensor>& res);
 void norm_bwd(const torch::Tensor& dy, const torch::Tensor& x,
               const torch::Tensor& w, const torch::Tensor& mean,
               const torch::Tensor& rstd, torch::Tensor& dx, torch::Tensor& dw,
-              torch::Tensor& db, hipStream_t st);
+              torch::Tensor& db, const c10::optional<torch::Tensor>& res,
+              hipStream_t st);
 
+// res: the gradient of x on its way round the norm, to be added to dx
 std::vector<torch::Tensor> layernorm_bwd(torch::Tensor dy, torch::Tensor x,
                                          torch::Tensor w, torch::Tensor mean,
-                                         torch::Tensor rstd) {
+                                         torch::Tensor rstd,
+                                         c10::optional<torch::Tensor> res) {
+  if (res && !(x.size(0) > 0 && norm_bwd_takes(dy, x, w, res))) {
+    auto out = layernorm_bwd(dy, x, w, mean, rstd, c10::nullopt);
+    out[0].add_(*res);
+    return out;
+  }
   CHECK_CUDA(dy); CHECK_CONTIG(dy); CHECK_CONTIG(x);
   const long R = x.size(0);
   const int D = (int)x.size(1);
@@ -281,8 +289,8 @@ std::vector<torch::Tensor> layernorm_bwd(torch::Tensor dy, torch::Tensor x,
   auto dw = torch::empty_like(w);
   auto db = torch::empty_like(w);
   auto stream = scaffold_stream();
-  if (R > 0 && norm_bwd_takes(dy, x, w)) {
-    norm_bwd(dy, x, w, mean, rstd, dx, dw, db, stream);
+  if (R > 0 && norm_bwd_takes(dy, x, w, res)) {
+    norm_bwd(dy, x, w, mean, rstd, dx, dw, db, res, stream);
     HIP_CHECK(hipGetLastError());
     return {dx, dw, db};
   }

@@ -293,23 +293,31 @@ std::vector<torch::Tensor> rmsnorm_fwd(torch::Tensor x, torch::Tensor w, double 
 }
 
 bool norm_bwd_takes(const torch::Tensor& dy, const torch::Tensor& x,
-                    const torch::Tensor& w);
+                    const torch::Tensor& w, const c10::optional<torch::Tensor>& res);
 void norm_bwd(const torch::Tensor& dy, const torch::Tensor& x,
               const torch::Tensor& w, const torch::Tensor& mean,
               const torch::Tensor& rstd, torch::Tensor& dx, torch::Tensor& dw,
-              torch::Tensor& db, hipStream_t st);
+              torch::Tensor& db, const c10::optional<torch::Tensor>& res,
+              hipStream_t st);
 
+// res: the gradient of x on its way round the norm, to be added to dx
 std::vector<torch::Tensor> rmsnorm_bwd(torch::Tensor dy, torch::Tensor x,
-                                       torch::Tensor w, torch::Tensor rstd) {
+                                       torch::Tensor w, torch::Tensor rstd,
+                                       c10::optional<torch::Tensor> res) {
+  if (res && !(x.size(0) > 0 && norm_bwd_takes(dy, x, w, res))) {
+    auto out = rmsnorm_bwd(dy, x, w, rstd, c10::nullopt);
+    out[0].add_(*res);
+    return out;
+  }
   CHECK_CUDA(dy); CHECK_CONTIG(dy); CHECK_CONTIG(x);
   const long R = x.size(0);
   const int D = (int)x.size(1);
   auto dx = torch::empty_like(x);
   auto dw = torch::empty_like(w);
   auto stream = scaffold_stream();
-  if (R > 0 && norm_bwd_takes(dy, x, w)) {
+  if (R > 0 && norm_bwd_takes(dy, x, w, res)) {
     torch::Tensor none;
-    norm_bwd(dy, x, w, none, rstd, dx, dw, none, stream);
+    norm_bwd(dy, x, w, none, rstd, dx, dw, none, res, stream);
     HIP_CHECK(hipGetLastError());
     return {dx, dw};
   }

@@ -16,6 +16,15 @@ import torch.nn as nn
 from .. import ops
 
 
+def unhooked(module: nn.Module, cls: type) -> bool:
+    """Whether a call of module is no more than cls.forward, which may then be
+    part of a larger op."""
+    return (type(module) is cls and "forward" not in vars(module)
+            and not (module._forward_hooks or module._forward_pre_hooks
+                     or module._backward_hooks or module._backward_pre_hooks
+                     or torch.nn.modules.module._has_any_global_hook()))
+
+
 class LayerNorm(nn.Module):
     def __init__(self, dim: int, eps: float = 1e-5):
         super().__init__()
@@ -25,6 +34,13 @@ class LayerNorm(nn.Module):
 
     def forward(self, x):
         return ops.layer_norm(x, self.weight, self.bias, self.eps)
+
+    @staticmethod
+    def fork(norm, x):
+        """norm(x), and x for the residual beside it."""
+        if not unhooked(norm, LayerNorm):
+            return norm(x), x
+        return ops.layer_norm_fork(x, norm.weight, norm.bias, norm.eps)
 
 
 class CausalSelfAttention(nn.Module):
@@ -83,8 +99,9 @@ class Block(nn.Module):
     def forward(self, x):
         # hot ops routed through scaffold.ops: K5 hand MFMA linears with
         # fused bias+GELU (fc) and fused residual-add (projections)
-        x = self.attn(self.ln1(x), residual=x)
-        h = self.ln2(x)
+        h, x = LayerNorm.fork(self.ln1, x)
+        x = self.attn(h, residual=x)
+        h, x = LayerNorm.fork(self.ln2, x)
         if self.moe is not None:
             B, S, C = h.shape
             return x + self.moe(h.reshape(B * S, C)).view(B, S, C)

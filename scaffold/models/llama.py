@@ -12,6 +12,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
+from .gpt2 import unhooked
 
 
 class RMSNorm(nn.Module):
@@ -22,6 +23,13 @@ class RMSNorm(nn.Module):
 
     def forward(self, x):
         return ops.rms_norm(x, self.weight, self.eps)
+
+    @staticmethod
+    def fork(norm, x):
+        """norm(x), and x for the residual beside it."""
+        if not unhooked(norm, RMSNorm):
+            return norm(x), x
+        return ops.rms_norm_fork(x, norm.weight, norm.eps)
 
 
 class LlamaAttention(nn.Module):
@@ -81,8 +89,9 @@ class LlamaBlock(nn.Module):
             self.w_down = nn.Linear(d_ff, d_model, bias=False)
 
     def forward(self, x, cos, sin):
-        x = self.attn(self.attn_norm(x), cos, sin, residual=x)
-        h = self.mlp_norm(x)
+        h, x = RMSNorm.fork(self.attn_norm, x)
+        x = self.attn(h, cos, sin, residual=x)
+        h, x = RMSNorm.fork(self.mlp_norm, x)
         if self.moe is not None:
             B, S, C = h.shape
             return x + self.moe(h.reshape(B * S, C)).view(B, S, C)

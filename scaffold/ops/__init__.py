@@ -27,7 +27,9 @@ from .lm import (Parts, clamped_glu, decay_tables, distance_bias, embed_norm,
 
 __all__ = [
     "layer_norm",
+    "layer_norm_fork",
     "rms_norm",
+    "rms_norm_fork",
     "rope_apply",
     "softmax_cross_entropy",
     "attention",
@@ -75,22 +77,46 @@ __all__ = [
 
 # ---------------------------------------------------------------- LayerNorm
 class _LayerNorm(torch.autograd.Function):
+    """fork: x is returned too, for a way round the norm; the gradient from
+    there is added in the backward's one pass over memory."""
+
     @staticmethod
-    def forward(ctx, x, weight, bias, eps):
+    def forward(ctx, x, weight, bias, eps, fork=False):
         m = require_ext()
         x2 = x.contiguous().view(-1, x.shape[-1])
         y, mean, rstd = m.layernorm_fwd(x2, weight, bias, eps)
         ctx.save_for_backward(x2, weight, mean, rstd)
         ctx.x_shape = x.shape
-        return y.view(x.shape)
+        ctx.set_materialize_grads(not fork)
+        return (y.view(x.shape), x) if fork else y.view(x.shape)
 
     @staticmethod
-    def backward(ctx, dy):
+    def backward(ctx, dy, dres=None):
+        if dy is None:
+            return dres, None, None, None, None
         x2, weight, mean, rstd = ctx.saved_tensors
         dy2 = dy.contiguous().view(-1, dy.shape[-1])
         m = require_ext()
-        dx, dw, db = m.layernorm_bwd(dy2, x2, weight, mean, rstd)
-        return dx.view(ctx.x_shape), dw, db, None
+        dx, dw, db = m.layernorm_bwd(dy2, x2, weight, mean, rstd,
+                                     _beside(dres, x2))
+        return _with(dx.view(ctx.x_shape), dres), dw, db, None, None
+
+
+def _beside(dres: Optional[torch.Tensor], x2: torch.Tensor
+            ) -> Optional[torch.Tensor]:
+    """dres for a kernel that has no gradient of its own, else _with() adds it."""
+    if dres is None or torch.is_grad_enabled():
+        return None
+    return dres.contiguous().view(x2.shape)
+
+
+def _with(dx: torch.Tensor, dres: Optional[torch.Tensor]) -> torch.Tensor:
+    return dx if dres is None or not torch.is_grad_enabled() else dx + dres
+
+
+def _forks(x: torch.Tensor) -> bool:
+    return (x.is_cuda and x.requires_grad and torch.is_grad_enabled()
+            and not torch.compiler.is_compiling() and not _transformed())
 
 
 def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor,
@@ -100,24 +126,38 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor,
     return F.layer_norm(x, (x.shape[-1],), weight, bias, eps)
 
 
+def layer_norm_fork(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor,
+                    eps: float = 1e-5) -> Tuple[torch.Tensor, torch.Tensor]:
+    """layer_norm(x), and x for a residual: where both have gradients, one kernel
+    adds them (csrc/kernels/norm_bwd.hip)."""
+    if _forks(x):
+        return _LayerNorm.apply(x, weight, bias, eps, True)
+    return layer_norm(x, weight, bias, eps), x
+
+
 # ----------------------------------------------------------------- RMSNorm
 class _RMSNorm(torch.autograd.Function):
+    """fork: as _LayerNorm's."""
+
     @staticmethod
-    def forward(ctx, x, weight, eps):
+    def forward(ctx, x, weight, eps, fork=False):
         m = require_ext()
         x2 = x.contiguous().view(-1, x.shape[-1])
         y, rstd = m.rmsnorm_fwd(x2, weight, eps)
         ctx.save_for_backward(x2, weight, rstd)
         ctx.x_shape = x.shape
-        return y.view(x.shape)
+        ctx.set_materialize_grads(not fork)
+        return (y.view(x.shape), x) if fork else y.view(x.shape)
 
     @staticmethod
-    def backward(ctx, dy):
+    def backward(ctx, dy, dres=None):
+        if dy is None:
+            return dres, None, None, None
         x2, weight, rstd = ctx.saved_tensors
         dy2 = dy.contiguous().view(-1, dy.shape[-1])
         m = require_ext()
-        dx, dw = m.rmsnorm_bwd(dy2, x2, weight, rstd)
-        return dx.view(ctx.x_shape), dw, None
+        dx, dw = m.rmsnorm_bwd(dy2, x2, weight, rstd, _beside(dres, x2))
+        return _with(dx.view(ctx.x_shape), dres), dw, None, None
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.Tensor:
@@ -126,6 +166,14 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.
     xf = x.float()
     y = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)
     return (y * weight.float()).to(x.dtype)
+
+
+def rms_norm_fork(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5
+                  ) -> Tuple[torch.Tensor, torch.Tensor]:
+    """rms_norm(x), and x for a residual, as layer_norm_fork()."""
+    if _forks(x):
+        return _RMSNorm.apply(x, weight, eps, True)
+    return rms_norm(x, weight, eps), x
 
 
 # -------------------------------------------------------------------- RoPE
