@@ -75,6 +75,9 @@ c10::optional<torch::Tensor> head_logits(const torch::Tensor& x, const torch::Te
 std::vector<torch::Tensor> head_grads(const torch::Tensor& d, const torch::Tensor& x,
                                       const torch::Tensor& w, bool want_x, bool want_w);
 c10::optional<torch::Tensor> input_grad(const torch::Tensor& dy, const torch::Tensor& w);
+c10::optional<torch::Tensor> residual_linear(const torch::Tensor& x, const torch::Tensor& w,
+                                             const c10::optional<torch::Tensor>& bias,
+                                             const torch::Tensor& res, bool last);
 std::vector<torch::Tensor> linear_fwd(torch::Tensor x, torch::Tensor w,
                                       c10::optional<torch::Tensor> bias,
                                       long epilogue,
@@ -185,6 +188,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("x"));
   m.def("input_grad", [](py::object dy, py::object w) { return exact(input_grad, dy, w); },
         "dY W where that is faster than a library, or None", py::arg("dy"), py::arg("w"));
+  m.def("residual_linear",
+        [](py::object x, py::object w, py::object bias, py::object res, bool last) {
+          return exact([&](const torch::Tensor& x, const torch::Tensor& w) -> c10::optional<torch::Tensor> {
+            if (!THPVariable_CheckExact(res.ptr()) ||
+                (!bias.is_none() && !THPVariable_CheckExact(bias.ptr())))
+              return c10::nullopt;
+            return residual_linear(x, w, bias.cast<c10::optional<torch::Tensor>>(),
+                                   res.cast<torch::Tensor>(), last);
+          }, x, w);
+        },
+        "x W^T + bias + res in one pass where that is faster, or None", py::arg("x"),
+        py::arg("w"), py::arg("bias"), py::arg("res"), py::arg("last"));
   m.def("head_logits", [](py::object x, py::object w) { return exact(head_logits, x, w); },
         "x W^T in rows of whole lines, or None", py::arg("x"), py::arg("w"));
   m.def("head_grads", &head_grads, "dL W and dL^T x of such logits", py::arg("d"),

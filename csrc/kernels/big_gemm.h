@@ -30,6 +30,7 @@
 struct BigArgs {
   const short *a, *b;            // operands, of rows of lda and ldb
   const short* bias;             // (N) or null; x w^T only
+  const short* res;              // (M, N) of rows of ldy, added to the result
   short* y;                      // (M, N) of rows of ldy
   long lda, ldb, ldy;
   int M, N, K;
@@ -38,7 +39,8 @@ struct BigArgs {
   bool stream;                   // the result goes past the caches
 };
 
-enum BigAct { BIG_NONE, BIG_GELU_ERF };
+// a residual is added before the result is rounded, or to the rounded result
+enum BigAct { BIG_NONE, BIG_GELU_ERF, BIG_RESIDUAL, BIG_RESIDUAL_LAST };
 
 namespace big {
 
@@ -264,11 +266,11 @@ gemm_kernel(BigArgs a) {
     int lane = l;
     asm volatile("" : "+v"(lane));
     const int lr = lane & 15, lg = lane >> 4;
-    // Sixteen rows from m on of the result as a buffer: what lies behind the last row is not
-    // stored, but counts as a store, as step() has it.  A lane's place is its row and
-    // column; one behind the last column lies outside of all.
-    auto rows = [&](int m) INLINE {
-      const unsigned long at = (unsigned long)(a.y + (long)min(m, a.M - 1) * a.ldy + n0);
+    // Sixteen rows from m on of the result (or what is added to it) as a buffer: what lies
+    // behind the last row is not stored, but counts as a store, as step() has it.  A lane's
+    // place is its row and column; one behind the last column lies outside of all.
+    auto rows = [&](const short* y, int m) INLINE {
+      const unsigned long at = (unsigned long)(y + (long)min(m, a.M - 1) * a.ldy + n0);
       const long size = m < a.M && n0 < a.N ? (min(16, a.M - m) - 1) * a.ldy + a.N - n0 : 0;
       return __builtin_amdgcn_make_buffer_rsrc(
           (void*)((unsigned long)same((unsigned)(at >> 32)) << 32 | same((unsigned)at)), 0,
@@ -290,7 +292,7 @@ gemm_kernel(BigArgs a) {
         short* mine = turned + wid * 16 * TURN;
         #pragma unroll
         for (int i = 0; i < MT; ++i) {
-          const auto to = rows(m0 + 16 * i);
+          const auto to = rows(a.y, m0 + 16 * i);
           #pragma unroll
           for (int j = 0; j < NT; ++j)
             *(u32x2*)(mine + lr * TURN + 16 * j + 4 * lg) =
@@ -309,15 +311,50 @@ gemm_kernel(BigArgs a) {
         if (a.bias)
           #pragma unroll
           for (int j = 0; j < NT; ++j) b[j] = bf2f(a.bias[min(n0 + lr * NT + j, a.N - 1)]);
+        // the residual, asked for AHEAD stores before it is taken; 8 of 16 bytes do not fit
+        // beside the next tile's operands
+        constexpr int AHEAD = NT == 8 ? 5 : 7;
+        constexpr bool RES = ACT == BIG_RESIDUAL || ACT == BIG_RESIDUAL_LAST;
+        unsigned add[RES ? AHEAD + 1 : 1][NT / 2];
+        auto ask = [&](int s) INLINE {
+          const auto from = rows(a.res, m0 + s / 4 * 16);
+          const unsigned place = at(4 * lg + s % 4, lr * NT);
+          unsigned* to = add[s % (AHEAD + 1)];
+          if constexpr (NT == 8) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(from, place, 0, 0);
+            #pragma unroll
+            for (int j = 0; j < 4; ++j) to[j] = v[j];
+          } else {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b96(from, place, 0, 0);
+            #pragma unroll
+            for (int j = 0; j < 3; ++j) to[j] = v[j];
+          }
+        };
+        if constexpr (RES)
+          #pragma unroll
+          for (int s = 0; s < AHEAD; ++s) ask(s);
         #pragma unroll
         for (int i = 0; i < MT; ++i) {
-          const auto to = rows(m0 + 16 * i);
+          const auto to = rows(a.y, m0 + 16 * i);
           #pragma unroll
           for (int r = 0; r < 4; ++r) {
+            if constexpr (RES)
+              if (4 * i + r + AHEAD < 4 * MT) ask(4 * i + r + AHEAD);
             unsigned v[NT / 2];
             #pragma unroll
-            for (int j = 0; j < NT / 2; ++j)
-              v[j] = cvt_pk_bf16(act(acc[i][2 * j][r] + b[2 * j]), act(acc[i][2 * j + 1][r] + b[2 * j + 1]));
+            for (int j = 0; j < NT / 2; ++j) {
+              float lo = acc[i][2 * j][r] + b[2 * j], hi = acc[i][2 * j + 1][r] + b[2 * j + 1];
+              if constexpr (ACT == BIG_RESIDUAL_LAST) {
+                const unsigned y = cvt_pk_bf16(lo, hi);
+                lo = __uint_as_float(y << 16);
+                hi = __uint_as_float(y & 0xffff0000u);
+              }
+              if constexpr (RES) {
+                lo += __uint_as_float(add[(4 * i + r) % (AHEAD + 1)][j] << 16);
+                hi += __uint_as_float(add[(4 * i + r) % (AHEAD + 1)][j] & 0xffff0000u);
+              }
+              v[j] = cvt_pk_bf16(act(lo), act(hi));
+            }
             const unsigned place = at(4 * lg + r, lr * NT);
             if constexpr (NT == 8)
               __builtin_amdgcn_raw_buffer_store_b128(u32x4{v[0], v[1], v[2], v[3]}, to, place, 0, AUX);

@@ -82,6 +82,53 @@ void big_gemm(const TileArgs& t, TileAct act, hipStream_t st) {
   else launch<false, false, 8, BIG_NONE>(a, st);
 }
 
+// x w^T + b + res; None where big_takes() says no.  One rounding, as linear_fwd has it, or (last)
+// two, as a product and a sum have, so that results are the same bits.  The residual comes in while
+// the results are stored, where a pass of its own reads the product and writes it again.  Of 37
+// sizes of 2336 to 65536 rows it takes, every one is faster.  In us, the product and a pass,
+// tiles of 128 (linear_fwd, of up to 1024 columns and depths) and this: 16384 x 768 x 768 38, 41
+// and 29, 65536 x 256 x 256 39, 30 and 27, 12288 x 1024 x 1024 42, 48 and 33; 16384 x 768 x 3072 85
+// and 73, 8040 x 2920 x 256 49 and 36, 26104 x 1032 x 3200 179 and 162.
+c10::optional<torch::Tensor> residual_linear(const torch::Tensor& x, const torch::Tensor& w,
+                                             const c10::optional<torch::Tensor>& bias,
+                                             const torch::Tensor& res, bool last) {
+  if (watched() || !x.is_cuda()) return c10::nullopt;
+  auto whole = [&](const torch::Tensor& t) {
+    return plain(t, x.device()) && t.is_contiguous();
+  };
+  if (x.dim() < 2 || w.dim() != 2 || !whole(x) || !whole(w) || !whole(res) ||
+      (bias && (!whole(*bias) || bias->dim() != 1 || bias->size(0) != w.size(0))) ||
+      x.numel() == 0 || x.size(-1) != w.size(1) || w.size(0) >= 1 << 30 ||
+      x.numel() / w.size(1) >= 1 << 30)
+    return c10::nullopt;
+  auto shape = x.sizes().vec();
+  shape.back() = w.size(0);
+  if (res.sizes() != c10::IntArrayRef(shape)) return c10::nullopt;
+  TileArgs t = {};
+  t.K = (int)w.size(1);
+  t.N = (int)w.size(0);
+  t.M = (int)(x.numel() / t.K);
+  t.x = (const short*)x.data_ptr();
+  t.w = (const short*)w.data_ptr();
+  t.bias = bias ? (const short*)bias->data_ptr() : nullptr;
+  t.ldx = t.K;
+  t.ldy = t.N;
+  if ((size_t)res.data_ptr() % 16 || !big_takes(t, TILE_NONE)) return c10::nullopt;
+  const c10::DeviceGuard guard(x.device());
+  auto y = torch::empty(shape, x.options());
+  t.y = (short*)y.data_ptr();
+  BigArgs a = of(t);
+  a.res = (const short*)res.data_ptr();
+  auto st = scaffold_stream();
+  const bool wide = width(a) == 8;
+  if (last && wide) launch<false, false, 8, BIG_RESIDUAL_LAST>(a, st);
+  else if (last) launch<false, false, 6, BIG_RESIDUAL_LAST>(a, st);
+  else if (wide) launch<false, false, 8, BIG_RESIDUAL>(a, st);
+  else launch<false, false, 6, BIG_RESIDUAL>(a, st);
+  HIP_CHECK(hipGetLastError());
+  return y;
+}
+
 // dW[N][K] = sum over t of dY[t][N] X[t][K] where that is faster than a library's, else None:
 // where tiles keep two thirds of the chip at work.  In us, library and this: 28672 x 4096 out
 // of 8192 rows 1646 and 1272, of 500 176 and 106; 4096 x 4096 out of 8192 240 and 188; 6144 x

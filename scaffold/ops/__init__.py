@@ -543,8 +543,10 @@ class _LinearResidualFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, b, res):
         m = require_ext()
-        x = x.contiguous()
-        (y,) = m.linear_fwd(x, w, b, 2, res.contiguous())
+        x, res = x.contiguous(), res.contiguous()
+        y = m.residual_linear(x, w, b, res, False) if _many(res) else None
+        if y is None:
+            (y,) = m.linear_fwd(x, w, b, 2, res)
         ctx.save_for_backward(x, w)
         ctx.has_bias = b is not None
         return y
@@ -585,6 +587,21 @@ def _product(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None
     return F.linear(x, w, b) if y is None else y
 
 
+def _many(y: torch.Tensor) -> bool:
+    """Whether a result may be large enough for big_gemm.hip, before its rule,
+    which takes longer, is asked."""
+    return y.numel() >= 8_200_000              # 0.6 of a round of 192 columns
+
+
+def _residual_product(x: torch.Tensor, w: torch.Tensor,
+                      b: Optional[torch.Tensor], res: torch.Tensor
+                      ) -> torch.Tensor:
+    """_product() + res, in one kernel where that is ours."""
+    y = (require_ext().residual_linear(x, w, b, res, True)
+         if _many(res) and not torch.compiler.is_compiling() else None)
+    return _product(x, w, b) + res if y is None else y
+
+
 class _LinearLib(torch.autograd.Function):
     """Forward by _product() with an explicit backward:
     rocBLAS matmuls for dX/dW plus the hand colsum kernel for the bias
@@ -592,10 +609,12 @@ class _LinearLib(torch.autograd.Function):
     costs nothing: its gradient is not made, and what only that needs not kept."""
 
     @staticmethod
-    def forward(ctx, x, w, b):
-        need_x, need_w, ctx.need_b = ctx.needs_input_grad
+    def forward(ctx, x, w, b, res=None):
+        need_x, need_w, ctx.need_b = ctx.needs_input_grad[:3]
         ctx.save_for_backward(x if need_w else None, w if need_x else None)
         ctx.x_shape = x.shape
+        if res is not None:
+            return _residual_product(x, w, b, res)
         return _product(x, w, b)
 
     @staticmethod
@@ -607,7 +626,8 @@ class _LinearLib(torch.autograd.Function):
             dx = _input_grad(dy2, w).view(ctx.x_shape)
         if x is not None:
             dw = _weight_grad(dy2, x.contiguous().view(-1, x.shape[-1]))
-        return dx, dw, _colsum(dy2) if ctx.need_b else None
+        db = _colsum(dy2) if ctx.need_b else None
+        return dx, dw, db, dy if ctx.needs_input_grad[3:] else None
 
 
 class _LinearGeluLib(torch.autograd.Function):
@@ -691,7 +711,11 @@ def linear_residual(x: torch.Tensor, w: torch.Tensor,
     if (x.is_cuda and x.dtype == w.dtype == torch.bfloat16
             and (b is None or b.dtype == torch.bfloat16)
             and torch.is_grad_enabled() and not _transformed()):
-        return _LinearLib.apply(x, w, b) + res     # gradients by own kernels
+        # gradients by own kernels
+        if (res.is_cuda and res.dtype == x.dtype
+                and res.shape == x.shape[:-1] + w.shape[:1]):
+            return _LinearLib.apply(x, w, b, res)
+        return _LinearLib.apply(x, w, b) + res
     return F.linear(x, w, b) + res
 
 

@@ -132,3 +132,63 @@ def test_rows_that_lie_far_apart():
     w = _rows(2048, 512)
     got = ops.require_ext().tile_linear(both[:, 512:], w)
     _close(got, both[:, 512:], w.t())
+
+
+@pytest.mark.parametrize("M,N,K,bias", [
+    (16001, 768, 768, True),          # 192 columns, the last tile of one row
+    (2500, 8184, 1408, False),        # the last of 120 columns
+    (16384, 768, 768, True),
+    (16129, 2056, 256, True),         # 256 columns, several tiles a block
+    (9000, 6664, 256, False)])        # past the caches
+def test_products_beside_a_residual(M, N, K, bias):
+    torch.manual_seed(M)
+    x, w, res = _rows(M, K), (_rows(N, K, 0.5) / K ** 0.5).contiguous(), _rows(M, N)
+    b = torch.randn(N, device="cuda").bfloat16() if bias else None
+    got = ops.require_ext().residual_linear(x, w, b, res, False)
+    # the residual and the bias are two more terms of each sum
+    want = x.double() @ w.double().t() + res.double() + (b.double() if bias else 0)
+    size = x.double().abs() @ w.double().abs().t() + res.double().abs() + (
+        b.double().abs() if bias else 0)
+    lim = 2.0 ** -8 * want.abs() + (K / 32 + 34) * 2.0 ** -24 * size
+    assert ((got.double() - want).abs() <= lim).all()
+    apart = ops.require_ext().tile_linear(x, w, b, 0) + res
+    assert torch.equal(ops.require_ext().residual_linear(x, w, b, res, True), apart)
+    if M % 128 == 0 and N % 128 == 0:
+        assert torch.equal(got, ops.require_ext().linear_fwd(x, w, b, 2, res)[0])
+
+
+def test_residuals_of_other_forms_are_left():
+    def f(*a):
+        return ops.require_ext().residual_linear(*a, False)
+
+    x, w, b, r = _rows(16384, 768), _rows(768, 768), _rows(1, 768)[0], _rows(16384, 768)
+    assert f(x, w, b, r) is not None and f(x.view(4, 4096, 768), w, b, r.view(4, 4096, 768)) is not None
+    odd = torch.cat([r[0, :1], r.flatten()])[1:].view_as(r)
+    for other in (r[:1], r[:, :1], r.float(), odd, r.cpu(), r.t().contiguous().t(),
+                  r.view(4, 4096, 768)):
+        assert f(x, w, b, other) is None
+
+
+@pytest.mark.parametrize("n", [768, 3072])
+def test_residual_layers_take_it(n, monkeypatch):
+    """Both layers that add a residual, and their gradients; a residual that is
+    spread over rows is added as before."""
+    ext, calls = ops.require_ext(), []
+    made = ext.residual_linear
+    monkeypatch.setattr(ext, "residual_linear",
+                        lambda *a: calls.append(made(*a)) or calls[-1])
+    torch.manual_seed(n)
+    x, r = (torch.randn(16384, k, device="cuda").bfloat16().requires_grad_() for k in (n, 768))
+    w = (torch.randn(768, n, device="cuda") / n ** 0.5).bfloat16().requires_grad_()
+    b = torch.randn(768, device="cuda").bfloat16().requires_grad_()
+    y = ops.linear_residual(x, w, b, r)
+    assert len(calls) == 1 and calls[0] is not None
+    dy = torch.randn_like(y)
+    got = torch.autograd.grad(y, (x, w, b, r), dy)
+    want = torch.autograd.grad(ops.linear(x, w, b), (x, w, b), dy)
+    assert all(map(torch.equal, got, (*want, dy)))
+    if n == 3072:
+        y = ops.linear_residual(x, w, b, r[:1])
+        assert torch.equal(y, ops.linear(x, w, b) + r[:1])
+        (got,) = torch.autograd.grad(y, r, dy)
+        assert got.shape == r.shape and not got[1:].any()
