@@ -58,8 +58,11 @@ DEVINL float other_half(float x) {
 // result is as near as with a float32 product, to five digits of its error
 // (heads of 64 and 128, 2 to 4096 rows, up to 4096 keys): its own rounding to
 // 8 bits is what there is.  An infinite value is NaN in what sees it.
-template <int D, bool SPLIT>
-__global__ void __launch_bounds__(64 * W, D == 64 && !SPLIT ? 4 : 2)
+//
+// KS = 2: the tiles of 64 keys go by turns to two groups of W waves, each with images of its
+// own, and the first puts both results together at the end.
+template <int D, bool SPLIT, int KS>
+__global__ void __launch_bounds__(64 * W * KS, D == 64 && !SPLIT ? 4 : 2)
 attn_fwd_mfma_kernel(const short* __restrict__ q, const short* __restrict__ k,
                    const short* __restrict__ v, short* __restrict__ o,
                    float* __restrict__ lse, int B, int H, int Hkv, int S,
@@ -69,10 +72,14 @@ attn_fwd_mfma_kernel(const short* __restrict__ q, const short* __restrict__ k,
   constexpr int NDT = D / 32;
   constexpr int CH = D / 8;          // 16-B chunks per row
   constexpr int SLOTS = CH / W;      // of a wave, of an image
-  __shared__ __attribute__((aligned(16))) short k0[64 * D], k1[64 * D];
-  __shared__ __attribute__((aligned(16))) short v0[64 * D], v1[64 * D];
+  static_assert(KS == 1 || SPLIT, "training's sums have an order");
+  __shared__ __attribute__((aligned(16))) short k0s[KS * 64 * D], k1s[KS * 64 * D];
+  __shared__ __attribute__((aligned(16))) short v0s[KS * 64 * D], v1s[KS * 64 * D];
 
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // 0..3
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wid = wave % W, group = KS > 1 ? wave / W : 0;
+  short *const k0 = k0s + group * 64 * D, *const k1 = k1s + group * 64 * D;
+  short *const v0 = v0s + group * 64 * D, *const v1 = v1s + group * 64 * D;
   const int l = threadIdx.x & 63;
   const int lq = l & 31;
   const int half = l >> 5;
@@ -110,7 +117,9 @@ attn_fwd_mfma_kernel(const short* __restrict__ q, const short* __restrict__ k,
   float m_run = LOWEST, l_run = 0.f;  // base-2 domain
 
   const int kv_end = causal ? min(Sk, off + q0 + 32 * STEP) : Sk;
-  const int n = (kv_end + 63) / 64;
+  // tiles of a group, and of the first, which has the most: all meet at its barriers
+  const int all = (kv_end + 63) / 64, most = (all + KS - 1) / KS;
+  const int n = (all - group + KS - 1) / KS;
 
   // Copies of K(t) and V(t) into LDS, as buffer loads: what lies behind the last
   // key reads as zero, a lane's place in a tile is the same in every tile, and,
@@ -261,11 +270,15 @@ attn_fwd_mfma_kernel(const short* __restrict__ q, const short* __restrict__ k,
   };
   // copies of a phase pair: K(u) and V(u - 1), for u up to n
   auto stage = [&](auto odd, int u) INLINE {
-    if (u < n) copy(odd ? k1 : k0, k + kb, ks.ss, ko, u);
-    copy(odd ? v0 : v1, v + vb, vs.ss, vo, u - 1);
+    if (u < n) copy(odd ? k1 : k0, k + kb, ks.ss, ko, KS * u + group);
+    copy(odd ? v0 : v1, v + vb, vs.ss, vo, KS * (u - 1) + group);
   };
   auto tile = [&](auto odd, auto first, int t) INLINE {
     constexpr bool O = decltype(odd)::value;
+    if (KS > 1 && t >= n) {
+      turn();
+      return;
+    }
     stage(std::integral_constant<bool, !O>{}, t + 1);
     __builtin_amdgcn_s_setprio(1);
     scores(O ? k1 : k0);
@@ -290,23 +303,50 @@ attn_fwd_mfma_kernel(const short* __restrict__ q, const short* __restrict__ k,
       }
     }
     __builtin_amdgcn_s_setprio(0);
-    softmax(t * 64);
+    softmax((KS * t + group) * 64);
     arrived();
     turn();
   };
   constexpr std::true_type yes;
   constexpr std::false_type no;
-  copy(k0, k + kb, ks.ss, ko, 0);
+  if (KS == 1 || n > 0) copy(k0, k + kb, ks.ss, ko, group);
   arrived();
   turn();
   tile(no, yes, 0);
-  for (int t = 1; t < n; t += 2) {
+  for (int t = 1; t < most; t += 2) {
     tile(yes, no, t);
-    if (t + 1 < n) tile(no, no, t + 1);
+    if (t + 1 < most) tile(no, no, t + 1);
   }
   if (n & 1) values(v0);
-  else values(v1);
+  else if (KS == 1 || n > 0) values(v1);
   if constexpr (SPLIT) l_run += other_half(l_run);
+
+  if constexpr (KS == 2) {
+    turn();                                // no image is read any more
+    float *lo = (float*)k0s, *hi = (float*)k1s, *sums = (float*)v0s;
+    const int at = wid * 64 + l;
+    if (group) {
+      #pragma unroll
+      for (int t = 0; t < NDT; ++t)
+        #pragma unroll
+        for (int r = 0; r < 16; ++r)
+          (t < NDT / 2 ? lo : hi)[(t % (NDT / 2) * 16 + r) * 64 * W + at] = oacc[t][r];
+      sums[at] = m_run;
+      sums[64 * W + at] = l_run;
+    }
+    turn();
+    if (group) return;
+    const float m1 = sums[at], l1 = sums[64 * W + at], m = fmaxf(m_run, m1);
+    const float f0 = __builtin_amdgcn_exp2f(m_run - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
+    m_run = m;
+    l_run = l_run * f0 + l1 * f1;
+    #pragma unroll
+    for (int t = 0; t < NDT; ++t)
+      #pragma unroll
+      for (int r = 0; r < 16; ++r)
+        oacc[t][r] = oacc[t][r] * f0 +
+                     (t < NDT / 2 ? lo : hi)[(t % (NDT / 2) * 16 + r) * 64 * W + at] * f1;
+  }
 
   // serving: -inf throughout is NaN, as in a softmax
   const float inv_l = SPLIT || l_run > 0.f ? 1.f / l_run : 0.f;
@@ -344,7 +384,25 @@ static void launch(const torch::Tensor& q, const torch::Tensor& k,
                    int Sk, float scale2, bool causal, hipStream_t st) {
   const int B = (int)q.size(0), H = (int)q.size(1), S = (int)q.size(2);
   const int nbx = SPLIT ? (S + ROWS - 1) / ROWS : (S + 2 * ROWS - 1) / (2 * ROWS) * 2;
-  hipLaunchKernelGGL((attn_fwd_mfma_kernel<D, SPLIT>), dim3(nbx * B * H), dim3(64 * W), 0,
+  auto kernel = attn_fwd_mfma_kernel<D, SPLIT, 1>;
+  int waves = W;
+  // Serving, blocks for no more than every unit: two groups of waves share the keys, so that
+  // a SIMD has two waves that nothing ties to each other between barriers.  In us, one group and
+  // two, heads of 64: 1 row of 12 heads x 1000 22.5 and 19.1, x 333 10.8 and 9.8, 4 x 12 x 600 16.9
+  // and 15.1, 12 x 1000 rows behind 2000 keys 57 and 44, 10 x 12 x 256 behind 700 23.3 and 20.7; of
+  // 128, 32 x 1000 32.3 and 28.8, 1000 rows behind 2000 84 and 74, 2 x 32 x 400 18.8 and 18.2.  Of
+  // few keys what the groups save goes into their meeting: 32 x 300 x 128 12.7 and 13.3, 4 x 12 x 317
+  // x 64 10.4 and 10.3.  With more blocks a unit has its two waves to a SIMD without: 8 x 12 x 317 x
+  // 64 (288 blocks) 11.7 and 14.1, 32 x 1200 behind 2000 keys (320) 100 and 114; causal heads of 64
+  // whose blocks differ most gain all the same (12 x 3000, 288, 56 and 45), 8 x 12 x 317 behind 700,
+  // as many, do not (28 and 34).
+  if constexpr (SPLIT) {
+    if (Sk > 320 && (long)nbx * B * H <= 256) {
+      kernel = attn_fwd_mfma_kernel<D, SPLIT, 2>;
+      waves = 2 * W;
+    }
+  }
+  hipLaunchKernelGGL(kernel, dim3(nbx * B * H), dim3(64 * waves), 0,
                      st, (const short*)q.data_ptr(), (const short*)k.data_ptr(),
                      (const short*)v.data_ptr(), (short*)o.data_ptr(), lse, B, H,
                      (int)k.size(1), S, Sk, scale2, causal ? 1 : 0, nbx, strides_of(q),

@@ -35,6 +35,41 @@ def test_prompt_attention_matches_float64(D, H, G, S, Sk):
     assert (got - want).norm() / want.norm() < 2.0 ** -9
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,S,Sk", [
+    (1, 2, 2, 320), (1, 2, 2, 321),       # five tiles of keys, and a sixth
+    (2, 3, 130, 385), (1, 2, 449, 449),   # one group has a tile more
+    (1, 1, 1025, 1025),
+    (8, 8, 512, 512), (8, 8, 513, 513)])  # 256 and 320 blocks
+def test_prompt_keys_in_two_groups(D, B, H, S, Sk):
+    from scaffold import ops
+
+    torch.manual_seed(S + D)
+    f = ops.require_ext().prompt_attention
+    q, k, v = (torch.randn(B, H, n, D, device="cuda").bfloat16() for n in (S, Sk, Sk))
+    v += 1
+    got = f(q, k, v, Sk).double()
+    s = q.double() @ k.double().transpose(2, 3).contiguous() / math.sqrt(D)
+    see = (torch.arange(Sk, device="cuda")
+           <= torch.arange(Sk - S, Sk, device="cuda").unsqueeze(1))
+    want = torch.softmax(s.masked_fill(~see, -math.inf), -1) @ v.double()
+    # the bounds of test_prompt_attention_matches_float64
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13).all()
+    assert (got - want).norm() / want.norm() < 2.0 ** -9
+    # all scores near the lowest float's exponent, the highest in either group's tiles
+    q, k = torch.full_like(q, 1e17), torch.full_like(k, -1e18)
+    for best in (0, 64, 70, 130):
+        if best > Sk - S:
+            break
+        k[:, :, best] = -9e17
+        got = f(q, k, v, Sk)
+        assert torch.equal(got, v[:, :, best:best + 1].expand_as(got))
+        k[:, :, best] = float("nan")
+        assert f(q, k, v, Sk).isnan().all()
+        k[:, :, best] = -1e18
+    assert f(q * 1e13, k * 1e13, v, Sk).isnan().all()
+
+
 @pytest.mark.parametrize("D,H,G", [(128, 4, 2), (64, 3, 3)])
 @pytest.mark.parametrize("S,Sk", [(1, 70), (5, 5), (64, 65), (257, 300)])
 def test_prompt_scores_far_below_zero(D, H, G, S, Sk):
