@@ -108,7 +108,8 @@ torch::Tensor prompt_attention(torch::Tensor q, torch::Tensor k,
 torch::Tensor skinny_linear_parts(torch::Tensor x, torch::Tensor w,
                                   c10::optional<torch::Tensor> bias);
 c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Tensor& w,
-                                         const c10::optional<torch::Tensor>& bias, long act);
+                                         const c10::optional<torch::Tensor>& bias, long act,
+                                         bool grad);
 torch::Tensor skinny_linear(torch::Tensor x, torch::Tensor w,
                             c10::optional<torch::Tensor> bias,
                             c10::optional<torch::Tensor> res, long act,
@@ -224,18 +225,19 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "sums over parts of the depth of a product of few rows", py::arg("x"),
         py::arg("w"), py::arg("bias") = py::none());
   m.def("tile_linear",
-        [](py::object x, py::object w, py::object bias, long act) {
+        [](py::object x, py::object w, py::object bias, long act, bool grad) {
           c10::optional<torch::Tensor> y;
           // classes and modes that override functions see torch's product
           if (at::impl::torch_function_mode_enabled()) return y;
           for (const auto* t : {&x, &w, &bias})
             if (!t->is_none() && !THPVariable_CheckExact(t->ptr())) return y;
           y = tile_linear(x.cast<torch::Tensor>(), w.cast<torch::Tensor>(),
-                          bias.cast<c10::optional<torch::Tensor>>(), act);
+                          bias.cast<c10::optional<torch::Tensor>>(), act, grad);
           return y;
         },
         "act(x w^T + b) of some hundred rows, or None; act: 0 none, 1 tanh-GELU, 2 erf-GELU",
-        py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("act") = 0);
+        py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("act") = 0,
+        py::arg("grad") = false);
   m.def("skinny_linear", &skinny_linear,
         "product of up to 64 rows with bias, residual, GELU or SwiGLU",
         py::arg("x"), py::arg("w"), py::arg("bias") = py::none(),

@@ -113,7 +113,8 @@ c10::optional<torch::Tensor> residual_linear(const torch::Tensor& x, const torch
   t.bias = bias ? (const short*)bias->data_ptr() : nullptr;
   t.ldx = t.K;
   t.ldy = t.N;
-  if ((size_t)res.data_ptr() % 16 || !big_takes(t, TILE_NONE)) return c10::nullopt;
+  if ((size_t)res.data_ptr() % 16 || t.K > BIG_DEPTH_OF_TRAINING || !big_takes(t, TILE_NONE))
+    return c10::nullopt;
   const c10::DeviceGuard guard(x.device());
   auto y = torch::empty(shape, x.options());
   t.y = (short*)y.data_ptr();
@@ -135,8 +136,8 @@ c10::optional<torch::Tensor> residual_linear(const torch::Tensor& x, const torch
 // 4096 out of 1000 66 and 52; but 608 x 12888 out of 11800 (0.60) 225 and 236.
 //
 // Sums run in the library's order, and the gradients are the same bits, but where it splits
-// the tiles of a last round.  Deep sums of few rounds whose last is half empty stay with it:
-// 4096 x 14336 out of 8192 rows would take 721 instead of 982, but 5000 of its 59 million
+// the tiles of a last round.  Deep sums of few rounds whose last is half empty stay with it (up
+// to 4096 rows deep it does not split them): 4096 x 14336 out of 8192 rows would take 721 instead of 982, but 5000 of its 59 million
 // gradients are rounded otherwise, after which a step of AdamW leaves the next gradients
 // 2 % apart, the most that bf16 lets them.  (128256 x 4096, the head, of 31 rounds, 7361 and
 // 5691: 5000 of 525 million, and 0.7 %.)
@@ -156,7 +157,7 @@ c10::optional<torch::Tensor> wide_weight_grad(const torch::Tensor& dy, const tor
   a.lda = N; a.ldb = a.ldy = K;
   const long tiles = up(N, 256) * up(K, 256), last = tiles % UNITS;
   if (at_work(a, rounds(a, 8)) < 0.66 ||
-      (T >= 8192 && tiles < 4 * UNITS && last > 0 && last <= UNITS / 2))
+      (T > 4096 && tiles < 4 * UNITS && last > 0 && last <= UNITS / 2))
     return c10::nullopt;
   // the operands' device, whichever is current: torch's product goes by it too
   const c10::DeviceGuard guard(dy.device());
@@ -171,6 +172,11 @@ c10::optional<torch::Tensor> wide_weight_grad(const torch::Tensor& dy, const tor
 // where tiles keep 0.72 of the chip at work, of 150 sizes every one.  In us, library and this:
 // 16384 rows, 768 from 3072 86 and 68, 3072 from 768 85 and 68, 8192 rows, 4096 from 28672 1400
 // and 1302, 14336 from 4096 716 and 642; but 2000 rows, 4096 from 28672 (0.60) 394 and 472.
+//
+// Of Llama-3-8B's products, 4096 and more deep, a library splits the last round of tiles at 6002
+// to 7800 rows, not up to 5120 nor at full rounds (8000 to 8192 rows): there this one's bits are the
+// same.  Elsewhere it is left out: 10000 of 30 million values rounded otherwise are 0.9 % of the
+// first step's gradients, and 4 % of the next's.
 c10::optional<torch::Tensor> input_grad(const torch::Tensor& dy, const torch::Tensor& w) {
   if (watched() || !dy.is_cuda() || !plain(dy, dy.device()) || !plain(w, dy.device()) ||
       dy.dim() != 2 || w.dim() != 2 || dy.size(1) != w.size(0) || !dy.is_contiguous() ||
@@ -186,7 +192,9 @@ c10::optional<torch::Tensor> input_grad(const torch::Tensor& dy, const torch::Te
   a.M = (int)M; a.N = (int)K; a.K = (int)N;
   a.lda = N; a.ldb = a.ldy = K;
   const int nt = columns(a);
-  if (at_work(a, rounds(a, nt)) < 0.72) return c10::nullopt;
+  if (at_work(a, rounds(a, nt)) < 0.72 ||
+      (N > BIG_DEPTH_OF_TRAINING && M > 5120 && up(M, 256) * up(K, 256) % UNITS != 0))
+    return c10::nullopt;
   const c10::DeviceGuard guard(dy.device());
   auto dx = torch::empty({M, K}, dy.options());
   a.y = (short*)dx.data_ptr();

@@ -269,7 +269,8 @@ void tile_gemm(const TileArgs& a, TileAct act, hipStream_t st) {
 // act(x w^T + b) of rows (..., K), act as TileAct, by these or by large tiles; None: not
 // what they are for
 c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Tensor& w,
-                                         const c10::optional<torch::Tensor>& bias, long act) {
+                                         const c10::optional<torch::Tensor>& bias, long act,
+                                         bool grad) {
   // what a plain kernel would not see: gradients, transforms, tensors of Python classes
   if (watched()) return c10::nullopt;
   auto plain = [&](const torch::Tensor& t) { return ::plain(t, x.device()); };
@@ -289,7 +290,7 @@ c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Te
   a.bias = bias.has_value() ? (const short*)bias->data_ptr() : nullptr;
   a.ldx = x.dim() == 2 ? x.stride(0) : a.K;
   a.ldy = a.N;
-  const bool big = big_takes(a, (TileAct)act);
+  const bool big = (!grad || a.K <= BIG_DEPTH_OF_TRAINING) && big_takes(a, (TileAct)act);
   if (!big && !tile_takes(a, (TileAct)act)) return c10::nullopt;
   // the operands' device, whichever is current: torch's product goes by it too
   const c10::DeviceGuard guard(x.device());

@@ -571,19 +571,20 @@ _HAND_GEMM_ALL = False  # flipped by benchmarks once the 8-phase core wins
 
 
 def _tiled(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None,
-           act: int = 0) -> Optional[torch.Tensor]:
+           act: int = 0, grad: bool = False) -> Optional[torch.Tensor]:
     """act(x w^T + b) of some hundred rows by tiles of our own, which take more of
     the chip there (both sides' times: csrc/kernels/tile_gemm.hip).  None for what
     they are not for, or where torch has to see the product."""
     if not x.is_cuda or torch.compiler.is_compiling() or ext() is None:
         return None
-    return ext().tile_linear(x, w, b, act)
+    return ext().tile_linear(x, w, b, act, grad)
 
 
-def _product(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None
-             ) -> torch.Tensor:
-    """F.linear without a graph, by tiles of our own where they are for it."""
-    y = _tiled(x, w, b)
+def _product(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None,
+             grad: bool = False) -> torch.Tensor:
+    """F.linear without a graph, by tiles of our own where they are for it; grad:
+    as the forward of a function that has one."""
+    y = _tiled(x, w, b, 0, grad)
     return F.linear(x, w, b) if y is None else y
 
 
@@ -599,7 +600,7 @@ def _residual_product(x: torch.Tensor, w: torch.Tensor,
     """_product() + res, in one kernel where that is ours."""
     y = (require_ext().residual_linear(x, w, b, res, True)
          if _many(res) and not torch.compiler.is_compiling() else None)
-    return _product(x, w, b) + res if y is None else y
+    return _product(x, w, b, True) + res if y is None else y
 
 
 class _LinearLib(torch.autograd.Function):
@@ -615,7 +616,7 @@ class _LinearLib(torch.autograd.Function):
         ctx.x_shape = x.shape
         if res is not None:
             return _residual_product(x, w, b, res)
-        return _product(x, w, b)
+        return _product(x, w, b, True)
 
     @staticmethod
     def backward(ctx, dy):
@@ -636,7 +637,7 @@ class _LinearGeluLib(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w, b):
-        pre = _product(x, w, b)
+        pre = _product(x, w, b, True)
         ctx.save_for_backward(x, w, b, pre)
         return F.gelu(pre, approximate="tanh")
 

@@ -192,3 +192,31 @@ def test_residual_layers_take_it(n, monkeypatch):
         assert torch.equal(y, ops.linear(x, w, b) + r[:1])
         (got,) = torch.autograd.grad(y, r, dy)
         assert got.shape == r.shape and not got[1:].any()
+
+
+def test_deep_products_of_training_are_the_library_s():
+    """Where a library splits the depth, its gradients are kept; without them
+    the kernel of tiles is as good."""
+    torch.manual_seed(0)
+    x, w = _rows(1000, 4096), (_rows(28672, 4096) / 64).contiguous()
+    f = ops.require_ext().tile_linear
+    assert f(x, w) is not None and f(x, w, None, 0, True) is None
+    want = F.linear(x, w)
+    assert torch.equal(ops.linear(x.requires_grad_(), w), want)
+    x, w, res = _rows(3000, 4096), (_rows(4096, 4096) / 64).contiguous(), _rows(3000, 4096)
+    assert torch.equal(ops.linear_residual(x.requires_grad_(), w, None, res),
+                       F.linear(x, w) + res)
+
+
+@pytest.mark.parametrize("T,own", [(4096, True), (5000, True), (6002, False), (8192, True)])
+def test_deep_gradients_are_the_library_s(T, own):
+    """The same bits where it does not split the depth, and its own elsewhere."""
+    ext = ops.require_ext()
+    torch.manual_seed(T)
+    w, x, dy = _rows(4096, 14336).contiguous(), _rows(T, 14336), _rows(T, 4096)
+    dx, dw = ext.input_grad(dy, w), ext.wide_weight_grad(dy, x)
+    assert (dx is not None) == own and (dw is not None) == (T == 4096)
+    if own:
+        assert torch.equal(dx, dy @ w)
+    if T == 4096:
+        assert torch.equal(dw, dy.t() @ x)
