@@ -137,10 +137,10 @@ c10::optional<torch::Tensor> residual_linear(const torch::Tensor& x, const torch
 //
 // Sums run in the library's order, and the gradients are the same bits, but where it splits
 // the tiles of a last round.  Deep sums of few rounds whose last is half empty stay with it (up
-// to 4096 rows deep it does not split them): 4096 x 14336 out of 8192 rows would take 721 instead of 982, but 5000 of its 59 million
-// gradients are rounded otherwise, after which a step of AdamW leaves the next gradients
-// 2 % apart, the most that bf16 lets them.  (128256 x 4096, the head, of 31 rounds, 7361 and
-// 5691: 5000 of 525 million, and 0.7 %.)
+// to 4096 rows deep it does not split them): 4096 x 14336 out of 8192 rows would take 721 instead
+// of 982, but 5000 of its 59 million gradients are rounded otherwise, after which a step of AdamW
+// leaves the next gradients 2 % apart, the most that bf16 lets them.  (128256 x 4096, the head, of
+// 31 rounds, 7361 and 5691: 5000 of 525 million, and 0.7 %.)
 c10::optional<torch::Tensor> wide_weight_grad(const torch::Tensor& dy, const torch::Tensor& x) {
   if (watched() || !dy.is_cuda() || !plain(dy, dy.device()) || !plain(x, dy.device()) ||
       dy.dim() != 2 || x.dim() != 2 || dy.size(0) != x.size(0) || !dy.is_contiguous() ||
