@@ -235,17 +235,21 @@ c10::optional<torch::Tensor> head_logits(const torch::Tensor& x, const torch::Te
 }
 
 // {d w, d^T x} of such logits' gradient d, zero behind its last column; undefined where not
-// wanted
+// wanted.  By torch where the rows lie otherwise: a saved tensor that a hook has copied comes
+// back with one row behind the other.
 std::vector<torch::Tensor> head_grads(const torch::Tensor& d, const torch::Tensor& x,
                                       const torch::Tensor& w, bool want_x, bool want_w) {
+  auto whole = [&](const torch::Tensor& t) {
+    return plain(t, d.device()) && t.dim() == 2 && t.is_contiguous() &&
+           (size_t)t.data_ptr() % 16 == 0;
+  };
+  if (watched() || !d.is_cuda() || !plain(d, d.device()) || d.dim() != 2 || !whole(x) ||
+      !whole(w) || x.size(0) != d.size(0) || w.size(0) != d.size(1) || x.size(1) != w.size(1) ||
+      x.size(1) % 8 || d.stride(1) != 1 || d.stride(0) != up(d.size(1), 128) * 128 ||
+      d.storage_offset() != 0 || (long)d.storage().nbytes() < 2 * d.size(0) * d.stride(0) ||
+      (size_t)d.data_ptr() % 16)
+    return {want_x ? at::mm(d, w) : torch::Tensor(), want_w ? at::mm(d.t(), x) : torch::Tensor()};
   const long R = d.size(0), V = w.size(0), K = w.size(1), ld = d.stride(0);
-  TORCH_CHECK(d.is_cuda() && d.scalar_type() == torch::kBFloat16 && d.dim() == 2 &&
-              d.size(1) == V && d.stride(1) == 1 && ld == up(V, 128) * 128 &&
-              d.storage_offset() == 0 && (long)d.storage().nbytes() >= 2 * R * ld &&
-              x.is_contiguous() && w.is_contiguous() && x.size(0) == R && x.size(1) == K &&
-              x.scalar_type() == torch::kBFloat16 && w.scalar_type() == torch::kBFloat16 &&
-              K % 8 == 0 && ((size_t)x.data_ptr() | (size_t)w.data_ptr()) % 16 == 0,
-              "head_grads: operands");
   const c10::DeviceGuard guard(d.device());
   auto st = scaffold_stream();
   torch::Tensor dx, dw;

@@ -783,7 +783,7 @@ class _HeadCE(torch.autograd.Function):
         x, w, logits, targets, lse = ctx.saved_tensors
         m = require_ext()
         need_x, need_w = ctx.needs_input_grad[:2]
-        h = x.view(-1, x.shape[-1])
+        h = x.contiguous().view(-1, x.shape[-1])
         d = m.softmax_xent_bwd(
             logits, targets, lse,
             dloss_dev=dloss.to(logits.device, torch.float32))

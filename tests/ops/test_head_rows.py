@@ -17,6 +17,22 @@ def _made(R, V, K):
     return x, w, torch.randint(0, V, (R,), device="cuda")
 
 
+def _gradient(x, w, t):
+    """The gradient of the logits, whose bits no layout changes."""
+    m = ops.require_ext()
+    logits = m.head_logits(x.detach(), w.detach())
+    return m.softmax_xent_bwd(logits, t, m.softmax_xent_fwd(logits, t)[1])
+
+
+def _close(got, a, b):
+    """got = a b, of which every partial sum is below the sum of sizes: the
+    result's rounding, and that of depth / 32 + 32 float32 sums."""
+    a, b = a.double().contiguous(), b.double()
+    want, size = a @ b, a.abs() @ b.abs()
+    lim = 2.0 ** -8 * want.abs() + (a.shape[1] / 32 + 32) * 2.0 ** -24 * size
+    assert got.shape == want.shape and ((got.double() - want).abs() <= lim).all()
+
+
 def _calls(monkeypatch):
     ext, calls = ops.require_ext(), []
     made = ext.head_grads
@@ -58,6 +74,27 @@ def test_the_same_bits_as_one_row_behind_the_other(monkeypatch):
     b = torch.autograd.grad(ops.softmax_cross_entropy(F.linear(x, w), t), (x, w))
     for g, h in zip(a, b):
         assert (g.double() - h.double()).norm() < 1e-3 * h.double().norm()
+
+
+@pytest.mark.parametrize("R,V,K", [(2047, 10001, 256), (2048, 15001, 768)])
+@pytest.mark.parametrize("how", ["host", "copy", "strides"])
+def test_saved_tensors_that_hooks_have_copied(R, V, K, how):
+    """Logits come back with one row behind the other, or as they were: the
+    gradients are the products they were."""
+    from torch.autograd.graph import save_on_cpu, saved_tensors_hooks
+
+    x, w, t = _made(R, V, K)
+    with {"host": save_on_cpu(),
+          "copy": saved_tensors_hooks(lambda s: s.clone(memory_format=torch.contiguous_format),
+                                      lambda s: s),
+          "strides": saved_tensors_hooks(
+              lambda s: s.clone(memory_format=torch.contiguous_format),
+              lambda s: F.pad(s, (0, 24))[..., :-24] if s.shape == (R, V) else s)}[how]:
+        loss = ops.lm_head_ce(x, w, t)
+    dx, dw = torch.autograd.grad(loss, (x, w))
+    d = _gradient(x, w, t)
+    _close(dx, d, w.detach())
+    _close(dw, d.t(), x.detach())
 
 
 def test_small_or_other_operands_go_the_general_way(monkeypatch):
