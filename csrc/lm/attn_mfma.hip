@@ -667,7 +667,9 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
     __syncthreads();
     if (part || !w_any) return;
     const float m1 = to[16 * NDT][l], mn = fmaxf(m_run, m1);
-    const float al = __builtin_amdgcn_exp2f(m_run - mn), be = __builtin_amdgcn_exp2f(m1 - mn);
+    // an infinite sink is the largest of all, and leaves nothing of what has scores
+    const float al = m_run == mn ? 1.f : __builtin_amdgcn_exp2f(m_run - mn);
+    const float be = __builtin_amdgcn_exp2f(m1 - mn);
     l_run = l_run * al + to[16 * NDT + 1][l] * be;
     #pragma unroll
     for (int i = 0; i < NDT; ++i)

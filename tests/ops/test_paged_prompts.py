@@ -62,3 +62,17 @@ def test_a_sink_that_is_no_number_shows(parts):
     assert got[:, 1].isnan().all()
     got[:, 1] = 0
     assert got.isfinite().all()
+
+
+@pytest.mark.parametrize("H,G,d,e", [(4, 2, 64, 64), (3, 3, 128, 64),
+                                     (64, 64, 64, 64), (128, 64, 128, 128)])
+def test_a_sink_above_all_leaves_nothing(H, G, d, e):
+    """Of its head, whether a page's keys are split (below 257 blocks) or not."""
+    T = 290
+    q, k, v = rnd(T, H, d, seed=1), rnd(T, G, d, seed=2), rnd(T, G, e, seed=3)
+    sink = rnd(H, seed=4)
+    sink[1] = math.inf
+    got = run_attention("cuda", torch.bfloat16, q, k, v, scale=d ** -0.5, size=0,
+                        sink=sink, parts=(T,))
+    assert not got[:, 1].any()
+    assert got.isfinite().all() and got[:, 0].any() and got[:, 2].any()
