@@ -255,8 +255,13 @@ gemm_kernel(BigArgs a) {
       step(no, no);
       step(yes, no);
     }
-    // the last products' results
-    asm volatile("s_nop 15\n\ts_nop 15");
+    // The last products' results, which take up to 18 wait states.  Every sum goes through a
+    // statement behind the wait, so that no read of it can be placed before that.
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    #pragma unroll
+    for (int i = 0; i < MT; ++i)
+      #pragma unroll
+      for (int j = 0; j < NT; ++j) asm volatile("" : "+a"(acc[i][j]));
     __builtin_amdgcn_sched_barrier(0);
     int m0, n0;
     place(t, m0, n0);
