@@ -441,6 +441,13 @@ def _colsum(dy2: torch.Tensor) -> torch.Tensor:
     return dy2.sum(0)
 
 
+def _unseen() -> bool:
+    """Whether nothing has to see a product of a backward: no graph, no transform,
+    no compiler, which traces it with gradients off."""
+    return not (torch.is_grad_enabled() or torch.compiler.is_compiling()
+                or _transformed())
+
+
 def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """dy^T x of contiguous rows.  The library splits the rows too little
     where dW has few tiles: in us, library and own kernel, 3072 x 768 out of
@@ -451,8 +458,7 @@ def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     16384 108 and 86.  Where tiles fill the chip, another: csrc/kernels/big_gemm.hip."""
     n, k = dy.shape[1], x.shape[1]
     many = n * k >= 11_000_000                 # tiles for two thirds of the chip
-    if (x.is_cuda and (many or x.shape[0] >= 8192)
-            and not torch.is_grad_enabled() and not _transformed()):
+    if x.is_cuda and (many or x.shape[0] >= 8192) and _unseen():
         small, large = min(n, k), max(n, k)
         if (small >= 64 and (small >= 256 or large <= 8192)
                 and dy.dtype == x.dtype == torch.bfloat16
@@ -470,8 +476,7 @@ def _input_grad(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """dy w of contiguous rows, by a kernel of our own where that is faster
     than the library's (both sides' times: csrc/kernels/big_gemm.hip)."""
     if (dy.shape[0] * w.shape[1] >= 9_900_000  # tiles for most of the chip
-            and dy.is_cuda and not torch.is_grad_enabled()
-            and not _transformed()):
+            and dy.is_cuda and _unseen()):
         dx = require_ext().input_grad(dy, w)
         if dx is not None:
             return dx
@@ -714,9 +719,11 @@ def linear_residual(x: torch.Tensor, w: torch.Tensor,
             and torch.is_grad_enabled() and not _transformed()):
         # gradients by own kernels
         if (res.is_cuda and res.dtype == x.dtype
-                and res.shape == x.shape[:-1] + w.shape[:1]):
+                and res.shape == x.shape[:-1] + w.shape[:1]
+                and not torch.compiler.is_compiling()):
             return _LinearLib.apply(x, w, b, res)
-        return _LinearLib.apply(x, w, b) + res
+        if b is not None:
+            return _LinearLib.apply(x, w, b) + res
     return F.linear(x, w, b) + res
 
 
