@@ -668,13 +668,13 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
     if (part || !w_any) return;
     const float m1 = to[16 * NDT][l], mn = fmaxf(m_run, m1);
     // an infinite sink is the largest of all, and leaves nothing of what has scores
-    const float al = m_run == mn ? 1.f : __builtin_amdgcn_exp2f(m_run - mn);
+    const float al = __builtin_amdgcn_exp2f(m_run == mn ? 0.f : m_run - mn);
     const float be = __builtin_amdgcn_exp2f(m1 - mn);
-    l_run = l_run * al + to[16 * NDT + 1][l] * be;
+    l_run = fmaf(l_run, al, to[16 * NDT + 1][l] * be);
     #pragma unroll
     for (int i = 0; i < NDT; ++i)
       #pragma unroll
-      for (int r = 0; r < 16; ++r) o[i][r] = o[i][r] * al + to[16 * i + r][l] * be;
+      for (int r = 0; r < 16; ++r) o[i][r] = fmaf(o[i][r], al, to[16 * i + r][l] * be);
   }
   if (row < t.y) {
     const float inv = l_run > 0.f ? a.out_scale / l_run : 0.f;
