@@ -409,6 +409,11 @@ attn_prefill_form_kernel(AttnArgs a, const int4* __restrict__ tiles,
 // waves of a SIMD, which add their results up at the end, for one wave alone has 8 cycles
 // an instruction and waits between products and softmax.  Two prompts of 1000 behind 1500,
 // 256 blocks, 47.6 -> 41.3 us.  (There, copies two pages ahead into three images take 51.)
+// Of few pages the adding up is more than that saves.  In us, KS = 1 and 2: two heads a
+// block, 16 of 128 on 4, 8 x 64 tokens (a page) 9.9 and 11.1, 4 x 128 (two) 11.8 and 13.0, 192
+// (three) 13.6-14.6 and 14.0-14.2, 2 x 193 14.0-15.3 and 14.4-14.6, 300 (five) 17.6 and 16.3-16.9;
+// of 64, 7.2 and 7.8, 8.6 and 8.7, 9.7 and 9.9, 10.6 and 10.5; one head, 8 of 128 9.8 and 10.1,
+// 11.9 and 11.6, 14.3 and 13.4; 3 of 64 7.1 and 7.0, 8.5 and 7.8, 9.5 and 8.7.
 template <int DK, int DV, int HPB, bool BIAS, int KS>
 __global__ void __launch_bounds__(HPB * 128 * KS, KS == 1 ? 2 : 1)
 attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
@@ -684,12 +689,19 @@ attn_prefill_kernel(AttnArgs a, const int4* __restrict__ tiles, int n_tiles) {
 
 constexpr unsigned UNITS = 256;          // compute units
 
+// pages that a tile sees at most
+int most_pages(const AttnArgs& a) {
+  const long reach = a.reach ? a.reach : (long)a.max_pages * LM_PAGE;
+  const long seen = a.size ? std::min(reach, a.size + LM_PAGE - 1l) : reach;
+  return (int)((seen + LM_PAGE - 1) / LM_PAGE);
+}
+
 // FORM 0: as stored; 1: with a bias by distance; 2: tied, with one; 3: window
 template <int DK, int DV, int HPB, int FORM>
 void go(const AttnArgs& a, const int4* tiles, int n, hipStream_t st) {
   const dim3 grid((unsigned)((long)n * a.G * (a.H / a.G / HPB)));
   if constexpr (FORM < 2) {
-    if (grid.x <= UNITS)
+    if (grid.x <= UNITS && most_pages(a) >= (HPB == 2 ? 5 : DV / 64))
       hipLaunchKernelGGL((attn_prefill_kernel<DK, DV, HPB, FORM == 1, 2>), grid,
                          dim3(HPB * 256), 0, st, a, tiles, n);
     else

@@ -361,9 +361,10 @@ Tensor paged_attention(Tensor qkv, Tensor kc, Tensor vc, Tensor table,
                        Tensor pos, Tensor slot, Tensor tiles, long n_dec,
                        OptTensor qw, OptTensor kw, OptTensor sink,
                        OptTensor slopes, long heads, long size, double scale,
-                       double eps, long max_len) {
+                       double eps, long max_len, long reach) {
   AttnArgs a = attn_args(qkv, kc, vc, table, qw, kw, sink, slopes, heads, size,
                          scale, eps);
+  a.reach = (int)std::max<long>(0, std::min(reach, max_len));
   return attend(a, qkv, pos, slot, tiles, n_dec, max_len);
 }
 
@@ -992,7 +993,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "post-norm, residual add and next pre-norm in one pass");
   m.def("gelu_erf", &gelu_erf, "exact GELU");
   m.def("paged_attention", &paged_attention,
-        "chunked causal attention with sink over a paged cache");
+        "chunked causal attention with sink over a paged cache; reach: prompt rows see "
+        "positions below it (0: not known)",
+        py::arg("qkv"), py::arg("kc"), py::arg("vc"), py::arg("table"), py::arg("pos"),
+        py::arg("slot"), py::arg("tiles"), py::arg("n_dec"), py::arg("qw"), py::arg("kw"),
+        py::arg("sink"), py::arg("slopes"), py::arg("heads"), py::arg("size"),
+        py::arg("scale"), py::arg("eps"), py::arg("max_len"), py::arg("reach") = 0);
   m.def("window_attention", &window_attention,
         "window attention with kept first tokens over a paged cache");
   m.def("gla", &gla, "gated linear attention over state slots");

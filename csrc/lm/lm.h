@@ -140,6 +140,7 @@ struct AttnArgs {
   int size;           // chunk or window length in tokens; 0 = plain causal
   float scale;
   float eps;
+  int reach;          // prompt rows see positions below it; 0: not known
 };
 // rows [row0, row0 + n): norm q in place, norm k into the cache, copy v
 void lm_attn_prep(const AttnArgs& a, const int* pos, const int* slot, int row0,

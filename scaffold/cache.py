@@ -83,7 +83,8 @@ class StepPlan:
     seqs  (m, 4): first tile, tiles, position of the portion, slot
     slot < 0 marks a row to skip (an idle slot of a fixed-width step).
     portions repeats the prompt portions for the host: first row, rows,
-    position of the first, slot."""
+    position of the first, slot; reach: the positions below it are all that
+    they see."""
     tokens: torch.Tensor           # (T,) int64
     pos: torch.Tensor              # (T,) int32
     slot: torch.Tensor             # (T,) int32
@@ -92,6 +93,7 @@ class StepPlan:
     n_dec: int
     rows: Optional[torch.Tensor]   # wanted rows, int32; None = every row
     portions: Sequence[Tuple[int, int, int, int]] = ()
+    reach: int = 0
     _spans: Dict[int, Tuple[torch.Tensor, torch.Tensor]] = field(
         default_factory=dict)
 
@@ -349,7 +351,9 @@ class PagedStateCache:
                 end += n
             tokens[at:end] = run[0] if len(run) == 1 else torch.cat(run)
         return (StepPlan(tokens, ps, sl, tl.view(nt, 4), sq.view(ns, 4),
-                         n_dec, rw, portions), [len(e[2]) for e in entries])
+                         n_dec, rw, portions,
+                         max((p0 + n for _, n, p0, _ in portions), default=0)),
+                [len(e[2]) for e in entries])
 
     def commit(self, entries: Sequence[Entry]) -> None:
         for slot, toks, _ in entries:

@@ -319,7 +319,7 @@ def paged_attention(qkv, cache, run, plan, *, heads, q_norm, k_norm, sink,
         return require_lm_ext().paged_attention(
             qkv, kc, vc, cache.table, plan.pos, plan.slot, plan.tiles,
             plan.n_dec, q_norm, k_norm, sink, slopes, heads, size, scale, eps,
-            cache.max_len)
+            cache.max_len, plan.reach)
     G, page, dim, vdim = kc.shape[1], kc.shape[2], kc.shape[3], vc.shape[3]
     q, k, v = torch.split(qkv, [heads * dim, G * dim, G * vdim], dim=1)
     q, k, v = (q.reshape(-1, heads, dim), k.reshape(-1, G, dim),

@@ -50,6 +50,55 @@ def test_as_many_blocks_as_units_and_more(H, G, d, parts):
     close(got, want.to(got.dtype).reshape(got.shape), torch.bfloat16)
 
 
+def _check(H, G, d, e, parts, size=0, sink=None, slopes=None):
+    T = sum(parts)
+    q, k, v = rnd(T, H, d, seed=1), rnd(T, G, d, seed=2), rnd(T, G, e, seed=3)
+    got = run_attention("cuda", torch.bfloat16, q, k, v, scale=d ** -0.5, size=size,
+                        sink=sink, parts=parts, slopes=slopes).double()
+    i, j = torch.arange(T, device="cuda").unsqueeze(1), torch.arange(T, device="cuda")
+    q, k, v = (t.transpose(0, 1).cuda() for t in (
+        q, k.repeat_interleave(H // G, 1), v.repeat_interleave(H // G, 1)))
+    x = q @ k.transpose(1, 2).contiguous() * d ** -0.5
+    if slopes is not None:
+        x = x - slopes.cuda().double().view(H, 1, 1) * (i - j)
+    x = x.masked_fill((j > i) | (j < i - i % size if size else j < 0), -math.inf)
+    none = torch.full((H,), -math.inf).double()
+    s = (none if sink is None else sink).cuda().view(H, 1, 1).expand(H, T, 1)
+    w = torch.softmax(torch.cat([x, s], 2), 2)[..., :-1]
+    want = (w @ v).transpose(0, 1)
+    # one rounding of the result; weights in two parts of 8 bits, the bias and the
+    # exponents of scores below 2^7 in float32
+    lim = 2.0 ** -8 * want.abs() + 2.0 ** -14 * (w @ v.abs()).transpose(0, 1) + 2.0 ** -20
+    assert ((got - want).abs() <= lim).all()
+
+
+FORMS = [(16, 4, 128, 128), (4, 2, 64, 64), (8, 2, 64, 128), (4, 2, 128, 64), (6, 3, 72, 104),
+         (3, 3, 128, 128), (3, 1, 64, 64), (5, 5, 64, 128), (3, 3, 128, 64), (3, 3, 104, 40)]
+
+
+@pytest.mark.parametrize("H,G,d,e", FORMS)
+@pytest.mark.parametrize("parts", [(64,), (65,), (256,), (257,), (30, 34, 33, 40)], ids=str)
+def test_few_pages(H, G, d, e, parts):
+    """As many pages as are not split yet, and one more: one (and none, values of 64), or
+    four with two heads a block."""
+    _check(H, G, d, e, parts, sink=rnd(H, seed=4, scale=2))
+    _check(H, G, d, e, parts, size=70, slopes=torch.rand(H) / 8)
+
+
+@pytest.mark.parametrize("H,G,d,e", FORMS)
+@pytest.mark.parametrize("what", ["plain", "sink", "none", "chunks", "slopes"])
+def test_many_blocks(H, G, d, e, what):
+    """More blocks than compute units, where pages are not split: as many copies of the
+    form's groups of heads as it takes for 5 and 9 tiles."""
+    for parts in ((257,), (60, 515)):
+        n = 257 // -(-max(parts) // 64) // G + 1
+        sink = rnd(n * H, seed=4, scale=2) if what in ("sink", "none", "chunks") else None
+        if what == "none":
+            sink[::2] = -math.inf
+        _check(n * H, n * G, d, e, parts, size=200 if what == "chunks" else 0, sink=sink,
+               slopes=torch.rand(n * H) / 8 if what == "slopes" else None)
+
+
 @pytest.mark.parametrize("parts", [(65,), (64, 1)], ids=str)
 def test_a_sink_that_is_no_number_shows(parts):
     """In its head, and in no other."""

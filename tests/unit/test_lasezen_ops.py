@@ -49,7 +49,7 @@ def test_embed_norm_and_gelu(dev, dt):
 
 # -------------------------------------------------------------- attention
 def run_attention(dev, dt, q, k, v, *, scale, size, sink, parts, qw=None,
-                  kw=None, eps=1e-6, cache=None, slot=None):
+                  kw=None, eps=1e-6, cache=None, slot=None, slopes=None):
     T, H, d = q.shape
     G, e = k.shape[1], v.shape[2]
     cache = cache or op_cache(KVSpec(G, d, e), dev, dt)
@@ -64,7 +64,8 @@ def run_attention(dev, dt, q, k, v, *, scale, size, sink, parts, qw=None,
             q_norm=None if qw is None else qw.to(dev, dt),
             k_norm=None if kw is None else kw.to(dev, dt),
             sink=None if sink is None else sink.to(dev, dt),
-            size=size, scale=scale, eps=eps))
+            size=size, scale=scale, eps=eps,
+            slopes=None if slopes is None else slopes.to(dev, torch.float32)))
         cache.commit(ent)
         at += n
     assert at == T
