@@ -268,48 +268,34 @@ void dispatch_norm(const NormArgs& a, bool f32, hipStream_t st) {
 }
 
 // Memory bounds it: 8192 x 8192 of bf16, read and written, 57 us with 8 bytes a load, blocks
-// with the whole grid's stride and erff(), whose instructions took as long; 42 (6.4 TB/s)
-// with U loads of 16 bytes in flight, a block's next to each other.  One load where that
-// leaves few blocks: 1000 x 1000 4.4 us with four, 3.8 with one.
-template <bool F32, int V, int U>
+// with the whole grid's stride and erff(), whose instructions took as long; 40 with one load
+// of 16 bytes a thread, a block's next to each other.  Four of those in flight are slower at
+// every size, behind the product that left the operand in the caches above all: 9640 x 1704
+// 17.3 us for 13.4, with its product of 256 deep 46.2 for 42.4.  Operands at odd places too:
+// vectors have an element's alignment, which a load of 16 bytes needs no more than.
+template <bool F32>
 __global__ void __launch_bounds__(256)
 gelu_erf_kernel(const void* in, void* out, long n) {
   typedef typename Num<F32>::E E;
-  struct alignas(V * sizeof(E)) Vec { E e[V]; };
-  const long first = ((long)blockIdx.x * U * 256 + threadIdx.x) * V;
-  Vec p[U];
-  #pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (first + u * 256 * V + V <= n) p[u] = *(const Vec*)((const E*)in + first + u * 256 * V);
-  #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const long at = first + u * 256 * V;
-    if (at + V <= n) {
-      #pragma unroll
-      for (int j = 0; j < V; ++j) p[u].e[j] = Num<F32>::down(gelu_erf(Num<F32>::up(p[u].e[j])));
-      *(Vec*)((E*)out + at) = p[u];
-    } else {
-      for (long i = at; i < n; ++i)              // the last few
-        ((E*)out)[i] = Num<F32>::down(gelu_erf(Num<F32>::up(((const E*)in)[i])));
-    }
+  constexpr int V = 16 / sizeof(E);
+  struct Vec { E e[V]; };
+  const long at = ((long)blockIdx.x * 256 + threadIdx.x) * V;
+  if (at + V <= n) {
+    Vec p = *(const Vec*)((const E*)in + at);
+    #pragma unroll
+    for (int j = 0; j < V; ++j) p.e[j] = Num<F32>::down(gelu_erf(Num<F32>::up(p.e[j])));
+    *(Vec*)((E*)out + at) = p;
+  } else {
+    for (long i = at; i < n; ++i)                // the last few
+      ((E*)out)[i] = Num<F32>::down(gelu_erf(Num<F32>::up(((const E*)in)[i])));
   }
 }
 
 template <bool F32>
 void launch_gelu_erf(const void* in, void* out, long n, hipStream_t st) {
-  constexpr int V = F32 ? 4 : 8;
-  auto go = [&](auto v, auto u) {
-    constexpr int VEC = decltype(v)::value, U = decltype(u)::value;
-    const long each = 256 * VEC * U;
-    hipLaunchKernelGGL((gelu_erf_kernel<F32, VEC, U>), dim3((unsigned)((n + each - 1) / each)),
-                       dim3(256), 0, st, in, out, n);
-  };
-  constexpr std::integral_constant<int, V> wide;
-  constexpr std::integral_constant<int, 4> four;
-  constexpr std::integral_constant<int, 1> one;
-  if (((size_t)in | (size_t)out) % 16) go(one, four);
-  else if (n >= 1024 * 1024 * V) go(wide, four);
-  else go(wide, one);
+  const long each = 256 * (F32 ? 4 : 8);
+  hipLaunchKernelGGL((gelu_erf_kernel<F32>), dim3((unsigned)((n + each - 1) / each)), dim3(256),
+                     0, st, in, out, n);
 }
 
 // act(g) * u of rows [g | u], each n wide
