@@ -266,6 +266,15 @@ void tile_gemm(const TileArgs& a, TileAct act, hipStream_t st) {
   else pick<TILE_NONE>(a, tile, st);
 }
 
+// Whether tile_linear() takes a product of that many rows that a gradient goes through
+bool tile_sizes(long M, long N, long K) {
+  if (M < 1 || M >= 1 << 30 || N < 1 || N >= 1 << 30 || K < 1 || K > 1 << 22) return false;
+  TileArgs a = {};
+  a.M = (int)M; a.N = (int)N; a.K = (int)K;
+  a.ldx = K; a.ldy = N;
+  return (K <= BIG_DEPTH_OF_TRAINING && big_takes(a, TILE_NONE)) || tile_takes(a, TILE_NONE);
+}
+
 // act(x w^T + b) of rows (..., K), act as TileAct, by these or by large tiles; None: not
 // what they are for
 c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Tensor& w,

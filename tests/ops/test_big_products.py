@@ -194,6 +194,40 @@ def test_residual_layers_take_it(n, monkeypatch):
         assert got.shape == r.shape and not got[1:].any()
 
 
+@pytest.mark.parametrize("M,N,K,own", [
+    (100, 1024, 2816, False), (256, 1792, 4096, False), (3200, 1408, 1664, False),
+    (255, 4096, 14336, False), (256, 4096, 14336, True), (500, 2048, 2048, True),
+    (8192, 256, 1032, True), (4096, 2056, 128, True), (4096, 64, 2560, True)])
+def test_residuals_without_a_bias_are_torch_s_where_nothing_is_ours(M, N, K, own):
+    x = torch.randn(M, K, device="cuda").bfloat16().requires_grad_()
+    w = (torch.randn(N, K, device="cuda") / K ** 0.5).bfloat16().requires_grad_()
+    res = torch.randn(M, N, device="cuda").bfloat16()
+    y = ops.linear_residual(x, w, None, res)
+    assert (type(y.grad_fn).__name__ == "_LinearLibBackward") == own
+    # two roundings, of which the first may differ
+    torch.testing.assert_close(y, F.linear(x, w) + res, rtol=2 ** -7, atol=2 ** -6)
+
+
+class Marked(torch.Tensor):
+    pass
+
+
+@pytest.mark.filterwarnings("ignore:.*torch.jit.trace:DeprecationWarning")
+def test_residuals_without_a_bias_that_torch_has_to_see():
+    x = torch.randn(4096, 2048, device="cuda").bfloat16().requires_grad_()
+    w = (torch.randn(2048, 2048, device="cuda") / 45).bfloat16().requires_grad_()
+    res = torch.randn(4096, 2048, device="cuda").bfloat16()
+    f = ops.linear_residual
+    assert type(f(x, w, None, res).grad_fn).__name__ == "_LinearLibBackward"
+    assert type(f(x, w, None, res.as_subclass(Marked)).grad_fn).__name__ != "_LinearLibBackward"
+    traced = torch.jit.trace(lambda x, w, r: f(x, w, None, r), (x, w, res), check_trace=False)
+    assert "PythonOp" not in str(traced.graph) and "_LinearLib" not in str(traced.graph)
+    # a weight of one row without its dimension
+    v = w.detach()[0].clone().requires_grad_()
+    (got,) = torch.autograd.grad(f(x, v, None, res[:, 0]).sum(), v)
+    assert got.shape == v.shape
+
+
 def test_deep_products_of_training_are_the_library_s():
     """Where a library splits the depth, its gradients are kept; without them
     the kernel of tiles is as good."""
