@@ -837,12 +837,13 @@ def lm_head_ce(x: torch.Tensor, w: torch.Tensor, targets: torch.Tensor
     t = targets.contiguous().view(-1)
     if x.is_cuda and _FUSED_CE:
         return _LmHeadCE.apply(x, w, t)
-    if x.is_cuda and not _transformed() and not torch.compiler.is_compiling():
-        x = x.contiguous()
-        logits = require_ext().head_logits(x.detach().view(-1, x.shape[-1]),
+    if (x.is_cuda and w.shape[0] % 8 and not _transformed()
+            and not torch.compiler.is_compiling()):
+        h = x.contiguous()
+        logits = require_ext().head_logits(h.detach().view(-1, h.shape[-1]),
                                            w.detach())
         if logits is not None:
-            return _HeadCE.apply(x, w, logits, t)
+            return _HeadCE.apply(h, w, logits, t)
     if x.is_cuda:
         # unfused: full logits through blaslt + K3 CE kernels
         return softmax_cross_entropy(linear(x, w), t)
