@@ -20,6 +20,7 @@ def unhooked(module: nn.Module, cls: type) -> bool:
     """Whether a call of module is no more than cls.forward, which may then be
     part of a larger op."""
     return (type(module) is cls and "forward" not in vars(module)
+            and module._compiled_call_impl is None
             and not (module._forward_hooks or module._forward_pre_hooks
                      or module._backward_hooks or module._backward_pre_hooks
                      or torch.nn.modules.module._has_any_global_hook()))

@@ -10,7 +10,7 @@ from scaffold.models.llama import RMSNorm
 
 @pytest.mark.parametrize("cls", [LayerNorm, RMSNorm])
 @pytest.mark.parametrize("how", ["plain", "hook", "pre", "backward", "global",
-                                 "subclass", "instance"])
+                                 "subclass", "instance", "compiled"])
 def test_norms_with_hooks_are_called(cls, how):
     calls = []
     norm = type("Other", (cls,), {"forward": lambda s, x: calls.append(1) or x})(8) \
@@ -28,6 +28,8 @@ def test_norms_with_hooks_are_called(cls, how):
             lambda *a: calls.append(1))
     elif how == "instance":
         norm.forward = lambda x: calls.append(1) or x
+    elif how == "compiled":
+        norm.compile(backend=lambda graph, _: calls.append(1) or graph.forward)
     try:
         y, same = cls.fork(norm, x)
         (y.sum() + same.sum()).backward()
