@@ -40,11 +40,43 @@ def _calls(monkeypatch):
     return calls
 
 
-@pytest.mark.parametrize("R,V,K", [
-    (2047, 10001, 256),      # both gradients by the library
-    (16384, 3001, 768),      # dx by the kernel
-    (2048, 15001, 768),      # dW by the kernel
-    (2049, 15007, 768)])
+SIZES = [(2047, 10001, 256),      # both gradients by the library
+         (16384, 3001, 768),      # dx by the kernel
+         (2048, 15001, 768),      # dW by the kernel
+         (2049, 15007, 768)]
+
+
+@pytest.mark.parametrize("R,V,K", SIZES)
+def test_each_number_of_each_step(R, V, K):
+    """The last rows and columns too, which are not whole eights: every logit, weight and
+    gradient against 64 bits, of the operands that its step was given."""
+    m = ops.require_ext()
+    x, w, t = _made(R, V, K)
+    x, w = x.detach(), w.detach()
+    logits = m.head_logits(x, w)
+    assert logits.shape == (R, V) and logits.stride() == (-(-V // 128) * 128, 1)
+    _close(logits, x, w.t())
+    loss, lse = m.softmax_xent_fwd(logits, t)
+    z = logits.double()
+    want = z.logsumexp(1)
+    # sums of V exponentials that are 2^-21 off, by 256 threads; logarithms below 2^5
+    off = (V / 256 + 40) * 2.0 ** -24
+    assert ((lse.double() - want).abs() <= off).all()
+    at = z.gather(1, t.unsqueeze(1)).squeeze(1)
+    assert ((loss.double() - (want - at)).abs() <= 2 * off).all()
+    d = m.softmax_xent_bwd(logits, t, lse)
+    assert d.stride() == logits.stride()
+    p = (z - want.unsqueeze(1)).exp()
+    want = p.scatter_add(1, t.unsqueeze(1), torch.full((R, 1), -1.0, device="cuda").double())
+    assert ((d.double() * R - want).abs() <= 2.0 ** -8 * want.abs() + 2 * off * p).all()
+    # which their gradients' products read
+    assert not d.as_strided((R, d.stride(0) - V), d.stride(), V).any()
+    dx, dw = m.head_grads(d, x, w, True, True)
+    _close(dx, d, w)
+    _close(dw, d.t(), x)
+
+
+@pytest.mark.parametrize("R,V,K", SIZES)
 def test_loss_and_gradients(R, V, K, monkeypatch):
     calls = _calls(monkeypatch)
     x, w, t = _made(R, V, K)
@@ -66,7 +98,8 @@ def test_loss_and_gradients(R, V, K, monkeypatch):
         assert abs(ops.lm_head_ce(x, w, t).item() - loss.item()) < 1e-6
 
 
-def test_the_same_bits_as_one_row_behind_the_other(monkeypatch):
+def test_as_near_as_one_row_behind_the_other(monkeypatch):
+    """Sums in another order: one rounding of 2^-9 in some hundred values."""
     calls = _calls(monkeypatch)
     x, w, t = _made(16384, 3001, 768)
     a = torch.autograd.grad(ops.lm_head_ce(x, w, t), (x, w))

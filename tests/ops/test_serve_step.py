@@ -9,10 +9,14 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("D,H,G", [(128, 8, 2), (64, 3, 3)])
+@pytest.mark.parametrize("D,H,G", [(128, 8, 2), (64, 3, 3), (64, 8, 2)])
 @pytest.mark.parametrize("S,Sk", [(1, 1), (2, 130), (63, 63), (64, 65),
-                                  (256, 256), (257, 300), (700, 1025)])
+                                  (256, 256), (257, 300), (700, 1025),
+                                  # keys in two groups of waves, one with a tile more
+                                  (1, 321), (130, 449), (257, 640), (500, 500)])
 def test_prompt_attention_matches_float64(D, H, G, S, Sk):
+    """Queries by token, keys and values in a cache with more behind them, heads that
+    share keys."""
     from scaffold import ops
 
     torch.manual_seed(S + D)
