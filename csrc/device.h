@@ -58,9 +58,9 @@ DEVINL void each(const F& f) {
   each_of(f, std::make_integer_sequence<int, N>{});
 }
 
-// Past the caches, or through them: for what is read or written once and is more than the
-// memory-side cache holds, 256 MB, so that this keeps what will be asked for again, and does
-// not have to write back before it takes something in.
+// Past the caches, or through them: for what is read or written once in passes whose operands
+// and results are together more than the memory-side cache holds, 256 MB, so that this keeps
+// what will be asked for again, and does not have to write back before it takes something in.
 template <bool PAST, typename V>
 DEVINL void put_to(V* to, V v) {
   if constexpr (PAST) __builtin_nontemporal_store(v, to);

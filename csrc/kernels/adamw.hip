@@ -141,11 +141,14 @@ adamw_few_kernel(const long* __restrict__ meta, int n, long total_vec4,
   }
 }
 
-// More places than this: moments and masters are more than the memory-side cache holds, and go
-// past it both ways, so that nothing is written back before something is read.  The new weights
-// go through it.  Through the cache and past, in us: 10 million elements 45 and 53, 25 million
-// 137 and 120, 60 million 320 and 265, 124 million 700 and 565 (6.2 TB/s), 400 million 2354 and
-// 2186; with the stores alone past it 717 for 124 million, with the loads alone 678.
+// More places than this (16.8 million elements, of which a step reads and writes 268 MB and more):
+// moments and masters go past the memory-side cache, of 256 MB, both ways, so that nothing is
+// written back before something is read.  The new weights go through it.  Where the line lies
+// depends on what the cache holds.  Through it and past it, in us, of bf16 gradients: step upon
+// step 10 million 45 and 53, 17 million 88 and 93, 22 million 117 and 115, 25 million 137 and 120,
+// 60 million 320 and 265, 124 million 700 and 565 (6.2 TB/s), 400 million 2354 and 2186; but
+// behind 1.2 GB that were written, as a backward leaves it, 17 million 116 and 100, 20 million 130 and
+// 116.  With the stores alone past it 717 for 124 million, with the loads alone 678.
 constexpr long PAST_CACHES = 4 << 20;    // places
 
 template <bool BF16, bool PAST>

@@ -146,12 +146,13 @@ c10::optional<torch::Tensor> residual_linear(const torch::Tensor& x, const torch
 // of 8192 rows 1646 and 1272, of 500 176 and 106; 4096 x 4096 out of 8192 240 and 188; 6144 x
 // 4096 out of 1000 66 and 52; but 608 x 12888 out of 11800 (0.60) 225 and 236.
 //
-// Sums run in the library's order, and the gradients are the same bits, but where it splits
+// Sums run in the order of the library (hipBLASLt of ROCm 7, at Llama-3-8B's widths; another
+// version or width may differ), and the gradients are the same bits, but where it splits
 // the tiles of a last round.  Deep sums of few rounds whose last is half empty stay with it (up
 // to 4096 rows deep it does not split them): 4096 x 14336 out of 8192 rows would take 721 instead
-// of 982, but 5000 of its 59 million gradients are rounded otherwise, after which a step of AdamW
-// leaves the next gradients 2 % apart, the most that bf16 lets them.  (128256 x 4096, the head, of
-// 31 rounds, 7361 and 5691: 5000 of 525 million, and 0.7 %.)
+// of 982, but 5000 of its 59 million gradients are rounded otherwise, no nearer to 64 bits or
+// farther, after which a step of AdamW leaves the next gradients 2 % apart, the most that bf16
+// lets them.  (128256 x 4096, the head, of 31 rounds, 7361 and 5691: 5000 of 525 million, and 0.7 %.)
 c10::optional<torch::Tensor> wide_weight_grad(const torch::Tensor& dy, const torch::Tensor& x) {
   if (watched() || !dy.is_cuda() || !plain(dy, dy.device()) || !plain(x, dy.device()) ||
       dy.dim() != 2 || x.dim() != 2 || dy.size(0) != x.size(0) || !dy.is_contiguous() ||
@@ -184,10 +185,11 @@ c10::optional<torch::Tensor> wide_weight_grad(const torch::Tensor& dy, const tor
 // 16384 rows, 768 from 3072 86 and 68, 3072 from 768 85 and 68, 8192 rows, 4096 from 28672 1400
 // and 1302, 14336 from 4096 716 and 642; but 2000 rows, 4096 from 28672 (0.60) 394 and 472.
 //
-// Of Llama-3-8B's products, 4096 and more deep, a library splits the last round of tiles at 6002
-// to 7800 rows, not up to 5120 nor at full rounds (8000 to 8192 rows): there this one's bits are the
-// same.  Elsewhere it is left out: 10000 of 30 million values rounded otherwise are 0.9 % of the
-// first step's gradients, and 4 % of the next's.
+// Of Llama-3-8B's products, 4096 and more deep, that library was seen to split the last round of
+// its tiles, of 256 x 256 whatever this one's are, at 6002 to 7800 rows, not up to 5120 nor at full
+// rounds (8000 to 8192 rows): there this one's bits are the same.  Elsewhere it is left out: 10000
+// of 30 million values rounded otherwise are 0.9 % of the first step's gradients, and 4 % of the
+// next's.
 c10::optional<torch::Tensor> input_grad(const torch::Tensor& dy, const torch::Tensor& w) {
   if (watched() || !dy.is_cuda() || !plain(dy, dy.device()) || !plain(w, dy.device()) ||
       dy.dim() != 2 || w.dim() != 2 || dy.size(1) != w.size(0) || !dy.is_contiguous() ||

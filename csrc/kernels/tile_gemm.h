@@ -21,9 +21,10 @@ void tile_gemm(const TileArgs& a, TileAct act, hipStream_t st);
 bool big_takes(const TileArgs& a, TileAct act);
 void big_gemm(const TileArgs& a, TileAct act, hipStream_t st);
 
-// Forward products that a gradient goes through.  A library splits the depth of some deep ones
-// (1000 x 28672 x 4096, 3000 x 28672 x 4096), whose sums then round otherwise: through 4 layers
-// of Llama-3-8B's width that is 2 % of the first step's gradients and 7 to 13 % of the next's,
-// as much as bf16 lets either side be off, for 4 to 9 % of such a product.  GPT-2's, of 768 and
-// 3072, end 0.8 % apart after two steps.
+// Forward products that a gradient goes through.  The library (hipBLASLt of ROCm 7) was seen to
+// split the depth of some deep ones (1000 x 28672 x 4096, 3000 x 28672 x 4096), whose sums then round
+// otherwise, no nearer to 64 bits: through 4 layers of Llama-3-8B's width that is 2 % of the first
+// step's gradients and 7 to 13 % of the next's, as much as bf16 lets either side be off, for 4 to
+// 9 % of such a product.  GPT-2's, of 768 and 3072, end 0.8 % apart after two steps.  The bound
+// keeps a training run the one it was with that library; no other width or version was looked at.
 constexpr int BIG_DEPTH_OF_TRAINING = 3072;

@@ -609,9 +609,10 @@ def _residual_product(x: torch.Tensor, w: torch.Tensor,
 
 
 class _LinearLib(torch.autograd.Function):
-    """Forward by _product() with an explicit backward:
-    rocBLAS matmuls for dX/dW plus the hand colsum kernel for the bias
-    gradient (torch's generic reduce measured ~1 TB/s there).  What is frozen
+    """Forward by _product(), or with a residual, and an explicit backward: dX
+    and dW by _input_grad() and _weight_grad(), kernels of our own or a library's
+    products, and the hand colsum kernel for the bias gradient (torch's generic
+    reduce measured ~1 TB/s there).  What is frozen
     costs nothing: its gradient is not made, and what only that needs not kept."""
 
     @staticmethod

@@ -1,4 +1,5 @@
-"""Passes over more than the memory-side cache holds, whose results go past it."""
+"""Passes whose operands and results are together more than the memory-side cache
+holds, and go past it: batch norm of 64 MB, AdamW of 16 million elements."""
 
 import pytest
 import torch
