@@ -128,6 +128,21 @@ def test_products(M, N, K, act, bias):
     assert ((got.double() - want).abs() <= lim + 2.0 ** -8 * want.abs()).all()
 
 
+@pytest.mark.parametrize("M,N,K,act,own", [
+    (7000, 1792, 1024, 0, True), (7000, 1792, 1152, 0, False),      # 0.75 of one round
+    (2456, 15360, 2048, 2, True), (2456, 15360, 2176, 2, False),    # 0.75 of three
+    (2456, 15368, 2176, 2, True)])
+def test_whole_tiles_of_part_of_a_round(M, N, K, act, own):
+    """Where a library is as quick; both ways are one rounding of the same sums."""
+    torch.manual_seed(M)
+    x, w = _rows(M, K), (_rows(N, K, 0.5) / K ** 0.5).contiguous()
+    assert (ops.require_ext().tile_linear(x, w, None, act) is not None) == own
+    if act == 0:
+        assert ops.require_ext().tile_sizes(M, N, K) == own
+        with torch.no_grad():
+            _close(ops.linear(x, w), x, w.t())
+
+
 def test_rows_that_lie_far_apart():
     torch.manual_seed(5)
     both = _rows(8000, 1024)
