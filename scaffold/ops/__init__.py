@@ -717,6 +717,9 @@ def _own(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor) -> bool:
     if not (w.dim() == 2 and type(x) in _PLAIN and type(w) in _PLAIN
             and type(res) in _PLAIN) or torch.jit.is_tracing():
         return False
+    if (torch.is_autocast_enabled("cuda")
+            and torch.get_autocast_dtype("cuda") != torch.bfloat16):
+        return False                           # the product is of that type
     n, k = w.shape
     rows = x.numel() // max(1, k)
     return rows > 0 and n > 0 and (
