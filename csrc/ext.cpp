@@ -183,8 +183,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("swiglu_bwd", &swiglu_bwd, "fused SwiGLU backward (dg, du)");
   m.def("save_shard_pinned", &save_shard_pinned,
         "stream tensors to a safetensors shard via pinned D2H (C6)");
-  m.def("weight_grad", &weight_grad, "dY^T X of few tiles, split over rows",
-        py::arg("dy"), py::arg("x"));
+  m.def("weight_grad",
+        [](py::object dy, py::object x) {
+          // modes that count or replace products see torch's
+          return exact([](const torch::Tensor& dy, const torch::Tensor& x) {
+            return c10::impl::dispatch_mode_enabled() ? c10::nullopt
+                                                      : c10::make_optional(weight_grad(dy, x));
+          }, dy, x);
+        },
+        "dY^T X of few tiles, split over rows, or None", py::arg("dy"), py::arg("x"));
   m.def("wide_weight_grad", [](py::object dy, py::object x) { return exact(wide_weight_grad, dy, x); },
         "weight_grad where that is faster than a library, or None", py::arg("dy"),
         py::arg("x"));

@@ -465,9 +465,10 @@ def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
                 and x.shape[0] >= 8192 and n % 8 == 0 and k % 8 == 0
                 and 0 < -(-n // 256) * -(-k // 256) <= 64
                 and dy.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0):
-            return require_ext().weight_grad(dy, x)
-        dw = require_ext().wide_weight_grad(dy, x) if many else None
-        if dw is not None:
+            dw = require_ext().weight_grad(dy, x)
+        else:
+            dw = require_ext().wide_weight_grad(dy, x) if many else None
+        if dw is not None:                     # None: torch has to see the product
             return dw
     return dy.t() @ x
 
