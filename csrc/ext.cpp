@@ -110,7 +110,7 @@ torch::Tensor skinny_linear_parts(torch::Tensor x, torch::Tensor w,
 c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Tensor& w,
                                          const c10::optional<torch::Tensor>& bias, long act,
                                          bool grad);
-bool tile_sizes(long M, long N, long K);
+bool residual_takes(const torch::Tensor& x, const torch::Tensor& w, const torch::Tensor& res);
 torch::Tensor skinny_linear(torch::Tensor x, torch::Tensor w,
                             c10::optional<torch::Tensor> bias,
                             c10::optional<torch::Tensor> res, long act,
@@ -246,8 +246,17 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "act(x w^T + b) of some hundred rows, or None; act: 0 none, 1 tanh-GELU, 2 erf-GELU",
         py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("act") = 0,
         py::arg("grad") = false);
-  m.def("tile_sizes", &tile_sizes,
-        "whether tile_linear takes M rows of K to N that a gradient goes through");
+  m.def("residual_takes",
+        [](py::object x, py::object w, py::object res) {
+          // classes and modes that override functions see torch's product
+          for (const auto* t : {&x, &w, &res})
+            if (!THPVariable_CheckExact(t->ptr())) return false;
+          return !at::impl::torch_function_mode_enabled() &&
+                 residual_takes(x.cast<torch::Tensor>(), w.cast<torch::Tensor>(),
+                                res.cast<torch::Tensor>());
+        },
+        "whether x w^T + res or a gradient of it may be a kernel's of ours", py::arg("x"),
+        py::arg("w"), py::arg("res"));
   m.def("skinny_linear", &skinny_linear,
         "product of up to 64 rows with bias, residual, GELU or SwiGLU",
         py::arg("x"), py::arg("w"), py::arg("bias") = py::none(),

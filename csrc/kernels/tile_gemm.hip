@@ -266,13 +266,26 @@ void tile_gemm(const TileArgs& a, TileAct act, hipStream_t st) {
   else pick<TILE_NONE>(a, tile, st);
 }
 
-// Whether tile_linear() takes a product of that many rows that a gradient goes through
-bool tile_sizes(long M, long N, long K) {
-  if (M < 1 || M >= 1 << 30 || N < 1 || N >= 1 << 30 || K < 1 || K > 1 << 22) return false;
+// Whether a kernel of ours may make x w^T + res, through which gradients go, or one of its
+// gradients: that is what an autograd function in torch's place is worth, with which the host
+// takes 13 us of 138 more both ways.
+bool residual_takes(const torch::Tensor& x, const torch::Tensor& w, const torch::Tensor& res) {
+  if (watched() || !x.is_cuda() || !memory(x, x.device()) || !memory(w, x.device()) ||
+      !memory(res, x.device()) || x.dim() < 1 || w.dim() != 2 || res.dim() != x.dim())
+    return false;
+  const long N = w.size(0), K = w.size(1);
+  if (N < 1 || N >= 1 << 30 || K < 1 || K > 1 << 22 || x.size(-1) != K || res.size(-1) != N)
+    return false;
+  const long M = x.numel() / K;
   TileArgs a = {};
   a.M = (int)M; a.N = (int)N; a.K = (int)K;
   a.ldx = K; a.ldy = N;
-  return (K <= BIG_DEPTH_OF_TRAINING && big_takes(a, TILE_NONE)) || tile_takes(a, TILE_NONE);
+  // results and input gradients of big_gemm.hip, and weight gradients, are no smaller
+  return M > 0 && M < 1 << 30 &&
+         res.sizes().slice(0, res.dim() - 1) == x.sizes().slice(0, x.dim() - 1) &&
+         (M * N >= 8200000 || M * K >= 9900000 || M >= 8192 ||
+          (M >= 256 && N * K >= 11000000) ||
+          (K <= BIG_DEPTH_OF_TRAINING && big_takes(a, TILE_NONE)) || tile_takes(a, TILE_NONE));
 }
 
 // act(x w^T + b) of rows (..., K), act as TileAct, by these or by large tiles; None: not

@@ -13,13 +13,18 @@ inline bool watched() {
           at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16);
 }
 
-// Nothing but memory on the device, of bf16, that no gradient is asked of: no wrapper, no
-// batch, no tensor of zeros without any.
-inline bool plain(const torch::Tensor& t, const torch::Device& device) {
+// Nothing but memory on the device, of bf16: no wrapper, no batch, no tensor of zeros without
+// any.
+inline bool memory(const torch::Tensor& t, const torch::Device& device) {
   const auto keys = t.key_set() - c10::autograd_dispatch_keyset -
                     c10::autocast_dispatch_keyset -
                     c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView);
   return keys == c10::DispatchKeySet(c10::DispatchKey::CUDA) &&
          t.scalar_type() == torch::kBFloat16 && t.device() == device &&
-         !t._fw_grad(0).defined() && !(at::GradMode::is_enabled() && t.requires_grad());
+         !t._fw_grad(0).defined();
+}
+
+// and no gradient asked of it
+inline bool plain(const torch::Tensor& t, const torch::Device& device) {
+  return memory(t, device) && !(at::GradMode::is_enabled() && t.requires_grad());
 }

@@ -708,27 +708,6 @@ def linear_gelu(x: torch.Tensor, w: torch.Tensor,
     return F.gelu(F.linear(x, w, b), approximate="tanh")
 
 
-_PLAIN = (torch.Tensor, torch.nn.Parameter)
-
-
-def _own(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor) -> bool:
-    """Whether a kernel of our own may make x w^T or a gradient of it, which is what
-    an autograd function in torch's place is worth: otherwise it takes the host
-    4 us of 29 more forward, 13 of 138 both ways."""
-    if not (w.dim() == 2 and type(x) in _PLAIN and type(w) in _PLAIN
-            and type(res) in _PLAIN) or torch.jit.is_tracing():
-        return False
-    if (torch.is_autocast_enabled("cuda")
-            and torch.get_autocast_dtype("cuda") != torch.bfloat16):
-        return False                           # the product is of that type
-    n, k = w.shape
-    rows = x.numel() // max(1, k)
-    return rows > 0 and n > 0 and (
-        rows * n >= 8_200_000 or rows * k >= 9_900_000 or rows >= 8192
-        or (rows >= 256 and n * k >= 11_000_000)
-        or require_ext().tile_sizes(rows, n, k))
-
-
 def linear_residual(x: torch.Tensor, w: torch.Tensor,
                     b: Optional[torch.Tensor], res: torch.Tensor) -> torch.Tensor:
     # measured >= hipBLASLt only for small N AND K (the square attn
@@ -736,18 +715,21 @@ def linear_residual(x: torch.Tensor, w: torch.Tensor,
     if x.is_cuda and _tile_ok(x, w) and (
             _HAND_GEMM_ALL or (w.shape[0] <= 1024 and w.shape[1] <= 1024)):
         return _LinearResidualFn.apply(x, w, b, res)
+    if b is None:
+        if (x.is_cuda and torch.is_grad_enabled()
+                and not torch.compiler.is_compiling()
+                and require_ext().residual_takes(x, w, res)
+                and not _transformed()):
+            return _LinearLib.apply(x, w, b, res)
     # one type throughout: autocast's float32 weights need torch's own backward
-    if (x.is_cuda and x.dtype == w.dtype == torch.bfloat16
-            and (b is None or b.dtype == torch.bfloat16)
+    elif (x.is_cuda and x.dtype == w.dtype == b.dtype == torch.bfloat16
             and torch.is_grad_enabled() and not _transformed()):
         # gradients by own kernels
-        if (res.is_cuda and res.dtype == x.dtype
+        if (_many(res) and res.is_cuda and res.dtype == x.dtype
                 and res.shape == x.shape[:-1] + w.shape[:1]
-                and not torch.compiler.is_compiling()
-                and (b is not None or _own(x, w, res))):
+                and not torch.compiler.is_compiling()):
             return _LinearLib.apply(x, w, b, res)
-        if b is not None:
-            return _LinearLib.apply(x, w, b) + res
+        return _LinearLib.apply(x, w, b) + res
     return F.linear(x, w, b) + res
 
 

@@ -138,7 +138,6 @@ def test_whole_tiles_of_part_of_a_round(M, N, K, act, own):
     x, w = _rows(M, K), (_rows(N, K, 0.5) / K ** 0.5).contiguous()
     assert (ops.require_ext().tile_linear(x, w, None, act) is not None) == own
     if act == 0:
-        assert ops.require_ext().tile_sizes(M, N, K) == own
         with torch.no_grad():
             _close(ops.linear(x, w), x, w.t())
 
