@@ -824,8 +824,9 @@ def lm_head_ce(x: torch.Tensor, w: torch.Tensor, targets: torch.Tensor
     t = targets.contiguous().view(-1)
     if x.is_cuda and _FUSED_CE:
         return _LmHeadCE.apply(x, w, t)
-    if (x.is_cuda and w.shape[0] % 8 and not _transformed()
-            and not torch.compiler.is_compiling()):
+    if (x.is_cuda and w.shape[0] % 8
+            and t.numel() * w.shape[0] >= 7_800_000   # big_gemm.hip's are no fewer
+            and not _transformed() and not torch.compiler.is_compiling()):
         h = x.contiguous()
         logits = require_ext().head_logits(h.detach().view(-1, h.shape[-1]),
                                            w.detach())
