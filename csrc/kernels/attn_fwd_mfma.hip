@@ -57,7 +57,8 @@ DEVINL float other_half(float x) {
 // hi + lo, 16 of float32's 24 significand bits (serving).  Against 64 bits the
 // result is as near as with a float32 product, to five digits of its error
 // (heads of 64 and 128, 2 to 4096 rows, up to 4096 keys): its own rounding to
-// 8 bits is what there is.  An infinite value is NaN in what sees it.
+// 8 bits is what there is.  An infinite value is infinite, or NaN where the weight's second
+// part is none or of the other sign, in what sees it.
 //
 // KS = 2: the tiles of 64 keys go by turns to two groups of W waves, each with images of its
 // own, and the first puts both results together at the end.
