@@ -153,24 +153,29 @@ c10::optional<torch::Tensor> residual_linear(const torch::Tensor& x, const torch
 // of 982, but 5000 of its 59 million gradients are rounded otherwise, no nearer to 64 bits or
 // farther, after which a step of AdamW leaves the next gradients 2 % apart, the most that bf16
 // lets them.  (128256 x 4096, the head, of 31 rounds, 7361 and 5691: 5000 of 525 million, and 0.7 %.)
+bool weight_grad_takes(long T, long N, long K) {
+  if (T < 256 || T >= 1l << 30 || N < 256 || K < 256 || N % 8 || K % 8 || N > 1l << 22 ||
+      K > 1l << 22)
+    return false;
+  BigArgs a = {};
+  a.M = (int)N; a.N = (int)K;
+  const long tiles = up(N, 256) * up(K, 256), last = tiles % UNITS;
+  return at_work(a, rounds(a, 8)) >= 0.66 &&
+         !(T > 4096 && tiles < 4 * UNITS && last > 0 && last <= UNITS / 2);
+}
+
 c10::optional<torch::Tensor> wide_weight_grad(const torch::Tensor& dy, const torch::Tensor& x) {
   if (watched() || !dy.is_cuda() || !plain(dy, dy.device()) || !plain(x, dy.device()) ||
       dy.dim() != 2 || x.dim() != 2 || dy.size(0) != x.size(0) || !dy.is_contiguous() ||
       !x.is_contiguous() || ((size_t)dy.data_ptr() | (size_t)x.data_ptr()) % 16)
     return c10::nullopt;
   const long T = x.size(0), N = dy.size(1), K = x.size(1);
-  if (T < 256 || T >= 1l << 30 || N < 256 || K < 256 || N % 8 || K % 8 || N > 1l << 22 ||
-      K > 1l << 22)
-    return c10::nullopt;
+  if (!weight_grad_takes(T, N, K)) return c10::nullopt;
   BigArgs a = {};
   a.a = (const short*)dy.data_ptr();
   a.b = (const short*)x.data_ptr();
   a.M = (int)N; a.N = (int)K; a.K = (int)T;
   a.lda = N; a.ldb = a.ldy = K;
-  const long tiles = up(N, 256) * up(K, 256), last = tiles % UNITS;
-  if (at_work(a, rounds(a, 8)) < 0.66 ||
-      (T > 4096 && tiles < 4 * UNITS && last > 0 && last <= UNITS / 2))
-    return c10::nullopt;
   // the operands' device, whichever is current: torch's product goes by it too
   const c10::DeviceGuard guard(dy.device());
   auto dw = torch::empty({N, K}, x.options());
@@ -190,28 +195,32 @@ c10::optional<torch::Tensor> wide_weight_grad(const torch::Tensor& dy, const tor
 // rounds (8000 to 8192 rows): there this one's bits are the same.  Elsewhere it is left out: 10000
 // of 30 million values rounded otherwise are 0.9 % of the first step's gradients, and 4 % of the
 // next's.
+bool input_grad_takes(long M, long N, long K) {
+  if (M < 256 || M >= 1l << 30 || N < 128 || N % 128 || N > 1l << 22 || K < 256 || K % 8 ||
+      K > 1l << 22)
+    return false;
+  BigArgs a = {};
+  a.M = (int)M; a.N = (int)K;
+  return at_work(a, rounds(a, columns(a))) >= 0.72 &&
+         !(N > BIG_DEPTH_OF_TRAINING && M > 5120 && up(M, 256) * up(K, 256) % UNITS != 0);
+}
+
 c10::optional<torch::Tensor> input_grad(const torch::Tensor& dy, const torch::Tensor& w) {
   if (watched() || !dy.is_cuda() || !plain(dy, dy.device()) || !plain(w, dy.device()) ||
       dy.dim() != 2 || w.dim() != 2 || dy.size(1) != w.size(0) || !dy.is_contiguous() ||
       !w.is_contiguous() || ((size_t)dy.data_ptr() | (size_t)w.data_ptr()) % 16)
     return c10::nullopt;
   const long M = dy.size(0), N = w.size(0), K = w.size(1);
-  if (M < 256 || M >= 1l << 30 || N < 128 || N % 128 || N > 1l << 22 || K < 256 || K % 8 ||
-      K > 1l << 22)
-    return c10::nullopt;
+  if (!input_grad_takes(M, N, K)) return c10::nullopt;
   BigArgs a = {};
   a.a = (const short*)dy.data_ptr();
   a.b = (const short*)w.data_ptr();
   a.M = (int)M; a.N = (int)K; a.K = (int)N;
   a.lda = N; a.ldb = a.ldy = K;
-  const int nt = columns(a);
-  if (at_work(a, rounds(a, nt)) < 0.72 ||
-      (N > BIG_DEPTH_OF_TRAINING && M > 5120 && up(M, 256) * up(K, 256) % UNITS != 0))
-    return c10::nullopt;
   const c10::DeviceGuard guard(dy.device());
   auto dx = torch::empty({M, K}, dy.options());
   a.y = (short*)dx.data_ptr();
-  if (nt == 6) launch<false, true, 6, BIG_NONE>(a, scaffold_stream());
+  if (columns(a) == 6) launch<false, true, 6, BIG_NONE>(a, scaffold_stream());
   else launch<false, true, 8, BIG_NONE>(a, scaffold_stream());
   HIP_CHECK(hipGetLastError());
   return dx;

@@ -20,6 +20,9 @@ void tile_gemm(const TileArgs& a, TileAct act, hipStream_t st);
 // The same for many tiles, no or the erf GELU: see big_gemm.hip
 bool big_takes(const TileArgs& a, TileAct act);
 void big_gemm(const TileArgs& a, TileAct act, hipStream_t st);
+// and whether dY (M, N) W (N, K) and dY^T X, X (M, K), are that kernel's
+bool input_grad_takes(long M, long N, long K);
+bool weight_grad_takes(long M, long N, long K);
 
 // Forward products that a gradient goes through.  The library (hipBLASLt of ROCm 7) was seen to
 // split the depth of some deep ones (1000 x 28672 x 4096, 3000 x 28672 x 4096), whose sums then round

@@ -266,9 +266,17 @@ void tile_gemm(const TileArgs& a, TileAct act, hipStream_t st) {
   else pick<TILE_NONE>(a, tile, st);
 }
 
-// Whether a kernel of ours may make x w^T + res, through which gradients go, or one of its
-// gradients: that is what an autograd function in torch's place is worth, with which the host
-// takes 13 us of 138 more both ways.
+// Whether an autograd function in torch's place is worth it for x w^T + res, through which
+// gradients go.  Where the product is a kernel's of ours the host takes no longer: both ways,
+// eager, 134 us of torch's and 126 at 666 x 3072 x 768, 123 at 3125.  Where only a gradient is, it
+// takes 13 to 30 us more, which the GPU has to have saved.  The large products' kernel: of 24
+// sizes of more than 20 G products every one is faster (885 x 4096 x 8192 194 and 172 us); of 22 of
+// 10 to 20 the mean is 0.93 and eight are 2 to 11 % slower (777 x 4096 x 4096 110 and 102, 890 x 2048
+// x 8192 130 and 143, whose GPU time is 118 and 107); of less they are 6 to 11 % slower (408 x 2048
+// x 5632 128 and 142, of the GPU 84 and 68).  Weight gradients of few tiles, for which a library's
+// time grows with the rows: 43764 x 344 x 712 347 and 202, 22184 x 456 x 480 202 and 159, 51357 x 64
+// x 96 180 and 162, of 29 sizes 0.71; of 43 below the line 1.03 (10381 x 488 x 432 147 and 164,
+// 25997 x 576 x 80 154 and 164).
 bool residual_takes(const torch::Tensor& x, const torch::Tensor& w, const torch::Tensor& res) {
   if (watched() || !x.is_cuda() || !memory(x, x.device()) || !memory(w, x.device()) ||
       !memory(res, x.device()) || x.dim() < 1 || w.dim() != 2 || res.dim() != x.dim())
@@ -277,15 +285,23 @@ bool residual_takes(const torch::Tensor& x, const torch::Tensor& w, const torch:
   if (N < 1 || N >= 1 << 30 || K < 1 || K > 1 << 22 || x.size(-1) != K || res.size(-1) != N)
     return false;
   const long M = x.numel() / K;
+  if (M < 1 || M >= 1 << 30 ||
+      res.sizes().slice(0, res.dim() - 1) != x.sizes().slice(0, x.dim() - 1))
+    return false;
   TileArgs a = {};
   a.M = (int)M; a.N = (int)N; a.K = (int)K;
   a.ldx = K; a.ldy = N;
-  // results and input gradients of big_gemm.hip, and weight gradients, are no smaller
-  return M > 0 && M < 1 << 30 &&
-         res.sizes().slice(0, res.dim() - 1) == x.sizes().slice(0, x.dim() - 1) &&
-         (M * N >= 8200000 || M * K >= 9900000 || M >= 8192 ||
-          (M >= 256 && N * K >= 11000000) ||
-          (K <= BIG_DEPTH_OF_TRAINING && big_takes(a, TILE_NONE)) || tile_takes(a, TILE_NONE));
+  if ((K <= BIG_DEPTH_OF_TRAINING && big_takes(a, TILE_NONE)) || tile_takes(a, TILE_NONE))
+    return true;
+  const bool dx = x.requires_grad(), dw = w.requires_grad();
+  if ((double)M * (double)N * (double)K >= 10e9 &&
+      ((dx && input_grad_takes(M, N, K)) || (dw && weight_grad_takes(M, N, K))))
+    return true;
+  // weight_grad.hip's
+  const long small = std::min(N, K), large = std::max(N, K);
+  return dw && (M >= 32768 || (M >= 8192 && M * (N + K) >= 20000000)) && N % 8 == 0 &&
+         K % 8 == 0 && small >= 64 && (small >= 256 || large <= 8192) &&
+         ((N + 255) / 256) * ((K + 255) / 256) <= 64;
 }
 
 // act(x w^T + b) of rows (..., K), act as TileAct, by these or by large tiles; None: not

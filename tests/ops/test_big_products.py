@@ -211,9 +211,17 @@ def test_residual_layers_take_it(n, monkeypatch):
 
 
 @pytest.mark.parametrize("M,N,K,own", [
-    (100, 1024, 2816, False), (256, 1792, 4096, False), (3200, 1408, 1664, False),
-    (255, 4096, 14336, False), (256, 4096, 14336, True), (500, 2048, 2048, True),
-    (8192, 256, 1032, True), (4096, 2056, 128, True), (4096, 64, 2560, True)])
+    # nothing, also where one is large enough to be asked about
+    (100, 1024, 2816, False), (3200, 1408, 1664, False), (4682, 2048, 1024, False),
+    (721, 3072, 5632, False), (255, 4096, 14336, False), (4096, 2056, 128, False),
+    # the product, by tiles
+    (500, 2048, 2048, True),
+    # a gradient alone, of less and of more than 10 G products
+    (408, 2048, 5632, False), (1800, 2048, 5632, True), (7015, 768, 1536, False),
+    (6628, 512, 3536, True),
+    # a weight gradient of few tiles, out of few and many rows
+    (8192, 256, 1032, False), (22184, 456, 480, True), (32767, 72, 104, False),
+    (32768, 72, 104, True), (40000, 56, 104, False)])
 def test_residuals_without_a_bias_are_torch_s_where_nothing_is_ours(M, N, K, own):
     x = torch.randn(M, K, device="cuda").bfloat16().requires_grad_()
     w = (torch.randn(N, K, device="cuda") / K ** 0.5).bfloat16().requires_grad_()
@@ -231,16 +239,17 @@ class Marked(torch.Tensor):
 @pytest.mark.filterwarnings("ignore:.*torch.jit.trace:DeprecationWarning",
                             "ignore::torch.jit.TracerWarning")
 def test_residuals_without_a_bias_that_torch_has_to_see():
-    x = torch.randn(4096, 2048, device="cuda").bfloat16().requires_grad_()
-    w = (torch.randn(2048, 2048, device="cuda") / 45).bfloat16().requires_grad_()
-    res = torch.randn(4096, 2048, device="cuda").bfloat16()
+    x = torch.randn(4096, 768, device="cuda").bfloat16().requires_grad_()
+    w = (torch.randn(3072, 768, device="cuda") / 28).bfloat16().requires_grad_()
+    res = torch.randn(4096, 3072, device="cuda").bfloat16()
     f = ops.linear_residual
     assert type(f(x, w, None, res).grad_fn).__name__ == "_LinearLibBackward"
     assert type(f(x, w, None, res.as_subclass(Marked)).grad_fn).__name__ != "_LinearLibBackward"
     traced = torch.jit.trace(lambda x, w, r: f(x, w, None, r), (x, w, res), check_trace=False)
     assert "PythonOp" not in str(traced.graph) and "_LinearLib" not in str(traced.graph)
     # a weight of one row without its dimension
-    v = w.detach()[0].clone().requires_grad_()
+    x = torch.randn(4096, 2048, device="cuda").bfloat16()
+    v = torch.randn(2048, device="cuda").bfloat16().requires_grad_()
     (got,) = torch.autograd.grad(f(x, v, None, res[:, 0]).sum(), v)
     assert got.shape == v.shape
 
