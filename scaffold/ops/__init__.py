@@ -456,28 +456,28 @@ def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     8192 rows take 120 and 116.  Tiles that are mostly empty are not worth it:
     8192 rows, 32 x 256 19 and 30, 64 x 64 45 and 30, 64 x 16384 63 and 75, 256 x
     16384 108 and 86.  Where tiles fill the chip, another: csrc/kernels/big_gemm.hip."""
-    n, k = dy.shape[1], x.shape[1]
-    many = n * k >= 11_000_000                 # tiles for two thirds of the chip
-    if x.is_cuda and (many or x.shape[0] >= 8192) and _unseen():
+    rows, n, k = x.shape[0], dy.shape[1], x.shape[1]
+    dw = None                                  # torch has to see the product
+    if x.is_cuda and n % 8 == 0 and k % 8 == 0:
         small, large = min(n, k), max(n, k)
-        if (small >= 64 and (small >= 256 or large <= 8192)
+        if (rows >= 8192 and small >= 64 and (small >= 256 or large <= 8192)
                 and dy.dtype == x.dtype == torch.bfloat16
-                and x.shape[0] >= 8192 and n % 8 == 0 and k % 8 == 0
-                and 0 < -(-n // 256) * -(-k // 256) <= 64
+                and -(-n // 256) * -(-k // 256) <= 64 and _unseen()
                 and dy.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0):
             dw = require_ext().weight_grad(dy, x)
-        else:
-            dw = require_ext().wide_weight_grad(dy, x) if many else None
-        if dw is not None:                     # None: torch has to see the product
-            return dw
-    return dy.t() @ x
+        elif (rows >= 256 and n * k >= 11_000_000   # tiles for two thirds of the chip
+              and _unseen()):
+            dw = require_ext().wide_weight_grad(dy, x)
+    return dy.t() @ x if dw is None else dw
 
 
 def _input_grad(dy: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """dy w of contiguous rows, by a kernel of our own where that is faster
-    than the library's (both sides' times: csrc/kernels/big_gemm.hip)."""
-    if (dy.shape[0] * w.shape[1] >= 9_900_000  # tiles for most of the chip
-            and dy.is_cuda and _unseen()):
+    than the library's (both sides' times: csrc/kernels/big_gemm.hip).  Sizes are
+    looked at first: in a backward's thread the rest takes 3 to 5 us."""
+    rows, n, k = dy.shape[0], w.shape[0], w.shape[1]
+    if (rows * k >= 9_900_000 and rows >= 256  # tiles for most of the chip
+            and n % 128 == 0 and dy.is_cuda and _unseen()):
         dx = require_ext().input_grad(dy, w)
         if dx is not None:
             return dx

@@ -106,6 +106,20 @@ def test_layers_take_it(act, monkeypatch):
     assert len(calls) == 1
 
 
+@pytest.mark.parametrize("M,N,K", [(300, 15001, 768), (255, 4096, 4096), (20000, 1000, 12),
+                                   (64, 264, 160000), (13000, 264, 768)])
+def test_sizes_that_are_no_kernel_s_are_not_asked_about(M, N, K, monkeypatch):
+    ext, calls = ops.require_ext(), []
+    for name in ("input_grad", "wide_weight_grad"):
+        monkeypatch.setattr(ext, name, lambda *a: calls.append(1))
+    x, w = _rows(M, K).requires_grad_(), (_rows(N, K) / K ** 0.5).requires_grad_()
+    y = ops.linear(x, w)
+    dy = torch.randn_like(y)
+    dx, dw = torch.autograd.grad(y, (x, w), dy)
+    assert not calls
+    assert dx.shape == x.shape and dw.shape == w.shape
+
+
 @pytest.mark.parametrize("M,N,K,act,bias", [
     (16129, 2056, 256, 0, True),      # tiles of 256 columns, several a block
     (16001, 768, 768, 0, True),       # of 192, the last of one row
