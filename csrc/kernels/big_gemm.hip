@@ -55,7 +55,8 @@ int width(const BigArgs& a) { return a.N % 24 ? 8 : columns(a); }
 
 // Where it is faster than a library on the whole: of 250 random sizes of 300 to 33000 rows the mean
 // is 0.79 of the library's time, with the erf GELU, of 150, 0.83; one in twelve is slower, by 2 to
-// 18 %, all of them with whole tiles of 128 columns, which a library is quick at.  In us,
+// 18 %, all of them with whole tiles of 128 columns, which a library is quick at (big_alone() leaves
+// it half of those; of 300 deeper than 512 then 15 are slower, by 2 to 14 %, all whole across).  In us,
 // library and this.  Shallow products, whose stores a library waits for: 16384 rows, 768 to
 // 2304 69 and 53, to 3072 78 and 67; 9208 x 1656 x 512 35 and 20; 1152 x 28168 x 896 (0.64) 79
 // and 74; but 8360 x 14088 x 128 83 and 92.  Deeper ones with tiles left over, for which 192
@@ -82,6 +83,18 @@ bool big_takes(const TileArgs& t, TileAct act) {
   }
   if (t.K <= 1280) return t.K >= 256 && busy >= (whole && t.K > 1024 ? 0.78 : 0.6);
   return t.K <= 4096 && busy >= 0.72 && busy <= 0.97;
+}
+
+// Alone, without a GELU or a residual, tiles that are whole across, as the library's are, gain
+// nothing in one round, nor, 1280 to 2048 deep, in two.  More than 512 deep, its time 1: of 39 sizes
+// in one round 1.03 (in us, 15215 x 1024 x 1152 31 and 33, 6038 x 2304 x 2560 54 and 57), of 16 in two
+// 1.00 (6383 x 4096 x 1664 71 and 79); but of 22 in two of other depths 0.94, of 107 in more 0.89, of
+// 156 with columns left over 0.82, none slower, and of 60 with tiles of 192 columns 0.85, none slower.
+bool big_alone(const TileArgs& t) {
+  const BigArgs a = of(t);
+  if (t.N % 256 || t.K <= 512 || width(a) == 6) return true;
+  const double r = rounds(a, 8);
+  return r > 2 || (r == 2 && (t.K <= 1280 || t.K > 2048));
 }
 
 void big_gemm(const TileArgs& t, TileAct act, hipStream_t st) {

@@ -19,6 +19,7 @@ void tile_gemm(const TileArgs& a, TileAct act, hipStream_t st);
 
 // The same for many tiles, no or the erf GELU: see big_gemm.hip
 bool big_takes(const TileArgs& a, TileAct act);
+bool big_alone(const TileArgs& a);        // and whether that pays for a product alone
 void big_gemm(const TileArgs& a, TileAct act, hipStream_t st);
 // and whether dY (M, N) W (N, K) and dY^T X, X (M, K), are that kernel's
 bool input_grad_takes(long M, long N, long K);

@@ -328,7 +328,8 @@ c10::optional<torch::Tensor> tile_linear(const torch::Tensor& x, const torch::Te
   a.bias = bias.has_value() ? (const short*)bias->data_ptr() : nullptr;
   a.ldx = x.dim() == 2 ? x.stride(0) : a.K;
   a.ldy = a.N;
-  const bool big = (!grad || a.K <= BIG_DEPTH_OF_TRAINING) && big_takes(a, (TileAct)act);
+  const bool big = (!grad || a.K <= BIG_DEPTH_OF_TRAINING) && big_takes(a, (TileAct)act) &&
+                   (act != TILE_NONE || big_alone(a));
   if (!big && !tile_takes(a, (TileAct)act)) return c10::nullopt;
   // the operands' device, whichever is current: torch's product goes by it too
   const c10::DeviceGuard guard(x.device());

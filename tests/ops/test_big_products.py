@@ -143,7 +143,11 @@ def test_products(M, N, K, act, bias):
 
 
 @pytest.mark.parametrize("M,N,K,act,own", [
-    (7000, 1792, 1024, 0, True), (7000, 1792, 1152, 0, False),      # 0.75 of one round
+    (10000, 2176, 1024, 0, True), (10000, 2176, 1152, 0, False),    # 0.65 of two rounds
+    (7000, 1792, 512, 0, True), (7000, 1792, 640, 0, False),        # whole across, one
+    (7000, 1920, 640, 0, True),
+    (6500, 4096, 1280, 0, True), (6500, 4096, 1408, 0, False),      # whole across, two
+    (6500, 4096, 2048, 0, False), (6500, 4096, 2176, 0, True),
     (2456, 15360, 2048, 2, True), (2456, 15360, 2176, 2, False),    # 0.75 of three
     (2456, 15368, 2176, 2, True)])
 def test_whole_tiles_of_part_of_a_round(M, N, K, act, own):
