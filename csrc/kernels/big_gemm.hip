@@ -56,7 +56,8 @@ int width(const BigArgs& a) { return a.N % 24 ? 8 : columns(a); }
 // Where it is faster than a library on the whole: of 250 random sizes of 300 to 33000 rows the mean
 // is 0.79 of the library's time, with the erf GELU, of 150, 0.83; one in twelve is slower, by 2 to
 // 18 %, all of them with whole tiles of 128 columns, which a library is quick at (big_alone() leaves
-// it half of those; of 300 deeper than 512 then 15 are slower, by 2 to 14 %, all whole across).  In us,
+// it most of those: deeper than 512, 56 of 400 were more than 2 % slower, and 15 of 300 still are, by
+// up to 14 %, all whole across).  In us,
 // library and this.  Shallow products, whose stores a library waits for: 16384 rows, 768 to
 // 2304 69 and 53, to 3072 78 and 67; 9208 x 1656 x 512 35 and 20; 1152 x 28168 x 896 (0.64) 79
 // and 74; but 8360 x 14088 x 128 83 and 92.  Deeper ones with tiles left over, for which 192
